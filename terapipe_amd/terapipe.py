@@ -90,6 +90,12 @@ class _StackBuffers:
         # the one-pass dK/dV kernel is 16-bit and has head dimensions 64 and 128; other runs keep gradient caches
         self.position_indexed = runner.suffix_dkdv and dtype != torch.float32 and Dh in (64, 128)
         self.fused_attn_bwd = runner.fused_attn_bwd
+        self.merge_slices = runner.merge_slices
+        # the pieces a step runs in
+        self.pieces = runner.seq_slices
+        if runner.merge_slices:
+            self.pieces = merged_slices(runner.seq_slices, max(runner.batch_slices), E,
+                                        runner.slice_streams if self.position_indexed else 1)
         gdt = torch.float32 if runner.fp32_grad_cache else dtype
         kw = dict(dtype=dtype, device=device)
         f32 = dict(dtype=torch.float32, device=device)
@@ -115,8 +121,9 @@ class _StackBuffers:
             else:
                 b["q"] = [torch.empty(R, E, **kw) for _ in range(nl)]
                 b["lse"] = [torch.empty(R * H, **f32) for _ in range(nl)]
-                b["d_o"] = torch.empty(max(runner.seq_slices) * Bs, E, **kw)
-                b["delta"] = torch.empty(max(runner.seq_slices) * Bs * H, **f32)
+                longest = max(runner.seq_slices + self.pieces)
+                b["d_o"] = torch.empty(longest * Bs, E, **kw)
+                b["delta"] = torch.empty(longest * Bs * H, **f32)
             # zero-filled once: rows beyond the current slice are read only under the causal mask, but
             # they must hold finite values (reference create_attn_cache zero-fills, transformer_models.py:257-261)
             b["cache"] = [torch.zeros(Bs * H, L, Dh, **kw) for _ in range(2 * nl)]
@@ -193,6 +200,37 @@ def _flat_views(flat, layout):
     return [{n: flat[o:o + int(np.prod(s))].view(s) for n, (o, s) in d.items()} for d in layout]
 
 
+# Rows (tokens x batch) from which a merged sequence is cut into two pieces on two streams, and the slices that stay as
+# they are (rows on average, hidden size): see merged_slices.
+MERGE_TWO_ROWS = 2048
+MERGE_KEEP_ROWS, MERGE_KEEP_HIDDEN = 256, 2048
+
+
+def merged_slices(seq_slices, batch, hidden, n_lanes):
+    """The pieces a single-stage step runs the sequence in: the whole sequence, or two halves on two streams.
+
+    Slices are the unit in which pipeline STAGES hand work to each other.  One runner holds every slice of its stage
+    from the start, and what its step computes does not depend on where the sequence is cut: every operation of a layer
+    but attention works row by row, and attention over the prefix and the slice is attention over the positions up to
+    the query's own.  A slice costs a pass over the stack's weights and a chain of launches, so the fewer the better: a
+    product of 64 rows is bound by reading its weight, one of 2048 by the matrix pipe.  Measured (16 bit, 2048 tokens):
+    64 slices of 32 x 2 rows of hidden 6144: 104.8 ms -> 46.1 as one piece, 44.8 as two; seven slices of 160-512 rows
+    of hidden 5120: 25.6 -> 23.0 / 22.2.  Four pieces are slower than two (48.5 / 23.0).  Two pieces of 1024 rows and
+    more fill each other's last waves of tiles and the attention launches' tails; below that one piece wins.  The cut
+    is at a whole 64-query block.
+
+    Slices of MERGE_KEEP_ROWS rows and more on a hidden size up to MERGE_KEEP_HIDDEN stay as they are: there the lanes'
+    products share the weights through the memory-side cache and merging gains least (8 x 256 rows of hidden 2048: 5.9 ms
+    -> 5.0), and the step keeps giving the bits of the same slices run one after the other."""
+    L = sum(seq_slices)
+    if L * batch >= MERGE_KEEP_ROWS * len(seq_slices) and hidden <= MERGE_KEEP_HIDDEN:
+        return list(seq_slices)
+    cut = (L // 2 + 63) // 64 * 64
+    if n_lanes > 1 and L * batch >= MERGE_TWO_ROWS and 0 < cut < L:
+        return [cut, L - cut]
+    return [L]
+
+
 def fused_backward_slices(seq_slices, n_lanes, window=None):
     """[(own_end, fused)] per sequence slice: the end of the positions whose delta a fused attention-backward launch
     of the slice takes itself (the slice and the n_lanes - 1 slices after it, whose launches may still be running),
@@ -254,8 +292,8 @@ def _run_program(program):
             raise _lib.TeraPipeHipError("replayed launch failed: %s" % (_lib.load().tp_last_error() or b"").decode())
 
 
-def _forward_body(runner, ws, act, bufs, states):
-    """Every (batch slice, sequence slice) through the whole layer stack, slice-major, reading the batch
+def _forward_body(runner, ws, act, bufs, states, pieces):
+    """Every (batch slice, sequence slice of `pieces`) through the whole layer stack, slice-major, reading the batch
     slices from bufs x[0] and leaving the outputs in bufs x[n_layers].  Launches kernels only (no
     allocation, no host synchronisation), so it can be recorded into a HIP graph.
 
@@ -275,7 +313,7 @@ def _forward_body(runner, ws, act, bufs, states):
         cache = pb["cache"]
         P = 0
         prev_done = None
-        for i, T in enumerate(runner.seq_slices):
+        for i, T in enumerate(pieces):
             r0, r1 = P * Bs, (P + T) * Bs
             sts, done = [], []
             st_i = lanes[i % len(lanes)] if lanes else main
@@ -324,14 +362,14 @@ def _forward_body(runner, ws, act, bufs, states):
         _wait_stream(main, st)
 
 
-def _backward_body(runner, ws, act, bufs, states):
+def _backward_body(runner, ws, act, bufs, states, pieces):
     """Reverse-order slices (terapipe.py:182-191 of the reference) reading the output gradient from bufs
     dx[n_layers], then one weight-gradient GEMM per weight and one reduction per vector parameter over
     all tokens, into bufs.wgrads / bufs.sgrads.  Launches kernels only."""
     layers = runner.layers
     nl, H = layers.n_layers, layers.num_attention_heads
     E, F = layers.embedding_dim, layers.ffn_embedding_dim
-    nb, ns = len(runner.batch_slices), len(runner.seq_slices)
+    nb, ns = len(runner.batch_slices), len(pieces)
     L = runner.seq_len
     ops.zero_(bufs.small)
     side = bufs.lanes
@@ -343,7 +381,7 @@ def _backward_body(runner, ws, act, bufs, states):
         _wait_stream(st, main)
     if early_dw:
         _wait_stream(bufs.dw_stream, main)
-    fusion = fused_backward_slices(runner.seq_slices, len(lanes))
+    fusion = fused_backward_slices(pieces, len(lanes))
     for b in reversed(range(nb)):
         Bs = runner.batch_slices[b]
         pb = bufs.per_batch[b]
@@ -351,7 +389,7 @@ def _backward_body(runner, ws, act, bufs, states):
         P = L
         later_done = None
         for i in reversed(range(ns)):
-            T = runner.seq_slices[i]
+            T = pieces[i]
             P -= T
             r0, r1 = P * Bs, (P + T) * Bs
             last = i == ns - 1
@@ -484,6 +522,42 @@ def _capture(fn, bufs):
     return g
 
 
+def _slice_states(runner, bufs, states, pieces):
+    """What the forward kept, slice by slice of runner.seq_slices (row ranges of the pieces' tensors)."""
+    if list(pieces) == runner.seq_slices:
+        return states.copy()
+    out = np.empty((len(runner.batch_slices), len(runner.seq_slices)), dtype="O")
+    nl, H = runner.layers.n_layers, runner.layers.num_attention_heads
+    for b, Bs in enumerate(runner.batch_slices):
+        pb, P = bufs.per_batch[b], 0
+        for i, T in enumerate(runner.seq_slices):
+            r0, r1 = P * Bs, (P + T) * Bs
+            out[b, i] = []
+            for l in range(nl):
+                st = core.SliceState()
+                for name in ("x", "mean1", "rstd1", "xn", "o", "h", "mean2", "rstd2", "hn", "a", "z"):
+                    t = pb[name][l]
+                    setattr(st, name, None if t is None else t[r0:r1])
+                if bufs.position_indexed:
+                    st.q, st.lse, st.q_bh_rows = pb["q"][l][:, P:], pb["lse"][l][:, P:], runner.seq_len
+                else:
+                    # compact per piece: [B * H, rows of the piece, ...]
+                    p0 = 0
+                    for n in pieces:
+                        if P < p0 + n:
+                            break
+                        p0 += n
+                    q = pb["q"][l][p0 * Bs:(p0 + n) * Bs].view(Bs * H, n, -1)
+                    lse = pb["lse"][l][p0 * Bs * H:(p0 + n) * Bs * H].view(Bs * H, n)
+                    st.q, st.lse, st.q_bh_rows = q[:, P - p0:], lse[:, P - p0:], n
+                st.stat_bh_rows = st.q_bh_rows
+                st.k_cache, st.v_cache = pb["cache"][2 * l], pb["cache"][2 * l + 1]
+                st.cache_len, st.T, st.B = P, T, Bs
+                out[b, i].append(st)
+            P += T
+    return out
+
+
 class _TeraPipeFunction(torch.autograd.Function):
     """One autograd node around the whole slice grid (see _forward_body / _backward_body)."""
 
@@ -494,7 +568,9 @@ class _TeraPipeFunction(torch.autograd.Function):
         ws = [dict(zip(core.PARAM_NAMES, flat_params[12 * i:12 * i + 12])) for i in range(nl)]
         act = [l.activation for l in layers.layers]
         bufs = runner._stack_buffers(inputs.dtype, inputs.device, ws)
-        nb, ns = len(runner.batch_slices), len(runner.seq_slices)
+        # slice timings are asked for slice by slice; otherwise the step runs in as few pieces as pay
+        pieces = bufs.pieces if runner.slice_timing is None else runner.seq_slices
+        nb, ns = len(runner.batch_slices), len(pieces)
         b0 = 0
         for b, Bs in enumerate(runner.batch_slices):
             # the batch slice as [L*Bs, E] rows (t, b_local): a copy, as grid_slice_batch_and_sequence makes
@@ -512,20 +588,20 @@ class _TeraPipeFunction(torch.autograd.Function):
             # second pass: run it and keep what it launched
             states = np.empty((nb, ns), dtype="O")
             with ops.CallRecorder(program=[]) as rec:
-                _forward_body(runner, ws, act, bufs, states)
+                _forward_body(runner, ws, act, bufs, states, pieces)
             bufs.fwd_program, bufs.states = rec.program, states
             bufs.program_stream = torch.cuda.current_stream().cuda_stream
         else:
             if replayable and bufs.fwd_program == 0:
                 bufs.fwd_program = 1
             states = np.empty((nb, ns), dtype="O")
-            _forward_body(runner, ws, act, bufs, states)
+            _forward_body(runner, ws, act, bufs, states, pieces)
             if runner.use_hip_graph:
                 bufs.states = states
-                bufs.fwd_graph = _capture(lambda: _forward_body(runner, ws, act, bufs, np.empty((nb, ns), dtype="O")), bufs)
+                bufs.fwd_graph = _capture(lambda: _forward_body(runner, ws, act, bufs, np.empty((nb, ns), dtype="O"), pieces), bufs)
         runner.last_caches = [pb["cache"] for pb in bufs.per_batch]
         if runner.keep_states:
-            runner.last_states = states.copy()
+            runner.last_states = _slice_states(runner, bufs, states, pieces)
         if nb == 1:
             y = bufs.per_batch[0]["x"][nl].view(runner.seq_len, runner.batch_slices[0], E).clone()
         else:
@@ -534,12 +610,14 @@ class _TeraPipeFunction(torch.autograd.Function):
         # the buffers hold ONE step's activations: a backward must run before the next forward overwrites them
         bufs.generation += 1
         ctx.generation = bufs.generation
+        ctx.pieces = pieces
         ctx.runner, ctx.ws, ctx.act, ctx.states, ctx.bufs = runner, ws, act, states, bufs
         return y
 
     @staticmethod
     def backward(ctx, grad_y):
         runner, ws, act, states, bufs = ctx.runner, ctx.ws, ctx.act, ctx.states, ctx.bufs
+        pieces = ctx.pieces
         if ctx.generation != bufs.generation or bufs is not runner._sbufs:
             raise RuntimeError("TeraPipe keeps the activations of one step in buffers that the next forward "
                                "reuses: this backward belongs to a forward that a later forward has overwritten")
@@ -572,16 +650,16 @@ class _TeraPipeFunction(torch.autograd.Function):
             bufs.wgrad_descs, bufs.recording = {}, True
             try:
                 with ops.CallRecorder(program=[]) as rec:
-                    _backward_body(runner, ws, act, bufs, states)
+                    _backward_body(runner, ws, act, bufs, states, pieces)
             finally:
                 bufs.recording = False
             bufs.bwd_program = rec.program
         else:
             if replayable and bufs.bwd_program == 0:
                 bufs.bwd_program = 1
-            _backward_body(runner, ws, act, bufs, states)
+            _backward_body(runner, ws, act, bufs, states, pieces)
             if runner.use_hip_graph:
-                bufs.bwd_graph = _capture(lambda: _backward_body(runner, ws, act, bufs, states), bufs)
+                bufs.bwd_graph = _capture(lambda: _backward_body(runner, ws, act, bufs, states, pieces), bufs)
         # vector-parameter gradients: one clone of the flat buffer (it is reused by the next step); weight
         # gradients: this backward's own storage, or a clone of the graph's static one
         sviews = _flat_views(bufs.sgrad_flat.clone(), bufs.sgrad_layout)
@@ -631,6 +709,12 @@ class TeraPipe(nn.Module):
     run through the stack side by side.  Same kernels, same arguments, same results; the overlap fills the
     chip where one chain of short kernels cannot, and GEMMs that stream the same weight at the same time
     share its way through the caches.  Default 3 (1 under use_hip_graph).
+    merge_slices: the step runs the sequence in one or two pieces instead of slice by slice (merged_slices says why and
+    when), with the same results up to rounding.  None (the default): where the caller leaves the way the step runs to
+    the runner.  A caller that sets slice_streams asks for its slices on that many streams (1: one after the other, as
+    on a stage that gets them one by one), suffix_dkdv=False and fp32_grad_cache=False for the hand-over of cache
+    gradients from slice to slice, several batch slices for that grid: those run as they are cut, and so does a step
+    whose slices are timed (slice_timing).
     launch_replay: the first step runs as written, the second also keeps every library call it makes (bound
     descriptor + stream handle) and every stream wait / event record in one list, and later steps re-issue
     that list: the same launches on the same streams without rebuilding descriptors, views and saved state
@@ -646,7 +730,7 @@ class TeraPipe(nn.Module):
 
     def __init__(self, layers, batch_size, seq_len, batch_slices, seq_slices, batch_dim=1, sequence_dim=0,
                  fp32_grad_cache=True, use_hip_graph=False, suffix_dkdv=True, slice_streams=None, launch_replay=None,
-                 fused_attn_bwd=True):
+                 fused_attn_bwd=True, merge_slices=None):
         super().__init__()
         assert sum(batch_slices) == batch_size and sum(seq_slices) == seq_len
         assert batch_dim == 1 and sequence_dim == 0, "layers take [seq, batch, embed] inputs"
@@ -658,6 +742,8 @@ class TeraPipe(nn.Module):
         self.use_hip_graph = use_hip_graph
         self.suffix_dkdv = suffix_dkdv
         self.fused_attn_bwd = bool(fused_attn_bwd)
+        self.merge_slices = bool(merge_slices) if merge_slices is not None else (
+            slice_streams is None and not use_hip_graph and suffix_dkdv and fp32_grad_cache and len(self.batch_slices) == 1)
         # defaults: three slice streams and launch replay; one stream and no replay under use_hip_graph
         self.slice_streams = int(slice_streams) if slice_streams is not None else (1 if use_hip_graph else 3)
         self.launch_replay = bool(launch_replay) if launch_replay is not None else not use_hip_graph
@@ -692,6 +778,7 @@ class TeraPipe(nn.Module):
         if (self._sbufs is None or self._sbufs.dtype != dtype or self._sbufs.device != device
                 or self._sbufs.slice_streams != self.slice_streams
                 or self._sbufs.fused_attn_bwd != self.fused_attn_bwd
+                or self._sbufs.merge_slices != self.merge_slices
                 or self._sbufs.param_ptrs != ptrs):     # recorded graphs / launches hold the parameter addresses
             self._sbufs = _StackBuffers(self, dtype, device, ws)
         return self._sbufs

@@ -1,0 +1,62 @@
+"""The pieces a default runner's step runs in: the rule on the CPU, and merged steps against the CPU oracle."""
+import pytest
+import torch
+
+import oracle
+from tests.util import assert_close, load_params_into, make_params
+
+
+def test_rule():
+    from terapipe_amd.terapipe import merged_slices
+    assert merged_slices([32] * 64, 1, 6144, 3) == [1024, 1024]
+    assert merged_slices([32] * 64, 1, 6144, 1) == [2048]
+    assert merged_slices([16] * 8, 2, 256, 3) == [128]
+    assert merged_slices([1031, 1032], 1, 5120, 3) == [1088, 975]
+    assert merged_slices([1023, 1024], 1, 5120, 3) == [2047]
+    assert merged_slices([256] * 8, 1, 2048, 3) == [256] * 8            # long slices, small weights: kept
+    assert merged_slices([255] * 8, 1, 2048, 3) == [2040]
+    assert merged_slices([256] * 8, 1, 2056, 3) == [1024, 1024]
+    assert merged_slices([40], 64, 4096, 3) == [40]                     # nothing to cut at a 64-query block
+
+
+def test_who_merges():
+    import terapipe_amd as ta
+    layers = ta.TransformerLayers(1, 64, 128, 1, dtype=torch.float16, device="cpu")
+    make = lambda bs=(2,), **kw: ta.TeraPipe(layers, 2, 64, list(bs), [32, 32], **kw).merge_slices
+    assert make() and make(launch_replay=False) and make(slice_streams=1, merge_slices=True)
+    assert not any(make(**kw) for kw in (dict(slice_streams=3), dict(use_hip_graph=True), dict(suffix_dkdv=False),
+                                         dict(fp32_grad_cache=False), dict(bs=(1, 1)), dict(merge_slices=False)))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("E,H,B,slices,dtype,pieces", [
+    (128, 2, 3, [7, 1, 30, 27], torch.float16, [65]),             # one piece, odd length
+    (128, 1, 32, [33, 31, 5], torch.bfloat16, [64, 5]),           # two pieces, a short second one
+    (160, 2, 16, [100, 31], torch.float16, [131]),                # head dimension 80: gradient caches
+    (128, 2, 3, [7, 1, 30, 27], torch.float32, [65]),             # gradient caches
+], ids=str)
+def test_merged_step_against_the_oracle(E, H, B, slices, dtype, pieces, monkeypatch):
+    """Three steps (eager, recorded, re-issued) of the default runner, GeLU so that no sign decision is involved."""
+    import terapipe_amd as ta
+    monkeypatch.setattr(ta.terapipe, "MERGE_KEEP_HIDDEN", 0)
+    L, nl = sum(slices), 2
+    ps = make_params(nl, E, 4 * E, dtype, seed=5)
+    layers = ta.TransformerLayers(nl, E, 4 * E, H, dtype=dtype, device="cuda", activation="gelu")
+    load_params_into(layers, ps, dtype)
+    runner = ta.TeraPipe(layers, B, L, [B], slices)
+    g = torch.Generator().manual_seed(9)
+    x, dy = torch.randn(L, B, E, generator=g).to(dtype), torch.randn(L, B, E, generator=g).to(dtype)
+    leaf = [{k: v.clone().requires_grad_(True) for k, v in p.items()} for p in ps]
+    yo, dxo, _ = oracle.terapipe_forward_backward(leaf, x.float(), dy.float(), H, [B], slices, activation="gelu")
+    for step in range(3):
+        for p in layers.parameters():
+            p.grad = None
+        xd = x.cuda().requires_grad_(True)
+        y = runner(xd)
+        y.backward(dy.cuda())
+        assert runner._sbufs.pieces == pieces
+        assert_close(y, yo, dtype, "step %d: y" % step)
+        assert_close(xd.grad, dxo, dtype, "step %d: dx" % step)
+        for l, layer in enumerate(layers.layers):
+            for name, p in layer.param_dict().items():
+                assert_close(p.grad, leaf[l][name].grad, dtype, "step %d: layer %d %s" % (step, l, name))
