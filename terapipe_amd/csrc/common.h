@@ -404,6 +404,27 @@ template <typename T, int ROWS, int COLS, int NT, bool ALONG_COLS, bool KM16 = f
     __device__ __forceinline__ void advance() { origin += step; }
 };
 
+// A ragged k of the tiles above: the k range's first len % BK positions make the FIRST tile, copied through registers
+// with zeros behind them (so that every tile after it is whole); `len` of them are valid from slide0 on.  Where k runs
+// along the tile's columns, len is a multiple of 8.  The caller waits (lgkmcnt) before it lets the tile be read.
+template <typename T, int ROWS, int COLS, int NT, bool ALONG_COLS, bool KM16>
+__device__ __forceinline__ void copy_ragged_tile(T* tile, const T* __restrict__ base, long ld, int fixed0, int fixed_max,
+                                                 int slide0, int len, int tid) {
+    constexpr int CPR = COLS / 8, N = ROWS * CPR / NT;
+#pragma unroll
+    for (int i = 0; i < N; ++i) {
+        const int p = i * NT + tid;
+        const int row = p / CPR, lc = (p % CPR) ^ swz16<COLS, KM16>(row);
+        const int sl = ALONG_COLS ? lc * 8 : row;
+        int fx = fixed0 + (ALONG_COLS ? row : lc * 8);
+        const int last = fixed_max - (ALONG_COLS ? 1 : 8);
+        fx = fx < last ? fx : last;
+        uint4 v = make_uint4(0, 0, 0, 0);
+        if (sl < len) v = *reinterpret_cast<const uint4*>(base + (ALONG_COLS ? (long)fx * ld + slide0 + sl : (long)(slide0 + sl) * ld + fx));
+        *reinterpret_cast<uint4*>(tile + p * 8) = v;
+    }
+}
+
 // error plumbing shared by the host-side entry points
 void set_error(const char* fmt, ...);
 

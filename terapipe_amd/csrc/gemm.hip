@@ -211,8 +211,10 @@ void gemm_tall_kernel(typename std::conditional<GROUPED, GemmGroupArgs, GemmArgs
     const int kend = min(a.K, kbeg + a.kper);
     DA da;
     DB db;
-    da.init(reinterpret_cast<const T*>(a.A), a.lda, m0, a.M, kbeg, BK, tid);
-    db.init(reinterpret_cast<const T*>(a.B), a.ldb, n0, a.N, kbeg, BK, tid);
+    const int nk = (kend - kbeg + BK - 1) / BK;
+    const int ragged = (kend - kbeg) % BK;      // a ragged k has its short tile first (copy_ragged_tile)
+    da.init(reinterpret_cast<const T*>(a.A), a.lda, m0, a.M, ragged ? kbeg + ragged - BK : kbeg, BK, tid);
+    db.init(reinterpret_cast<const T*>(a.B), a.ldb, n0, a.N, ragged ? kbeg + ragged - BK : kbeg, BK, tid);
     const unsigned lds0 = lds_addr(smem);
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);
     auto issue = [&](int stage) {
@@ -262,9 +264,17 @@ void gemm_tall_kernel(typename std::conditional<GROUPED, GemmGroupArgs, GemmArgs
         }
     }
 
-    const int nk = (kend - kbeg) / BK;          // whole tiles only (the plan guarantees it)
+    if (ragged) {
+        copy_ragged_tile<T, AR, AC, NT, AKM, MI16 && AKM>(tiles, reinterpret_cast<const T*>(a.A), a.lda, m0, a.M, kbeg, ragged, tid);
+        copy_ragged_tile<T, BR, BC, NT, BKM, MI16 && BKM>(tiles + A_ELEMS, reinterpret_cast<const T*>(a.B), a.ldb, n0, a.N, kbeg, ragged, tid);
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+        da.advance();
+        db.advance();
+    } else {
+        issue(0);
+    }
 #pragma unroll
-    for (int s = 0; s < STAGES - 1; ++s)
+    for (int s = 1; s < STAGES - 1; ++s)
         if (s < nk) issue(s);
 
     constexpr int NSET = MI16 ? 1 : 2;
@@ -525,10 +535,13 @@ static bool tile_cfg(int id, TileCfg& c) {
     case 41: c = {224, 128, 64, 3}; return true;   // 2 x 2 waves of 112 x 64
     case 42: c = {160, 128, 64, 3}; return true;   // 2 x 2 waves of 80 x 64
     case 43: c = {224, 160, 64, 3}; return true;   // 2 x 2 waves of 112 x 80 (NT only, like 6 and 7)
+    // gemm_wide_kernel: eight waves (2 x 4) of 128 x 64, software-pipelined
+    case 44: c = {256, 256, 64, 2}; return true;   // NT and NN
     default: return false;
     }
 }
 static constexpr int kFirstStreamCfg = 21, kLastStreamCfg = 40;
+static constexpr int kWideCfg = 44;
 
 // Measured plans: for NT / NN the weight extents (N, K) match exactly and M (tokens of the slice) picks the
 // nearest measured M at or above it (at least half of it, so that a much shorter slice falls through to the
@@ -566,6 +579,60 @@ static void finish_plan(const tp_gemm_desc* d, GemmPlan& p, int bk, int nsplit) 
     long per = (kt + nsplit - 1) / nsplit;
     p.kper = (int)(per * bk);
     p.nsplit = (int)((d->K + p.kper - 1) / p.kper);
+}
+
+// The time (us) of `tiles` workgroups of a tile configuration over k: rounds of one workgroup per CU, each a fixed part
+// (prologue, epilogue) and a part per k; a partly filled round runs somewhat faster per k (less traffic, higher clocks).
+// Fitted to a sweep of 198 products (hidden 1024 to 6144; 1024, 2048 and 4096 rows; all three operand orders; alone on
+// the chip): the per-k part is flops at 1.16 to 1.47 PFLOP/s of the whole chip.  Where the operands outgrow the
+// memory-side cache the smaller tiles, which read them more often, fall behind (`spill`).
+struct TileCost { int cfg, bm, bn; float fixed, per_k, per_k_spill; };
+static const TileCost kTileCost[] = {
+    {16, 128, 128, 4.8f, 0.0068f, 0.0084f},
+    {14, 192, 128, 6.8f, 0.0088f, 0.0101f},
+    {15, 256, 128, 12.0f, 0.0115f, 0.0125f},
+    {kWideCfg, 256, 256, 12.0f, 0.0228f, 0.0232f},     // NT, NN
+    {2, 256, 256, 11.5f, 0.0248f, 0.0248f},            // TN
+};
+static float tile_time(const TileCost& c, long tiles, float k, bool spill) {
+    const float per_k = spill ? c.per_k_spill : c.per_k;
+    const long full = tiles / kNumCU, rest = tiles % kNumCU;
+    return full * (c.fixed + per_k * k) + (rest ? c.fixed + per_k * k * (0.72f + 0.28f * rest / kNumCU) : 0.f);
+}
+static bool tile_serves(const TileCost& c, int op, int K) {
+    if (op == TP_GEMM_TN) return c.cfg != 14 && c.cfg != kWideCfg;
+    return c.cfg != 2 && (c.cfg != kWideCfg || K >= 64);
+}
+
+// Products of more than 512 rows and parameter gradients: the tile and the k split with the smallest estimate.  A split
+// costs its fp32 partial sums (written and read once at 5.5 TB/s) and the launch that adds them.  The rules this replaces
+// named 256 x 256 tiles from 192 of them on and split or shrank them otherwise, without regard for the last round: the
+// estimate's choice takes 0.61 to 1.0 of their time (1024 x 5120 x 20480: 284 -> 188 us; 4096 x 1600 x 6400: 117 -> 80).
+static void plan_large(const tp_gemm_desc* d, int& cfg, int& ns) {
+    const float K = (float)d->K;
+    // an LM head's data gradient (k = vocabulary): 48 to 63 tiles of 256 x 256 on a long k, split to one round
+    const long t256 = (long)((d->M + 255) / 256) * ((d->N + 255) / 256);
+    if (d->op != TP_GEMM_TN && d->K >= 8192 && t256 >= 48 && t256 < 64) {
+        cfg = kWideCfg;
+        ns = (int)(kNumCU / t256);
+        return;
+    }
+    const bool spill = 2.0 * ((double)d->M + d->N) * d->K > 225e6;
+    // 64 x 64 tiles, two per CU: below 512 of them the larger tiles leave most of the chip idle
+    const long t64 = (long)((d->M + 63) / 64) * ((d->N + 63) / 64);
+    float best = t64 <= kNumCU ? 4.6f + 0.0038f * K : (float)((t64 + 511) / 512) * (3.5f + 0.0066f * K);
+    cfg = 8;
+    ns = 1;
+    for (const TileCost& c : kTileCost) {
+        if (!tile_serves(c, d->op, d->K)) continue;
+        const long tiles = (long)((d->M + c.bm - 1) / c.bm) * ((d->N + c.bn - 1) / c.bn);
+        for (int n = 1; n <= 8; ++n) {
+            if (n > 1 && (d->K / n < 512 || tiles * n > 2 * kNumCU)) break;
+            float t = tile_time(c, tiles * n, K / n, spill);
+            if (n > 1) t += 4.f + (float)((double)n * d->M * d->N * 8 / 5.5e6);
+            if (t < best) { best = t; cfg = c.cfg; ns = n; }
+        }
+    }
 }
 
 static GemmPlan plan_gemm(const tp_gemm_desc* d) {
@@ -636,43 +703,15 @@ static GemmPlan plan_gemm(const tp_gemm_desc* d) {
             if (d->K / ns3 >= 4096 || t128 > kNumCU) { cfg = 3; ns = ns3; }
             else { cfg = 13; ns = splits_for(t128, 2048); }
         }
-    } else if ((d->op == TP_GEMM_TN || d->M >= 512) && d->K % 64 == 0 && t256 >= 192) {
-        // parameter gradients of a whole step, and any product of 512 rows or more with that many tiles (the LM
-        // head): 256 x 256 tiles by eight waves (half the bytes per flop of a 128 x 128 tile through the
-        // 64 B/clk vector-memory path into LDS); the parameter gradients on 16 x 16 x 32 blocks with the 32-wide
-        // k-tile in four stages (timed inside steps of four geometries: 1 to 5 % under the 32 x 32 blocks)
-        cfg = d->op == TP_GEMM_TN ? 2 : 19;
-    } else if (d->op != TP_GEMM_TN && d->M >= 512 && d->K % 64 == 0 && t256 >= 48 && d->K >= 8192) {
-        // the same tiles on a long k with too few of them for the chip (the LM head's data gradient, k =
-        // vocabulary): k is split to about one workgroup per CU
-        cfg = 19;
-        ns = (int)((256 + t256 - 1) / t256);
-        int maxs = d->K / 2048;
-        if (ns > maxs) ns = maxs;
-        if (ns > 8) ns = 8;
-    } else if (t128 >= 144) {
-        // short activations: the deeper ring keeps the weight stream going; parameter gradients (both
-        // operands fetched with transpose reads): 128 x 128 x 32, four stages, two workgroups per CU
-        cfg = d->op == TP_GEMM_TN ? 10 : (d->M <= 256 ? 13 : 5);
-        if (t128 < 224) {
-            ns = (int)(448 / t128);
-            int maxs = d->K / 1024;
-            if (ns > maxs) ns = maxs;
-        }
     } else {
-        cfg = 8;
-        if (t64 < 384) {
-            ns = (int)(512 / t64);
-            int maxs = d->K / 3072;
-            if (ns > maxs) ns = maxs;
-        }
+        plan_large(d, cfg, ns);
     }
     // The pipelined 16 x 16 x 32 tiles in place of the 32 x 32 ones the rules above name, where a sweep over other
     // geometries (hidden 3072, 4096, 8192; 128 to 512 rows; 144 slice products) has them ahead: 128 x 128 for
     // 128 x 128 (0.94 to 0.99 of the time), 192 x 128 for 128 x 256 at 129 to 192 rows and at 257 to 384 (0.83 to 0.91),
     // 256 x 128 above 384 rows (0.92), and the 160- and 224-row tiles where they end with the slice (0.95 to 1.0 of
     // the padded tile's time on the 13B shapes); a k-split stays within one round of workgroups of the new tile.
-    if (d->op != TP_GEMM_TN && d->K % 64 == 0 && (cfg == 13 || cfg == 3)) {
+    if (d->op != TP_GEMM_TN && d->M <= 512 && (cfg == 13 || cfg == 3)) {
         int bm = 128, bn = 128, to = 16;
         if (cfg == 3) {
             // row tiles that end with the slice where whole 16-row blocks allow it: 160 (one or two tiles), 192 (one
@@ -696,15 +735,18 @@ static GemmPlan plan_gemm(const tp_gemm_desc* d) {
     TileCfg tc;
     if (forced_cfg >= 0 && tile_cfg(forced_cfg, tc)) cfg = forced_cfg;
     if (forced_split) ns = forced_split;
-    // the tall tiles load whole k-tiles only, and the 160 / 192 wide ones exist for the k-major weight (NT)
-    // (a token-major tile 160 or 192 wide has no XOR swizzle: the chunk index would leave the row)
-    if ((cfg == 6 || cfg == 7 || cfg == 43) && (d->K % 64 || d->op != TP_GEMM_NT)) cfg = 5;
-    if ((cfg == 41 || cfg == 42) && (d->K % 64 || d->op == TP_GEMM_TN)) cfg = 5;
-    if (((cfg >= 14 && cfg <= 20) || cfg == 2) && (d->K % 64 || (cfg == 17 && d->op != TP_GEMM_NT) || (cfg == 14 && d->op == TP_GEMM_TN))) cfg = 5;
-    // the streaming kernel: NT and NN only, whole 64-wide k-tiles only; tiles whose width is not a power of two need
-    // the k-major weight (NT)
+    // The tiles that exist for some operand orders only (a token-major tile 160 or 192 wide has no XOR swizzle: the chunk
+    // index would leave the row; the streaming and the wide kernel have no TN form).  A ragged k: the weight-streaming
+    // and the 32 x 32-block tall tiles load whole k-tiles only; the pipelined tiles copy the ragged part first, but a tile
+    // FORCED through the descriptor keeps to whole k-tiles (it falls back to the 128 x 128 tile).
+    const bool ragged = d->K % 64 != 0, forced = forced_cfg >= 0;
+    if ((cfg == 6 || cfg == 7 || cfg == 43) && ((ragged && forced) || d->op != TP_GEMM_NT)) cfg = 5;
+    if ((cfg == 41 || cfg == 42 || cfg == 14) && ((ragged && forced) || d->op == TP_GEMM_TN)) cfg = 5;
+    if ((cfg == 15 || cfg == 16 || cfg == 2) && ragged && forced) cfg = 5;
+    if (cfg == kWideCfg && ((ragged && forced) || d->op == TP_GEMM_TN || d->K < 64)) cfg = 5;
+    if (cfg >= 17 && cfg <= 20 && (ragged || (cfg == 17 && d->op != TP_GEMM_NT))) cfg = 5;
     if (cfg >= kFirstStreamCfg && cfg <= kLastStreamCfg &&
-        (d->op == TP_GEMM_TN || d->K % 64 || ((cfg == 24 || cfg == 25) && d->op != TP_GEMM_NT))) cfg = 5;
+        (d->op == TP_GEMM_TN || ragged || ((cfg == 24 || cfg == 25) && d->op != TP_GEMM_NT))) cfg = 5;
     p.cfg = cfg;
     tile_cfg(cfg, tc);
     p.gx = (d->N + tc.bn - 1) / tc.bn;
@@ -747,6 +789,8 @@ static bool launch_gemm(const tp_gemm_desc* d, const GemmPlan& p, const GemmArgs
         if (!launch_gemm_stream(p.cfg, d->op, d->dtype, dim3(p.gx, p.gy, p.nsplit), a, s)) return false;
     } else if (is_pipe_cfg(p.cfg) && d->dtype != TP_F32) {
         if (!launch_gemm_pipe(p.cfg, d->op, d->dtype, dim3(p.gx, p.gy, p.nsplit), a, s)) return false;
+    } else if (p.cfg == kWideCfg && d->dtype != TP_F32) {
+        if (!launch_gemm_wide(d->op, d->dtype, dim3(p.gx, p.gy, p.nsplit), a, s)) return false;
     } else {
         switch (d->op) {
         case TP_GEMM_NT: launch_cfg<T, true, true>(p, a, s); break;
@@ -861,23 +905,36 @@ static GemmArgs fill_args(const tp_gemm_desc* d, const GemmPlan& p, void* worksp
     return a;
 }
 
-// One launch for the whole group when every member is a 16-bit TN product (parameter gradients) of the same dtype
-// whose k is a whole number of 64-wide tiles and the group's largest member plans to a 256 x 256 tile with
-// unsplit k.
-// The tile configuration of the single launch that runs the group, or 0 when it runs member by member.
+// One launch for the whole group when every member is a 16-bit TN product (parameter gradients) of the same dtype and
+// k (whole 64-wide k-tiles), on the tile with the smallest estimate for all members' tiles together (or the largest
+// member's measured or forced one; the 256 x 256 tile unless another is a tenth ahead): the configuration of that
+// launch, or 0 when the group runs member by member.
 static int group_cfg(const tp_gemm_desc* descs, int n) {
     if (n < 2 || n > kGroupMax) return 0;
     int big = 0;
     for (int i = 0; i < n; ++i) {
         const tp_gemm_desc& d = descs[i];
-        if (d.op != TP_GEMM_TN || d.dtype != descs[0].dtype || d.dtype == TP_F32 || d.K % 64 != 0 ||
+        if (d.op != TP_GEMM_TN || d.dtype != descs[0].dtype || d.dtype == TP_F32 || d.K != descs[0].K || d.K % 64 != 0 ||
             d.reserved != descs[0].reserved ||      // a forced plan (tuning, tests) must be the same for all members
             d.defer_reduce != 0 || d.epilogue == TP_EPI_QKV_SCATTER)
             return 0;
         if ((double)d.M * d.N > (double)descs[big].M * descs[big].N) big = i;
     }
-    const GemmPlan pb = plan_gemm(&descs[big]);
-    return ((pb.cfg == 2 || pb.cfg == 15 || pb.cfg == 19 || pb.cfg == 20) && pb.nsplit == 1) ? pb.cfg : 0;
+    if (descs[0].reserved || find_tuned(&descs[big])) {
+        const GemmPlan pb = plan_gemm(&descs[big]);
+        return ((pb.cfg == 2 || pb.cfg == 15 || pb.cfg == 16 || pb.cfg == 19 || pb.cfg == 20) && pb.nsplit == 1) ? pb.cfg : 0;
+    }
+    const bool spill = 2.0 * ((double)descs[big].M + descs[big].N) * descs[0].K > 225e6;
+    int cfg = 0;
+    float best = 0.f;
+    for (const TileCost& c : kTileCost) {
+        if (!tile_serves(c, TP_GEMM_TN, descs[0].K)) continue;
+        long tiles = 0;
+        for (int i = 0; i < n; ++i) tiles += (long)((descs[i].M + c.bm - 1) / c.bm) * ((descs[i].N + c.bn - 1) / c.bn);
+        const float t = tile_time(c, tiles, (float)descs[0].K, spill) * (c.cfg == 2 ? 0.9f : 1.f);
+        if (!cfg || t < best) { best = t; cfg = c.cfg; }
+    }
+    return cfg;
 }
 
 template <typename T>
@@ -902,7 +959,7 @@ static bool launch_group(const tp_gemm_desc* descs, int n, int cfg, hipStream_t 
     for (int i = n; i < kGroupMax; ++i) { ga.g[i] = ga.g[0]; ga.first_tile[i] = tiles; ga.tiles_x[i] = 1; ga.tiles_y[i] = 1; }
     ga.n = n;
     if (cfg == 2) gemm_tall_kernel<T, AKM, BKM, 256, 256, 32, 4, 2, 4, true, true><<<dim3(tiles), 512, 0, s>>>(ga);
-    else if (cfg == 15) return launch_gemm_pipe_group(cfg, descs[0].dtype, tiles, ga, s);
+    else if (cfg == 15 || cfg == 16) return launch_gemm_pipe_group(cfg, descs[0].dtype, tiles, ga, s);
     else if (cfg == 19) gemm_tall_kernel<T, AKM, BKM, 256, 256, 64, 4, 2, 2, true><<<dim3(tiles), 512, 0, s>>>(ga);
     else gemm_tall_kernel<T, AKM, BKM, 256, 256, 32, 4, 2, 4, true><<<dim3(tiles), 512, 0, s>>>(ga);
     return true;

@@ -71,11 +71,12 @@ void gemm_pipe_kernel(typename std::conditional<GROUPED, GemmGroupArgs, GemmArgs
     const int m0 = tile_y * BM, n0 = tile_x * BN;
     const int kbeg = tile_z * a.kper;
     const int kend = min(a.K, kbeg + a.kper);
-    const int nk = (kend - kbeg) / BK;          // whole tiles only (the plan guarantees it)
+    const int nk = (kend - kbeg + BK - 1) / BK;
+    const int ragged = (kend - kbeg) % BK;      // a ragged k has its short tile first (copy_ragged_tile)
     DA da;
     DB db;
-    da.init(reinterpret_cast<const T*>(a.A), a.lda, m0, a.M, kbeg, BK, tid);
-    db.init(reinterpret_cast<const T*>(a.B), a.ldb, n0, a.N, kbeg, BK, tid);
+    da.init(reinterpret_cast<const T*>(a.A), a.lda, m0, a.M, ragged ? kbeg + ragged - BK : kbeg, BK, tid);
+    db.init(reinterpret_cast<const T*>(a.B), a.ldb, n0, a.N, ragged ? kbeg + ragged - BK : kbeg, BK, tid);
     const unsigned lds0 = lds_addr(smem);
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);
 
@@ -151,12 +152,20 @@ void gemm_pipe_kernel(typename std::conditional<GROUPED, GemmGroupArgs, GemmArgs
 #pragma unroll
     for (int s = 0; s < STAGES; ++s)
         if (s < nk) {
+            if (s == 0 && ragged) {
+                copy_ragged_tile<T, AR, AC, NT, AKM, AKM>(tiles, reinterpret_cast<const T*>(a.A), a.lda, m0, a.M, kbeg, ragged, tid);
+                copy_ragged_tile<T, BR, BC, NT, BKM, BKM>(tiles + A_ELEMS, reinterpret_cast<const T*>(a.B), a.ldb, n0, a.N, kbeg, ragged, tid);
+                da.advance();
+                db.advance();
+                continue;
+            }
             const unsigned sA = lds0 + (unsigned)(s * STAGE_ELEMS * 2);
             da.issue(sA, wave_u);
             db.issue(sA + (unsigned)(A_ELEMS * 2), wave_u);
         }
     if (nk >= STAGES) wait_vmcnt<NLOAD * (STAGES - 1)>();
     else wait_vmcnt<0>();
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // (a copied tile's stores)
     __builtin_amdgcn_s_barrier();
     asm volatile("" ::: "memory");
     static_for<NF>([&](auto fc) __attribute__((always_inline)) {
@@ -268,10 +277,17 @@ bool launch_gemm_pipe(int cfg, int op, int dtype, dim3 grid, const GemmArgs& a, 
 }
 
 bool launch_gemm_pipe_group(int cfg, int dtype, int tiles, const GemmGroupArgs& ga, hipStream_t s) {
-    if (cfg != 15) return false;
-    if (dtype == TP_F16) gemm_pipe_kernel<f16, false, false, 256, 128, 4, 1, 3, true><<<dim3(tiles), 256, 0, s>>>(ga);
-    else if (dtype == TP_BF16) gemm_pipe_kernel<bf16, false, false, 256, 128, 4, 1, 3, true><<<dim3(tiles), 256, 0, s>>>(ga);
-    else return false;
+    if (dtype == TP_F16) {
+        if (cfg == 15) gemm_pipe_kernel<f16, false, false, 256, 128, 4, 1, 3, true><<<dim3(tiles), 256, 0, s>>>(ga);
+        else if (cfg == 16) gemm_pipe_kernel<f16, false, false, 128, 128, 2, 2, 3, true><<<dim3(tiles), 256, 0, s>>>(ga);
+        else return false;
+    } else if (dtype == TP_BF16) {
+        if (cfg == 15) gemm_pipe_kernel<bf16, false, false, 256, 128, 4, 1, 3, true><<<dim3(tiles), 256, 0, s>>>(ga);
+        else if (cfg == 16) gemm_pipe_kernel<bf16, false, false, 128, 128, 2, 2, 3, true><<<dim3(tiles), 256, 0, s>>>(ga);
+        else return false;
+    } else {
+        return false;
+    }
     return true;
 }
 
