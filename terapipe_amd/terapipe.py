@@ -94,8 +94,7 @@ class _StackBuffers:
         # the pieces a step runs in
         self.pieces = runner.seq_slices
         if runner.merge_slices:
-            self.pieces = merged_slices(runner.seq_slices, max(runner.batch_slices), E,
-                                        runner.slice_streams if self.position_indexed else 1)
+            self.pieces = merged_slices(runner.seq_slices, max(runner.batch_slices), E)
         gdt = torch.float32 if runner.fp32_grad_cache else dtype
         kw = dict(dtype=dtype, device=device)
         f32 = dict(dtype=torch.float32, device=device)
@@ -200,35 +199,30 @@ def _flat_views(flat, layout):
     return [{n: flat[o:o + int(np.prod(s))].view(s) for n, (o, s) in d.items()} for d in layout]
 
 
-# Rows (tokens x batch) from which a merged sequence is cut into two pieces on two streams, and the slices that stay as
-# they are (rows on average, hidden size): see merged_slices.
-MERGE_TWO_ROWS = 2048
-MERGE_KEEP_ROWS, MERGE_KEEP_HIDDEN = 256, 2048
+# The slices that stay as they are (rows of one on average, rows of all, hidden size): see merged_slices.
+MERGE_KEEP_ROWS, MERGE_KEEP_TOTAL, MERGE_KEEP_HIDDEN = 256, 2048, 2048
 
 
-def merged_slices(seq_slices, batch, hidden, n_lanes):
-    """The pieces a single-stage step runs the sequence in: the whole sequence, or two halves on two streams.
+def merged_slices(seq_slices, batch, hidden):
+    """The pieces a single-stage step runs the sequence in: the whole sequence as one, but for the exception below.
 
     Slices are the unit in which pipeline STAGES hand work to each other.  One runner holds every slice of its stage
     from the start, and what its step computes does not depend on where the sequence is cut: every operation of a layer
     but attention works row by row, and attention over the prefix and the slice is attention over the positions up to
     the query's own.  A slice costs a pass over the stack's weights and a chain of launches, so the fewer the better: a
     product of 64 rows is bound by reading its weight, one of 2048 by the matrix pipe.  Measured (16 bit, 2048 tokens):
-    64 slices of 32 x 2 rows of hidden 6144: 104.8 ms -> 46.1 as one piece, 44.8 as two; seven slices of 160-512 rows
-    of hidden 5120: 25.6 -> 23.0 / 22.2.  Four pieces are slower than two (48.5 / 23.0).  Two pieces of 1024 rows and
-    more fill each other's last waves of tiles and the attention launches' tails; below that one piece wins.  The cut
-    is at a whole 64-query block.
+    64 slices of 32 x 2 rows of hidden 6144: 104.8 ms -> 44.7; seven slices of 160-512 rows of hidden 5120: 25.9 ->
+    21.0.  Two pieces on two streams, which fill each other's last waves of tiles, are level or slower with the tiles
+    chosen for whole rounds of the chip (44.7 and 22.3; hidden 4096: 8.8 against 8.2).
 
-    Slices of MERGE_KEEP_ROWS rows and more on a hidden size up to MERGE_KEEP_HIDDEN stay as they are: there the lanes'
-    products share the weights through the memory-side cache and merging gains least (8 x 256 rows of hidden 2048: 5.9 ms
-    -> 5.0), and the step keeps giving the bits of the same slices run one after the other."""
-    L = sum(seq_slices)
-    if L * batch >= MERGE_KEEP_ROWS * len(seq_slices) and hidden <= MERGE_KEEP_HIDDEN:
+    Slices of MERGE_KEEP_ROWS rows and more, MERGE_KEEP_TOTAL together, on a hidden size up to MERGE_KEEP_HIDDEN stay as
+    they are: there the lanes' products share the weights through the memory-side cache and merging gains least
+    (8 x 256 rows of hidden 2048: 6.0 ms -> 4.6), and the step keeps giving the bits of the same slices run one after
+    the other."""
+    rows = sum(seq_slices) * batch
+    if MERGE_KEEP_ROWS * len(seq_slices) <= rows <= MERGE_KEEP_TOTAL and hidden <= MERGE_KEEP_HIDDEN:
         return list(seq_slices)
-    cut = (L // 2 + 63) // 64 * 64
-    if n_lanes > 1 and L * batch >= MERGE_TWO_ROWS and 0 < cut < L:
-        return [cut, L - cut]
-    return [L]
+    return [sum(seq_slices)]
 
 
 def fused_backward_slices(seq_slices, n_lanes, window=None):
@@ -709,7 +703,7 @@ class TeraPipe(nn.Module):
     run through the stack side by side.  Same kernels, same arguments, same results; the overlap fills the
     chip where one chain of short kernels cannot, and GEMMs that stream the same weight at the same time
     share its way through the caches.  Default 3 (1 under use_hip_graph).
-    merge_slices: the step runs the sequence in one or two pieces instead of slice by slice (merged_slices says why and
+    merge_slices: the step runs the sequence in one piece instead of slice by slice (merged_slices says why and
     when), with the same results up to rounding.  None (the default): where the caller leaves the way the step runs to
     the runner.  A caller that sets slice_streams asks for its slices on that many streams (1: one after the other, as
     on a stage that gets them one by one), suffix_dkdv=False and fp32_grad_cache=False for the hand-over of cache

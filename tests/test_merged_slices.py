@@ -8,15 +8,12 @@ from tests.util import assert_close, load_params_into, make_params
 
 def test_rule():
     from terapipe_amd.terapipe import merged_slices
-    assert merged_slices([32] * 64, 1, 6144, 3) == [1024, 1024]
-    assert merged_slices([32] * 64, 1, 6144, 1) == [2048]
-    assert merged_slices([16] * 8, 2, 256, 3) == [128]
-    assert merged_slices([1031, 1032], 1, 5120, 3) == [1088, 975]
-    assert merged_slices([1023, 1024], 1, 5120, 3) == [2047]
-    assert merged_slices([256] * 8, 1, 2048, 3) == [256] * 8            # long slices, small weights: kept
-    assert merged_slices([255] * 8, 1, 2048, 3) == [2040]
-    assert merged_slices([256] * 8, 1, 2056, 3) == [1024, 1024]
-    assert merged_slices([40], 64, 4096, 3) == [40]                     # nothing to cut at a 64-query block
+    assert merged_slices([32] * 64, 1, 6144) == [2048]
+    assert merged_slices([16] * 8, 2, 256) == [128]
+    assert merged_slices([256] * 8, 1, 2048) == [256] * 8               # long slices, small weights: kept
+    assert merged_slices([255] * 8, 1, 2048) == [2040]
+    assert merged_slices([256] * 8, 1, 2056) == [2048]
+    assert merged_slices([256] * 8, 2, 2048) == [2048]
 
 
 def test_who_merges():
@@ -30,9 +27,9 @@ def test_who_merges():
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("E,H,B,slices,dtype,pieces", [
-    (128, 2, 3, [7, 1, 30, 27], torch.float16, [65]),             # one piece, odd length
-    (128, 1, 32, [33, 31, 5], torch.bfloat16, [64, 5]),           # two pieces, a short second one
-    (160, 2, 16, [100, 31], torch.float16, [131]),                # head dimension 80: gradient caches
+    (128, 2, 3, [7, 1, 30, 27], torch.float16, [65]),             # odd length
+    (128, 1, 32, [33, 31, 5], torch.bfloat16, [69]),              # more than 2048 rows
+    (160, 2, 16, [100, 31], torch.float16, [131]),                # head dimension 80
     (128, 2, 3, [7, 1, 30, 27], torch.float32, [65]),             # gradient caches
 ], ids=str)
 def test_merged_step_against_the_oracle(E, H, B, slices, dtype, pieces, monkeypatch):
