@@ -340,6 +340,9 @@ int tp_adam_step(const tp_adam_desc* desc, void* stream);
  * LayerNorm / bias gradients into parameter .grad tensors (autograd's sum over slices). */
 int tp_accum_cast(void* dst, const float* src, int64_t n, int accumulate, int dtype, void* stream);
 /* acc[N] += column sums of x[M, N] (fp32 accumulators). */
+/* The same for n (at most 8) tensors whose fp32 sums lie one after the other in src, sizes[i] values each, in one launch. */
+int tp_accum_cast_parts(void* const* dst, const int32_t* sizes, int n, const float* src, int accumulate, int dtype,
+                        void* stream);
 int tp_colsum_acc(const void* x, int64_t ldx, float* acc, int M, int N, int dtype, void* stream);
 /* fills n 32-bit words with zero (a kernel, so it can be recorded into a HIP graph) */
 int tp_zero_words(void* dst, int64_t n_words, void* stream);
@@ -354,6 +357,56 @@ int tp_zero_words(void* dst, int64_t n_words, void* stream);
    stages operand tiles through LDS. */
 int tp_fill_probe(const void* big, int64_t big_bytes, const void* small_region, int64_t small_bytes,
                   int hits_per_miss, int workgroups, int batches_per_wave, int64_t row_stride, void* stream);
+
+/* ---------------------------------------------------------------------------------------------
+ * Whole layers per call: the launches of TransformerLayer.forward (transformer_models.py:273-285) and of its backward,
+ * built from one descriptor instead of one call each.  Same kernels and results as the single calls.
+ * ------------------------------------------------------------------------------------------- */
+typedef struct tp_layer_desc {
+    int32_t dtype, T, batch, heads, hidden, ffn;
+    int32_t activation;                 /* 0 = ReLU, 1 = GeLU */
+    int32_t cache_len;                  /* P */
+    int64_t cache_rows;                 /* L_max */
+    /* attn_ln gain, offset; in_proj weight, bias; out_proj weight, bias; fc_ln gain, offset; fc1 weight, bias; fc2
+       weight, bias */
+    const void* w[12];
+    const void* x;                      /* [T*B, E] */
+    void* k_cache; void* v_cache;       /* [B*H, L_max, Dh]; rows [P, P+T) are written */
+    /* what the forward leaves for the backward: rows of T*B ([B*H, T, Dh] q, [B*H, T] lse) */
+    void* xn; float* mean1; float* rstd1;
+    void* q; void* o; float* lse;
+    void* h; float* mean2; float* rstd2;
+    void* hn; void* a; void* z;         /* z: GeLU's pre-activation, NULL for ReLU */
+    void* out;                          /* [T*B, E] */
+} tp_layer_desc;
+
+/* n layers in a chain (layers[i].x == layers[i-1].out).  Layers may share every buffer but x and out (forward only). */
+size_t tp_layers_fwd_workspace_bytes(const tp_layer_desc* layers, int n);
+int tp_layers_fwd(const tp_layer_desc* layers, int n, void* workspace, size_t workspace_bytes, void* stream);
+
+typedef struct tp_layer_bwd_desc {
+    tp_layer_desc f;
+    const void* dout;                   /* [T*B, E] */
+    void* dz1; void* dhn; void* dh; void* d_o; void* dqkv; void* dxn;   /* intermediate gradients, rows of T*B */
+    void* dx;                           /* [T*B, E] */
+    float* delta;                       /* [B*H, T] */
+    float* small_acc;                   /* fp32 sums of the eight vector-parameter gradients, one after the other:
+                                           attn_ln gain, offset, in_proj bias, out_proj bias, fc_ln gain, offset, fc1
+                                           bias, fc2 bias */
+    void* dk_cache; void* dv_cache;     /* see tp_attn_desc; NULL without caches */
+    int32_t grad_cache_dtype, accumulate_prefix, has_incoming, zero_slice_rows;
+    int64_t wg_rows;                    /* rows of the weight-gradient products below; 0: leave them out */
+    const void* wg_dqkv; const void* wg_xn; const void* wg_dh; const void* wg_o;
+    const void* wg_dz1; const void* wg_hn; const void* wg_dout; const void* wg_a;
+    void* wg_out[4];                    /* in_proj, out_proj, fc1, fc2 */
+    int32_t wg_accumulate;              /* 1: += */
+    int32_t small_zero;                 /* 1: small_acc starts from zero */
+    void* small_out[8];                 /* where the sums go, cast (small_out[0] NULL: nowhere) */
+    int32_t small_accumulate;           /* 1: += */
+    int32_t reserved;
+} tp_layer_bwd_desc;
+size_t tp_layer_bwd_workspace_bytes(const tp_layer_bwd_desc* d);
+int tp_layer_bwd(const tp_layer_bwd_desc* d, void* workspace, size_t workspace_bytes, void* stream);
 
 #ifdef __cplusplus
 }

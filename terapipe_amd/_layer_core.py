@@ -4,9 +4,12 @@ terapipe.py.  Follows TransformerLayer.forward (transformer_models.py:273-285 of
 MultiheadLMAttentionWithCache.forward (:214-255); every arithmetic step is a call into
 libterapipe_hip.so through terapipe_amd.ops.
 """
+import ctypes
+import struct
+
 import torch
 
-from . import ops
+from . import _lib, ops
 from ._lib import (TP_EPI_BIAS_GELU, TP_EPI_BIAS_RELU, TP_EPI_BIAS_RESIDUAL, TP_EPI_GELU_GRAD, TP_EPI_QKV_SCATTER,
                    TP_EPI_RELU_GRAD, TP_GEMM_NN, TP_GEMM_NT)
 
@@ -203,3 +206,123 @@ def layer_bwd(w, st, dout, heads, gk, gv, accumulate_prefix, has_incoming, zero_
     dx = ops.layernorm_bwd(dxn_in, st.x, st.mean1, st.rstd1, w["attn_ln.weight"], dh, None, None, None, None,
                            out=buf.dx)
     return dx.view(T, B, E)
+
+
+# ------------------------------------------------------------------------------------------------
+# whole layers per library call (tp_layers_fwd, tp_layer_bwd): what the layer-level surface and the forward-only path use.
+# A layer is nine to fifteen launches; issued one by one through ops.py each costs about 11 us of Python, which bounds
+# short slices from the host.
+# ------------------------------------------------------------------------------------------------
+_FWD_PACK = struct.Struct("8iq28Q")            # tp_layer_desc
+_BWD_PACK = struct.Struct("12Q4iq8Q4Q2i8Q2i")  # tp_layer_bwd_desc after its tp_layer_desc
+_ACTIVATIONS = {"relu": 0, "gelu": 1}
+
+
+class _Arena:
+    """Byte offsets (multiples of 256) of a set of buffers inside one allocation."""
+    __slots__ = ("off", "total")
+
+    def __init__(self, sizes):
+        self.off, self.total = {}, 0
+        for name, nbytes in sizes:
+            self.off[name] = self.total
+            self.total += (nbytes + 255) // 256 * 256
+
+
+class LayerGeometry:
+    """Sizes of one layer call and where its buffers lie.  Forward: what the backward reads again.  Backward: the
+    intermediate gradients and the fp32 sums of the vector-parameter gradients."""
+    __slots__ = ("T", "B", "E", "F", "H", "dtype", "es", "M", "activation", "fwd", "bwd", "n_small", "dt")
+    _cache = {}
+
+    def __init__(self, T, B, E, F, H, dtype, activation):
+        self.T, self.B, self.E, self.F, self.H, self.dtype, self.activation = T, B, E, F, H, dtype, activation
+        self.es, self.M, self.dt = dtype.itemsize, T * B, ops.tp_dtype(dtype)
+        M, es = self.M, self.es
+        rows = lambda width: M * width * es
+        self.n_small = small_acc_numel(E, F)
+        self.fwd = _Arena([("xn", rows(E)), ("mean1", 4 * M), ("rstd1", 4 * M), ("q", rows(E)), ("o", rows(E)),
+                           ("lse", 4 * M * H), ("h", rows(E)), ("mean2", 4 * M), ("rstd2", 4 * M), ("hn", rows(E)),
+                           ("a", rows(F)), ("z", rows(F) if activation == "gelu" else 0)])
+        self.bwd = _Arena([("dz1", rows(F)), ("dhn", rows(E)), ("dh", rows(E)), ("d_o", rows(E)), ("dqkv", rows(3 * E)),
+                           ("dxn", rows(E)), ("delta", 4 * M * H), ("small", 4 * self.n_small)])
+
+    @classmethod
+    def of(cls, T, B, E, F, H, dtype, activation):
+        key = (T, B, E, F, H, dtype, activation)
+        g = cls._cache.get(key)
+        if g is None:
+            if activation not in _ACTIVATIONS:
+                raise ValueError("activation must be 'relu' or 'gelu'")
+            if len(cls._cache) >= 512:
+                cls._cache.clear()
+            g = cls._cache[key] = cls(*key)
+        return g
+
+    def pack_fwd(self, image, at, cache_len, cache_rows, w_ptrs, x, k, v, base, out, over=None):
+        """Writes a tp_layer_desc at byte `at` of `image`.  base: address of the forward arena; over: addresses that take
+        the place of the arena's."""
+        o = self.fwd.off
+        p = {n: base + o[n] for n in o}
+        if over:
+            p.update(over)
+        _FWD_PACK.pack_into(image, at, self.dt, self.T, self.B, self.H, self.E, self.F, _ACTIVATIONS[self.activation],
+                            cache_len, cache_rows, *w_ptrs, x, k, v, p["xn"], p["mean1"], p["rstd1"], p["q"], p["o"],
+                            p["lse"], p["h"], p["mean2"], p["rstd2"], p["hn"], p["a"],
+                            p["z"] if self.activation == "gelu" else 0, out)
+
+
+def _address(image):
+    return ctypes.addressof(ctypes.c_char.from_buffer(image))
+
+
+def layers_fwd(images, n, device):
+    """tp_layers_fwd on n packed descriptors, on the current stream."""
+    lib = _lib.load()
+    ptr = _address(images)
+    stream = ops._stream()
+    need = lib.tp_layers_fwd_workspace_bytes(ptr, n)
+    ws = ops.Workspace.get(need, device, stream) if need else None
+    _lib.check(lib.tp_layers_fwd(ptr, n, ops._p(ws), ws.numel() if ws is not None else 0, stream), "tp_layers_fwd")
+    ops._record("layers_fwd", n, lambda s=None, ws=ws, keep=images: lib.tp_layers_fwd(
+        ptr, n, ops._p(ws), ws.numel() if ws is not None else 0, ops._on(s)))
+
+
+def layer_bwd_native(image, device):
+    """tp_layer_bwd on a packed tp_layer_bwd_desc, on the current stream."""
+    lib = _lib.load()
+    ptr = _address(image)
+    stream = ops._stream()
+    need = lib.tp_layer_bwd_workspace_bytes(ptr)
+    ws = ops.Workspace.get(need, device, stream) if need else None
+    _lib.check(lib.tp_layer_bwd(ptr, ops._p(ws), ws.numel() if ws is not None else 0, stream), "tp_layer_bwd")
+    ops._record("layer_bwd", 1, lambda s=None, ws=ws, keep=image: lib.tp_layer_bwd(
+        ptr, ops._p(ws), ws.numel() if ws is not None else 0, ops._on(s)))
+
+
+def stack_forward_only(layers, x, caches, cache_len):
+    """The forward of a chain of layers without anything kept for a backward, as one library call: all layers share one
+    set of intermediate buffers.  layers: [(12 parameters in PARAM_NAMES order, heads, activation)], equal geometry;
+    caches: [(k, v)] per layer.  Returns the output [T, B, E]."""
+    T, B, E = x.shape
+    ops._require_cuda(x)
+    x = x.contiguous()
+    n = len(layers)
+    F = layers[0][0][8].shape[0]
+    geo = LayerGeometry.of(T, B, E, F, layers[0][1], x.dtype, layers[0][2])
+    row = geo.M * E * geo.es
+    step = (row + 255) // 256 * 256
+    # one allocation: the arena and, from two layers on, the outputs between the layers in turn
+    arena = torch.empty(geo.fwd.total + (2 if n > 2 else n - 1) * step, dtype=torch.uint8, device=x.device)
+    out = torch.empty_like(x)
+    base = arena.data_ptr()
+    image = bytearray(n * _FWD_PACK.size)
+    src = x.data_ptr()
+    for i, (params, _, _) in enumerate(layers):
+        k, v = caches[i]
+        dst = out.data_ptr() if i == n - 1 else base + geo.fwd.total + (i & 1) * step
+        geo.pack_fwd(image, i * _FWD_PACK.size, cache_len, k.shape[1], [p.data_ptr() for p in params], src, k.data_ptr(),
+                     v.data_ptr(), base, dst)
+        src = dst
+    layers_fwd(image, n, x.device)
+    return out

@@ -96,6 +96,26 @@ class AdamDesc(ctypes.Structure):
     ]
 
 
+class LayerDesc(ctypes.Structure):
+    """Mirror of ``tp_layer_desc``."""
+    _fields_ = [(n, c_int32) for n in ("dtype", "T", "batch", "heads", "hidden", "ffn", "activation", "cache_len")] + [
+        ("cache_rows", c_int64), ("w", c_void_p * 12)] + [
+        (n, c_void_p) for n in ("x", "k_cache", "v_cache", "xn", "mean1", "rstd1", "q", "o", "lse", "h", "mean2", "rstd2",
+                                "hn", "a", "z", "out")]
+
+
+class LayerBwdDesc(ctypes.Structure):
+    """Mirror of ``tp_layer_bwd_desc``."""
+    _fields_ = [("f", LayerDesc)] + [
+        (n, c_void_p) for n in ("dout", "dz1", "dhn", "dh", "d_o", "dqkv", "dxn", "dx", "delta", "small_acc", "dk_cache",
+                                "dv_cache")] + [
+        (n, c_int32) for n in ("grad_cache_dtype", "accumulate_prefix", "has_incoming", "zero_slice_rows")] + [
+        ("wg_rows", c_int64)] + [
+        (n, c_void_p) for n in ("wg_dqkv", "wg_xn", "wg_dh", "wg_o", "wg_dz1", "wg_hn", "wg_dout", "wg_a")] + [
+        ("wg_out", c_void_p * 4), ("wg_accumulate", c_int32), ("small_zero", c_int32), ("small_out", c_void_p * 8),
+        ("small_accumulate", c_int32), ("reserved", c_int32)]
+
+
 # every symbol include/terapipe_hip.h declares: name -> (restype, argtypes)
 SYMBOLS = {
     "tp_version": (c_int, []),
@@ -128,6 +148,11 @@ SYMBOLS = {
     "tp_adam_check_table": (c_int, [c_void_p, c_int, c_int]),
     "tp_adam_step": (c_int, [ctypes.POINTER(AdamDesc), c_void_p]),
     "tp_accum_cast": (c_int, [c_void_p, c_void_p, c_int64, c_int, c_int, c_void_p]),
+    "tp_accum_cast_parts": (c_int, [c_void_p, c_void_p, c_int, c_void_p, c_int, c_int, c_void_p]),
+    "tp_layers_fwd_workspace_bytes": (c_size_t, [c_void_p, c_int]),
+    "tp_layers_fwd": (c_int, [c_void_p, c_int, c_void_p, c_size_t, c_void_p]),
+    "tp_layer_bwd_workspace_bytes": (c_size_t, [c_void_p]),
+    "tp_layer_bwd": (c_int, [c_void_p, c_void_p, c_size_t, c_void_p]),
     "tp_colsum_acc": (c_int, [c_void_p, c_int64, c_void_p, c_int, c_int, c_int, c_void_p]),
     "tp_zero_words": (c_int, [c_void_p, c_int64, c_void_p]),
     "tp_fill_probe": (c_int, [c_void_p, c_int64, c_void_p, c_int64, c_int, c_int, c_int, c_int64, c_void_p]),

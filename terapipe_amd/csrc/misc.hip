@@ -27,6 +27,21 @@ __global__ __launch_bounds__(256) void accum_cast_kernel(T* __restrict__ dst, co
     }
 }
 
+struct CastParts { void* dst[8]; int first_block[9]; int size[8]; int first[8]; };
+template <typename T>
+__global__ __launch_bounds__(256) void accum_cast_parts_kernel(CastParts parts, const float* __restrict__ src, int accumulate) {
+    void* dst = parts.dst[0];
+    int first_block = 0, size = parts.size[0], first = 0;
+#pragma unroll
+    for (int i = 1; i < 8; ++i)     // (constant indices only)
+        if ((int)blockIdx.x >= parts.first_block[i]) { dst = parts.dst[i]; first_block = parts.first_block[i]; size = parts.size[i]; first = parts.first[i]; }
+    const int i = ((int)blockIdx.x - first_block) * 256 + threadIdx.x;
+    if (i >= size) return;
+    float v = src[first + i];
+    if (accumulate) v += Elem<T>::to_float(reinterpret_cast<T*>(dst)[i]);
+    reinterpret_cast<T*>(dst)[i] = Elem<T>::from_float(v);
+}
+
 // one thread per column, 32 rows per block; partial sums go to the fp32 accumulators with atomics
 template <typename T>
 __global__ __launch_bounds__(256) void colsum_acc_kernel(const T* __restrict__ x, long ldx, float* acc, int M, int N) {
@@ -116,6 +131,32 @@ extern "C" int tp_accum_cast(void* dst, const float* src, int64_t n, int accumul
     default: accum_cast_kernel<bf16><<<grid, 256, 0, s>>>((bf16*)dst, src, n, accumulate); break;
     }
     return launch_status("tp_accum_cast");
+}
+
+extern "C" int tp_accum_cast_parts(void* const* dst, const int32_t* sizes, int n, const float* src, int accumulate, int dtype,
+                                   void* stream) {
+    using namespace tp;
+    if (!dst || !sizes || !src || n < 1 || n > 8) { set_error("tp_accum_cast_parts: bad argument (n=%d)", n); return TP_ERR_ARG; }
+    if (dtype < TP_F32 || dtype > TP_BF16) { set_error("tp_accum_cast_parts: bad dtype %d", dtype); return TP_ERR_ARG; }
+    CastParts p;
+    int blocks = 0, first = 0;
+    for (int i = 0; i < n; ++i) {
+        if (!dst[i] || sizes[i] <= 0) { set_error("tp_accum_cast_parts: part %d: null pointer or bad size", i); return TP_ERR_ARG; }
+        p.dst[i] = dst[i]; p.size[i] = sizes[i]; p.first[i] = first; p.first_block[i] = blocks;
+        blocks += (sizes[i] + 255) / 256;
+        first += sizes[i];
+    }
+    for (int i = n; i < 8; ++i) { p.dst[i] = p.dst[0]; p.size[i] = 0; p.first[i] = 0; p.first_block[i] = blocks; }
+    p.first_block[8] = blocks;
+    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    switch (dtype) {
+    case TP_F32: accum_cast_parts_kernel<float><<<blocks, 256, 0, s>>>(p, src, accumulate); break;
+    case TP_F16: accum_cast_parts_kernel<f16><<<blocks, 256, 0, s>>>(p, src, accumulate); break;
+    default: accum_cast_parts_kernel<bf16><<<blocks, 256, 0, s>>>(p, src, accumulate); break;
+    }
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) { set_error("tp_accum_cast_parts: launch failed: %s", hipGetErrorString(e)); return TP_ERR_LAUNCH; }
+    return TP_OK;
 }
 
 extern "C" int tp_colsum_acc(const void* x, int64_t ldx, float* acc, int M, int N, int dtype, void* stream) {

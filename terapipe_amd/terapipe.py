@@ -17,7 +17,7 @@ from . import _layer_core as core
 from . import _lib
 from . import ops
 from ._lib import TP_EPI_ACCUMULATE, TP_EPI_STORE, TP_GEMM_TN
-from .transformer_models import ModelParallelTransformerLayer, grid_slice_batch_and_sequence
+from .transformer_models import ModelParallelTransformerLayer, _check_cache, grid_slice_batch_and_sequence
 
 
 def loss_func(y):
@@ -64,12 +64,25 @@ class TransformerLayers(nn.Module):
         return cache
 
     def forward(self, x, cache, cache_len):
+        if not torch.is_grad_enabled() and self.n_layers:
+            return self._forward_only(x, cache, cache_len), list(cache[:2 * self.n_layers])
         cache_outputs = []
         for layer_id in range(self.n_layers):
             k_input, v_input = cache[2 * layer_id], cache[2 * layer_id + 1]
             x, (k_output, v_output) = self.layers[layer_id](x, (k_input, v_input), cache_len)
             cache_outputs += [k_output, v_output]
         return x, cache_outputs
+
+    def _forward_only(self, x, cache, cache_len):
+        """All layers as one library call (evaluation, generation: no backward follows)."""
+        T, B, E = x.shape
+        assert E == self.embedding_dim
+        stack, caches = [], []
+        for i, layer in enumerate(self.layers):
+            attn = layer._modules["attn"]
+            caches.append(_check_cache((cache[2 * i], cache[2 * i + 1]), B, attn.num_heads, attn.head_dim, cache_len + T, x.dtype))
+            stack.append((layer.param_list(), attn.num_heads, layer.activation))
+        return core.stack_forward_only(stack, x, caches, cache_len)
 
     def create_inputs(self, batch_size, seq_len, device="cuda", random=False):
         fn = torch.randn if random else torch.empty
@@ -787,6 +800,5 @@ class TeraPipe(nn.Module):
         assert inputs.size(self.sequence_dim) == self.seq_len and inputs.size(self.batch_dim) == self.batch_size
         flat = []
         for layer in self.layers.layers:
-            p = layer.param_dict()
-            flat += [p[n] for n in core.PARAM_NAMES]
+            flat += layer.param_list()
         return _TeraPipeFunction.apply(self, inputs, *flat)

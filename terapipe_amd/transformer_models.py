@@ -9,6 +9,7 @@ a separate _AssignCache op, with the same in-place, alias-returning semantics an
 contract (reference transformer_models.py:177-193).
 """
 import warnings
+import weakref
 
 import numpy as np
 import torch
@@ -188,53 +189,123 @@ def _grads_can_go_in_place(w):
     return True
 
 
+def _engine_adds_to_grad(ctx, w, first):
+    """Whether the backward pass under way is going to add this node's gradients to the parameters' .grad and nobody looks
+    at them on the way: then the kernels can add them.  ctx.next_functions[first:] are the parameters' AccumulateGrad
+    nodes; under torch.autograd.grad they do not run (the query raises for captured leaves), and a hook on a parameter or
+    a graph of the backward itself (create_graph) needs the gradients as tensors."""
+    if torch.is_grad_enabled():
+        return False
+    nodes = ctx.next_functions[first:]
+    try:
+        for p, (node, _) in zip(w.values(), nodes):
+            if p._backward_hooks or getattr(p, "_post_accumulate_grad_hooks", None) or getattr(node, "variable", None) is not p \
+                    or not torch._C._will_engine_execute_node(node):
+                return False
+    except RuntimeError:
+        return False
+    return True
+
+
 class _GradOptions:
     """How a layer's backward hands its parameter gradients to autograd (TransformerLayer's two switches) and,
-    for deferred weight gradients, the sequences whose backward is under way (keyed by their K cache)."""
-    __slots__ = ("in_place", "defer", "pending")
+    for deferred weight gradients, the sequences under way (keyed by their K cache): the rows their forward has filled
+    and the gradients of those whose backward runs."""
+    __slots__ = ("in_place", "defer", "pending", "inputs")
 
     def __init__(self):
         self.in_place, self.defer, self.pending = False, False, {}
+        self.inputs = weakref.WeakValueDictionary()     # the slices' graphs own them
 
 
-class _PendingGrads:
-    """Deferred weight gradients of one sequence in one layer: the output gradients and inputs of the four
-    linears for every position whose slice has run its backward (rows [low, rows); the reverse-slice order
-    fills them from the end), and the fp32 sums of the vector-parameter gradients so far."""
-    __slots__ = ("rows", "low", "dqkv", "dh", "dz1", "dout", "xn", "o", "hn", "a", "acc")
+class _SequenceInputs:
+    """Deferred weight gradients: the inputs of the four linears of one sequence in one layer, position-indexed; the
+    forward of a slice writes its rows (the next slice starts at `rows`)."""
+    __slots__ = ("rows", "xn", "o", "hn", "a", "__weakref__")
 
     def __init__(self, rows, E, F, dtype, device):
         new = lambda n: torch.empty(rows, n, dtype=dtype, device=device)
-        self.rows = self.low = rows
-        self.dqkv, self.dh, self.dz1, self.dout = new(3 * E), new(E), new(F), new(E)
+        self.rows = 0
         self.xn, self.o, self.hn, self.a = new(E), new(E), new(E), new(F)
-        self.acc = torch.zeros(core.small_acc_numel(E, F), dtype=torch.float32, device=device)
+
+
+class _PendingGrads:
+    """Deferred weight gradients of one sequence in one layer: the output gradients of the four linears for every
+    position whose slice has run its backward (rows [low, rows); the reverse-slice order fills them from the end), and
+    the fp32 sums of the vector-parameter gradients so far."""
+    __slots__ = ("rows", "low", "inputs", "dqkv", "dh", "dz1", "dout", "acc")
+
+    def __init__(self, rows, inputs, E, F, dtype, device):
+        new = lambda n: torch.empty(rows, n, dtype=dtype, device=device)
+        self.rows = self.low = rows
+        self.inputs = inputs
+        self.dqkv, self.dh, self.dz1, self.dout = new(3 * E), new(E), new(F), new(E)
+        self.acc = torch.empty(core.small_acc_numel(E, F), dtype=torch.float32, device=device)
+
+
+class _SliceKept:
+    """The forward's kept activations as tensors, for whoever inspects a graph (the kernels work on addresses)."""
+    __slots__ = ("geo", "arena", "seq", "cache_len")
+
+    def __init__(self, geo, arena, seq, cache_len):
+        self.geo, self.arena, self.seq, self.cache_len = geo, arena, seq, cache_len
+
+    @property
+    def a(self):
+        g = self.geo
+        if self.seq is not None:
+            return self.seq.a[self.cache_len * g.B:self.cache_len * g.B + g.M]
+        at = g.fwd.off["a"]
+        return self.arena[at:at + g.M * g.F * g.es].view(g.dtype).view(g.M, g.F)
 
 
 class _LayerFunction(torch.autograd.Function):
     """One whole layer over one slice.  Inputs: x, k_cache, v_cache (or None, None), then the 12
     parameters in core.PARAM_NAMES order.  Outputs: out, and the two caches when given.
 
-    Backward of a slice: the data gradients (core.layer_bwd), then the four weight gradients as one grouped
-    library call and the eight vector-parameter gradients as one launch.  opts (_GradOptions):
-    in_place -- where every parameter already has a .grad, add the gradients to it inside those launches (the
-    GEMM's accumulate epilogue, one rounding) and hand autograd None, instead of returning twelve tensors that
-    autograd adds to .grad one elementwise kernel each;
-    defer -- keep the slice's dY / X rows and take the weight gradients once per sequence, over all its rows, in
-    the backward of the slice at position 0 (the last one the reverse-slice order reaches); the slices before
-    it hand autograd None for the parameters."""
+    Forward and backward are one library call each (tp_layers_fwd, tp_layer_bwd).  The backward of a slice: the data
+    gradients, the eight vector-parameter gradients as one launch, the four weight gradients as one grouped one.
+    Where every parameter already has a .grad that the engine is going to add to (_engine_adds_to_grad), or with
+    opts.in_place, the kernels add the gradients to it (the GEMM's accumulate epilogue, one rounding) and autograd gets
+    None, instead of twelve tensors that autograd adds one elementwise kernel each.  opts.defer -- keep the slice's dY / X
+    rows and take the weight gradients once per sequence, over all its rows, in the backward of the slice at position 0
+    (the last one the reverse-slice order reaches); the slices before it hand autograd None for the parameters."""
 
     @staticmethod
     def forward(ctx, heads, cache_len, activation, opts, x, k_cache, v_cache, *params):
-        w = dict(zip(core.PARAM_NAMES, params))
         T, B, E = x.shape
-        Dh = E // heads
+        ops._require_cuda(x, *params)
+        dt, dev = x.dtype, x.device
+        F = params[8].shape[0]
         ctx.has_cache = k_cache is not None
         if not ctx.has_cache:
-            k_cache, v_cache = _temp_cache(B, heads, T, Dh, x)
-        out, st = core.layer_fwd(w, x.contiguous(), heads, k_cache, v_cache, cache_len, activation)
-        ctx.st, ctx.w, ctx.heads, ctx.activation = st, w, heads, activation
-        ctx.opts = opts
+            k_cache, v_cache = _temp_cache(B, heads, T, E // heads, x)
+        x = x.contiguous()
+        geo = core.LayerGeometry.of(T, B, E, F, heads, dt, activation)
+        arena = torch.empty(geo.fwd.total, dtype=torch.uint8, device=dev)
+        out = torch.empty(T, B, E, dtype=dt, device=dev)
+        seq, over = None, None
+        if opts.defer and ctx.has_cache:
+            # the slice's rows of the sequence's buffers; a slice that does not continue a sequence starts one
+            r0, r1 = cache_len * B, (cache_len + T) * B
+            key = k_cache.data_ptr()
+            seq = opts.inputs.get(key)
+            if seq is None or cache_len == 0 or seq.rows != r0 or seq.xn.shape[0] < r1:
+                seq = None
+                if cache_len == 0:
+                    seq = opts.inputs[key] = _SequenceInputs(k_cache.shape[1] * B, E, F, dt, dev)
+            if seq is not None:
+                seq.rows = r1
+                over = {n: getattr(seq, n)[r0:].data_ptr() for n in ("xn", "o", "hn", "a")}
+        image = bytearray(core._FWD_PACK.size + core._BWD_PACK.size)
+        geo.pack_fwd(image, 0, cache_len, k_cache.shape[1], [p.data_ptr() for p in params], x.data_ptr(),
+                     k_cache.data_ptr(), v_cache.data_ptr(), arena.data_ptr(), out.data_ptr(), over)
+        core.layers_fwd(image, 1, dev)
+        ctx.geo, ctx.cache_len, ctx.opts = geo, cache_len, opts
+        ctx.image = image               # the descriptor's addresses stay valid: what they point to is kept
+        ctx.kept = (x, k_cache, v_cache, arena, seq)
+        ctx.st = _SliceKept(geo, arena, seq, cache_len)
+        ctx.w = params
         ctx.set_materialize_grads(False)
         if ctx.has_cache:
             # the caches were written through their raw pointers (as `cache.data[index] = value` does,
@@ -244,11 +315,13 @@ class _LayerFunction(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, dout, dk_out=None, dv_out=None):
-        st, w, heads, opts = ctx.st, ctx.w, ctx.heads, ctx.opts
-        E = st.x.shape[1]
-        F = w["fc1.weight"].shape[0]
+        geo, opts, cache_len = ctx.geo, ctx.opts, ctx.cache_len
+        x, k_cache, v_cache, arena, seq = ctx.kept
+        w = dict(zip(core.PARAM_NAMES, ctx.w))
+        T, B, E, F, M, dt, dev = geo.T, geo.B, geo.E, geo.F, geo.M, geo.dtype, x.device
         if dout is None:
-            dout = torch.zeros(st.T, st.B, E, dtype=st.x.dtype, device=st.x.device)
+            dout = torch.zeros(T, B, E, dtype=dt, device=dev)
+        dout = dout.contiguous()
         gk = gv = None
         has_incoming = False
         if ctx.has_cache:
@@ -257,70 +330,74 @@ class _LayerFunction(torch.autograd.Function):
                 gk, gv = dk_out.clone(), (dv_out.clone() if dv_out is not None else torch.zeros_like(dk_out))
                 has_incoming = True
             else:
-                gk, gv = torch.zeros_like(st.k_cache), torch.zeros_like(st.v_cache)
-        M, dt, dev = st.T * st.B, st.x.dtype, dout.device
-        dout = dout.contiguous()
-        dout2d = dout.view(M, E)
-        new = lambda n: torch.empty(M, n, dtype=dt, device=dev)
-        pend = None
-        if opts.defer and ctx.has_cache:
+                both = torch.zeros((2,) + k_cache.shape, dtype=dt, device=dev)
+                gk, gv = both[0], both[1]
+        buf = torch.empty(geo.bwd.total, dtype=torch.uint8, device=dev)
+        dx = torch.empty(T, B, E, dtype=dt, device=dev)
+        base, off = buf.data_ptr(), geo.bwd.off
+        p = {n: base + off[n] for n in off}
+        fo, fbase = geo.fwd.off, arena.data_ptr()
+        # addresses of the four linears' inputs over the rows of the weight-gradient products
+        xs = {n: fbase + fo[n] for n in ("xn", "o", "hn", "a")}
+        rows, dy = M, dout.data_ptr()
+        pend, done, fresh = None, True, True
+        if opts.defer and ctx.has_cache and (seq is not None or cache_len == 0):
             # rows [r0, r1) of the sequence's position-indexed gradient buffers
-            r0, r1 = st.cache_len * st.B, (st.cache_len + st.T) * st.B
-            key = st.k_cache.data_ptr()
+            r0, r1 = cache_len * B, (cache_len + T) * B
+            key = k_cache.data_ptr()
             pend = opts.pending.get(key)
-            if pend is None or pend.low != r1:
+            if pend is None or pend.low != r1 or pend.inputs is not seq:
                 # the last slice of a sequence opens it; an entry that does not end where this slice begins belongs
                 # to a sequence whose backward was abandoned or skipped a slice
                 if pend is not None and pend.low < pend.rows:
                     warnings.warn("defer_weight_grads: the backward of a sequence stopped at row %d and never reached "
                                   "its first slice; its weight gradients are dropped" % pend.low)
-                pend = opts.pending[key] = _PendingGrads(r1, E, F, dt, dev)
-            buf = core.Bufs(dz1=pend.dz1[r0:r1], dhn=new(E), dh=pend.dh[r0:r1], dqkv=pend.dqkv[r0:r1], dxn=new(E))
-        else:
-            buf = core.Bufs(dz1=new(F), dhn=new(E), dh=new(E), dqkv=new(3 * E), dxn=new(E))
-        dx = core.layer_bwd(w, st, dout, heads, gk, gv, accumulate_prefix=True, has_incoming=has_incoming,
-                            zero_slice_rows=has_incoming, activation=ctx.activation, buf=buf)
-        acc = pend.acc if pend is not None else torch.zeros(core.small_acc_numel(E, F), dtype=torch.float32,
-                                                            device=dev)
-        sv = core.small_acc_views(acc, E, F)
-        ops.vec_param_grads([(buf.dqkv, sv["attn.in_proj.bias"]),
-                             (buf.dh, sv["attn.out_proj.bias"]),
-                             (buf.dz1, sv["fc1.bias"]),
-                             (dout2d, sv["fc2.bias"]),
-                             (buf.dxn, st.x, st.mean1, st.rstd1, sv["attn_ln.weight"], sv["attn_ln.bias"]),
-                             (buf.dhn, st.h, st.mean2, st.rstd2, sv["fc_ln.weight"], sv["fc_ln.bias"])])
-        ctx.st = None
-        no_param_grads = (None, None, None, None, dx, gk, gv) + (None,) * len(core.PARAM_NAMES)
-        if pend is not None:
-            pend.dout[r0:r1].copy_(dout2d)
-            pend.xn[r0:r1].copy_(st.xn)
-            pend.o[r0:r1].copy_(st.o.view(M, E))
-            pend.hn[r0:r1].copy_(st.hn)
-            pend.a[r0:r1].copy_(st.a)
+                pend = opts.pending[key] = _PendingGrads(r1, seq, E, F, dt, dev)
+            else:
+                fresh = False
+            p["dz1"], p["dh"], p["dqkv"] = (t[r0:].data_ptr() for t in (pend.dz1, pend.dh, pend.dqkv))
+            p["small"] = pend.acc.data_ptr()
+            if r1 - r0 < pend.rows:
+                pend.dout[r0:r1].copy_(dout.view(M, E))
+            else:
+                pend.dout = dout                # the whole sequence in one slice
             pend.low = r0
-            if r0 > 0:
-                return no_param_grads
-            del opts.pending[key]
-            K = pend.rows
-            pairs = ((pend.dqkv, pend.xn), (pend.dh, pend.o), (pend.dz1, pend.hn), (pend.dout, pend.a))
-        else:
-            K = M
-            pairs = ((buf.dqkv, st.xn), (buf.dh, st.o.view(M, E)), (buf.dz1, st.hn), (dout2d, st.a))
-        in_place = opts.in_place and _grads_can_go_in_place(w)
-        epi = TP_EPI_ACCUMULATE if in_place else TP_EPI_STORE
-        wgrad = {n: (w[n].grad if in_place else torch.empty_like(w[n])) for n in core.BIG_PARAMS}
-        ops.gemm_grouped([(TP_GEMM_TN, dy, xin, wgrad[n].shape[0], wgrad[n].shape[1], K, wgrad[n], epi)
-                          for n, (dy, xin) in zip(("attn.in_proj.weight", "attn.out_proj.weight", "fc1.weight",
-                                                   "fc2.weight"), pairs)])
-        if in_place:
-            for n in core.SMALL_PARAMS:
-                ops.accum_cast(w[n].grad, sv[n], True)
-            return no_param_grads
-        flat = torch.empty(acc.numel(), dtype=dt, device=dev)
-        ops.accum_cast(flat, acc, False)
-        grads = core.small_acc_views(flat, E, F)
-        grads.update(wgrad)
-        return no_param_grads[:7] + tuple(grads[n] for n in core.PARAM_NAMES)
+            done = r0 == 0
+            if done:
+                del opts.pending[key]
+                if opts.inputs.get(key) is seq:
+                    del opts.inputs[key]
+                rows = pend.rows
+        in_place = done and (opts.in_place or _engine_adds_to_grad(ctx, w, 3 if ctx.has_cache else 1)) \
+            and _grads_can_go_in_place(w)
+        wg_out, small_out, wg = (0,) * 4, (0,) * 8, (0,) * 8
+        grads = {}
+        if done:
+            if in_place:
+                grads = {n: t.grad for n, t in w.items()}
+            else:
+                flat = torch.empty(geo.n_small, dtype=dt, device=dev)
+                grads = core.small_acc_views(flat, E, F)
+                for n in core.BIG_PARAMS:
+                    grads[n] = torch.empty_like(w[n])
+            wg_out = tuple(grads[n].data_ptr() for n in core.BIG_PARAMS)
+            small_out = tuple(grads[n].data_ptr() for n in core.SMALL_PARAMS)
+            if pend is not None:
+                s = pend.inputs
+                wg = (pend.dqkv.data_ptr(), s.xn.data_ptr(), pend.dh.data_ptr(), s.o.data_ptr(), pend.dz1.data_ptr(),
+                      s.hn.data_ptr(), pend.dout.data_ptr(), s.a.data_ptr())
+            else:
+                wg = (p["dqkv"], xs["xn"], p["dh"], xs["o"], p["dz1"], xs["hn"], dy, xs["a"])
+        core._BWD_PACK.pack_into(ctx.image, core._FWD_PACK.size, dy, p["dz1"], p["dhn"], p["dh"], p["d_o"], p["dqkv"],
+                                 p["dxn"], dx.data_ptr(), p["delta"], p["small"],
+                                 0 if gk is None else gk.data_ptr(), 0 if gv is None else gv.data_ptr(),
+                                 geo.dt, 1, int(has_incoming), int(has_incoming), rows if done else 0, *wg, *wg_out,
+                                 int(in_place), int(fresh), *small_out, int(in_place), 0)
+        core.layer_bwd_native(ctx.image, dev)
+        ctx.kept = ctx.image = ctx.w = ctx.st = None
+        if not done or in_place:
+            return (None, None, None, None, dx, gk, gv) + (None,) * len(core.PARAM_NAMES)
+        return (None, None, None, None, dx, gk, gv) + tuple(grads[n] for n in core.PARAM_NAMES)
 
 
 class _AttentionFunction(torch.autograd.Function):
@@ -453,28 +530,43 @@ class TransformerLayer(nn.Module):
         self.fc1 = ColumnParallelLinear(embedding_dim, ffn_embedding_dim, gather_output=False, device=device)
         self.fc2 = RowParallelLinear(ffn_embedding_dim, embedding_dim, input_is_parallel=True, device=device)
 
+    def param_list(self):
+        """The 12 parameter tensors in core.PARAM_NAMES order."""
+        try:
+            # (straight from the modules' dictionaries: attribute look-ups through nn.Module cost as much as a launch)
+            m = self._modules
+            attn = m["attn"]._modules
+            lin, out, fc1, fc2 = (t._parameters for t in (attn["in_proj"], attn["out_proj"], m["fc1"], m["fc2"]))
+            ln1, ln2 = m["attn_ln"]._parameters, m["fc_ln"]._parameters
+            return [ln1["weight"], ln1["bias"], lin["weight"], lin["bias"], out["weight"], out["bias"], ln2["weight"],
+                    ln2["bias"], fc1["weight"], fc1["bias"], fc2["weight"], fc2["bias"]]
+        except KeyError:        # a parametrized module computes its weight
+            return [self.attn_ln.weight, self.attn_ln.bias, self.attn.in_proj.weight, self.attn.in_proj.bias,
+                    self.attn.out_proj.weight, self.attn.out_proj.bias, self.fc_ln.weight, self.fc_ln.bias,
+                    self.fc1.weight, self.fc1.bias, self.fc2.weight, self.fc2.bias]
+
     def param_dict(self):
         """The 12 parameter tensors keyed by their state-dict names."""
-        return {"attn_ln.weight": self.attn_ln.weight, "attn_ln.bias": self.attn_ln.bias,
-                "attn.in_proj.weight": self.attn.in_proj.weight, "attn.in_proj.bias": self.attn.in_proj.bias,
-                "attn.out_proj.weight": self.attn.out_proj.weight, "attn.out_proj.bias": self.attn.out_proj.bias,
-                "fc_ln.weight": self.fc_ln.weight, "fc_ln.bias": self.fc_ln.bias,
-                "fc1.weight": self.fc1.weight, "fc1.bias": self.fc1.bias,
-                "fc2.weight": self.fc2.weight, "fc2.bias": self.fc2.bias}
+        return dict(zip(core.PARAM_NAMES, self.param_list()))
 
     def forward(self, x, full_cache=None, cache_len=0):
-        tgt_len, bsz, embed_dim = x.size()
-        assert embed_dim == self.attn.embed_dim
+        tgt_len, bsz, embed_dim = x.shape
+        attn = self._modules["attn"]
+        assert embed_dim == attn.embed_dim
         k = v = None
         if full_cache is not None:
-            k, v = _check_cache(full_cache, bsz, self.attn.num_heads, self.attn.head_dim, cache_len + tgt_len, x.dtype)
+            k, v = _check_cache(full_cache, bsz, attn.num_heads, attn.head_dim, cache_len + tgt_len, x.dtype)
         else:
             assert cache_len == 0
-        p = self.param_dict()
+        params = self.param_list()
+        if not torch.is_grad_enabled():
+            # nothing to keep for a backward
+            kv = (k, v) if k is not None else _temp_cache(bsz, attn.num_heads, tgt_len, attn.head_dim, x)
+            out = core.stack_forward_only([(params, attn.num_heads, self.activation)], x, [kv], cache_len)
+            return out, None if k is None else (k, v)
         opts = self._grad_options
         opts.in_place, opts.defer = bool(self.accumulate_grads_in_place), bool(self.defer_weight_grads)
-        res = _LayerFunction.apply(self.attn.num_heads, cache_len, self.activation, opts,
-                                   x, k, v, *[p[n] for n in core.PARAM_NAMES])
+        res = _LayerFunction.apply(attn.num_heads, cache_len, self.activation, opts, x, k, v, *params)
         if full_cache is not None:
             return res[0], (res[1], res[2])
         return res, None
