@@ -542,6 +542,7 @@ static bool tile_cfg(int id, TileCfg& c) {
 }
 static constexpr int kFirstStreamCfg = 21, kLastStreamCfg = 40;
 static constexpr int kWideCfg = 44;
+static constexpr int kSkinnyRows = 32;
 
 // Measured plans: for NT / NN the weight extents (N, K) match exactly and M (tokens of the slice) picks the
 // nearest measured M at or above it (at least half of it, so that a much shorter slice falls through to the
@@ -685,8 +686,12 @@ static GemmPlan plan_gemm(const tp_gemm_desc* d) {
             else { cfg = 8; ns = splits_for(t64, 2048); }
         } else if (small_weight) {
             // 64 x 64 tiles reach the CU count without splitting k
-            cfg = (d->M <= 256 && d->K % 128 == 0) ? 12 : 8;
+            // (more than one per CU of a k-tile of 64: 64 x 64 x 64 up to two, the pipelined 128 x 128 tile beyond and on a
+            // longer k: 512 x 4800 x 1600 25.4 -> 14.5 us, 256 x 5120 x 1280 16.1 -> 11.1; 512 x 1600 x 6400 34.7 -> 27.4)
+            cfg = (d->M <= 256 && d->K % 128 == 0 && t64 <= kNumCU) ? 12 : 8;
             ns = t64 >= 96 ? 1 : splits_for(t64, 2048);
+            if (t64 > 2 * kNumCU || (t64 > kNumCU && d->K >= 1536)) cfg = 16;
+            else if (d->M > 256 && d->K >= 6144) { cfg = 16; ns = splits_for(t128, 1536); }
         } else if (d->M <= 128) {
             const int ns13 = splits_for(t128, 1536);
             if (t128 > kNumCU) { cfg = 3; ns = splits_for(t3, 2048); }                      // many column tiles: 128 x 256
@@ -782,10 +787,20 @@ static void launch_cfg(const GemmPlan& p, const GemmArgs& a, hipStream_t s) {
     }
 }
 
+// Forward products of up to kSkinnyRows rows on a weight of up to 4096 x 4096 run without LDS tiles: the plan's k splits,
+// whatever its tile.  (Beyond, both are bound by the weight stream and the tile kernels read the activation less often:
+// 16 rows on 20480 x 5120 37 us against 45.  A forced tile, and column sums, take the tile kernels.)
+static inline bool runs_skinny(const tp_gemm_desc* d) {
+    return d->op == TP_GEMM_NT && d->dtype != TP_F32 && d->M <= kSkinnyRows && (long)d->N * d->K <= (16L << 20) &&
+           (d->reserved & 0xff) == 0 && !d->colsum_acc;
+}
+
 // false: the plan names a (tile configuration, op, dtype) that no kernel is built for -- nothing was launched
 template <typename T>
 static bool launch_gemm(const tp_gemm_desc* d, const GemmPlan& p, const GemmArgs& a, hipStream_t s) {
-    if (p.cfg >= kFirstStreamCfg && p.cfg <= kLastStreamCfg) {
+    if (runs_skinny(d)) {
+        launch_gemm_skinny(d->dtype, a, s);
+    } else if (p.cfg >= kFirstStreamCfg && p.cfg <= kLastStreamCfg) {
         if (!launch_gemm_stream(p.cfg, d->op, d->dtype, dim3(p.gx, p.gy, p.nsplit), a, s)) return false;
     } else if (is_pipe_cfg(p.cfg) && d->dtype != TP_F32) {
         if (!launch_gemm_pipe(p.cfg, d->op, d->dtype, dim3(p.gx, p.gy, p.nsplit), a, s)) return false;

@@ -155,6 +155,8 @@ __device__ __forceinline__ void xcd_tile3(int t, int tx, int ty, int tz, int& ti
 bool launch_gemm_pipe(int cfg, int op, int dtype, dim3 grid, const GemmArgs& a, hipStream_t s);
 // A grouped launch (TN, token-major operands) of `tiles` workgroups on the pipelined 256 x 128 (15) or 128 x 128 (16) tile.
 bool launch_gemm_pipe_group(int cfg, int dtype, int tiles, const GemmGroupArgs& ga, hipStream_t s);
+// Products of up to 32 rows (gemm_skinny.hip; NT, 16-bit): whole k ranges per workgroup, k splits as the arguments say.
+void launch_gemm_skinny(int dtype, const GemmArgs& a, hipStream_t s);
 // The eight-wave 256 x 256 tile of gemm_wide.hip (tile configuration 44; NT and NN).
 bool launch_gemm_wide(int op, int dtype, dim3 grid, const GemmArgs& a, hipStream_t s);
 

@@ -52,3 +52,13 @@ def test_ragged_k_split(op):
     """A last split that is shorter than a k-tile."""
     _run(op, 600, 800, 1024 + 40, torch.bfloat16, ksplit=None)
     _run(op, 2048, 1024, 8192 + 24, torch.float16)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(1, 8, 8), (1, 2048, 2048), (5, 24, 264), (16, 1000, 2056), (17, 4096, 1024), (31, 520, 5128),
+                                   (4, 2048, 8192), (3, 15360, 1032), (32, 16, 40)], ids=str)
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=str)
+def test_few_rows(M, N, K, dtype):
+    """The kernel for up to 32 rows: one, two and four weight tiles per workgroup, a short last one, k tails, k splits."""
+    _run("NT", M, N, K, dtype)
+    _run("NT", M, N, K, dtype, None, 3 if K >= 192 else 1)
