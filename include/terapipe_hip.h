@@ -239,10 +239,10 @@ int tp_attn_prefix_bwd(const tp_attn_desc* d, void* workspace, size_t workspace_
  * Query position t in [key_begin, q_end) sees key position s <= t.  Writes the k and v parts of dqkv. */
 typedef struct tp_attn_suffix_desc {
     int32_t dtype;                      /* TP_F16 or TP_BF16 */
-    int32_t batch, heads, head_dim;     /* head_dim 64 or 128 */
+    int32_t batch, heads, head_dim;     /* head_dim 64 or 128, with odd_head_dims also 80 or 96 */
     int32_t key_begin, key_count;       /* P, T of the slice whose keys these are */
     int32_t q_end;                      /* queries [key_begin, q_end) take part */
-    int32_t reserved;
+    int32_t odd_head_dims;              /* nonzero: 80 and 96 are taken as well (0 refuses them, as a zeroed descriptor did) */
     int64_t cache_rows;                 /* rows per (b,h) of k_cache, v_cache */
     int64_t q_bh_rows;                  /* rows per (b,h) of q_all */
     int64_t stat_bh_rows;               /* entries per (b,h) of lse_all, delta_all */

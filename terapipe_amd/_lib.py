@@ -64,7 +64,7 @@ class AttnSuffixDesc(ctypes.Structure):
     """Mirror of ``tp_attn_suffix_desc``."""
     _fields_ = [
         ("dtype", c_int32), ("batch", c_int32), ("heads", c_int32), ("head_dim", c_int32),
-        ("key_begin", c_int32), ("key_count", c_int32), ("q_end", c_int32), ("reserved", c_int32),
+        ("key_begin", c_int32), ("key_count", c_int32), ("q_end", c_int32), ("odd_head_dims", c_int32),
         ("cache_rows", c_int64), ("q_bh_rows", c_int64), ("stat_bh_rows", c_int64),
         ("k_cache", c_void_p), ("v_cache", c_void_p),
         ("q_all", c_void_p), ("d_o_all", c_void_p),

@@ -505,13 +505,41 @@ static inline unsigned xcd_grid(int BH, int nblocks) { return 8u * ((BH + 7) / 8
 
 // ---- shared pieces of the second-generation 16-bit attention kernels -------------------------------
 
+// LDS tiles of these kernels have rows of 64 or 128 elements (the swizzle's power of two).  Head dimensions between (80,
+// 96) take rows of 128 whose last chunks are never loaded: their products run over the dimension's own k-steps of 16,
+// and the output blocks of 32 columns may end past it (columns 80 to 95 of a head of 80 are computed on whatever the
+// LDS holds there and not stored).
+template <int DH> __host__ __device__ constexpr int tile_pitch() { return DH <= 64 ? 64 : 128; }
+constexpr unsigned kNoChunk = 0xffffffffu;      // a lane whose chunk of the tile row lies past the head dimension
+template <int DH> __device__ __forceinline__ void load_chunk_lds(unsigned off, const void* base, unsigned lds_wave_base) {
+    if (DH == tile_pitch<DH>() || off != kNoChunk) dma16_saddr_lds(off, base, lds_wave_base);
+}
+
+// Adds the NW waves' [32][DH] blocks that acc_to_lds_rows left one behind the other, four columns a thread and turn
+// (consecutive threads along a row), and hands f(row, column, sum) each piece.
+template <int DH, int NW, typename F> __device__ __forceinline__ void sum_rows(const float* ebuf, int tid, F&& f) {
+    constexpr int LD = (DH + 31) / 32 * 32 + 4, PIECES = 32 * DH / 4, NT = NW * 64;
+#pragma unroll
+    for (int p0 = 0; p0 < PIECES; p0 += NT) {
+        const int p = p0 + tid, row = p / (DH / 4), col = (p % (DH / 4)) * 4;
+        if (PIECES % NT != 0 && p >= PIECES) break;
+        float4 acc = make_float4(0.f, 0.f, 0.f, 0.f);
+#pragma unroll
+        for (int w = 0; w < NW; ++w) {
+            const float4 v = *reinterpret_cast<const float4*>(ebuf + (w * 32 + row) * LD + col);
+            acc.x += v.x; acc.y += v.y; acc.z += v.z; acc.w += v.w;
+        }
+        f(row, col, acc);
+    }
+}
+
 // Wave-private transpose of a [DH x 32] fp32 accumulator set (register j of block db = row db*32 +
 // acc_row(j, g), column lane & 31) into row-major [32][DH] through LDS, so that global memory is then
 // touched in full rows.  `buf` is the wave's own 32 x (DH + 4) floats.  After the call lane l holds, for
 // i in [0, DH / 8): row 2 * i' ... see rows_read.
 template <int DH>
 __device__ __forceinline__ void acc_to_lds_rows(const float16v* acc, float* buf, int lane) {
-    constexpr int NDB = DH / 32, LD = DH + 4;
+    constexpr int NDB = (DH + 31) / 32, LD = NDB * 32 + 4;
     const int g = lane >> 5, li = lane & 31;
 #pragma unroll
     for (int db = 0; db < NDB; ++db)
@@ -534,15 +562,15 @@ template <typename T, typename GT, int DH, int NW, int STAGES>
 __global__ __launch_bounds__(NW * 64) void attn_bwd_dkdv2_kernel(AttnArgs a) {
     typedef Elem<T> E;
     static_assert(sizeof(T) == 2, "direct-to-LDS kernels are for fp16 / bf16");
-    constexpr int NDB = DH / 32, NKS = DH / 16;
-    constexpr int TILE = 32 * DH;                       // elements of one Q or dO tile
-    constexpr int CPR = DH / 8;                         // 16-byte chunks per row
+    constexpr int NDB = (DH + 31) / 32, NKS = DH / 16, PITCH = tile_pitch<DH>();
+    constexpr int TILE = 32 * PITCH;                       // elements of one Q or dO tile
+    constexpr int CPR = PITCH / 8;                         // 16-byte chunks per row
     constexpr int NLD = 32 * CPR / (NW * 64);           // loads per thread per tile
     static_assert(32 * CPR % (NW * 64) == 0, "tile must split evenly");
     constexpr int NLOAD = 2 * NLD;
     static_assert(NLOAD * (STAGES - 1) <= 63, "too many loads in flight for vmcnt");
     constexpr int RING_BYTES = STAGES * 2 * TILE * 2;
-    constexpr int EPI_LD = DH + 4;
+    constexpr int EPI_LD = NDB * 32 + 4;
     constexpr int EPI_BYTES = NW * 32 * EPI_LD * 4;
     constexpr int SMEM = RING_BYTES > EPI_BYTES ? RING_BYTES : EPI_BYTES;
     __shared__ __attribute__((aligned(16))) unsigned char smem[SMEM];
@@ -577,13 +605,13 @@ __global__ __launch_bounds__(NW * 64) void attn_bwd_dkdv2_kernel(AttnArgs a) {
     // compile-time offsets from these)
     const T* pkm[NKS];
 #pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) pkm[ks] = ring + km_offset<T, DH>(li, ks * 16, lane);
+    for (int ks = 0; ks < NKS; ++ks) pkm[ks] = ring + km_offset<T, PITCH>(li, ks * 16, lane);
     const T* ptr0[NDB];
     const T* ptr1[NDB];
 #pragma unroll
     for (int db = 0; db < NDB; ++db) {
         int o0, o1;
-        tr_offsets<T, DH, true>(0, db * 32, lane, o0, o1);
+        tr_offsets<T, PITCH, true>(0, db * 32, lane, o0, o1);
         ptr0[db] = ring + o0;
         ptr1[db] = ring + o1;
     }
@@ -593,9 +621,9 @@ __global__ __launch_bounds__(NW * 64) void attn_bwd_dkdv2_kernel(AttnArgs a) {
 #pragma unroll
     for (int i = 0; i < NLD; ++i) {
         const int p = (i * NW + wave) * 64 + lane;
-        const int r = p / CPR, lc = (p % CPR) ^ swz16<DH>(r);
-        qoff[i] = (unsigned)(r * DH * 2 + lc * 16);
-        dooff[i] = (unsigned)(r * ldo_bytes + lc * 16);
+        const int r = p / CPR, lc = (p % CPR) ^ swz16<PITCH>(r);
+        qoff[i] = lc < DH / 8 ? (unsigned)(r * DH * 2 + lc * 16) : kNoChunk;
+        dooff[i] = lc < DH / 8 ? (unsigned)(r * ldo_bytes + lc * 16) : kNoChunk;
     }
     const char* Qb = uniform_ptr(reinterpret_cast<const char*>(reinterpret_cast<const T*>(a.q) + (long)bh * a.q_bhs));
     const char* dOb = uniform_ptr(reinterpret_cast<const char*>(reinterpret_cast<const T*>(a.d_o) + (long)b * EE + (long)h * DH));
@@ -613,24 +641,24 @@ __global__ __launch_bounds__(NW * 64) void attn_bwd_dkdv2_kernel(AttnArgs a) {
             const char* sq = Qb + (long)row0 * (DH * 2);
             const char* sd = dOb + (long)row0 * ldo_bytes;
 #pragma unroll
-            for (int i = 0; i < NLD; ++i) dma16_saddr_lds(qoff[i], sq, dq_ + i * NW * 1024);
+            for (int i = 0; i < NLD; ++i) load_chunk_lds<DH>(qoff[i], sq, dq_ + i * NW * 1024);
 #pragma unroll
-            for (int i = 0; i < NLD; ++i) dma16_saddr_lds(dooff[i], sd, dq_ + TILE * 2 + i * NW * 1024);
+            for (int i = 0; i < NLD; ++i) load_chunk_lds<DH>(dooff[i], sd, dq_ + TILE * 2 + i * NW * 1024);
         } else {
             const int last = T_ - 1;
 #pragma unroll
             for (int i = 0; i < NLD; ++i) {
                 const int p = (i * NW + wave) * 64 + lane;
-                const int r = p / CPR, lc = (p % CPR) ^ swz16<DH>(r);
+                const int r = p / CPR, lc = (p % CPR) ^ swz16<PITCH>(r);
                 const int rr = min(row0 + r, last);
-                dma16_saddr_lds((unsigned)(rr * DH * 2 + lc * 16), Qb, dq_ + i * NW * 1024);
+                load_chunk_lds<DH>(lc < DH / 8 ? (unsigned)(rr * DH * 2 + lc * 16) : kNoChunk, Qb, dq_ + i * NW * 1024);
             }
 #pragma unroll
             for (int i = 0; i < NLD; ++i) {
                 const int p = (i * NW + wave) * 64 + lane;
-                const int r = p / CPR, lc = (p % CPR) ^ swz16<DH>(r);
+                const int r = p / CPR, lc = (p % CPR) ^ swz16<PITCH>(r);
                 const int rr = min(row0 + r, last);
-                dma16_saddr_lds((unsigned)(rr * ldo_bytes + lc * 16), dOb, dq_ + TILE * 2 + i * NW * 1024);
+                load_chunk_lds<DH>(lc < DH / 8 ? (unsigned)(rr * ldo_bytes + lc * 16) : kNoChunk, dOb, dq_ + TILE * 2 + i * NW * 1024);
             }
         }
     };
@@ -718,8 +746,8 @@ __global__ __launch_bounds__(NW * 64) void attn_bwd_dkdv2_kernel(AttnArgs a) {
                     for (int hs = 0; hs < 2; ++hs)
 #pragma unroll
                         for (int db = 0; db < NDB; ++db) {
-                            ado[hs][db] = load_tr<T>(ptr0[db] + so + TILE + hs * 16 * DH, ptr1[db] + so + TILE + hs * 16 * DH);
-                            aq[hs][db] = load_tr<T>(ptr0[db] + so + hs * 16 * DH, ptr1[db] + so + hs * 16 * DH);
+                            ado[hs][db] = load_tr<T>(ptr0[db] + so + TILE + hs * 16 * PITCH, ptr1[db] + so + TILE + hs * 16 * PITCH);
+                            aq[hs][db] = load_tr<T>(ptr0[db] + so + hs * 16 * PITCH, ptr1[db] + so + hs * 16 * PITCH);
                         }
                     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -795,7 +823,7 @@ __global__ __launch_bounds__(NW * 64) void attn_bwd_dkdv2_kernel(AttnArgs a) {
 // dK/dV kernel that follows on the stream.
 // LDS bytes of the dQ workgroup: NW private rings of two stages of K + V, reused for the reduction
 template <int DH, int NW> constexpr int dq2_smem_bytes() {
-    constexpr int ring = NW * 2 * 2 * 32 * DH * 2, epi = NW * 32 * (DH + 4) * 4;
+    constexpr int ring = NW * 2 * 2 * 32 * tile_pitch<DH>() * 2, epi = NW * 32 * ((DH + 31) / 32 * 32 + 4) * 4;
     return ring > epi ? ring : epi;
 }
 
@@ -804,14 +832,14 @@ template <typename T, int DH, int NW>
 __device__ __forceinline__ void attn_bwd_dq2_body(const AttnArgs& a, unsigned char* smem, int wg_id) {
     typedef Elem<T> E;
     static_assert(sizeof(T) == 2, "direct-to-LDS kernels are for fp16 / bf16");
-    constexpr int NDB = DH / 32, NKS = DH / 16;
-    constexpr int TILE = 32 * DH;                       // elements of one K or V tile
-    constexpr int CPR = DH / 8;
+    constexpr int NDB = (DH + 31) / 32, NKS = DH / 16, PITCH = tile_pitch<DH>();
+    constexpr int TILE = 32 * PITCH;                       // elements of one K or V tile
+    constexpr int CPR = PITCH / 8;
     constexpr int NLD = 32 * CPR / 64;                  // loads per lane per tile (one wave loads a whole tile)
     constexpr int NLOAD = 2 * NLD;
     static_assert(NLOAD <= 63, "too many loads in flight for vmcnt");
     constexpr int WAVE_RING = 2 * 2 * TILE * 2;         // bytes: two stages of K + V
-    constexpr int EPI_LD = DH + 4;
+    constexpr int EPI_LD = NDB * 32 + 4;
 
     const int tid = threadIdx.x, lane = tid & 63, g = lane >> 5, li = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -835,13 +863,13 @@ __device__ __forceinline__ void attn_bwd_dq2_body(const AttnArgs& a, unsigned ch
     // lane-constant LDS addresses inside stage 0's K tile
     const T* pkm[NKS];
 #pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) pkm[ks] = ring + km_offset<T, DH>(li, ks * 16, lane);
+    for (int ks = 0; ks < NKS; ++ks) pkm[ks] = ring + km_offset<T, PITCH>(li, ks * 16, lane);
     const T* ptr0[NDB];
     const T* ptr1[NDB];
 #pragma unroll
     for (int db = 0; db < NDB; ++db) {
         int o0, o1;
-        tr_offsets<T, DH, true>(0, db * 32, lane, o0, o1);
+        tr_offsets<T, PITCH, true>(0, db * 32, lane, o0, o1);
         ptr0[db] = ring + o0;
         ptr1[db] = ring + o1;
     }
@@ -849,8 +877,8 @@ __device__ __forceinline__ void attn_bwd_dq2_body(const AttnArgs& a, unsigned ch
 #pragma unroll
     for (int i = 0; i < NLD; ++i) {
         const int p = i * 64 + lane;
-        const int r = p / CPR, lc = (p % CPR) ^ swz16<DH>(r);
-        koff[i] = (unsigned)(r * DH * 2 + lc * 16);
+        const int r = p / CPR, lc = (p % CPR) ^ swz16<PITCH>(r);
+        koff[i] = lc < DH / 8 ? (unsigned)(r * DH * 2 + lc * 16) : kNoChunk;
     }
     const char* Kb = uniform_ptr(reinterpret_cast<const char*>(reinterpret_cast<const T*>(a.kc) + (long)bh * a.cache_rows * DH));
     const char* Vb = uniform_ptr(reinterpret_cast<const char*>(reinterpret_cast<const T*>(a.vc) + (long)bh * a.cache_rows * DH));
@@ -863,24 +891,24 @@ __device__ __forceinline__ void attn_bwd_dq2_body(const AttnArgs& a, unsigned ch
             const char* sk = Kb + (long)row0 * (DH * 2);
             const char* sv = Vb + (long)row0 * (DH * 2);
 #pragma unroll
-            for (int i = 0; i < NLD; ++i) dma16_saddr_lds(koff[i], sk, dst + i * 1024);
+            for (int i = 0; i < NLD; ++i) load_chunk_lds<DH>(koff[i], sk, dst + i * 1024);
 #pragma unroll
-            for (int i = 0; i < NLD; ++i) dma16_saddr_lds(koff[i], sv, dst + TILE * 2 + i * 1024);
+            for (int i = 0; i < NLD; ++i) load_chunk_lds<DH>(koff[i], sv, dst + TILE * 2 + i * 1024);
         } else {
             const int last = S - 1;
 #pragma unroll
             for (int i = 0; i < NLD; ++i) {
                 const int p = i * 64 + lane;
-                const int r = p / CPR, lc = (p % CPR) ^ swz16<DH>(r);
-                const unsigned off = (unsigned)(min(row0 + r, last) * DH * 2 + lc * 16);
-                dma16_saddr_lds(off, Kb, dst + i * 1024);
+                const int r = p / CPR, lc = (p % CPR) ^ swz16<PITCH>(r);
+                const unsigned off = lc < DH / 8 ? (unsigned)(min(row0 + r, last) * DH * 2 + lc * 16) : kNoChunk;
+                load_chunk_lds<DH>(off, Kb, dst + i * 1024);
             }
 #pragma unroll
             for (int i = 0; i < NLD; ++i) {
                 const int p = i * 64 + lane;
-                const int r = p / CPR, lc = (p % CPR) ^ swz16<DH>(r);
-                const unsigned off = (unsigned)(min(row0 + r, last) * DH * 2 + lc * 16);
-                dma16_saddr_lds(off, Vb, dst + TILE * 2 + i * 1024);
+                const int r = p / CPR, lc = (p % CPR) ^ swz16<PITCH>(r);
+                const unsigned off = lc < DH / 8 ? (unsigned)(min(row0 + r, last) * DH * 2 + lc * 16) : kNoChunk;
+                load_chunk_lds<DH>(off, Vb, dst + TILE * 2 + i * 1024);
             }
         }
     };
@@ -966,7 +994,7 @@ __device__ __forceinline__ void attn_bwd_dq2_body(const AttnArgs& a, unsigned ch
         for (int hs = 0; hs < 2; ++hs)
 #pragma unroll
             for (int db = 0; db < NDB; ++db)
-                ak[hs][db] = load_tr<T>(ptr0[db] + so + hs * 16 * DH, ptr1[db] + so + hs * 16 * DH);
+                ak[hs][db] = load_tr<T>(ptr0[db] + so + hs * 16 * PITCH, ptr1[db] + so + hs * 16 * PITCH);
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int hs = 0; hs < 2; ++hs)
@@ -988,23 +1016,11 @@ __device__ __forceinline__ void attn_bwd_dq2_body(const AttnArgs& a, unsigned ch
     float* ebuf = reinterpret_cast<float*>(smem);
     acc_to_lds_rows<DH>(dq, ebuf + wave * 32 * EPI_LD, lane);
     __syncthreads();
-    // thread -> (row, 16 consecutive columns) for DH = 128 with 256 threads; generally 32*DH/(NW*64) columns
-    constexpr int CPT = 32 * DH / (NW * 64);             // columns per thread
-    static_assert(CPT % 4 == 0 && DH % CPT == 0, "bad reduction split");
-    const int row = tid / (DH / CPT), c0 = (tid % (DH / CPT)) * CPT;
-    if (q0 + row < T_) {
-        T* dst = reinterpret_cast<T*>(a.dqkv) + ((long)(q0 + row) * a.B + b) * (3 * EE) + (long)h * 3 * DH + c0;
-#pragma unroll
-        for (int c = 0; c < CPT; c += 4) {
-            float4 acc4 = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-            for (int w = 0; w < NW; ++w) {
-                const float4 v = *reinterpret_cast<const float4*>(ebuf + (w * 32 + row) * EPI_LD + c0 + c);
-                acc4.x += v.x; acc4.y += v.y; acc4.z += v.z; acc4.w += v.w;
-            }
-            store4<T>(dst + c, acc4.x * a.qscale, acc4.y * a.qscale, acc4.z * a.qscale, acc4.w * a.qscale);
-        }
-    }
+    sum_rows<DH, NW>(ebuf, tid, [&](int row, int col, float4 v) {
+        if (q0 + row < T_)
+            store4<T>(reinterpret_cast<T*>(a.dqkv) + ((long)(q0 + row) * a.B + b) * (3 * EE) + (long)h * 3 * DH + col,
+                      v.x * a.qscale, v.y * a.qscale, v.z * a.qscale, v.w * a.qscale);
+    });
 }
 
 template <typename T, int DH, int NW>
@@ -1024,14 +1040,14 @@ template <typename T, int DH, int NW, int STG = 2>
 __global__ __launch_bounds__(NW * 64) void attn_fwd2_kernel(AttnArgs a) {
     typedef Elem<T> E;
     static_assert(sizeof(T) == 2, "direct-to-LDS kernels are for fp16 / bf16");
-    constexpr int NDB = DH / 32, NKS = DH / 16;
-    constexpr int TILE = 32 * DH;
-    constexpr int CPR = DH / 8;
+    constexpr int NDB = (DH + 31) / 32, NKS = DH / 16, PITCH = tile_pitch<DH>();
+    constexpr int TILE = 32 * PITCH;
+    constexpr int CPR = PITCH / 8;
     constexpr int NLD = 32 * CPR / 64;
     constexpr int NLOAD = 2 * NLD;
     static_assert(NLOAD <= 63, "too many loads in flight for vmcnt");
     constexpr int WAVE_RING = STG * 2 * TILE * 2;        // bytes: STG stages of K + V
-    constexpr int EPI_LD = DH + 4;
+    constexpr int EPI_LD = NDB * 32 + 4;
     constexpr int STAT_FLOATS = 2 * NW * 32;
     constexpr int EPI_BYTES = (STAT_FLOATS + NW * 32 * EPI_LD) * 4;
     constexpr int SMEM = NW * WAVE_RING > EPI_BYTES ? NW * WAVE_RING : EPI_BYTES;
@@ -1066,13 +1082,13 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd2_kernel(AttnArgs a) {
 
     const T* pkm[NKS];
 #pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) pkm[ks] = ring + km_offset<T, DH>(li, ks * 16, lane);
+    for (int ks = 0; ks < NKS; ++ks) pkm[ks] = ring + km_offset<T, PITCH>(li, ks * 16, lane);
     const T* ptr0[NDB];
     const T* ptr1[NDB];
 #pragma unroll
     for (int db = 0; db < NDB; ++db) {
         int o0, o1;
-        tr_offsets<T, DH, true>(0, db * 32, lane, o0, o1);
+        tr_offsets<T, PITCH, true>(0, db * 32, lane, o0, o1);
         ptr0[db] = ring + TILE + o0;          // inside the V tile
         ptr1[db] = ring + TILE + o1;
     }
@@ -1080,8 +1096,8 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd2_kernel(AttnArgs a) {
 #pragma unroll
     for (int i = 0; i < NLD; ++i) {
         const int p = i * 64 + lane;
-        const int r = p / CPR, lc = (p % CPR) ^ swz16<DH>(r);
-        koff[i] = (unsigned)(r * DH * 2 + lc * 16);
+        const int r = p / CPR, lc = (p % CPR) ^ swz16<PITCH>(r);
+        koff[i] = lc < DH / 8 ? (unsigned)(r * DH * 2 + lc * 16) : kNoChunk;
     }
     const char* Kb = uniform_ptr(reinterpret_cast<const char*>(reinterpret_cast<const T*>(a.kc) + (long)bh * a.cache_rows * DH));
     const char* Vb = uniform_ptr(reinterpret_cast<const char*>(reinterpret_cast<const T*>(a.vc) + (long)bh * a.cache_rows * DH));
@@ -1094,24 +1110,24 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd2_kernel(AttnArgs a) {
             const char* sk = Kb + (long)row0 * (DH * 2);
             const char* sv = Vb + (long)row0 * (DH * 2);
 #pragma unroll
-            for (int i = 0; i < NLD; ++i) dma16_saddr_lds(koff[i], sk, dst + i * 1024);
+            for (int i = 0; i < NLD; ++i) load_chunk_lds<DH>(koff[i], sk, dst + i * 1024);
 #pragma unroll
-            for (int i = 0; i < NLD; ++i) dma16_saddr_lds(koff[i], sv, dst + TILE * 2 + i * 1024);
+            for (int i = 0; i < NLD; ++i) load_chunk_lds<DH>(koff[i], sv, dst + TILE * 2 + i * 1024);
         } else {
             const int last = S - 1;
 #pragma unroll
             for (int i = 0; i < NLD; ++i) {
                 const int p = i * 64 + lane;
-                const int r = p / CPR, lc = (p % CPR) ^ swz16<DH>(r);
-                const unsigned off = (unsigned)(min(row0 + r, last) * DH * 2 + lc * 16);
-                dma16_saddr_lds(off, Kb, dst + i * 1024);
+                const int r = p / CPR, lc = (p % CPR) ^ swz16<PITCH>(r);
+                const unsigned off = lc < DH / 8 ? (unsigned)(min(row0 + r, last) * DH * 2 + lc * 16) : kNoChunk;
+                load_chunk_lds<DH>(off, Kb, dst + i * 1024);
             }
 #pragma unroll
             for (int i = 0; i < NLD; ++i) {
                 const int p = i * 64 + lane;
-                const int r = p / CPR, lc = (p % CPR) ^ swz16<DH>(r);
-                const unsigned off = (unsigned)(min(row0 + r, last) * DH * 2 + lc * 16);
-                dma16_saddr_lds(off, Vb, dst + TILE * 2 + i * 1024);
+                const int r = p / CPR, lc = (p % CPR) ^ swz16<PITCH>(r);
+                const unsigned off = lc < DH / 8 ? (unsigned)(min(row0 + r, last) * DH * 2 + lc * 16) : kNoChunk;
+                load_chunk_lds<DH>(off, Vb, dst + TILE * 2 + i * 1024);
             }
         }
     };
@@ -1151,7 +1167,7 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd2_kernel(AttnArgs a) {
         for (int hs = 0; hs < 2; ++hs)
 #pragma unroll
             for (int db = 0; db < NDB; ++db)
-                av[hs][db] = load_tr<T>(ptr0[db] + so + hs * 16 * DH, ptr1[db] + so + hs * 16 * DH);
+                av[hs][db] = load_tr<T>(ptr0[db] + so + hs * 16 * PITCH, ptr1[db] + so + hs * 16 * PITCH);
         __builtin_amdgcn_sched_barrier(0);
         float16v sacc;
 #pragma unroll
@@ -1247,24 +1263,11 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd2_kernel(AttnArgs a) {
         else a.lse[(long)bh * a.st_bhs + tq] = lse_wg;
     }
     __syncthreads();
-    constexpr int CPT = 32 * DH / (NW * 64);
-    static_assert(CPT % 4 == 0 && DH % CPT == 0, "bad reduction split");
-    const int row = tid / (DH / CPT), c0 = (tid % (DH / CPT)) * CPT;
-    if (q0 + row < T_) {
-        T* dst = reinterpret_cast<T*>(a.o) + ((long)(q0 + row) * a.B + b) * EE + (long)h * DH + c0;
-        float* pdst = a.part_o + (prow0 + q0 + row) * DH + c0;
-#pragma unroll
-        for (int c = 0; c < CPT; c += 4) {
-            float4 acc4 = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-            for (int w = 0; w < NW; ++w) {
-                const float4 v = *reinterpret_cast<const float4*>(ebuf + (w * 32 + row) * EPI_LD + c0 + c);
-                acc4.x += v.x; acc4.y += v.y; acc4.z += v.z; acc4.w += v.w;
-            }
-            if (partial) *reinterpret_cast<float4*>(pdst + c) = acc4;
-            else store4<T>(dst + c, acc4.x, acc4.y, acc4.z, acc4.w);
-        }
-    }
+    sum_rows<DH, NW>(ebuf, tid, [&](int row, int col, float4 v) {
+        if (q0 + row >= T_) return;
+        if (partial) *reinterpret_cast<float4*>(a.part_o + (prow0 + q0 + row) * DH + col) = v;
+        else store4<T>(reinterpret_cast<T*>(a.o) + ((long)(q0 + row) * a.B + b) * EE + (long)h * DH + col, v.x, v.y, v.z, v.w);
+    });
 }
 
 // Forward for slices of 64 queries and more.  A workgroup owns 64 queries of one (batch, head) -- two blocks of 32 --
@@ -1282,13 +1285,13 @@ template <typename T, int DH, int NW>
 __global__ __launch_bounds__(NW * 64) void attn_fwd3_kernel(AttnArgs a) {
     typedef Elem<T> E;
     static_assert(sizeof(T) == 2, "direct-to-LDS kernels are for fp16 / bf16");
-    constexpr int NDB = DH / 32, NKS = DH / 16;
-    constexpr int TILE = 32 * DH;
-    constexpr int CPR = DH / 8;
+    constexpr int NDB = (DH + 31) / 32, NKS = DH / 16, PITCH = tile_pitch<DH>();
+    constexpr int TILE = 32 * PITCH;
+    constexpr int CPR = PITCH / 8;
     constexpr int NLD = 32 * CPR / 64;                   // loads per K or V tile and lane
     static_assert(3 * NLD <= 63, "too many loads in flight for vmcnt");
     constexpr int WAVE_RING = 2 * 2 * TILE * 2;          // bytes: two stages of K + V
-    constexpr int EPI_LD = DH + 4;
+    constexpr int EPI_LD = NDB * 32 + 4;
     constexpr int STAT_FLOATS = 2 * NW * 32;
     constexpr int EPI_BYTES = (STAT_FLOATS + NW * 32 * EPI_LD) * 4;
     constexpr int SMEM = NW * WAVE_RING > EPI_BYTES ? NW * WAVE_RING : EPI_BYTES;
@@ -1322,13 +1325,13 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd3_kernel(AttnArgs a) {
 
     const T* pkm[NKS];
 #pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) pkm[ks] = ring + km_offset<T, DH>(li, ks * 16, lane);
+    for (int ks = 0; ks < NKS; ++ks) pkm[ks] = ring + km_offset<T, PITCH>(li, ks * 16, lane);
     const T* ptr0[NDB];
     const T* ptr1[NDB];
 #pragma unroll
     for (int db = 0; db < NDB; ++db) {
         int o0, o1;
-        tr_offsets<T, DH, true>(0, db * 32, lane, o0, o1);
+        tr_offsets<T, PITCH, true>(0, db * 32, lane, o0, o1);
         ptr0[db] = ring + TILE + o0;          // inside the V tile
         ptr1[db] = ring + TILE + o1;
     }
@@ -1336,8 +1339,8 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd3_kernel(AttnArgs a) {
 #pragma unroll
     for (int i = 0; i < NLD; ++i) {
         const int p = i * 64 + lane;
-        const int r = p / CPR, lc = (p % CPR) ^ swz16<DH>(r);
-        koff[i] = (unsigned)(r * DH * 2 + lc * 16);
+        const int r = p / CPR, lc = (p % CPR) ^ swz16<PITCH>(r);
+        koff[i] = lc < DH / 8 ? (unsigned)(r * DH * 2 + lc * 16) : kNoChunk;
     }
     const char* Kb = uniform_ptr(reinterpret_cast<const char*>(reinterpret_cast<const T*>(a.kc) + (long)bh * a.cache_rows * DH));
     const char* Vb = uniform_ptr(reinterpret_cast<const char*>(reinterpret_cast<const T*>(a.vc) + (long)bh * a.cache_rows * DH));
@@ -1351,15 +1354,15 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd3_kernel(AttnArgs a) {
         if (row0 + 32 <= S) {
             const char* sb = base + (long)row0 * (DH * 2);
 #pragma unroll
-            for (int i = 0; i < NLD; ++i) dma16_saddr_lds(koff[i], sb, dst + i * 1024);
+            for (int i = 0; i < NLD; ++i) load_chunk_lds<DH>(koff[i], sb, dst + i * 1024);
         } else {
             const int last = S - 1;
 #pragma unroll
             for (int i = 0; i < NLD; ++i) {
                 const int p = i * 64 + lane;
-                const int r = p / CPR, lc = (p % CPR) ^ swz16<DH>(r);
-                const unsigned off = (unsigned)(min(row0 + r, last) * DH * 2 + lc * 16);
-                dma16_saddr_lds(off, base, dst + i * 1024);
+                const int r = p / CPR, lc = (p % CPR) ^ swz16<PITCH>(r);
+                const unsigned off = lc < DH / 8 ? (unsigned)(min(row0 + r, last) * DH * 2 + lc * 16) : kNoChunk;
+                load_chunk_lds<DH>(off, base, dst + i * 1024);
             }
         }
     };
@@ -1470,7 +1473,7 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd3_kernel(AttnArgs a) {
         for (int hs = 0; hs < 2; ++hs)
 #pragma unroll
             for (int db = 0; db < NDB; ++db)
-                av[hs][db] = load_tr<T>(ptr0[db] + so + hs * 16 * DH, ptr1[db] + so + hs * 16 * DH);
+                av[hs][db] = load_tr<T>(ptr0[db] + so + hs * 16 * PITCH, ptr1[db] + so + hs * 16 * PITCH);
         float16v n0, n1;
         scores(son, n0, n1);
         uint4 p0[2], p1[2];
@@ -1499,8 +1502,6 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd3_kernel(AttnArgs a) {
     float* sL = sM + NW * 32;
     float* ebuf = sL + NW * 32;
     const bool partial = a.nsplit > 1;
-    constexpr int CPT = 32 * DH / (NW * 64);
-    static_assert(CPT % 4 == 0 && DH % CPT == 0, "bad reduction split");
     auto finish = [&](float16v* oacc, float m, float lsum, int qb0, int tq, bool qok) {
         __syncthreads();       // every wave is done with its ring (or with the previous block's merge)
         const float lw = lsum + __shfl_xor(lsum, 32, 64);
@@ -1539,22 +1540,11 @@ __global__ __launch_bounds__(NW * 64) void attn_fwd3_kernel(AttnArgs a) {
             else a.lse[(long)bh * a.st_bhs + tq] = lse_wg;
         }
         __syncthreads();
-        const int row = tid / (DH / CPT), c0 = (tid % (DH / CPT)) * CPT;
-        if (qb0 + row < T_) {
-            T* dst = reinterpret_cast<T*>(a.o) + ((long)(qb0 + row) * a.B + b) * EE + (long)h * DH + c0;
-            float* pdst = a.part_o + (prow0 + qb0 + row) * DH + c0;
-#pragma unroll
-            for (int c = 0; c < CPT; c += 4) {
-                float4 acc4 = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-                for (int w = 0; w < NW; ++w) {
-                    const float4 v = *reinterpret_cast<const float4*>(ebuf + (w * 32 + row) * EPI_LD + c0 + c);
-                    acc4.x += v.x; acc4.y += v.y; acc4.z += v.z; acc4.w += v.w;
-                }
-                if (partial) *reinterpret_cast<float4*>(pdst + c) = acc4;
-                else store4<T>(dst + c, acc4.x, acc4.y, acc4.z, acc4.w);
-            }
-        }
+        sum_rows<DH, NW>(ebuf, tid, [&](int row, int col, float4 v) {
+            if (qb0 + row >= T_) return;
+            if (partial) *reinterpret_cast<float4*>(a.part_o + (prow0 + qb0 + row) * DH + col) = v;
+            else store4<T>(reinterpret_cast<T*>(a.o) + ((long)(qb0 + row) * a.B + b) * EE + (long)h * DH + col, v.x, v.y, v.z, v.w);
+        });
     };
     finish(oacc0, m0, l0, q0, tq0, qok0);
     if (two) finish(oacc1, m1, l1, q0 + 32, tq1, qok1);
@@ -1577,7 +1567,7 @@ struct SuffixArgs {
 
 // LDS bytes of the dK/dV workgroup: NW private rings of two stages of Q + dO and of (lse, delta) rows
 template <int DH, int NW> constexpr int suffix_smem_bytes() {
-    constexpr int ring = NW * (2 * 2 * 32 * DH * 2 + 2 * 256), epi = NW * 32 * (DH + 4) * 4;
+    constexpr int ring = NW * (2 * 2 * 32 * tile_pitch<DH>() * 2 + 2 * 256), epi = NW * 32 * ((DH + 31) / 32 * 32 + 4) * 4;
     return ring > epi ? ring : epi;
 }
 
@@ -1589,15 +1579,15 @@ template <typename T, int DH, int NW, bool OWN_DELTA>
 __device__ __forceinline__ void attn_suffix_dkdv_body(const SuffixArgs& a, unsigned char* smem, float* own, int wg_id) {
     typedef Elem<T> E;
     static_assert(sizeof(T) == 2, "direct-to-LDS kernels are for fp16 / bf16");
-    constexpr int NDB = DH / 32, NKS = DH / 16;
-    constexpr int TILE = 32 * DH;                       // elements of one Q or dO tile
-    constexpr int CPR = DH / 8;
+    constexpr int NDB = (DH + 31) / 32, NKS = DH / 16, PITCH = tile_pitch<DH>();
+    constexpr int TILE = 32 * PITCH;                       // elements of one Q or dO tile
+    constexpr int CPR = PITCH / 8;
     constexpr int NLD = 32 * CPR / 64;
     constexpr int NLOAD = 2 * NLD + 1;                  // Q, dO and the stats row
     static_assert(NLOAD <= 63, "too many loads in flight for vmcnt");
     constexpr int WAVE_RING = 2 * 2 * TILE * 2;         // bytes: two stages of Q + dO
     constexpr int STAT_BYTES = 2 * 256;                 // per wave: two stages of 32 lse + 32 delta
-    constexpr int EPI_LD = DH + 4;
+    constexpr int EPI_LD = NDB * 32 + 4;
 
     const int tid = threadIdx.x, lane = tid & 63, g = lane >> 5, li = lane & 31;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -1620,13 +1610,13 @@ __device__ __forceinline__ void attn_suffix_dkdv_body(const SuffixArgs& a, unsig
 
     const T* pkm[NKS];
 #pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) pkm[ks] = ring + km_offset<T, DH>(li, ks * 16, lane);
+    for (int ks = 0; ks < NKS; ++ks) pkm[ks] = ring + km_offset<T, PITCH>(li, ks * 16, lane);
     const T* ptr0[NDB];
     const T* ptr1[NDB];
 #pragma unroll
     for (int db = 0; db < NDB; ++db) {
         int o0, o1;
-        tr_offsets<T, DH, true>(0, db * 32, lane, o0, o1);
+        tr_offsets<T, PITCH, true>(0, db * 32, lane, o0, o1);
         ptr0[db] = ring + o0;
         ptr1[db] = ring + o1;
     }
@@ -1635,9 +1625,9 @@ __device__ __forceinline__ void attn_suffix_dkdv_body(const SuffixArgs& a, unsig
 #pragma unroll
     for (int i = 0; i < NLD; ++i) {
         const int p = i * 64 + lane;
-        const int r = p / CPR, lc = (p % CPR) ^ swz16<DH>(r);
-        qoff[i] = (unsigned)(r * DH * 2 + lc * 16);
-        dooff[i] = (unsigned)(r * ldo_bytes + lc * 16);
+        const int r = p / CPR, lc = (p % CPR) ^ swz16<PITCH>(r);
+        qoff[i] = lc < DH / 8 ? (unsigned)(r * DH * 2 + lc * 16) : kNoChunk;
+        dooff[i] = lc < DH / 8 ? (unsigned)(r * ldo_bytes + lc * 16) : kNoChunk;
     }
     const char* Qb = uniform_ptr(reinterpret_cast<const char*>(reinterpret_cast<const T*>(a.q) + (long)bh * a.q_bhs));
     const char* dOb = uniform_ptr(reinterpret_cast<const char*>(reinterpret_cast<const T*>(a.d_o) + (long)b * EE + (long)h * DH));
@@ -1651,22 +1641,22 @@ __device__ __forceinline__ void attn_suffix_dkdv_body(const SuffixArgs& a, unsig
             const char* sq = Qb + (long)row0 * (DH * 2);
             const char* sd = dOb + (long)row0 * ldo_bytes;
 #pragma unroll
-            for (int i = 0; i < NLD; ++i) dma16_saddr_lds(qoff[i], sq, dst + i * 1024);
+            for (int i = 0; i < NLD; ++i) load_chunk_lds<DH>(qoff[i], sq, dst + i * 1024);
 #pragma unroll
-            for (int i = 0; i < NLD; ++i) dma16_saddr_lds(dooff[i], sd, dst + TILE * 2 + i * 1024);
+            for (int i = 0; i < NLD; ++i) load_chunk_lds<DH>(dooff[i], sd, dst + TILE * 2 + i * 1024);
         } else {
             const int last = Lq - 1;
 #pragma unroll
             for (int i = 0; i < NLD; ++i) {
                 const int p = i * 64 + lane;
-                const int r = p / CPR, lc = (p % CPR) ^ swz16<DH>(r);
-                dma16_saddr_lds((unsigned)(min(row0 + r, last) * DH * 2 + lc * 16), Qb, dst + i * 1024);
+                const int r = p / CPR, lc = (p % CPR) ^ swz16<PITCH>(r);
+                load_chunk_lds<DH>(lc < DH / 8 ? (unsigned)(min(row0 + r, last) * DH * 2 + lc * 16) : kNoChunk, Qb, dst + i * 1024);
             }
 #pragma unroll
             for (int i = 0; i < NLD; ++i) {
                 const int p = i * 64 + lane;
-                const int r = p / CPR, lc = (p % CPR) ^ swz16<DH>(r);
-                dma16_saddr_lds((unsigned)(min(row0 + r, last) * ldo_bytes + lc * 16), dOb, dst + TILE * 2 + i * 1024);
+                const int r = p / CPR, lc = (p % CPR) ^ swz16<PITCH>(r);
+                load_chunk_lds<DH>(lc < DH / 8 ? (unsigned)(min(row0 + r, last) * ldo_bytes + lc * 16) : kNoChunk, dOb, dst + TILE * 2 + i * 1024);
             }
         }
         dma4(statb + min(row0 + li, Lq - 1), stat_lds + stage * 256);
@@ -1789,8 +1779,8 @@ __device__ __forceinline__ void attn_suffix_dkdv_body(const SuffixArgs& a, unsig
         for (int hs = 0; hs < 2; ++hs)
 #pragma unroll
             for (int db = 0; db < NDB; ++db) {
-                ado[hs][db] = load_tr<T>(ptr0[db] + so + TILE + hs * 16 * DH, ptr1[db] + so + TILE + hs * 16 * DH);
-                aq[hs][db] = load_tr<T>(ptr0[db] + so + hs * 16 * DH, ptr1[db] + so + hs * 16 * DH);
+                ado[hs][db] = load_tr<T>(ptr0[db] + so + TILE + hs * 16 * PITCH, ptr1[db] + so + TILE + hs * 16 * PITCH);
+                aq[hs][db] = load_tr<T>(ptr0[db] + so + hs * 16 * PITCH, ptr1[db] + so + hs * 16 * PITCH);
             }
         __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
@@ -1814,27 +1804,15 @@ __device__ __forceinline__ void attn_suffix_dkdv_body(const SuffixArgs& a, unsig
     __syncthreads();       // every wave is done with its ring: the space is reused for the reduction
 
     float* ebuf = reinterpret_cast<float*>(smem);
-    constexpr int CPT = 32 * DH / (NW * 64);
-    static_assert(CPT % 4 == 0 && DH % CPT == 0, "bad reduction split");
-    const int row = tid / (DH / CPT), c0 = (tid % (DH / CPT)) * CPT;
 #pragma unroll
     for (int which = 0; which < 2; ++which) {
         acc_to_lds_rows<DH>(which == 0 ? dk : dv, ebuf + wave * 32 * EPI_LD, lane);
         __syncthreads();
-        if (key0 + row < S) {
-            T* dst = reinterpret_cast<T*>(a.dqkv) + ((long)(key0 + row - P) * a.B + b) * (3 * EE) + (long)h * 3 * DH +
-                     (which + 1) * DH + c0;
-#pragma unroll
-            for (int c = 0; c < CPT; c += 4) {
-                float4 acc4 = make_float4(0.f, 0.f, 0.f, 0.f);
-#pragma unroll
-                for (int w = 0; w < NW; ++w) {
-                    const float4 v = *reinterpret_cast<const float4*>(ebuf + (w * 32 + row) * EPI_LD + c0 + c);
-                    acc4.x += v.x; acc4.y += v.y; acc4.z += v.z; acc4.w += v.w;
-                }
-                store4<T>(dst + c, acc4.x, acc4.y, acc4.z, acc4.w);
-            }
-        }
+        sum_rows<DH, NW>(ebuf, tid, [&](int row, int col, float4 v) {
+            if (key0 + row < S)
+                store4<T>(reinterpret_cast<T*>(a.dqkv) + ((long)(key0 + row - P) * a.B + b) * (3 * EE) + (long)h * 3 * DH +
+                          (which + 1) * DH + col, v.x, v.y, v.z, v.w);
+        });
         __syncthreads();   // the buffer is rewritten by the next pass
     }
 }
@@ -1867,7 +1845,7 @@ static constexpr int kNumCU = 256;
 
 // head dimensions of the 16-bit kernels with direct global->LDS loads; the others run, in every dtype, on the
 // register-staged kernels, whose LDS tiles pad the head dimension to whole 32-column blocks
-static inline bool tiled16(int head_dim) { return head_dim == 64 || head_dim == 128; }
+constexpr bool tiled16(int head_dim) { return head_dim == 64 || head_dim == 80 || head_dim == 96 || head_dim == 128; }
 static inline bool known_head_dim(int hd) { return hd == 16 || hd == 32 || hd == 64 || hd == 80 || hd == 96 || hd == 128; }
 
 // calls f(std::integral_constant<int, hd>) for a known head dimension
@@ -1875,6 +1853,15 @@ template <typename F> static void for_head_dim(int hd, F&& f) {
     switch (hd) {
     case 16: f(std::integral_constant<int, 16>()); break;
     case 32: f(std::integral_constant<int, 32>()); break;
+    case 64: f(std::integral_constant<int, 64>()); break;
+    case 80: f(std::integral_constant<int, 80>()); break;
+    case 96: f(std::integral_constant<int, 96>()); break;
+    default: f(std::integral_constant<int, 128>()); break;
+    }
+}
+
+template <typename F> static void for_tiled_dim(int hd, F&& f) {
+    switch (hd) {
     case 64: f(std::integral_constant<int, 64>()); break;
     case 80: f(std::integral_constant<int, 80>()); break;
     case 96: f(std::integral_constant<int, 96>()); break;
@@ -1971,7 +1958,7 @@ static AttnArgs make_args(const tp_attn_desc* d) {
 template <typename T, int DH>
 static void launch_fwd(const FwdPlan& p, const AttnArgs& a, hipStream_t s) {
     dim3 grid(p.qblocks, a.B * a.H, p.nsplit);
-    if constexpr (sizeof(T) == 2 && (DH == 64 || DH == 128)) {
+    if constexpr (sizeof(T) == 2 && tiled16(DH)) {
         const dim3 g2(xcd_grid(a.B * a.H, (a.T + 31) / 32), p.nsplit);
         if (p.bn == 64) attn_fwd3_kernel<T, DH, 4><<<dim3(xcd_grid(a.B * a.H, (a.T + 63) / 64), p.nsplit), 256, 0, s>>>(a);
         else if (p.bn == 8) attn_fwd2_kernel<T, DH, 8, 1><<<g2, 512, 0, s>>>(a);
@@ -1991,7 +1978,7 @@ template <typename T, typename GT, int DH>
 static void launch_bwd(const AttnArgs& a, hipStream_t s) {
     const int S = a.P + a.T;
     long rows = (long)a.T * a.B * a.H;
-    constexpr bool kTiled16 = sizeof(T) == 2 && (DH == 64 || DH == 128);
+    constexpr bool kTiled16 = sizeof(T) == 2 && tiled16(DH);
     if constexpr (kTiled16) {
         // dQ first: it also leaves delta for the dK/dV kernel
         attn_bwd_dq2_kernel<T, DH, 4><<<xcd_grid(a.B * a.H, (a.T + 31) / 32), 256, 0, s>>>(a);
@@ -2113,13 +2100,11 @@ extern "C" int tp_attn_suffix_dkdv(const tp_attn_suffix_desc* d, void* stream) {
     SuffixArgs a = make_suffix_args(d);
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     const unsigned grid = xcd_grid(d->batch * d->heads, (d->key_count + 31) / 32);
-    if (d->dtype == TP_F16) {
-        if (d->head_dim == 64) attn_suffix_dkdv_kernel<f16, 64, 4><<<grid, 256, 0, s>>>(a);
-        else attn_suffix_dkdv_kernel<f16, 128, 4><<<grid, 256, 0, s>>>(a);
-    } else {
-        if (d->head_dim == 64) attn_suffix_dkdv_kernel<bf16, 64, 4><<<grid, 256, 0, s>>>(a);
-        else attn_suffix_dkdv_kernel<bf16, 128, 4><<<grid, 256, 0, s>>>(a);
-    }
+    for_tiled_dim(d->head_dim, [&](auto dh) {
+        constexpr int DH = decltype(dh)::value;
+        if (d->dtype == TP_F16) attn_suffix_dkdv_kernel<f16, DH, 4><<<grid, 256, 0, s>>>(a);
+        else attn_suffix_dkdv_kernel<bf16, DH, 4><<<grid, 256, 0, s>>>(a);
+    });
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) { set_error("%s: launch failed: %s", who, hipGetErrorString(e)); return TP_ERR_LAUNCH; }
     return TP_OK;
@@ -2157,13 +2142,11 @@ extern "C" int tp_attn_bwd_fused(const tp_attn_desc* d, const tp_attn_suffix_des
     const int n_dq = (int)xcd_grid(d->batch * d->heads, (d->T + 31) / 32);
     const unsigned grid = (unsigned)n_dq + xcd_grid(d->batch * d->heads, (d->T + 31) / 32);
     const size_t dyn = (size_t)((own_len + 31) / 32) * 32 * sizeof(float);
-    if (d->dtype == TP_F16) {
-        if (d->head_dim == 64) attn_bwd_fused_kernel<f16, 64><<<grid, 256, dyn, s>>>(a, sa, n_dq);
-        else attn_bwd_fused_kernel<f16, 128><<<grid, 256, dyn, s>>>(a, sa, n_dq);
-    } else {
-        if (d->head_dim == 64) attn_bwd_fused_kernel<bf16, 64><<<grid, 256, dyn, s>>>(a, sa, n_dq);
-        else attn_bwd_fused_kernel<bf16, 128><<<grid, 256, dyn, s>>>(a, sa, n_dq);
-    }
+    for_tiled_dim(d->head_dim, [&](auto dh) {
+        constexpr int DH = decltype(dh)::value;
+        if (d->dtype == TP_F16) attn_bwd_fused_kernel<f16, DH><<<grid, 256, dyn, s>>>(a, sa, n_dq);
+        else attn_bwd_fused_kernel<bf16, DH><<<grid, 256, dyn, s>>>(a, sa, n_dq);
+    });
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) { set_error("%s: launch failed: %s", who, hipGetErrorString(e)); return TP_ERR_LAUNCH; }
     return TP_OK;
@@ -2173,7 +2156,10 @@ static int validate_suffix(const tp_attn_suffix_desc* d, const char* who) {
     using namespace tp;
     if (!d) { set_error("%s: null descriptor", who); return TP_ERR_ARG; }
     if (d->dtype != TP_F16 && d->dtype != TP_BF16) { set_error("%s: dtype %d not supported (fp16 / bf16)", who, d->dtype); return TP_ERR_UNSUPPORTED; }
-    if (d->head_dim != 64 && d->head_dim != 128) { set_error("%s: head_dim %d not supported (64 or 128)", who, d->head_dim); return TP_ERR_UNSUPPORTED; }
+    if (!tiled16(d->head_dim) || (!d->odd_head_dims && d->head_dim != 64 && d->head_dim != 128)) {
+        set_error("%s: head_dim %d not supported (64 or 128; with odd_head_dims 80 or 96)", who, d->head_dim);
+        return TP_ERR_UNSUPPORTED;
+    }
     if (d->batch <= 0 || d->heads <= 0 || d->key_begin < 0 || d->key_count <= 0 || d->q_end < d->key_begin + d->key_count) {
         set_error("%s: bad geometry B=%d H=%d keys [%d, +%d) q_end=%d", who, d->batch, d->heads, d->key_begin, d->key_count, d->q_end);
         return TP_ERR_ARG;

@@ -328,7 +328,7 @@ def attn_suffix_dkdv(k_cache, v_cache, q_all, d_o_all, lse_all, delta_all, dqkv,
     d = _lib.AttnSuffixDesc()
     d.dtype = tp_dtype(q_all.dtype)
     d.batch, d.heads, d.head_dim = batch, heads, head_dim
-    d.key_begin, d.key_count, d.q_end = key_begin, key_count, q_end
+    d.key_begin, d.key_count, d.q_end, d.odd_head_dims = key_begin, key_count, q_end, 1
     d.cache_rows, d.q_bh_rows, d.stat_bh_rows = k_cache.shape[1], q_all.shape[1], lse_all.shape[1]
     d.k_cache, d.v_cache = k_cache.data_ptr(), v_cache.data_ptr()
     d.q_all, d.d_o_all = q_all.data_ptr(), d_o_all.data_ptr()
@@ -363,7 +363,7 @@ def attn_bwd_fused(q, k_cache, v_cache, o, lse, d_o, dqkv, batch, heads, head_di
     sd = _lib.AttnSuffixDesc()
     sd.dtype = d.dtype
     sd.batch, sd.heads, sd.head_dim = batch, heads, head_dim
-    sd.key_begin, sd.key_count, sd.q_end = cache_len, T, q_end
+    sd.key_begin, sd.key_count, sd.q_end, sd.odd_head_dims = cache_len, T, q_end, 1
     sd.cache_rows, sd.q_bh_rows, sd.stat_bh_rows = k_cache.shape[1], q_all.shape[1], lse_all.shape[1]
     sd.k_cache, sd.v_cache = k_cache.data_ptr(), v_cache.data_ptr()
     sd.q_all, sd.d_o_all = q_all.data_ptr(), d_o_all.data_ptr()

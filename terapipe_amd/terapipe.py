@@ -100,8 +100,8 @@ class _StackBuffers:
         nl, E, F, H = layers.n_layers, layers.embedding_dim, layers.ffn_embedding_dim, layers.num_attention_heads
         L, Dh = runner.seq_len, layers.embedding_dim // layers.num_attention_heads
         self.dtype, self.device = dtype, device
-        # the one-pass dK/dV kernel is 16-bit and has head dimensions 64 and 128; other runs keep gradient caches
-        self.position_indexed = runner.suffix_dkdv and dtype != torch.float32 and Dh in (64, 128)
+        # the one-pass dK/dV kernel is 16-bit and has head dimensions 64 to 128; other runs keep gradient caches
+        self.position_indexed = runner.suffix_dkdv and dtype != torch.float32 and Dh in (64, 80, 96, 128)
         self.fused_attn_bwd = runner.fused_attn_bwd
         self.merge_slices = runner.merge_slices
         # the pieces a step runs in
