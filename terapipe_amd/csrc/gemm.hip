@@ -430,37 +430,44 @@ __global__ __launch_bounds__(WM * WN * 64) void gemm_kernel(GemmArgs a) {
 }
 
 // Sums the split-K partials and applies the epilogue.  A block of 256 threads covers 256 columns
-// (32 threads x 8 columns) by 32 rows (8 row lanes x 4 rows); column sums are combined across the
-// row lanes in LDS so that they cost one atomic per column per block.
+// (32 threads x 8 columns) by 8 rows, one vector of 8 columns a thread; column sums are combined across the
+// rows in LDS so that they cost one atomic per column per block.  Bound by the latency of its loads (4 partial
+// sums of 256 x 2048 are 8 MB, 1.6 us of bandwidth): four rows a thread, one split at a time, took 14.0 us.
+// One row a thread with four splits' loads in flight takes 7.2.
 template <typename T>
 __global__ __launch_bounds__(256) void gemm_splitk_reduce_kernel(GemmArgs a) {
     __shared__ float cs[8][256];
     const int cl = threadIdx.x & 31, rl = threadIdx.x >> 5;
     const int col0 = (blockIdx.x * 32 + cl) * 8;
-    const int rbase = blockIdx.y * 32;
+    const int row = blockIdx.y * 8 + rl;
     float csum[8];
 #pragma unroll
     for (int e = 0; e < 8; ++e) csum[e] = 0.f;
-    if (col0 < a.N) {
+    if (col0 < a.N && row < a.M) {
+        float v[8];
 #pragma unroll
-        for (int rr = 0; rr < 4; ++rr) {
-            const int row = rbase + rr * 8 + rl;
-            if (row < a.M) {
-                float v[8];
+        for (int e = 0; e < 8; ++e) v[e] = 0.f;
+        const long plane = (long)a.M * a.N;
+        const float* src = a.partial + (long)row * a.N + col0;
+        // four splits' loads under way at a time (the partial sums are added in the order of the splits)
+        for (int z = 0; z < a.nsplit; z += 4) {
+            float4 p[4][2];
 #pragma unroll
-                for (int e = 0; e < 8; ++e) v[e] = 0.f;
-                for (int z = 0; z < a.nsplit; ++z) {
-                    const float* src = a.partial + ((long)z * a.M + row) * a.N + col0;
-                    float4 p0 = *reinterpret_cast<const float4*>(src);
-                    float4 p1 = *reinterpret_cast<const float4*>(src + 4);
-                    v[0] += p0.x; v[1] += p0.y; v[2] += p0.z; v[3] += p0.w;
-                    v[4] += p1.x; v[5] += p1.y; v[6] += p1.z; v[7] += p1.w;
+            for (int u = 0; u < 4; ++u)
+                if (z + u < a.nsplit) {
+                    p[u][0] = *reinterpret_cast<const float4*>(src + (z + u) * plane);
+                    p[u][1] = *reinterpret_cast<const float4*>(src + (z + u) * plane + 4);
                 }
-                epilogue_vec8<T>(a, row, col0, v);
 #pragma unroll
-                for (int e = 0; e < 8; ++e) csum[e] += v[e];
-            }
+            for (int u = 0; u < 4; ++u)
+                if (z + u < a.nsplit) {
+                    v[0] += p[u][0].x; v[1] += p[u][0].y; v[2] += p[u][0].z; v[3] += p[u][0].w;
+                    v[4] += p[u][1].x; v[5] += p[u][1].y; v[6] += p[u][1].z; v[7] += p[u][1].w;
+                }
         }
+        epilogue_vec8<T>(a, row, col0, v);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) csum[e] = v[e];
     }
     if (a.colsum) {
 #pragma unroll
@@ -814,7 +821,7 @@ static bool launch_gemm(const tp_gemm_desc* d, const GemmPlan& p, const GemmArgs
         }
     }
     if (p.nsplit > 1 && !d->defer_reduce) {
-        dim3 grid((d->N + 255) / 256, (d->M + 31) / 32);
+        dim3 grid((d->N + 255) / 256, (d->M + 7) / 8);
         gemm_splitk_reduce_kernel<T><<<grid, 256, 0, s>>>(a);
     }
     return true;
