@@ -280,6 +280,15 @@ int tp_embedding_bwd(const int64_t* ids, const void* dout, float* dweight_acc, i
  * GEMM): loss[m] = logsumexp(logits[m, :V]) - logits[m, target[m]], and logits is overwritten IN PLACE with
  * its gradient (softmax - onehot(target)) * grad_scale (padding columns 0), the way the reference overwrites
  * its input with the softmax (:65-74) and returns it scaled as grad_input (:79-99). */
+/* dweight[ids[m], :] += dout[m, :] in `dtype`, every row's sum taken in fp32 and rounded once; no atomics.  M <= 8192, E whole
+   16-byte chunks. */
+int tp_embedding_bwd_rows(const int64_t* ids, const void* dout, void* dweight, int M, int E, int V, int dtype, void* stream);
+/* The two halves of tp_cross_entropy.  Loss: logits are read only; max_sum[2m], [2m+1] = the row's maximum and
+   sum exp(z - maximum).  Gradient, from those: logits[m, v] <- (softmax - onehot) * scale[m], padding columns <- 0. */
+int tp_cross_entropy_loss(const void* logits, int64_t ld, const int64_t* target, float* loss, float* max_sum, int M, int V,
+                          int dtype, void* stream);
+int tp_cross_entropy_grad(void* logits, int64_t ld, const int64_t* target, const float* max_sum, const float* scale, int M,
+                          int V, int Vpad, int dtype, void* stream);
 int tp_cross_entropy(void* logits, int64_t ld, const int64_t* target, float* loss, int M, int V, int Vpad,
                      float grad_scale, int dtype, void* stream);
 /* x[m, :N] *= scale[m] in place: the per-token grad_output factor of the cross-entropy backward (:97) */

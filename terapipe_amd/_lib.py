@@ -143,6 +143,9 @@ SYMBOLS = {
     "tp_embedding_fwd": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p]),
     "tp_embedding_bwd": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p]),
     "tp_cross_entropy": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_int, c_int, c_int, c_float, c_int, c_void_p]),
+    "tp_embedding_bwd_rows": (c_int, [c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_void_p]),
+    "tp_cross_entropy_loss": (c_int, [c_void_p, c_int64, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_void_p]),
+    "tp_cross_entropy_grad": (c_int, [c_void_p, c_int64] + [c_void_p] * 3 + [c_int] * 4 + [c_void_p]),
     "tp_scale_rows": (c_int, [c_void_p, c_int64, c_void_p, c_int, c_int, c_int, c_void_p]),
     "tp_plan_slices": (c_int, [c_void_p, c_int, c_int, c_int, ctypes.c_double] + [c_void_p] * 5),
     "tp_adam_check_table": (c_int, [c_void_p, c_int, c_int]),

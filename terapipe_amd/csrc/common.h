@@ -360,7 +360,7 @@ __device__ __forceinline__ void dma4(const void* gptr, unsigned lds_wave_base) {
 // Tile loads for full tiles only: the lane's chunk is a loop-invariant 32-bit byte offset from a wave-uniform
 // tile origin that advances by a scalar step, so a tile costs one VGPR per load and no vector ALU work.
 // Coordinates of the fixed axis beyond the matrix are CLAMPED to the last valid row / chunk (the caller never
-// stores results that depend on them); the sliding axis must be a whole number of tiles.
+// stores results that depend on them; the last chunk may reach past the matrix into its row's padding); the sliding axis must be a whole number of tiles.
 template <typename T, int ROWS, int COLS, int NT, bool ALONG_COLS, bool KM16 = false> struct ClampTileDma {
     static constexpr int CPR = COLS / 8;
     static constexpr int TOTAL = ROWS * CPR;
@@ -380,7 +380,7 @@ template <typename T, int ROWS, int COLS, int NT, bool ALONG_COLS, bool KM16 = f
             const int lc = pc ^ swz16<COLS, KM16>(row);
             int fx = ALONG_COLS ? row : lc * 8;
             const int sl = ALONG_COLS ? lc * 8 : row;
-            const int last = fixed_max - (ALONG_COLS ? 1 : 8) - fixed0;
+            const int last = (ALONG_COLS ? fixed_max - 1 : (fixed_max + 7) / 8 * 8 - 8) - fixed0;
             fx = fx < last ? fx : last;
             off[i] = (unsigned)((ALONG_COLS ? (long)fx * ld + sl : (long)sl * ld + fx) * (long)sizeof(T));
         }
@@ -404,9 +404,10 @@ template <typename T, int ROWS, int COLS, int NT, bool ALONG_COLS, bool KM16 = f
     __device__ __forceinline__ void advance() { origin += step; }
 };
 
-// A ragged k of the tiles above: the k range's first len % BK positions make the FIRST tile, copied through registers
-// with zeros behind them (so that every tile after it is whole); `len` of them are valid from slide0 on.  Where k runs
-// along the tile's columns, len is a multiple of 8.  The caller waits (lgkmcnt) before it lets the tile be read.
+// A ragged k of the tiles above: the LAST len % BK positions of the k range make the FIRST tile, copied through registers
+// with zeros behind them (so that every tile after it is whole); `len` of them are valid from slide0 on.  A chunk along k
+// that begins inside and ends past len is loaded as it is: where len is no multiple of 8, the other operand's rows there
+// are zeros.  The caller waits (lgkmcnt) before it lets the tile be read.
 template <typename T, int ROWS, int COLS, int NT, bool ALONG_COLS, bool KM16>
 __device__ __forceinline__ void copy_ragged_tile(T* tile, const T* __restrict__ base, long ld, int fixed0, int fixed_max,
                                                  int slide0, int len, int tid) {
@@ -417,7 +418,7 @@ __device__ __forceinline__ void copy_ragged_tile(T* tile, const T* __restrict__ 
         const int row = p / CPR, lc = (p % CPR) ^ swz16<COLS, KM16>(row);
         const int sl = ALONG_COLS ? lc * 8 : row;
         int fx = fixed0 + (ALONG_COLS ? row : lc * 8);
-        const int last = fixed_max - (ALONG_COLS ? 1 : 8);
+        const int last = ALONG_COLS ? fixed_max - 1 : (fixed_max + 7) / 8 * 8 - 8;
         fx = fx < last ? fx : last;
         uint4 v = make_uint4(0, 0, 0, 0);
         if (sl < len) v = *reinterpret_cast<const uint4*>(base + (ALONG_COLS ? (long)fx * ld + slide0 + sl : (long)(slide0 + sl) * ld + fx));

@@ -213,8 +213,8 @@ void gemm_tall_kernel(typename std::conditional<GROUPED, GemmGroupArgs, GemmArgs
     DB db;
     const int nk = (kend - kbeg + BK - 1) / BK;
     const int ragged = (kend - kbeg) % BK;      // a ragged k has its short tile first (copy_ragged_tile)
-    da.init(reinterpret_cast<const T*>(a.A), a.lda, m0, a.M, ragged ? kbeg + ragged - BK : kbeg, BK, tid);
-    db.init(reinterpret_cast<const T*>(a.B), a.ldb, n0, a.N, ragged ? kbeg + ragged - BK : kbeg, BK, tid);
+    da.init(reinterpret_cast<const T*>(a.A), a.lda, m0, a.M, ragged ? kbeg - BK : kbeg, BK, tid);
+    db.init(reinterpret_cast<const T*>(a.B), a.ldb, n0, a.N, ragged ? kbeg - BK : kbeg, BK, tid);
     const unsigned lds0 = lds_addr(smem);
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);
     auto issue = [&](int stage) {
@@ -265,8 +265,8 @@ void gemm_tall_kernel(typename std::conditional<GROUPED, GemmGroupArgs, GemmArgs
     }
 
     if (ragged) {
-        copy_ragged_tile<T, AR, AC, NT, AKM, MI16 && AKM>(tiles, reinterpret_cast<const T*>(a.A), a.lda, m0, a.M, kbeg, ragged, tid);
-        copy_ragged_tile<T, BR, BC, NT, BKM, MI16 && BKM>(tiles + A_ELEMS, reinterpret_cast<const T*>(a.B), a.ldb, n0, a.N, kbeg, ragged, tid);
+        copy_ragged_tile<T, AR, AC, NT, AKM, MI16 && AKM>(tiles, reinterpret_cast<const T*>(a.A), a.lda, m0, a.M, kend - ragged, ragged, tid);
+        copy_ragged_tile<T, BR, BC, NT, BKM, MI16 && BKM>(tiles + A_ELEMS, reinterpret_cast<const T*>(a.B), a.ldb, n0, a.N, kend - ragged, ragged, tid);
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         da.advance();
         db.advance();
@@ -635,7 +635,7 @@ static void plan_large(const tp_gemm_desc* d, int& cfg, int& ns) {
         if (!tile_serves(c, d->op, d->K)) continue;
         const long tiles = (long)((d->M + c.bm - 1) / c.bm) * ((d->N + c.bn - 1) / c.bn);
         for (int n = 1; n <= 8; ++n) {
-            if (n > 1 && (d->K / n < 512 || tiles * n > 2 * kNumCU)) break;
+            if (n > 1 && (d->N % 8 || d->K / n < 512 || tiles * n > 2 * kNumCU)) break;
             float t = tile_time(c, tiles * n, K / n, spill);
             if (n > 1) t += 4.f + (float)((double)n * d->M * d->N * 8 / 5.5e6);
             if (t < best) { best = t; cfg = c.cfg; ns = n; }
@@ -657,6 +657,7 @@ static GemmPlan plan_gemm(const tp_gemm_desc* d) {
             nsplit = (int)(want < maxs ? want : maxs);
             if (nsplit > 16) nsplit = 16;
         }
+        if (d->N % 8) nsplit = 1;       // (partial sums are rows of N)
         finish_plan(d, p, 16, nsplit);
         return p;
     }
@@ -759,6 +760,7 @@ static GemmPlan plan_gemm(const tp_gemm_desc* d) {
     if (cfg >= 17 && cfg <= 20 && (ragged || (cfg == 17 && d->op != TP_GEMM_NT))) cfg = 5;
     if (cfg >= kFirstStreamCfg && cfg <= kLastStreamCfg &&
         (d->op == TP_GEMM_TN || ragged || ((cfg == 24 || cfg == 25) && d->op != TP_GEMM_NT))) cfg = 5;
+    if (d->N % 8) ns = 1;               // (partial sums are rows of N)
     p.cfg = cfg;
     tile_cfg(cfg, tc);
     p.gx = (d->N + tc.bn - 1) / tc.bn;
@@ -838,14 +840,21 @@ static int validate_gemm(const tp_gemm_desc* d) {
     // contiguous extents of the operands as stored
     int a_cols = d->op == TP_GEMM_TN ? d->M : d->K;
     int b_cols = d->op == TP_GEMM_NT ? d->K : d->N;
-    if (a_cols % ch || b_cols % ch || d->lda % ch || d->ldb % ch) {
+    // A's contiguous extent may end inside a chunk that its row holds in full where what it multiplies is bounded by
+    // rows: k of NN (the weight's rows past k count as zeros; A's columns there have to be finite), M of TN
+    const bool a_ragged = d->op != TP_GEMM_NT && d->lda >= (a_cols + ch - 1) / ch * ch;
+    if ((a_cols % ch && !a_ragged) || b_cols % ch || d->lda % ch || d->ldb % ch) {
         set_error("tp_gemm: contiguous extents / leading dimensions must be multiples of %d elements "
                   "(A cols %d lda %ld, B cols %d ldb %ld)", ch, a_cols, (long)d->lda, b_cols, (long)d->ldb);
         return TP_ERR_UNSUPPORTED;
     }
     if (d->lda < a_cols || d->ldb < b_cols) { set_error("tp_gemm: leading dimension smaller than row"); return TP_ERR_ARG; }
     if (((uintptr_t)d->A | (uintptr_t)d->B) & 15) { set_error("tp_gemm: operands must be 16-byte aligned"); return TP_ERR_ARG; }
-    if (d->N % 8) { set_error("tp_gemm: N=%d must be a multiple of 8", d->N); return TP_ERR_UNSUPPORTED; }
+    // N of a plain NT product may end inside a chunk that C's row holds in full (the columns past N get the last one's values)
+    if (d->N % 8 && (d->op != TP_GEMM_NT || d->epilogue != TP_EPI_STORE || d->defer_reduce || d->colsum_acc || d->ldc < (d->N + 7) / 8 * 8)) {
+        set_error("tp_gemm: N=%d must be a multiple of 8", d->N);
+        return TP_ERR_UNSUPPORTED;
+    }
     if (d->defer_reduce && ((d->epilogue != TP_EPI_STORE && d->epilogue != TP_EPI_BIAS_RESIDUAL) || d->colsum_acc)) {
         set_error("tp_gemm: defer_reduce needs the STORE or BIAS_RESIDUAL epilogue and no colsum_acc");
         return TP_ERR_ARG;

@@ -75,8 +75,8 @@ void gemm_pipe_kernel(typename std::conditional<GROUPED, GemmGroupArgs, GemmArgs
     const int ragged = (kend - kbeg) % BK;      // a ragged k has its short tile first (copy_ragged_tile)
     DA da;
     DB db;
-    da.init(reinterpret_cast<const T*>(a.A), a.lda, m0, a.M, ragged ? kbeg + ragged - BK : kbeg, BK, tid);
-    db.init(reinterpret_cast<const T*>(a.B), a.ldb, n0, a.N, ragged ? kbeg + ragged - BK : kbeg, BK, tid);
+    da.init(reinterpret_cast<const T*>(a.A), a.lda, m0, a.M, ragged ? kbeg - BK : kbeg, BK, tid);
+    db.init(reinterpret_cast<const T*>(a.B), a.ldb, n0, a.N, ragged ? kbeg - BK : kbeg, BK, tid);
     const unsigned lds0 = lds_addr(smem);
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);
 
@@ -153,8 +153,8 @@ void gemm_pipe_kernel(typename std::conditional<GROUPED, GemmGroupArgs, GemmArgs
     for (int s = 0; s < STAGES; ++s)
         if (s < nk) {
             if (s == 0 && ragged) {
-                copy_ragged_tile<T, AR, AC, NT, AKM, AKM>(tiles, reinterpret_cast<const T*>(a.A), a.lda, m0, a.M, kbeg, ragged, tid);
-                copy_ragged_tile<T, BR, BC, NT, BKM, BKM>(tiles + A_ELEMS, reinterpret_cast<const T*>(a.B), a.ldb, n0, a.N, kbeg, ragged, tid);
+                copy_ragged_tile<T, AR, AC, NT, AKM, AKM>(tiles, reinterpret_cast<const T*>(a.A), a.lda, m0, a.M, kend - ragged, ragged, tid);
+                copy_ragged_tile<T, BR, BC, NT, BKM, BKM>(tiles + A_ELEMS, reinterpret_cast<const T*>(a.B), a.ldb, n0, a.N, kend - ragged, ragged, tid);
                 da.advance();
                 db.advance();
                 continue;

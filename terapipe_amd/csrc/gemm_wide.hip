@@ -52,8 +52,8 @@ void gemm_wide_kernel(GemmArgs a) {
     const int nk = (klen + BK - 1) / BK, ragged = klen % BK;       // a ragged k has its short tile first (copy_ragged_tile)
     DA da;
     DB db;
-    da.init(reinterpret_cast<const T*>(a.A), a.lda, m0, a.M, ragged ? kbeg + ragged - BK : kbeg, BK, tid);
-    db.init(reinterpret_cast<const T*>(a.B), a.ldb, n0, a.N, ragged ? kbeg + ragged - BK : kbeg, BK, tid);
+    da.init(reinterpret_cast<const T*>(a.A), a.lda, m0, a.M, ragged ? kbeg - BK : kbeg, BK, tid);
+    db.init(reinterpret_cast<const T*>(a.B), a.ldb, n0, a.N, ragged ? kbeg - BK : kbeg, BK, tid);
     const unsigned lds0 = lds_addr(smem);
     const int wave_u = __builtin_amdgcn_readfirstlane(wave);
 
@@ -136,8 +136,8 @@ void gemm_wide_kernel(GemmArgs a) {
 
     // prologue: both buffers get a k-tile; k-tile 0 is waited for and its first sub-step fetched
     if (ragged) {
-        copy_ragged_tile<T, AR, AC, NT, AKM, AKM>(tiles, reinterpret_cast<const T*>(a.A), a.lda, m0, a.M, kbeg, ragged, tid);
-        copy_ragged_tile<T, BR, BC, NT, BKM, BKM>(tiles + A_ELEMS, reinterpret_cast<const T*>(a.B), a.ldb, n0, a.N, kbeg, ragged, tid);
+        copy_ragged_tile<T, AR, AC, NT, AKM, AKM>(tiles, reinterpret_cast<const T*>(a.A), a.lda, m0, a.M, kbeg + klen - ragged, ragged, tid);
+        copy_ragged_tile<T, BR, BC, NT, BKM, BKM>(tiles + A_ELEMS, reinterpret_cast<const T*>(a.B), a.ldb, n0, a.N, kbeg + klen - ragged, ragged, tid);
         da.advance();
         db.advance();
     } else {
@@ -159,7 +159,7 @@ void gemm_wide_kernel(GemmArgs a) {
 
     // The loop body is one straight line (a branch in it costs register copies): the last two k-tiles load the last
     // k-tile again into a buffer that nothing reads any more, and the last one's fetches for "the next" are not used.
-    // (A single ragged k-tile loads the 64 positions before its end: the plan gives this tile no k below 64.)
+    // (A single ragged k-tile loads the 64 positions before it: the plan gives this tile no k below 64.)
     unsigned stage = lds0;
     for (int kt = 0; kt < nk; ++kt) {
         if (kt + 2 >= nk) {

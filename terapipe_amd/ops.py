@@ -486,6 +486,49 @@ def cross_entropy_(logits, target, V, grad_scale=1.0):
     return loss
 
 
+EMBEDDING_ROWS_MAX = 8192       # tokens of one embedding_bwd_rows_ call
+
+
+def embedding_rows_fit(ids, dout):
+    """Whether embedding_bwd_rows_ takes the call: rows of whole 16-byte chunks, aligned, and not too many of them."""
+    return ids.numel() <= EMBEDDING_ROWS_MAX and dout.shape[1] * dout.element_size() % 16 == 0 and dout.data_ptr() % 16 == 0
+
+
+def embedding_bwd_rows_(ids, dout, dweight):
+    """dweight [V, E] += scatter of dout [M, E] by ids, in dweight's own dtype (one rounding per row)."""
+    _require_cuda(ids, dout, dweight)
+    V, E = dweight.shape
+    lib = _lib.load()
+    _lib.check(lib.tp_embedding_bwd_rows(_p(ids), _p(dout), _p(dweight), ids.numel(), E, V, tp_dtype(dout.dtype), _stream()),
+               "tp_embedding_bwd_rows")
+    return dweight
+
+
+def cross_entropy_loss(logits, target, V):
+    """Per-row loss (fp32 [M]) of logits [M, >= V] and what cross_entropy_grad_ needs again (fp32 [M, 2])."""
+    _require_cuda(logits, target)
+    M = logits.shape[0]
+    loss = torch.empty(M, dtype=torch.float32, device=logits.device)
+    stats = torch.empty(M, 2, dtype=torch.float32, device=logits.device)
+    lib = _lib.load()
+    _lib.check(lib.tp_cross_entropy_loss(_p(logits), logits.stride(0), _p(target), _p(loss), _p(stats), M, V,
+                                         tp_dtype(logits.dtype), _stream()), "tp_cross_entropy_loss")
+    return loss, stats
+
+
+def cross_entropy_grad_(logits, target, stats, scale, V):
+    """logits [M, Vpad] <- (softmax - onehot) * scale[m], its columns from V on <- 0."""
+    _require_cuda(logits, target, stats, scale)
+    M, Vpad = logits.shape
+    lib = _lib.load()
+    for m0 in range(0, M, 65535):
+        m1 = min(M, m0 + 65535)
+        _lib.check(lib.tp_cross_entropy_grad(_p(logits[m0:m1]), logits.stride(0), _p(target[m0:m1]), _p(stats[m0:m1]),
+                                             _p(scale[m0:m1]), m1 - m0, V, Vpad, tp_dtype(logits.dtype), _stream()),
+                   "tp_cross_entropy_grad")
+    return logits
+
+
 def scale_rows_(x2d, scale_f32):
     _require_cuda(x2d, scale_f32)
     lib = _lib.load()

@@ -17,6 +17,7 @@ import torch.nn as nn
 
 from . import _layer_core as core
 from . import ops
+from ._autograd import engine_adds_to_grad
 from ._lib import TP_EPI_ACCUMULATE, TP_EPI_BIAS, TP_EPI_STORE, TP_GEMM_NN, TP_GEMM_NT, TP_GEMM_TN
 
 # reference transformer_models.py:16 -- kept for callers that import it; the kernels mask by index.
@@ -189,24 +190,6 @@ def _grads_can_go_in_place(w):
     return True
 
 
-def _engine_adds_to_grad(ctx, w, first):
-    """Whether the backward pass under way is going to add this node's gradients to the parameters' .grad and nobody looks
-    at them on the way: then the kernels can add them.  ctx.next_functions[first:] are the parameters' AccumulateGrad
-    nodes; under torch.autograd.grad they do not run (the query raises for captured leaves), and a hook on a parameter or
-    a graph of the backward itself (create_graph) needs the gradients as tensors."""
-    if torch.is_grad_enabled():
-        return False
-    nodes = ctx.next_functions[first:]
-    try:
-        for p, (node, _) in zip(w.values(), nodes):
-            if p._backward_hooks or getattr(p, "_post_accumulate_grad_hooks", None) or getattr(node, "variable", None) is not p \
-                    or not torch._C._will_engine_execute_node(node):
-                return False
-    except RuntimeError:
-        return False
-    return True
-
-
 class _GradOptions:
     """How a layer's backward hands its parameter gradients to autograd (TransformerLayer's two switches) and,
     for deferred weight gradients, the sequences under way (keyed by their K cache): the rows their forward has filled
@@ -265,7 +248,7 @@ class _LayerFunction(torch.autograd.Function):
 
     Forward and backward are one library call each (tp_layers_fwd, tp_layer_bwd).  The backward of a slice: the data
     gradients, the eight vector-parameter gradients as one launch, the four weight gradients as one grouped one.
-    Where every parameter already has a .grad that the engine is going to add to (_engine_adds_to_grad), or with
+    Where every parameter already has a .grad that the engine is going to add to (_autograd.engine_adds_to_grad), or with
     opts.in_place, the kernels add the gradients to it (the GEMM's accumulate epilogue, one rounding) and autograd gets
     None, instead of twelve tensors that autograd adds one elementwise kernel each.  opts.defer -- keep the slice's dY / X
     rows and take the weight gradients once per sequence, over all its rows, in the backward of the slice at position 0
@@ -368,7 +351,7 @@ class _LayerFunction(torch.autograd.Function):
                 if opts.inputs.get(key) is seq:
                     del opts.inputs[key]
                 rows = pend.rows
-        in_place = done and (opts.in_place or _engine_adds_to_grad(ctx, w, 3 if ctx.has_cache else 1)) \
+        in_place = done and (opts.in_place or engine_adds_to_grad(ctx, ctx.w, 3 if ctx.has_cache else 1)) \
             and _grads_can_go_in_place(w)
         wg_out, small_out, wg = (0,) * 4, (0,) * 8, (0,) * 8
         grads = {}

@@ -8,7 +8,8 @@ import torch.nn as nn
 from torch.nn import init
 
 from . import ops
-from ._lib import TP_EPI_STORE, TP_GEMM_NN, TP_GEMM_NT, TP_GEMM_TN
+from ._autograd import engine_adds_to_grad, grad_to_add_to
+from ._lib import TP_EPI_ACCUMULATE, TP_EPI_STORE, TP_GEMM_NN, TP_GEMM_NT, TP_GEMM_TN
 
 
 class _EmbeddingFunction(torch.autograd.Function):
@@ -16,19 +17,28 @@ class _EmbeddingFunction(torch.autograd.Function):
     def forward(ctx, ids, weight):
         flat = ids.reshape(-1).contiguous()
         out = ops.embedding_fwd(flat, weight)
-        ctx.save_for_backward(flat)
-        ctx.wshape, ctx.wdtype = weight.shape, weight.dtype
+        ctx.flat, ctx.weight = flat, weight
         return out.view(*ids.shape, weight.shape[1])
 
     @staticmethod
     def backward(ctx, dout):
-        (flat,) = ctx.saved_tensors
-        acc = torch.empty(ctx.wshape, dtype=torch.float32, device=dout.device)
+        """Into an existing .grad the rows that occur are added where they lie (a tied LM head has left its gradient
+        there by then: no dense gradient of the lookup is made, and none is added); otherwise they go into zeros."""
+        flat, weight = ctx.flat, ctx.weight
+        dout = dout.reshape(flat.numel(), -1).contiguous()
+        if ops.embedding_rows_fit(flat, dout):
+            grad = grad_to_add_to(ctx, weight, 1)
+            if grad is not None and grad.data_ptr() % 16 == 0:
+                ops.embedding_bwd_rows_(flat, dout, grad)
+                return None, None
+            dw = torch.zeros(weight.shape, dtype=weight.dtype, device=dout.device)
+            return None, ops.embedding_bwd_rows_(flat, dout, dw)
+        acc = torch.empty(weight.shape, dtype=torch.float32, device=dout.device)
         ops.zero_(acc)
-        ops.embedding_bwd(flat, dout.reshape(flat.numel(), -1).contiguous(), acc)
-        if ctx.wdtype == torch.float32:
+        ops.embedding_bwd(flat, dout, acc)
+        if weight.dtype == torch.float32:
             return None, acc
-        dw = torch.empty(ctx.wshape, dtype=ctx.wdtype, device=dout.device)
+        dw = torch.empty_like(weight)
         ops.accum_cast(dw, acc, False)
         return None, dw
 
@@ -51,43 +61,52 @@ class VocabParallelEmbedding(nn.Module):
         return _EmbeddingFunction.apply(input_, self.weight)
 
 
-VOCAB_PAD = 64      # the 256-row GEMM tiles take whole 64-wide k-tiles: the data-gradient GEMM has k = vocabulary
+VOCAB_PAD = 64      # logits rows are whole 128-byte lines
 
 
 def _pad_vocab(n):
     return (n + VOCAB_PAD - 1) // VOCAB_PAD * VOCAB_PAD
 
 
+def _as_operand(weight):
+    """The weight where a GEMM can read it: itself, or a copy where it is strided or not 16-byte aligned."""
+    weight = weight.contiguous()
+    return weight.clone() if weight.data_ptr() % 16 else weight
+
+
 class _LMHeadFunction(torch.autograd.Function):
-    """logits = h W^T with the vocabulary padded to a multiple of 64 columns for the GEMMs (the padding rows
-    of the weight copy are zero; the padding columns of the logits are ignored by the loss)."""
+    """logits = h W^T, rows padded to a multiple of 64 columns (zeros; the loss ignores them)."""
 
     @staticmethod
     def forward(ctx, h2d, weight):
         V, E = weight.shape
         Vp = _pad_vocab(V)
-        wp = weight
-        if Vp != V:
-            wp = torch.zeros(Vp, E, dtype=weight.dtype, device=weight.device)
-            wp[:V].copy_(weight)
         h2d = h2d.contiguous()
         logits = torch.empty(h2d.shape[0], Vp, dtype=h2d.dtype, device=h2d.device)
-        ops.gemm(TP_GEMM_NT, h2d, wp, h2d.shape[0], Vp, E, C=logits, epilogue=TP_EPI_STORE)
-        ctx.save_for_backward(h2d, wp)
-        ctx.V = V
+        ops.gemm(TP_GEMM_NT, h2d, _as_operand(weight), h2d.shape[0], V, E, C=logits, epilogue=TP_EPI_STORE)
+        if Vp != V:
+            logits[:, V:].zero_()
+        ctx.save_for_backward(h2d, weight)
         return logits
 
     @staticmethod
     def backward(ctx, dlogits):
-        h2d, wp = ctx.saved_tensors
+        h2d, weight = ctx.saved_tensors
         M, E = h2d.shape
-        Vp = wp.shape[0]
+        V = weight.shape[0]
         dlogits = dlogits.contiguous()
         dh = torch.empty_like(h2d)
-        ops.gemm(TP_GEMM_NN, dlogits, wp, M, E, Vp, C=dh)
-        dwp = torch.empty_like(wp)
-        ops.gemm(TP_GEMM_TN, dlogits, h2d, Vp, E, M, C=dwp)
-        return dh, dwp[:ctx.V]
+        ops.gemm(TP_GEMM_NN, dlogits, _as_operand(weight), M, E, V, C=dh)
+        grad = grad_to_add_to(ctx, weight, 1)
+        if grad is not None and grad.data_ptr() % 16 == 0:
+            ops.gemm(TP_GEMM_TN, dlogits, h2d, V, E, M, C=grad, epilogue=TP_EPI_ACCUMULATE)
+            return dh, None
+        dw = torch.empty(weight.shape, dtype=weight.dtype, device=weight.device)
+        ops.gemm(TP_GEMM_TN, dlogits, h2d, V, E, M, C=dw)
+        if weight.grad is None and engine_adds_to_grad(ctx, (weight,), 1):
+            weight.grad = dw        # as the engine would; an embedding tied to this weight adds its rows to it
+            return dh, None
+        return dh, dw
 
 
 def lm_head_logits(h2d, weight):
@@ -97,29 +116,37 @@ def lm_head_logits(h2d, weight):
 
 
 class _CrossEntropyFunction(torch.autograd.Function):
+    """Forward: the per-token losses, one read of the logits.  Backward: the logits become their gradient, scaled, in one
+    read and one write (the reference keeps its softmax in the logits' memory and scales it, :74, :97)."""
+
     @staticmethod
     def forward(ctx, logits, target, vocab_size):
         shape = target.shape
         l2 = logits.reshape(-1, logits.shape[-1])
         if not l2.is_contiguous():
             raise ValueError("vocab_parallel_cross_entropy overwrites its logits in place and needs them contiguous")
-        loss = ops.cross_entropy_(l2, target.reshape(-1).contiguous(), vocab_size, 1.0)
-        # l2 now holds softmax - onehot, as the reference keeps its softmax (:74).  The overwrite goes through
-        # the raw pointer: the logits are the output of a GEMM whose backward does not read them.
-        ctx.g2 = l2.detach()
+        flat = target.reshape(-1).contiguous()
+        loss, stats = ops.cross_entropy_loss(l2, flat, vocab_size)
+        # (the overwrite goes through the raw pointer: the logits are the output of a GEMM whose backward does not read
+        # them)
+        ctx.kept = l2.detach(), flat, stats, vocab_size
         ctx.lshape = logits.shape
         return loss.view(shape)
 
     @staticmethod
     def backward(ctx, grad_output):
-        g2 = ctx.g2
-        ops.scale_rows_(g2, grad_output.reshape(-1).to(torch.float32).contiguous())
-        return g2.view(ctx.lshape), None, None
+        l2, flat, stats, vocab_size = ctx.kept
+        scale = grad_output.reshape(-1).to(torch.float32).contiguous()
+        if flat is None:            # a second backward: the logits are gone, their gradient is scaled once more
+            ops.scale_rows_(l2, scale)
+            return l2.view(ctx.lshape), None, None
+        ctx.kept = l2, None, None, None
+        return ops.cross_entropy_grad_(l2, flat, stats, scale, vocab_size).view(ctx.lshape), None, None
 
 
 def vocab_parallel_cross_entropy(vocab_parallel_logits, target, vocab_size=None):
-    """Per-token loss log(sum exp logits) - logits[target] (mpu/cross_entropy.py:109-110).  Like the reference
-    it overwrites the logits (there with the softmax, here directly with softmax - onehot).  vocab_size:
-    number of valid leading columns when the logits come from lm_head_logits with a padded vocabulary."""
+    """Per-token loss log(sum exp logits) - logits[target] (mpu/cross_entropy.py:109-110).  Like the reference's, its
+    backward overwrites the logits (with their gradient).  vocab_size: number of valid leading columns when the logits
+    come from lm_head_logits with a padded vocabulary."""
     V = vocab_parallel_logits.shape[-1] if vocab_size is None else vocab_size
     return _CrossEntropyFunction.apply(vocab_parallel_logits, target, V)

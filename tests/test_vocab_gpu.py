@@ -1,0 +1,100 @@
+"""The kernels of the two ends of the stack at their edges: gradient rows of the embedding, loss and gradient of the
+cross-entropy, products over a vocabulary that is no multiple of 8, and where their gradients end up."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from tests.util import assert_close
+
+DEV = "cuda"
+DTYPES = pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16], ids=str)
+pytestmark = pytest.mark.gpu
+
+
+@DTYPES
+@pytest.mark.parametrize("M,E,V", [(1, 8, 1), (511, 264, 3), (513, 2056, 700), (1100, 16, 2000), (8192, 64, 5)], ids=str)
+def test_embedding_rows(dtype, M, E, V):
+    from terapipe_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(M)
+    ids = torch.randint(-1, V + 1, (M,), generator=g, device=DEV)       # ids outside the vocabulary add nothing
+    dout = (torch.randn(M, E, generator=g, device=DEV) / 16).to(dtype)
+    dw = torch.randn(V, E, generator=g, device=DEV).to(dtype)
+    inside = (ids >= 0) & (ids < V)
+    ref = dw.double().index_add(0, ids[inside], dout.double()[inside])
+    ops.embedding_bwd_rows_(ids, dout, dw)
+    assert_close(dw, ref, dtype, "rows")
+
+
+@DTYPES
+@pytest.mark.parametrize("M,V,ld,shift", [(1, 1, 8, 0), (3, 8192, 8192, 0), (5, 8191, 8200, 0), (2, 40001, 40064, 0),
+                                          (7, 777, 779, 0), (4, 1000, 1008, 1)], ids=str)
+def test_loss_and_gradient(dtype, M, V, ld, shift):
+    """Whole and ragged chunks; rows of odd length and rows that are not aligned take the scalar kernels."""
+    from terapipe_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(V)
+    buf = (torch.randn(M * ld + shift, generator=g, device=DEV) * 3).to(dtype)
+    z = buf[shift:].view(M, ld)
+    target = torch.randint(0, V, (M,), generator=g, device=DEV)
+    scale = torch.rand(M, generator=g, device=DEV)
+    zr = z[:, :V].double().clone().requires_grad_(True)
+    ref = F.cross_entropy(zr, target, reduction="none")
+    (ref * scale.double()).sum().backward()
+    loss, stats = ops.cross_entropy_loss(z, target, V)
+    assert_close(loss, ref, torch.float32, "loss", 1.0 if dtype == torch.float32 else 10.0)
+    ops.cross_entropy_grad_(z, target, stats, scale, V)
+    assert_close(z[:, :V], zr.grad, dtype, "gradient")
+    assert not z[:, V:].any()
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=str)
+@pytest.mark.parametrize("V", [1, 9, 257, 4097, 50257])
+@pytest.mark.parametrize("M", [1, 40, 300])
+def test_ragged_vocabulary(dtype, V, M):
+    """N of NT, k of NN and M of TN, none a multiple of 8."""
+    import terapipe_amd as ta
+    E = 256
+    g = torch.Generator(device=DEV).manual_seed(V + M)
+    h = torch.randn(M, E, generator=g, device=DEV).to(dtype).requires_grad_(True)
+    w = (torch.randn(V, E, generator=g, device=DEV) * 0.05).to(dtype).requires_grad_(True)
+    logits = ta.lm_head_logits(h, w)
+    assert not logits[:, V:].any()
+    dl = torch.randn(logits.shape, generator=g, device=DEV).to(dtype)
+    dl[:, V:] = 0
+    logits.backward(dl)
+    hd, wd = h.detach().double(), w.detach().double()
+    assert_close(logits[:, :V], hd @ wd.t(), dtype, "logits")
+    assert_close(h.grad, dl[:, :V].double() @ wd, dtype, "dh")
+    assert_close(w.grad, dl[:, :V].double().t() @ hd, dtype, "dw")
+
+
+@DTYPES
+@pytest.mark.parametrize("tied", [False, True])
+def test_where_gradients_go(dtype, tied):
+    """Into fresh and into existing gradients, of tied and of separate weights, with autograd's hooks and with
+    torch.autograd.grad: all the same sums."""
+    import terapipe_amd as ta
+    V, E, M = 203, 64, 90
+    g = torch.Generator().manual_seed(3)
+    emb = ta.VocabParallelEmbedding(V, E, device=DEV, dtype=dtype)
+    head = emb.weight if tied else torch.nn.Parameter(torch.randn(V, E, generator=g).mul(0.1).to(dtype).to(DEV))
+    params = [emb.weight] if tied else [emb.weight, head]
+    ids, target = (torch.randint(0, V, (M,), generator=g).to(DEV) for _ in range(2))
+
+    def loss():
+        return ta.vocab_parallel_cross_entropy(ta.lm_head_logits(emb(ids) * 4, head), target, vocab_size=V).sum()
+
+    ws = [p.detach().double().requires_grad_(True) for p in params]
+    F.cross_entropy(F.embedding(ids, ws[0]) * 4 @ ws[-1].t(), target, reduction="sum").backward()
+    for got, w in zip(torch.autograd.grad(loss(), params), ws):
+        assert_close(got, w.grad, dtype, "torch.autograd.grad")
+    assert all(p.grad is None for p in params)
+    for times in (1, 2):
+        loss().backward()
+        for p, w in zip(params, ws):
+            assert_close(p.grad, times * w.grad, dtype, "backward %d" % times)
+    seen = []
+    handle = params[0].register_hook(lambda t: seen.append(t.detach().clone()))
+    loss().backward()
+    handle.remove()
+    assert_close(sum(seen), ws[0].grad, dtype, "what a hook sees")
+    assert_close(params[0].grad, 3 * ws[0].grad, dtype, "backward with a hook")
