@@ -107,7 +107,7 @@ class _StackBuffers:
         # the pieces a step runs in
         self.pieces = runner.seq_slices
         if runner.merge_slices:
-            self.pieces = merged_slices(runner.seq_slices, max(runner.batch_slices), E)
+            self.pieces = [L]       # (merges says when and why)
         gdt = torch.float32 if runner.fp32_grad_cache else dtype
         kw = dict(dtype=dtype, device=device)
         f32 = dict(dtype=torch.float32, device=device)
@@ -216,12 +216,12 @@ def _flat_views(flat, layout):
     return [{n: flat[o:o + int(np.prod(s))].view(s) for n, (o, s) in d.items()} for d in layout]
 
 
-# The slices that stay as they are (rows of one on average, rows of all, hidden size): see merged_slices.
-MERGE_KEEP_ROWS, MERGE_KEEP_TOTAL, MERGE_KEEP_HIDDEN = 256, 2048, 2048
+# Where a runner with slice_streams=1 merges too (rows of a slice on average, rows of all, hidden size): see merges.
+MERGE_ONE_STREAM_ROWS, MERGE_ONE_STREAM_TOTAL, MERGE_ONE_STREAM_HIDDEN = 256, 2048, 2048
 
 
-def merged_slices(seq_slices, batch, hidden):
-    """The pieces a single-stage step runs the sequence in: the whole sequence as one, but for the exception below.
+def merges(seq_slices, batch, hidden, slice_streams):
+    """Whether a single-stage step runs the sequence in one piece.  slice_streams: what the caller set, None if nothing.
 
     Slices are the unit in which pipeline STAGES hand work to each other.  One runner holds every slice of its stage
     from the start, and what its step computes does not depend on where the sequence is cut: every operation of a layer
@@ -232,14 +232,16 @@ def merged_slices(seq_slices, batch, hidden):
     21.0.  Two pieces on two streams, which fill each other's last waves of tiles, are level or slower with the tiles
     chosen for whole rounds of the chip (44.7 and 22.3; hidden 4096: 8.8 against 8.2).
 
-    Slices of MERGE_KEEP_ROWS rows and more, MERGE_KEEP_TOTAL together, on a hidden size up to MERGE_KEEP_HIDDEN stay as
-    they are: there the lanes' products share the weights through the memory-side cache and merging gains least
-    (8 x 256 rows of hidden 2048: 6.0 ms -> 4.6), and the step keeps giving the bits of the same slices run one after
-    the other."""
+    A caller that sets slice_streams asks for slices on that many streams.  The exception: one stream, slices of
+    MERGE_ONE_STREAM_ROWS rows and more, MERGE_ONE_STREAM_TOTAL together, on a hidden size up to MERGE_ONE_STREAM_HIDDEN.
+    A slice of that size fills a row of tiles but not the chip, which one stream leaves idle otherwise (8 x 256 rows of
+    hidden 2048 on three streams: 6.0 ms, in one piece 4.6), and a runner on one stream gives the same bits there as the
+    default one, whose launches it is the plain version of."""
+    if slice_streams is None:
+        return True
     rows = sum(seq_slices) * batch
-    if MERGE_KEEP_ROWS * len(seq_slices) <= rows <= MERGE_KEEP_TOTAL and hidden <= MERGE_KEEP_HIDDEN:
-        return list(seq_slices)
-    return [sum(seq_slices)]
+    return (slice_streams == 1 and MERGE_ONE_STREAM_ROWS * len(seq_slices) <= rows <= MERGE_ONE_STREAM_TOTAL
+            and hidden <= MERGE_ONE_STREAM_HIDDEN)
 
 
 def fused_backward_slices(seq_slices, n_lanes, window=None):
@@ -720,10 +722,10 @@ class TeraPipe(nn.Module):
     run through the stack side by side.  Same kernels, same arguments, same results; the overlap fills the
     chip where one chain of short kernels cannot, and GEMMs that stream the same weight at the same time
     share its way through the caches.  Default 3 (1 under use_hip_graph).
-    merge_slices: the step runs the sequence in one piece instead of slice by slice (merged_slices says why and
-    when), with the same results up to rounding.  None (the default): where the caller leaves the way the step runs to
-    the runner.  A caller that sets slice_streams asks for its slices on that many streams (1: one after the other, as
-    on a stage that gets them one by one), suffix_dkdv=False and fp32_grad_cache=False for the hand-over of cache
+    merge_slices: the step runs the sequence in one piece instead of slice by slice (merges says why and when), with
+    the same results up to rounding.  None (the default): where the caller leaves the way the step runs to the runner.
+    A caller that sets slice_streams asks for its slices on that many streams (1: one after the other, as on a stage
+    that gets them one by one; but see merges), suffix_dkdv=False and fp32_grad_cache=False for the hand-over of cache
     gradients from slice to slice, several batch slices for that grid: those run as they are cut, and so does a step
     whose slices are timed (slice_timing).
     launch_replay: the first step runs as written, the second also keeps every library call it makes (bound
@@ -754,7 +756,8 @@ class TeraPipe(nn.Module):
         self.suffix_dkdv = suffix_dkdv
         self.fused_attn_bwd = bool(fused_attn_bwd)
         self.merge_slices = bool(merge_slices) if merge_slices is not None else (
-            slice_streams is None and not use_hip_graph and suffix_dkdv and fp32_grad_cache and len(self.batch_slices) == 1)
+            merges(self.seq_slices, batch_size, layers.embedding_dim, slice_streams)
+            and not use_hip_graph and suffix_dkdv and fp32_grad_cache and len(self.batch_slices) == 1)
         # defaults: three slice streams and launch replay; one stream and no replay under use_hip_graph
         self.slice_streams = int(slice_streams) if slice_streams is not None else (1 if use_hip_graph else 3)
         self.launch_replay = bool(launch_replay) if launch_replay is not None else not use_hip_graph

@@ -7,13 +7,11 @@ from tests.util import assert_close, load_params_into, make_params
 
 
 def test_rule():
-    from terapipe_amd.terapipe import merged_slices
-    assert merged_slices([32] * 64, 1, 6144) == [2048]
-    assert merged_slices([16] * 8, 2, 256) == [128]
-    assert merged_slices([256] * 8, 1, 2048) == [256] * 8               # long slices, small weights: kept
-    assert merged_slices([255] * 8, 1, 2048) == [2040]
-    assert merged_slices([256] * 8, 1, 2056) == [2048]
-    assert merged_slices([256] * 8, 2, 2048) == [2048]
+    from terapipe_amd.terapipe import merges
+    for case in (([32] * 64, 1, 6144), ([16] * 8, 2, 256), ([256] * 8, 1, 2048), ([2048] * 2, 8, 8192)):
+        assert merges(*case, None) and not merges(*case, 3)
+    assert merges([256] * 8, 1, 2048, 1)                # long slices, small weights: on one stream too
+    assert not any(merges(*case, 1) for case in (([255] * 8, 1, 2048), ([256] * 8, 1, 2056), ([256] * 8, 2, 2048)))
 
 
 def test_who_merges():
@@ -32,10 +30,9 @@ def test_who_merges():
     (160, 2, 16, [100, 31], torch.float16, [131]),                # head dimension 80
     (128, 2, 3, [7, 1, 30, 27], torch.float32, [65]),             # gradient caches
 ], ids=str)
-def test_merged_step_against_the_oracle(E, H, B, slices, dtype, pieces, monkeypatch):
+def test_merged_step_against_the_oracle(E, H, B, slices, dtype, pieces):
     """Three steps (eager, recorded, re-issued) of the default runner, GeLU so that no sign decision is involved."""
     import terapipe_amd as ta
-    monkeypatch.setattr(ta.terapipe, "MERGE_KEEP_HIDDEN", 0)
     L, nl = sum(slices), 2
     ps = make_params(nl, E, 4 * E, dtype, seed=5)
     layers = ta.TransformerLayers(nl, E, 4 * E, H, dtype=dtype, device="cuda", activation="gelu")
