@@ -104,7 +104,7 @@ def build_model(w, device):
         for p in layers.parameters():
             if p.dim() == 2:   # weights N(0, std); biases stay 0, LayerNorm gamma 1 / beta 0
                 p.copy_((torch.randn(p.shape, generator=g) * w["std"]).to(dt))
-    runner = ta.TeraPipe(layers, w["B"], w["L"], [w["B"]], w["slices"], slice_streams=1, launch_replay=False)
+    runner = ta.TeraPipe(layers, w["B"], w["L"], [w["B"]], w["slices"])
     x = torch.randn(w["L"], w["B"], w["E"], generator=g).to(dt).to(device)
     R = torch.randn(w["L"], w["B"], w["E"], generator=g).to(dt).to(device)
     return layers, runner, x, R
@@ -344,14 +344,18 @@ def _graph_ms(fns, reps=3):
 
 def measure_workload(name, args, device, detail):
     """Times `name`: tokens/s over args.steps steps after args.warmup, then (unless --no-roofline) the kernel
-    times of one recorded step per kind.  detail: also per GEMM shape."""
+    times of one recorded step per kind.  detail: also per GEMM shape.  The runner is the one a user constructs: it runs
+    the workload's slices in one piece.  With --slice-streams they run slice by slice on that many streams; without it
+    both sliced forms are timed beside the figure."""
     from terapipe_amd import ops
     w = WORKLOADS[name]
     args = argparse.Namespace(**vars(args))
+    merge = args.slice_streams is None
     args.slice_streams = args.slice_streams or w.get("streams", 3)
     layers, runner, x, R = build_model(w, device)
     runner.use_hip_graph = args.graph
     runner.slice_streams = args.slice_streams
+    runner.merge_slices = merge
     runner.fused_attn_bwd = not args.two_launch_attn_bwd
     runner.launch_replay = not (args.graph or args.no_launch_replay)
     warmup, steps = (args.warmup, args.steps) if detail else (3, 5)
@@ -374,7 +378,12 @@ def measure_workload(name, args, device, detail):
            "ms_per_step": elapsed * 1e3 / steps, "tokens_per_s": w["L"] * w["B"] * steps / elapsed,
            "ms_per_step_std": (sum((t - mean) ** 2 for t in per_step) / steps) ** 0.5,
            "ms_per_step_min": min(per_step), "ms_per_step_max": max(per_step),
-           "slice_streams": args.slice_streams}
+           "pieces": 1 if merge else len(w["slices"]), "slice_streams": 1 if merge else args.slice_streams}
+    if merge and not args.no_one_stream:
+        runner.merge_slices = False
+        mss = timed_steps(lambda: one_step(layers, runner, x, R), 3, 5)
+        res["ms_per_step_sliced"], res["tokens_per_s_sliced"] = mss, w["L"] * w["B"] / (mss * 1e-3)
+        res["sliced_slice_streams"] = args.slice_streams
     if args.slice_streams > 1 and not args.graph and not args.no_one_stream:
         # the same step with ONE slice stream: slice i+1 starts when slice i has left the stack, as on a pipeline
         # stage that receives its slices from an upstream stage (terapipe.py:249-264); recorded launches re-issued
@@ -383,6 +392,7 @@ def measure_workload(name, args, device, detail):
         res["ms_per_step_one_stream"] = ms1
         res["tokens_per_s_one_stream"] = w["L"] * w["B"] / (ms1 * 1e-3)
         runner.slice_streams = args.slice_streams
+        runner.merge_slices = merge
     if detail and w["dtype"] != "f32" and not args.no_layer_surface:
         msl = timed_steps(lambda: layer_surface_step(layers, x, R, w), 2, 4)
         msi = timed_steps(lambda: layer_surface_step(layers, x, R, w, in_place=True), 2, 4)
@@ -410,6 +420,15 @@ def measure_workload(name, args, device, detail):
     # include the time the GPU waits for the host).
     runner.use_hip_graph = False
     runner.launch_replay = False
+    # (the attention roofline is stated for the workload's slices: its calls come from a sliced step)
+    runner.merge_slices = False
+    for p in layers.parameters():
+        p.grad = None
+    with ops.CallRecorder() as sliced_rec:
+        one_step(layers, runner, x, R)
+    torch.cuda.synchronize()
+    sliced_keep = runner._sbufs, [p.grad for p in layers.parameters()]
+    runner.merge_slices = merge
     with ops.CallRecorder() as rec:
         one_step(layers, runner, x, R)
     torch.cuda.synchronize()
@@ -419,7 +438,7 @@ def measure_workload(name, args, device, detail):
     es = 4 if w["dtype"] == "f32" else 2
     peak = PEAK_MFMA_FP32 if w["dtype"] == "f32" else PEAK_MFMA_16BIT
 
-    def calls_of(tag):
+    def calls_of(tag, rec=rec):
         # "attn_bwd" covers both launches of the attention backward of a slice: delta + dQ, and the
         # one-pass dK/dV over all later positions
         return [c for c in rec.calls if c[0] == tag or (tag == "attn_bwd" and c[0] == "attn_bwd_dkdv")]
@@ -486,7 +505,7 @@ def measure_workload(name, args, device, detail):
         roof["per_gemm_note"] = ("avg_us is the launch alone on the chip with the plan the step uses; in_step_pick marks "
                                  "the shapes whose plan was chosen by timing whole steps on the slice streams (fewer k "
                                  "splits than the fastest plan alone), so vendor_us may be below avg_us there")
-    if args.slice_streams > 1:
+    if args.slice_streams > 1 and not merge:
         # the same GEMM calls as the step issues them: spread over the slice streams, so that a launch
         # which fills part of the chip runs beside its neighbours'.  Launched from the host (closures
         # bound to their descriptors), bracketed by two events on the current stream.  Every chain has a
@@ -522,9 +541,9 @@ def measure_workload(name, args, device, detail):
     res["roofline"] = roof
     attn = {}
     kt = {"gemm": round(g_ms, 3)}
-    has_suffix = any(c[0] == "attn_bwd_dkdv" for c in rec.calls)
+    has_suffix = any(c[0] == "attn_bwd_dkdv" for c in sliced_rec.calls)
     for tag in ("attn_fwd", "attn_bwd"):
-        calls = calls_of(tag)
+        calls = calls_of(tag, sliced_rec)
         ms = _graph_ms([fn for _, _, fn in calls]) if calls else 0.0
         metas = [m for t, m, _ in calls if t == tag]     # one per slice and layer
         nbytes = sum(attn_bytes_per_call(es, w["B"], w["H"], w["E"], T, P, tag == "attn_bwd") for (_b, _h, _d, T, P) in metas)
@@ -532,6 +551,10 @@ def measure_workload(name, args, device, detail):
         attn[tag] = {"calls": len(metas), "launches_per_call": 2 if tag == "attn_bwd" and has_suffix else 1,
                      "kernel_ms_per_step": ms, "algorithmic_GB_per_step": nbytes / 1e9,
                      "achieved_GBps": gbs, "frac_of_hbm_peak": gbs * 1e9 / PEAK_HBM}
+        if merge:
+            calls = calls_of(tag)
+            ms = _graph_ms([fn for _, _, fn in calls]) if calls else 0.0
+            attn[tag]["kernel_ms_per_step_in_one_piece"] = ms
         kt[tag] = round(ms, 3)
     for tag in ("layernorm_fwd", "layernorm_bwd"):
         calls = calls_of(tag)
@@ -539,7 +562,7 @@ def measure_workload(name, args, device, detail):
     res["roofline_attention"] = {"bound": "hbm", "peak": PEAK_HBM / 1e9, "unit": "GB/s",
                                  "slice_tokens": sorted(set(w["slices"])), **attn}
     res["kernel_time_ms_per_step"] = kt
-    del recorded_grads
+    del recorded_grads, sliced_keep
     return res, (layers, runner, x, R)
 
 
@@ -703,8 +726,8 @@ def main():
                     help="also run one plain 256 MiB device fill and one 256 MiB copy before the steps: the "
                          "known-size kernels that rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE readings are scaled by")
     ap.add_argument("--slice-streams", type=int, default=None,
-                    help="streams the runner spreads consecutive slices over (default: the workload's own, 3 except "
-                         "C2's 4; 1 = one chain of kernels); slice "
+                    help="run slice by slice, with consecutive slices spread over this many streams (default: the slices in "
+                         "one piece; the sliced figure beside it uses 3 streams, C2's 4; 1 = one chain of kernels); slice "
                          "i+1 of layer l runs beside slice i of layer l+1, which fills the CUs the short kernels "
                          "of one slice leave idle")
     ap.add_argument("--optimizer", action="store_true",
@@ -771,14 +794,17 @@ def main():
                    "launch": "HIP-graph replay of forward and of backward" if args.graph else
                              ("eager, every kernel launched from the host" if args.no_launch_replay else
                               "eager, recorded launches re-issued from the host"),
-                   "slice_streams": res["slice_streams"]},
+                   "pieces": res["pieces"], "slice_streams": res["slice_streams"]},
     }
-    for k in ("ms_per_step_one_stream", "tokens_per_s_one_stream", "layer_surface", "roofline", "kernel_time_ms_per_step"):
+    for k in ("ms_per_step_sliced", "tokens_per_s_sliced", "sliced_slice_streams", "ms_per_step_one_stream", "tokens_per_s_one_stream", "layer_surface", "roofline", "kernel_time_ms_per_step"):
         if k in res:
             out[k] = res[k]
     if "ms_per_step_one_stream" in res:
-        out["one_stream_note"] = ("value / ms_per_step overlap three consecutive slices on three streams of the one GPU; "
-                                  "*_one_stream run one slice at a time, as a pipeline stage fed by an upstream stage does")
+        out["one_stream_note"] = ("value / ms_per_step: the runner as constructed by default; pieces = 1: it runs the "
+                                  "sequence's slices in one piece on one stream, every position's forward, backward and "
+                                  "parameter gradients as in the sliced step; *_sliced overlap consecutive slices on "
+                                  "sliced_slice_streams streams; *_one_stream run one slice at a time, as a pipeline stage "
+                                  "fed by an upstream stage does")
     if "roofline_attention" in res:
         out["roofline_attention"] = dict(res["roofline_attention"], workload=args.workload)
     if args.optimizer and w["dtype"] != "f32":
