@@ -387,6 +387,8 @@ typedef struct tp_layer_desc {
     void* h; float* mean2; float* rstd2;
     void* hn; void* a; void* z;         /* z: GeLU's pre-activation, NULL for ReLU */
     void* out;                          /* [T*B, E] */
+    int64_t ldw[4];                     /* elements from row to row of the in_proj, out_proj, fc1 and fc2 weight;
+                                           0: the rows lie one after the other */
 } tp_layer_desc;
 
 /* n layers in a chain (layers[i].x == layers[i-1].out).  Layers may share every buffer but x and out (forward only). */

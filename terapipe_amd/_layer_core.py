@@ -213,9 +213,22 @@ def layer_bwd(w, st, dout, heads, gk, gv, accumulate_prefix, has_incoming, zero_
 # A layer is nine to fifteen launches; issued one by one through ops.py each costs about 11 us of Python, which bounds
 # short slices from the host.
 # ------------------------------------------------------------------------------------------------
-_FWD_PACK = struct.Struct("8iq28Q")            # tp_layer_desc
+_FWD_PACK = struct.Struct("8iq28Q4q")          # tp_layer_desc
 _BWD_PACK = struct.Struct("12Q4iq8Q4Q2i8Q2i")  # tp_layer_bwd_desc after its tp_layer_desc
 _ACTIVATIONS = {"relu": 0, "gelu": 1}
+
+
+def operands(params):
+    """(addresses, ldw) of a layer's 12 parameters in PARAM_NAMES order, as tp_layer_desc has them.  A weight may be a
+    column range of a wider matrix; what no kernel can read is refused."""
+    ldw = [0, 0, 0, 0]
+    for i, p in enumerate(params):
+        if not p.is_contiguous():
+            if p.dim() != 2 or p.stride(1) != 1 or p.stride(0) < p.shape[1]:
+                raise _lib.TeraPipeHipError("%s: strides %s; a vector, and each row of a weight, has to be contiguous"
+                                            % (PARAM_NAMES[i], tuple(p.stride())))
+            ldw[(2, 4, 8, 10).index(i)] = p.stride(0)
+    return [p.data_ptr() for p in params], ldw
 
 
 class _Arena:
@@ -259,9 +272,10 @@ class LayerGeometry:
             g = cls._cache[key] = cls(*key)
         return g
 
-    def pack_fwd(self, image, at, cache_len, cache_rows, w_ptrs, x, k, v, base, out, over=None):
-        """Writes a tp_layer_desc at byte `at` of `image`.  base: address of the forward arena; over: addresses that take
+    def pack_fwd(self, image, at, cache_len, cache_rows, params, x, k, v, base, out, over=None):
+        """Writes a tp_layer_desc at byte `at` of `image`.  params: the layer's 12; base: address of the forward arena; over: addresses that take
         the place of the arena's."""
+        w_ptrs, ldw = operands(params)
         o = self.fwd.off
         p = {n: base + o[n] for n in o}
         if over:
@@ -269,7 +283,7 @@ class LayerGeometry:
         _FWD_PACK.pack_into(image, at, self.dt, self.T, self.B, self.H, self.E, self.F, _ACTIVATIONS[self.activation],
                             cache_len, cache_rows, *w_ptrs, x, k, v, p["xn"], p["mean1"], p["rstd1"], p["q"], p["o"],
                             p["lse"], p["h"], p["mean2"], p["rstd2"], p["hn"], p["a"],
-                            p["z"] if self.activation == "gelu" else 0, out)
+                            p["z"] if self.activation == "gelu" else 0, out, *ldw)
 
 
 def _address(image):
@@ -321,7 +335,7 @@ def stack_forward_only(layers, x, caches, cache_len):
     for i, (params, _, _) in enumerate(layers):
         k, v = caches[i]
         dst = out.data_ptr() if i == n - 1 else base + geo.fwd.total + (i & 1) * step
-        geo.pack_fwd(image, i * _FWD_PACK.size, cache_len, k.shape[1], [p.data_ptr() for p in params], src, k.data_ptr(),
+        geo.pack_fwd(image, i * _FWD_PACK.size, cache_len, k.shape[1], params, src, k.data_ptr(),
                      v.data_ptr(), base, dst)
         src = dst
     layers_fwd(image, n, x.device)

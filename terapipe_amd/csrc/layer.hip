@@ -9,12 +9,16 @@ namespace tp {
 
 enum { W_LN1_G, W_LN1_B, W_QKV, B_QKV, W_OUT, B_OUT, W_LN2_G, W_LN2_B, W_FC1, B_FC1, W_FC2, B_FC2 };
 
-static tp_gemm_desc gemm_desc(const tp_layer_desc& l, int op, int epi, int M, int N, int K, const void* A, const void* B, void* C) {
+enum { LD_QKV, LD_OUT, LD_FC1, LD_FC2, LD_DENSE = -1 };
+
+// weight: which of the layer's weights B is (its rows may be a column range of a wider matrix), LD_DENSE: none of them
+static tp_gemm_desc gemm_desc(const tp_layer_desc& l, int op, int epi, int M, int N, int K, const void* A, const void* B, void* C,
+                              int weight = LD_DENSE) {
     tp_gemm_desc d = {};
     d.op = op; d.dtype = l.dtype; d.epilogue = epi;
     d.M = M; d.N = N; d.K = K;
     d.A = A; d.lda = op == TP_GEMM_TN ? M : K;
-    d.B = B; d.ldb = op == TP_GEMM_NT ? K : N;
+    d.B = B; d.ldb = weight != LD_DENSE && l.ldw[weight] ? l.ldw[weight] : op == TP_GEMM_NT ? K : N;
     d.C = C; d.ldc = N;
     return d;
 }
@@ -58,17 +62,17 @@ static ForwardPlan forward_plan(const tp_layer_desc& l) {
     const int M = l.T * l.batch, E = l.hidden, F = l.ffn;
     ForwardPlan p;
     p.attn = attn_desc(l);
-    p.qkv = gemm_desc(l, TP_GEMM_NT, TP_EPI_QKV_SCATTER, M, 3 * E, E, l.xn, l.w[W_QKV], nullptr);
+    p.qkv = gemm_desc(l, TP_GEMM_NT, TP_EPI_QKV_SCATTER, M, 3 * E, E, l.xn, l.w[W_QKV], nullptr, LD_QKV);
     p.qkv.bias = l.w[B_QKV];
     p.qkv.q = l.q; p.qkv.k_cache = l.k_cache; p.qkv.v_cache = l.v_cache;
     p.qkv.batch = l.batch; p.qkv.heads = l.heads; p.qkv.head_dim = E / l.heads;
     p.qkv.cache_len = l.cache_len; p.qkv.cache_rows = l.cache_rows; p.qkv.q_scale = p.attn.q_scale;
-    p.out = gemm_desc(l, TP_GEMM_NT, TP_EPI_BIAS_RESIDUAL, M, E, E, l.o, l.w[W_OUT], l.h);
+    p.out = gemm_desc(l, TP_GEMM_NT, TP_EPI_BIAS_RESIDUAL, M, E, E, l.o, l.w[W_OUT], l.h, LD_OUT);
     p.out.bias = l.w[B_OUT]; p.out.residual = l.x; p.out.ldr = E;
-    p.fc1 = gemm_desc(l, TP_GEMM_NT, l.activation ? TP_EPI_BIAS_GELU : TP_EPI_BIAS_RELU, M, F, E, l.hn, l.w[W_FC1], l.a);
+    p.fc1 = gemm_desc(l, TP_GEMM_NT, l.activation ? TP_EPI_BIAS_GELU : TP_EPI_BIAS_RELU, M, F, E, l.hn, l.w[W_FC1], l.a, LD_FC1);
     p.fc1.bias = l.w[B_FC1];
     if (l.activation) { p.fc1.aux_out = l.z; p.fc1.ldauxo = F; }
-    p.fc2 = gemm_desc(l, TP_GEMM_NT, TP_EPI_BIAS_RESIDUAL, M, E, F, l.a, l.w[W_FC2], l.out);
+    p.fc2 = gemm_desc(l, TP_GEMM_NT, TP_EPI_BIAS_RESIDUAL, M, E, F, l.a, l.w[W_FC2], l.out, LD_FC2);
     p.fc2.bias = l.w[B_FC2]; p.fc2.residual = l.h; p.fc2.ldr = E;
     return p;
 }
@@ -78,11 +82,11 @@ static BackwardPlan backward_plan(const tp_layer_bwd_desc& b) {
     const tp_layer_desc& l = b.f;
     const int M = l.T * l.batch, E = l.hidden, F = l.ffn;
     BackwardPlan p;
-    p.dz1 = gemm_desc(l, TP_GEMM_NN, l.activation ? TP_EPI_GELU_GRAD : TP_EPI_RELU_GRAD, M, F, E, b.dout, l.w[W_FC2], b.dz1);
+    p.dz1 = gemm_desc(l, TP_GEMM_NN, l.activation ? TP_EPI_GELU_GRAD : TP_EPI_RELU_GRAD, M, F, E, b.dout, l.w[W_FC2], b.dz1, LD_FC2);
     p.dz1.aux = l.activation ? l.z : l.a; p.dz1.ldaux = F;
-    p.dhn = gemm_desc(l, TP_GEMM_NN, TP_EPI_STORE, M, E, F, b.dz1, l.w[W_FC1], b.dhn);
-    p.d_o = gemm_desc(l, TP_GEMM_NN, TP_EPI_STORE, M, E, E, b.dh, l.w[W_OUT], b.d_o);
-    p.dxn = gemm_desc(l, TP_GEMM_NN, TP_EPI_STORE, M, E, 3 * E, b.dqkv, l.w[W_QKV], b.dxn);
+    p.dhn = gemm_desc(l, TP_GEMM_NN, TP_EPI_STORE, M, E, F, b.dz1, l.w[W_FC1], b.dhn, LD_FC1);
+    p.d_o = gemm_desc(l, TP_GEMM_NN, TP_EPI_STORE, M, E, E, b.dh, l.w[W_OUT], b.d_o, LD_OUT);
+    p.dxn = gemm_desc(l, TP_GEMM_NN, TP_EPI_STORE, M, E, 3 * E, b.dqkv, l.w[W_QKV], b.dxn, LD_QKV);
     const int K = (int)b.wg_rows, epi = b.wg_accumulate ? TP_EPI_ACCUMULATE : TP_EPI_STORE;
     p.wg[0] = gemm_desc(l, TP_GEMM_TN, epi, 3 * E, E, K, b.wg_dqkv, b.wg_xn, b.wg_out[0]);
     p.wg[1] = gemm_desc(l, TP_GEMM_TN, epi, E, E, K, b.wg_dh, b.wg_o, b.wg_out[1]);

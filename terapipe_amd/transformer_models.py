@@ -281,8 +281,8 @@ class _LayerFunction(torch.autograd.Function):
                 seq.rows = r1
                 over = {n: getattr(seq, n)[r0:].data_ptr() for n in ("xn", "o", "hn", "a")}
         image = bytearray(core._FWD_PACK.size + core._BWD_PACK.size)
-        geo.pack_fwd(image, 0, cache_len, k_cache.shape[1], [p.data_ptr() for p in params], x.data_ptr(),
-                     k_cache.data_ptr(), v_cache.data_ptr(), arena.data_ptr(), out.data_ptr(), over)
+        geo.pack_fwd(image, 0, cache_len, k_cache.shape[1], params, x.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
+                     arena.data_ptr(), out.data_ptr(), over)
         core.layers_fwd(image, 1, dev)
         ctx.geo, ctx.cache_len, ctx.opts = geo, cache_len, opts
         ctx.image = image               # the descriptor's addresses stay valid: what they point to is kept

@@ -1,0 +1,77 @@
+"""What a layer's kernels are handed: strides of the parameters."""
+import pytest
+import torch
+
+from tests.util import assert_close
+
+
+def _layer(E, H, F, dtype, activation="gelu", seed=3, device="cuda"):
+    import terapipe_amd as ta
+    torch.manual_seed(seed)
+    layer = ta.ModelParallelTransformerLayer(E, F, H, device=device, activation=activation).to(dtype)
+    with torch.no_grad():
+        for p in layer.parameters():
+            p.add_(torch.randn_like(p) * 0.02)
+    return layer
+
+
+def _replace_weights(layer, change):
+    for m in (layer.attn.in_proj, layer.attn.out_proj, layer.fc1, layer.fc2):
+        m.weight = torch.nn.Parameter(change(m.weight.detach()))
+
+
+def _column_range(w, before=8, after=16):
+    """w as columns [before, before + K) of a wider matrix of other values."""
+    wide = torch.full((w.shape[0], before + w.shape[1] + after), 7.0, dtype=w.dtype, device=w.device)
+    wide[:, before:before + w.shape[1]] = w
+    return wide[:, before:before + w.shape[1]]
+
+
+def _forward_backward(layer, x, dy, P=3):
+    B, L = x.shape[1], P + x.shape[0]
+    H, Dh = layer.attn.num_heads, layer.attn.head_dim
+    g = torch.Generator(device="cuda").manual_seed(1)
+    caches = [torch.randn(B * H, L, Dh, generator=g, device="cuda").to(x.dtype).requires_grad_() for _ in range(2)]
+    x = x.clone().requires_grad_()
+    y, _ = layer(x, tuple(caches), P)
+    y.backward(dy)
+    with torch.no_grad():
+        y0, _ = layer(x, tuple(c.detach() for c in caches), P)
+    return [y.detach(), y0, x.grad] + [c.grad for c in caches] + [p.grad for p in layer.param_list()]
+
+
+def test_addresses_and_row_pitches():
+    from terapipe_amd import _layer_core as core
+    from terapipe_amd import _lib
+    layer = _layer(64, 1, 128, torch.float16, device="cpu")
+    ptrs, ldw = core.operands(layer.param_list())
+    assert ptrs == [p.data_ptr() for p in layer.param_list()] and ldw == [0] * 4
+    _replace_weights(layer, _column_range)
+    ptrs, ldw = core.operands(layer.param_list())
+    assert ptrs == [p.data_ptr() for p in layer.param_list()] and ldw == [64 + 24] * 3 + [128 + 24]
+    for change in (lambda w: w.t().contiguous().t(), lambda w: w[:1].expand(w.shape), lambda w: torch.cat([w, w], 1)[:, ::2]):
+        _replace_weights(layer, change)
+        with pytest.raises(_lib.TeraPipeHipError, match="in_proj.weight: strides"):
+            core.operands(layer.param_list())
+    layer = _layer(64, 1, 128, torch.float16, device="cpu")
+    layer.fc1.bias = torch.nn.Parameter(torch.zeros(256, dtype=torch.float16)[::2])
+    with pytest.raises(_lib.TeraPipeHipError, match="fc1.bias: strides"):
+        core.operands(layer.param_list())
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("T,dtype", [(5, torch.float16), (70, torch.bfloat16), (9, torch.float32)], ids=str)
+def test_weights_that_are_column_ranges(T, dtype):
+    """The same bits as from dense weights, with and without gradients (the sums over rows of the vector parameters'
+    gradients are atomic: their order is not fixed)."""
+    x, dy = (torch.randn(T, 2, 128, device="cuda").to(dtype) for _ in range(2))
+    layer = _layer(128, 2, 512, dtype)
+    ref = _forward_backward(layer, x, dy)
+    _replace_weights(layer, _column_range)
+    layer.zero_grad()
+    got = _forward_backward(layer, x, dy)
+    for i, (a, b) in enumerate(zip(got, ref)):
+        if a.dim() > 1:
+            assert torch.equal(a, b), "tensor %d" % i
+        else:
+            assert_close(a, b, dtype, "tensor %d" % i, 1.0 if dtype == torch.float32 else 0.1)
