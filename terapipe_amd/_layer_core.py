@@ -316,27 +316,25 @@ def layer_bwd_native(image, device):
 
 def stack_forward_only(layers, x, caches, cache_len):
     """The forward of a chain of layers without anything kept for a backward, as one library call: all layers share one
-    set of intermediate buffers.  layers: [(12 parameters in PARAM_NAMES order, heads, activation)], equal geometry;
-    caches: [(k, v)] per layer.  Returns the output [T, B, E]."""
+    set of intermediate buffers.  layers: [(12 parameters in PARAM_NAMES order, heads, activation)], each with its own
+    FFN width, heads and activation; caches: [(k, v)] per layer.  Returns the output [T, B, E]."""
     T, B, E = x.shape
     ops._require_cuda(x)
     x = x.contiguous()
     n = len(layers)
-    F = layers[0][0][8].shape[0]
-    geo = LayerGeometry.of(T, B, E, F, layers[0][1], x.dtype, layers[0][2])
-    row = geo.M * E * geo.es
-    step = (row + 255) // 256 * 256
+    geos = [LayerGeometry.of(T, B, E, params[8].shape[0], heads, x.dtype, activation) for params, heads, activation in layers]
+    shared = max(g.fwd.total for g in geos)
+    step = (T * B * E * geos[0].es + 255) // 256 * 256
     # one allocation: the arena and, from two layers on, the outputs between the layers in turn
-    arena = torch.empty(geo.fwd.total + (2 if n > 2 else n - 1) * step, dtype=torch.uint8, device=x.device)
+    arena = torch.empty(shared + (2 if n > 2 else n - 1) * step, dtype=torch.uint8, device=x.device)
     out = torch.empty_like(x)
     base = arena.data_ptr()
     image = bytearray(n * _FWD_PACK.size)
     src = x.data_ptr()
     for i, (params, _, _) in enumerate(layers):
         k, v = caches[i]
-        dst = out.data_ptr() if i == n - 1 else base + geo.fwd.total + (i & 1) * step
-        geo.pack_fwd(image, i * _FWD_PACK.size, cache_len, k.shape[1], params, src, k.data_ptr(),
-                     v.data_ptr(), base, dst)
+        dst = out.data_ptr() if i == n - 1 else base + shared + (i & 1) * step
+        geos[i].pack_fwd(image, i * _FWD_PACK.size, cache_len, k.shape[1], params, src, k.data_ptr(), v.data_ptr(), base, dst)
         src = dst
     layers_fwd(image, n, x.device)
     return out

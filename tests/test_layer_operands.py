@@ -75,3 +75,21 @@ def test_weights_that_are_column_ranges(T, dtype):
             assert torch.equal(a, b), "tensor %d" % i
         else:
             assert_close(a, b, dtype, "tensor %d" % i, 1.0 if dtype == torch.float32 else 0.1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32], ids=str)
+def test_forward_only_stack_of_unequal_layers(dtype):
+    """FFN width, heads and activation are each layer's own, also where no gradients are asked for."""
+    import terapipe_amd as ta
+    E, T, B, P = 256, 6, 2, 5
+    layers = ta.TransformerLayers(4, E, 4 * E, 4, dtype=dtype, device="cuda")
+    shapes = [(4, 4 * E, "relu"), (2, 2 * E, "gelu"), (4, 6 * E, "gelu"), (4, E, "relu")]
+    for i, (H, F, activation) in enumerate(shapes):
+        layers.layers[i] = _layer(E, H, F, dtype, activation, seed=i)
+    x = torch.randn(T, B, E, device="cuda").to(dtype)
+    caches = [torch.randn(c.shape, device="cuda").to(dtype) for c in layers.create_cache(B, P + T)]
+    ref, _ = layers(x, [c.clone().requires_grad_() for c in caches], P)
+    with torch.no_grad():
+        got, _ = layers(x, caches, P)
+    assert_close(got, ref, dtype, "y", 1.0 if dtype == torch.float32 else 0.1)
