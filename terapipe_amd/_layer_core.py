@@ -231,6 +231,16 @@ def operands(params):
     return [p.data_ptr() for p in params], ldw
 
 
+def require_operands(x, params, k_cache, v_cache):
+    """The library gets addresses only: everything a layer reads or writes is in GPU memory and of x's type."""
+    ops._require_cuda(x, k_cache, v_cache)
+    dtype = x.dtype
+    for i, p in enumerate(params):
+        if not p.is_cuda or p.dtype is not dtype:
+            ops._require_cuda(p)
+            raise _lib.TeraPipeHipError("%s is %s, the layer's input %s" % (PARAM_NAMES[i], p.dtype, dtype))
+
+
 class _Arena:
     """Byte offsets (multiples of 256) of a set of buffers inside one allocation."""
     __slots__ = ("off", "total")
@@ -319,7 +329,8 @@ def stack_forward_only(layers, x, caches, cache_len):
     set of intermediate buffers.  layers: [(12 parameters in PARAM_NAMES order, heads, activation)], each with its own
     FFN width, heads and activation; caches: [(k, v)] per layer.  Returns the output [T, B, E]."""
     T, B, E = x.shape
-    ops._require_cuda(x)
+    for (params, _, _), (k, v) in zip(layers, caches):
+        require_operands(x, params, k, v)
     x = x.contiguous()
     n = len(layers)
     geos = [LayerGeometry.of(T, B, E, params[8].shape[0], heads, x.dtype, activation) for params, heads, activation in layers]

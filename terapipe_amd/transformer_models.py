@@ -257,7 +257,7 @@ class _LayerFunction(torch.autograd.Function):
     @staticmethod
     def forward(ctx, heads, cache_len, activation, opts, x, k_cache, v_cache, *params):
         T, B, E = x.shape
-        ops._require_cuda(x, *params)
+        core.require_operands(x, params, k_cache, v_cache)
         dt, dev = x.dtype, x.device
         F = params[8].shape[0]
         ctx.has_cache = k_cache is not None

@@ -93,3 +93,28 @@ def test_forward_only_stack_of_unequal_layers(dtype):
     with torch.no_grad():
         got, _ = layers(x, caches, P)
     assert_close(got, ref, dtype, "y", 1.0 if dtype == torch.float32 else 0.1)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("grad", [False, True])
+def test_host_memory_and_other_types_are_refused(grad):
+    """Nothing is launched: parameters or caches in host memory, and parameters of another type than the input."""
+    from terapipe_amd import _lib
+    layer = _layer(128, 2, 512, torch.float16)
+    x = torch.randn(3, 1, 128, device="cuda").half()
+    caches = [torch.zeros(2, 4, 64, dtype=torch.float16, device="cuda") for _ in range(2)]
+    with torch.set_grad_enabled(grad):
+        layer(x, tuple(caches), 0)
+        for i in range(2):
+            with pytest.raises(_lib.TeraPipeHipError, match="no CPU path"):
+                layer(x, tuple(c.cpu() if i == j else c for j, c in enumerate(caches)), 0)
+        with pytest.raises(_lib.TeraPipeHipError, match="no CPU path"):
+            layer(x.cpu(), tuple(caches), 0)
+        for name in ("fc1.weight", "fc_ln.bias"):
+            module = getattr(layer, name.split(".")[0])
+            kept = getattr(module, name.split(".")[1])
+            for other, message in ((kept.detach().cpu(), "no CPU path"), (kept.detach().float(), name + " is torch.float32")):
+                setattr(module, name.split(".")[1], torch.nn.Parameter(other))
+                with pytest.raises(_lib.TeraPipeHipError, match=message):
+                    layer(x, tuple(caches), 0)
+            setattr(module, name.split(".")[1], kept)
