@@ -183,10 +183,11 @@ def _temp_cache(B, H, T, Dh, like):
 
 
 def _grads_can_go_in_place(w):
-    """Every parameter of the layer already has a dense .grad of its own dtype to add to."""
-    for p in w.values():
-        g = p.grad
-        if g is None or g.dtype != p.dtype or g.shape != p.shape or not g.is_contiguous():
+    """Every parameter of the layer already has a dense .grad of its own dtype to add to, where the kernels can write it."""
+    for n, p in w.items():
+        g = p.grad if p.is_leaf else None
+        if g is None or g.dtype != p.dtype or g.shape != p.shape or g.layout != torch.strided or not g.is_contiguous() \
+                or (n in core.BIG_PARAMS and g.data_ptr() % 16):
             return False
     return True
 
@@ -249,9 +250,10 @@ class _LayerFunction(torch.autograd.Function):
 
     Forward and backward are one library call each (tp_layers_fwd, tp_layer_bwd).  The backward of a slice: the data
     gradients, the eight vector-parameter gradients as one launch, the four weight gradients as one grouped one.
-    Where every parameter already has a .grad that the engine is going to add to (_autograd.engine_adds_to_grad), or with
-    opts.in_place, the kernels add the gradients to it (the GEMM's accumulate epilogue, one rounding) and autograd gets
-    None, instead of twelve tensors that autograd adds one elementwise kernel each.  opts.defer -- keep the slice's dY / X
+    Where every parameter already has a .grad that the engine is going to add to on this node's stream
+    (_autograd.engine_adds_to_grad: a slice loop's second backward is the first that can know), or with opts.in_place, the
+    kernels add the gradients to it (the GEMM's accumulate epilogue, one rounding) and autograd gets None, instead of
+    twelve tensors that autograd adds one elementwise kernel each.  opts.defer -- keep the slice's dY / X
     rows and take the weight gradients once per sequence, over all its rows, in the backward of the slice at position 0
     (the last one the reverse-slice order reaches); the slices before it hand autograd None for the parameters."""
 
@@ -495,7 +497,8 @@ class TransformerLayer(nn.Module):
     # Two switches for loops that call .backward() / autograd.backward slice by slice, as the reference's does
     # (torch.autograd.grad would see None for the parameters, and post-accumulate-grad hooks may not fire):
     # accumulate_grads_in_place -- the backward of a slice adds its parameter gradients to existing .grad tensors
-    # inside the gradient kernels instead of returning them to autograd (same sums, one rounding fewer);
+    # inside the gradient kernels instead of returning them to autograd (same sums, one rounding fewer), wherever it
+    # runs: the caller keeps every forward of the layer, and its backward passes, on one stream;
     # defer_weight_grads -- with a cache, the weight gradients of a sequence are taken once, over all its rows, in
     # the backward of the slice at cache_len 0, which the reverse-slice order reaches last; .grad is complete when
     # that backward returns, and every slice of the sequence must run its backward, last slice first.
