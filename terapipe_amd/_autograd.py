@@ -1,4 +1,6 @@
 """What the autograd functions of the package ask the engine that runs their backward."""
+import weakref
+
 import torch
 
 from . import ops
@@ -53,11 +55,47 @@ def engine_adds_to_grad(ctx, params, first):
     return ours
 
 
-def grad_to_add_to(ctx, param, first):
-    """param.grad if the kernels may add to it in place of the engine (engine_adds_to_grad); otherwise None."""
-    if not engine_adds_to_grad(ctx, (param,), first):
+_LOOKUPS = "terapipe_amd lookups"       # in the metadata of the node a weight's gradient goes to: see note_lookup
+_TAKEN = object()
+
+
+def note_lookup(node, index):
+    """Remembers an autograd node whose backward adds a few rows to a dense gradient (an embedding): a product with the same
+    weight may hand it that gradient (take_on).  node.next_functions[index] is the weight's."""
+    weight, _ = node.next_functions[index]
+    if weight is not None:
+        node.stream, node.task, node.handed = ops._stream(), None, None
+        seen = weight.metadata.setdefault(_LOOKUPS, [])
+        seen[:] = [s for s in seen if s[0]() is not None] + [(weakref.ref(node), index)]
+
+
+def lookup_to_hand_to(ctx, index):
+    """A node (note_lookup) of the same weight, on the same stream, that is still to run in the backward pass under way, or
+    None.  What it is handed becomes part of the one gradient it returns, so the engine sees the same sum as from two nodes:
+    nothing of where that sum goes (.grad, a hook, torch.autograd.grad) is different."""
+    weight = ctx.next_functions[index]
+    if torch.is_grad_enabled() or weight[0] is None:
         return None
-    g = param.grad
-    if g is None or g.dtype != param.dtype or g.shape != param.shape or not g.is_contiguous() or g.is_sparse:
-        return None
-    return g
+    task, stream = torch._C._current_graph_task_id(), ops._stream()
+    for ref, at in weight[0].metadata.get(_LOOKUPS, ()):
+        node = ref()
+        if node is None or node.next_functions[at] != weight or node.stream != stream:
+            continue
+        if node.task != task:           # (what it was handed in a pass that broke off is dropped)
+            try:
+                if not torch._C._will_engine_execute_node(node):
+                    continue
+            except RuntimeError:
+                continue
+            node.task, node.handed = task, None
+        if node.handed is not _TAKEN:
+            return node
+    return None
+
+
+def taken_on(ctx):
+    """In the backward of a node (note_lookup): the gradient it was handed, its own from now on, or None."""
+    task = torch._C._current_graph_task_id()
+    handed = ctx.handed if ctx.task == task else None
+    ctx.task, ctx.handed = task, _TAKEN
+    return handed

@@ -8,7 +8,7 @@ import torch.nn as nn
 from torch.nn import init
 
 from . import ops
-from ._autograd import engine_adds_to_grad, grad_to_add_to
+from ._autograd import lookup_to_hand_to, note_lookup, taken_on
 from ._lib import TP_EPI_ACCUMULATE, TP_EPI_STORE, TP_GEMM_NN, TP_GEMM_NT, TP_GEMM_TN
 
 
@@ -17,29 +17,27 @@ class _EmbeddingFunction(torch.autograd.Function):
     def forward(ctx, ids, weight):
         flat = ids.reshape(-1).contiguous()
         out = ops.embedding_fwd(flat, weight)
-        ctx.flat, ctx.weight = flat, weight
+        ctx.save_for_backward(flat)
+        ctx.wshape, ctx.wdtype = weight.shape, weight.dtype
         return out.view(*ids.shape, weight.shape[1])
 
     @staticmethod
     def backward(ctx, dout):
-        """Into an existing .grad the rows that occur are added where they lie (a tied LM head has left its gradient
-        there by then: no dense gradient of the lookup is made, and none is added); otherwise they go into zeros."""
-        flat, weight = ctx.flat, ctx.weight
+        """The rows that occur are added to the gradient that an LM head tied to this weight has handed over (no dense
+        gradient of the lookup is made then, and none is added), otherwise to zeros."""
+        (flat,) = ctx.saved_tensors
         dout = dout.reshape(flat.numel(), -1).contiguous()
+        handed = taken_on(ctx)
         if ops.embedding_rows_fit(flat, dout):
-            grad = grad_to_add_to(ctx, weight, 1)
-            if grad is not None and grad.data_ptr() % 16 == 0:
-                ops.embedding_bwd_rows_(flat, dout, grad)
-                return None, None
-            dw = torch.zeros(weight.shape, dtype=weight.dtype, device=dout.device)
+            dw = torch.zeros(ctx.wshape, dtype=ctx.wdtype, device=dout.device) if handed is None else handed
             return None, ops.embedding_bwd_rows_(flat, dout, dw)
-        acc = torch.empty(weight.shape, dtype=torch.float32, device=dout.device)
+        acc = torch.empty(ctx.wshape, dtype=torch.float32, device=dout.device)
         ops.zero_(acc)
         ops.embedding_bwd(flat, dout, acc)
-        if weight.dtype == torch.float32:
+        if handed is None and ctx.wdtype == torch.float32:
             return None, acc
-        dw = torch.empty_like(weight)
-        ops.accum_cast(dw, acc, False)
+        dw = torch.empty(ctx.wshape, dtype=ctx.wdtype, device=dout.device) if handed is None else handed
+        ops.accum_cast(dw, acc, handed is not None)
         return None, dw
 
 
@@ -58,7 +56,10 @@ class VocabParallelEmbedding(nn.Module):
         init_method(self.weight)
 
     def forward(self, input_):
-        return _EmbeddingFunction.apply(input_, self.weight)
+        out = _EmbeddingFunction.apply(input_, self.weight)
+        if out.grad_fn is not None:
+            note_lookup(out.grad_fn, 1)
+        return out
 
 
 VOCAB_PAD = 64      # logits rows are whole 128-byte lines
@@ -97,14 +98,14 @@ class _LMHeadFunction(torch.autograd.Function):
         dlogits = dlogits.contiguous()
         dh = torch.empty_like(h2d)
         ops.gemm(TP_GEMM_NN, dlogits, _as_operand(weight), M, E, V, C=dh)
-        grad = grad_to_add_to(ctx, weight, 1)
-        if grad is not None and grad.data_ptr() % 16 == 0:
-            ops.gemm(TP_GEMM_TN, dlogits, h2d, V, E, M, C=grad, epilogue=TP_EPI_ACCUMULATE)
+        tied = lookup_to_hand_to(ctx, 1)        # an embedding of the same weight adds its rows to what it is handed
+        if tied is not None and tied.handed is not None:
+            ops.gemm(TP_GEMM_TN, dlogits, h2d, V, E, M, C=tied.handed, epilogue=TP_EPI_ACCUMULATE)
             return dh, None
         dw = torch.empty(weight.shape, dtype=weight.dtype, device=weight.device)
         ops.gemm(TP_GEMM_TN, dlogits, h2d, V, E, M, C=dw)
-        if weight.grad is None and engine_adds_to_grad(ctx, (weight,), 1):
-            weight.grad = dw        # as the engine would; an embedding tied to this weight adds its rows to it
+        if tied is not None:
+            tied.handed = dw
             return dh, None
         return dh, dw
 
