@@ -202,6 +202,11 @@ class _GradOptions:
         self.in_place, self.defer, self.pending = False, False, {}
         self.inputs = weakref.WeakValueDictionary()     # the slices' graphs own them
 
+    def __reduce__(self):
+        # the switches are set anew by every forward, and a sequence under way belongs to the graphs of its slices: a copied
+        # or unpickled layer starts with neither
+        return _GradOptions, ()
+
 
 class _SequenceInputs:
     """Deferred weight gradients: the inputs of the four linears of one sequence in one layer, position-indexed; the

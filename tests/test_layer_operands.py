@@ -118,3 +118,17 @@ def test_host_memory_and_other_types_are_refused(grad):
                 with pytest.raises(_lib.TeraPipeHipError, match=message):
                     layer(x, tuple(caches), 0)
             setattr(module, name.split(".")[1], kept)
+
+
+def test_a_layer_can_be_copied_and_pickled():
+    import copy
+    import io
+    layer = _layer(64, 1, 128, torch.float16, device="cpu")
+    layer._grad_options.pending[7] = object()
+    f = io.BytesIO()
+    torch.save(layer, f)
+    f.seek(0)
+    for other in (copy.deepcopy(layer), torch.load(f, weights_only=False)):
+        assert all(torch.equal(a, b) for a, b in zip(other.param_list(), layer.param_list()))
+        assert not other._grad_options.pending and not other._grad_options.inputs
+        assert other._grad_options is not layer._grad_options
