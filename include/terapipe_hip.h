@@ -147,7 +147,13 @@ typedef struct tp_gemm_desc {
                                            workspace and write nothing else; the LayerNorm that consumes C sums them,
                                            applies bias / residual and writes C (tp_layernorm_fwd/bwd_partials).
                                            Without a split the GEMM completes as usual. */
-    int32_t reserved4;
+    int32_t ragged;                     /* 1: three extents may end inside a 16-byte chunk whose row holds it in full (lda,
+                                           ldc cover it, in the last row too): N of a plain TP_GEMM_NT (STORE, no column
+                                           sums; up to the next multiple of 8) -- C's columns from N to there are
+                                           OVERWRITTEN --, k of TP_GEMM_NN -- A's columns from K to the end of the chunk
+                                           are read and have to be finite; what they multiply is zero -- and M of
+                                           TP_GEMM_TN -- A's columns past M are read, no result depends on them.
+                                           0: extents that are no whole chunks are refused. */
 } tp_gemm_desc;
 
 /* number of k splits the plan uses for this product (1 = none; 0 = invalid descriptor) */

@@ -36,7 +36,7 @@ class GemmDesc(ctypes.Structure):
         ("cache_rows", c_int64),
         ("q_scale", c_float), ("reserved", c_int32),
         ("q_bh_rows", c_int64),
-        ("defer_reduce", c_int32), ("reserved4", c_int32),
+        ("defer_reduce", c_int32), ("ragged", c_int32),
     ]
 
 

@@ -840,9 +840,9 @@ static int validate_gemm(const tp_gemm_desc* d) {
     // contiguous extents of the operands as stored
     int a_cols = d->op == TP_GEMM_TN ? d->M : d->K;
     int b_cols = d->op == TP_GEMM_NT ? d->K : d->N;
-    // A's contiguous extent may end inside a chunk that its row holds in full where what it multiplies is bounded by
-    // rows: k of NN (the weight's rows past k count as zeros; A's columns there have to be finite), M of TN
-    const bool a_ragged = d->op != TP_GEMM_NT && d->lda >= (a_cols + ch - 1) / ch * ch;
+    // With `ragged`, A's contiguous extent may end inside a chunk that its row holds in full where what it multiplies is
+    // bounded by rows: k of NN (the weight's rows past k count as zeros; A's columns there have to be finite), M of TN
+    const bool a_ragged = d->ragged && d->op != TP_GEMM_NT && d->lda >= (a_cols + ch - 1) / ch * ch;
     if ((a_cols % ch && !a_ragged) || b_cols % ch || d->lda % ch || d->ldb % ch) {
         set_error("tp_gemm: contiguous extents / leading dimensions must be multiples of %d elements "
                   "(A cols %d lda %ld, B cols %d ldb %ld)", ch, a_cols, (long)d->lda, b_cols, (long)d->ldb);
@@ -850,8 +850,8 @@ static int validate_gemm(const tp_gemm_desc* d) {
     }
     if (d->lda < a_cols || d->ldb < b_cols) { set_error("tp_gemm: leading dimension smaller than row"); return TP_ERR_ARG; }
     if (((uintptr_t)d->A | (uintptr_t)d->B) & 15) { set_error("tp_gemm: operands must be 16-byte aligned"); return TP_ERR_ARG; }
-    // N of a plain NT product may end inside a chunk that C's row holds in full (the columns past N get the last one's values)
-    if (d->N % 8 && (d->op != TP_GEMM_NT || d->epilogue != TP_EPI_STORE || d->defer_reduce || d->colsum_acc || d->ldc < (d->N + 7) / 8 * 8)) {
+    // with `ragged`, so may N of a plain NT product in C's rows (the columns past N get the last one's values)
+    if (d->N % 8 && (!d->ragged || d->op != TP_GEMM_NT || d->epilogue != TP_EPI_STORE || d->defer_reduce || d->colsum_acc || d->ldc < (d->N + 7) / 8 * 8)) {
         set_error("tp_gemm: N=%d must be a multiple of 8", d->N);
         return TP_ERR_UNSUPPORTED;
     }

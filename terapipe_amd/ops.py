@@ -174,14 +174,16 @@ def layernorm_bwd(dy, x2d, mean, rstd, gamma, dres, dgamma_acc, dbeta_acc, colsu
 
 
 def gemm(op, A, B, M, N, K, C=None, epilogue=TP_EPI_STORE, bias=None, residual=None, aux=None, aux_out=None,
-         colsum_acc=None, qkv=None, tile_cfg=None, ksplit=None, defer_reduce=False, desc_sink=None):
+         colsum_acc=None, qkv=None, tile_cfg=None, ksplit=None, defer_reduce=False, desc_sink=None, ragged=False):
     """Runs one GEMM.  A, B, C, residual, aux are 2-D row-major tensors (stride(1) == 1).
     qkv = dict(q, k_cache, v_cache, batch, heads, head_dim, cache_len, cache_rows, q_scale).
     tile_cfg / ksplit force a tile configuration / k-split count (tuning and tests); default automatic.
     defer_reduce (STORE / BIAS_RESIDUAL epilogues): if the plan splits k, C is left unwritten and a
     PendingReduce is returned for the LayerNorm call that consumes C; otherwise C as usual.
     desc_sink: a list that receives the call's descriptor (the one a recorded replay re-issues), for callers
-    that re-point C before a replay."""
+    that re-point C before a replay.
+    ragged: N of NT, k of NN and M of TN may be no multiple of 8; what lies in C's (NT) or A's rows from there to the
+    next one is overwritten or read (tp_gemm_desc.ragged)."""
     _require_cuda(A, B, C)
     d = GemmDesc()
     d.op, d.dtype, d.epilogue = op, tp_dtype(A.dtype), epilogue
@@ -198,6 +200,7 @@ def gemm(op, A, B, M, N, K, C=None, epilogue=TP_EPI_STORE, bias=None, residual=N
     if aux_out is not None:
         d.aux_out, d.ldauxo = aux_out.data_ptr(), aux_out.stride(0)
     d.colsum_acc = _p(colsum_acc)
+    d.ragged = int(ragged)
     if qkv is not None:
         d.q, d.k_cache, d.v_cache = qkv["q"].data_ptr(), qkv["k_cache"].data_ptr(), qkv["v_cache"].data_ptr()
         d.batch, d.heads, d.head_dim = qkv["batch"], qkv["heads"], qkv["head_dim"]

@@ -84,7 +84,8 @@ class _LMHeadFunction(torch.autograd.Function):
         Vp = _pad_vocab(V)
         h2d = h2d.contiguous()
         logits = torch.empty(h2d.shape[0], Vp, dtype=h2d.dtype, device=h2d.device)
-        ops.gemm(TP_GEMM_NT, h2d, _as_operand(weight), h2d.shape[0], V, E, C=logits, epilogue=TP_EPI_STORE)
+        ops.gemm(TP_GEMM_NT, h2d, _as_operand(weight), h2d.shape[0], V, E, C=logits, epilogue=TP_EPI_STORE,
+                 ragged=True)
         if Vp != V:
             logits[:, V:].zero_()
         ctx.save_for_backward(h2d, weight)
@@ -97,13 +98,13 @@ class _LMHeadFunction(torch.autograd.Function):
         V = weight.shape[0]
         dlogits = dlogits.contiguous()
         dh = torch.empty_like(h2d)
-        ops.gemm(TP_GEMM_NN, dlogits, _as_operand(weight), M, E, V, C=dh)
+        ops.gemm(TP_GEMM_NN, dlogits, _as_operand(weight), M, E, V, C=dh, ragged=True)
         tied = lookup_to_hand_to(ctx, 1)        # an embedding of the same weight adds its rows to what it is handed
         if tied is not None and tied.handed is not None:
-            ops.gemm(TP_GEMM_TN, dlogits, h2d, V, E, M, C=tied.handed, epilogue=TP_EPI_ACCUMULATE)
+            ops.gemm(TP_GEMM_TN, dlogits, h2d, V, E, M, C=tied.handed, epilogue=TP_EPI_ACCUMULATE, ragged=True)
             return dh, None
         dw = torch.empty(weight.shape, dtype=weight.dtype, device=weight.device)
-        ops.gemm(TP_GEMM_TN, dlogits, h2d, V, E, M, C=dw)
+        ops.gemm(TP_GEMM_TN, dlogits, h2d, V, E, M, C=dw, ragged=True)
         if tied is not None:
             tied.handed = dw
             return dh, None

@@ -125,3 +125,27 @@ def test_forced_tiles_that_load_whole_k_tiles_fall_back_on_a_ragged_k():
         assert _forced_plan("TN", 1024, 1024, 1024, cfg)[0] == 5, cfg
     assert _forced_plan("NN", 128, 1024, 1024, 24)[0] == 5                      # 80-wide tiles: NT only
     assert _forced_plan("NN", 224, 1024, 1024, 43)[0] == 5                      # 160-wide pipelined tile: NT only
+
+
+@pytest.mark.parametrize("op,M,N,K,ld", [("NT", 16, 13, 64, 24), ("NN", 16, 64, 13, 24), ("TN", 13, 64, 16, 24)])
+@pytest.mark.parametrize("dtype", [0, 1, 2])
+def test_extents_inside_a_chunk_are_asked_for(lib, op, M, N, K, ld, dtype):
+    """N of NT, k of NN, M of TN: refused unless the descriptor says that the rest of the chunk may be touched, and then only
+    where the rows hold it; other epilogues, deferred sums and column sums never take a ragged N."""
+    from terapipe_amd import _lib as L
+
+    def plan(ragged=1, ld=ld, **fields):
+        d = L.GemmDesc()
+        d.op, d.dtype, d.M, d.N, d.K, d.ragged = {"NT": L.TP_GEMM_NT, "NN": L.TP_GEMM_NN, "TN": L.TP_GEMM_TN}[op], dtype, M, N, K, ragged
+        d.A = d.B = d.C = d.bias = d.colsum_acc = 4096
+        d.colsum_acc = None
+        d.lda = 64 if op == "NT" else ld
+        d.ldb, d.ldc = 64, ld if op == "NT" else 64
+        for name, value in fields.items():
+            setattr(d, name, value)
+        return lib.tp_gemm_plan(ctypes.byref(d), None, None)
+
+    assert plan() == 0 and plan(ragged=0) == 2          # TP_ERR_UNSUPPORTED
+    assert plan(ld=13) == 2                             # rows that do not hold the chunk
+    if op == "NT":
+        assert plan(epilogue=L.TP_EPI_BIAS) == plan(defer_reduce=1) == plan(colsum_acc=4096) == 2

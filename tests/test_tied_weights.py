@@ -15,7 +15,7 @@ def calls(monkeypatch):
     from terapipe_amd._lib import TP_EPI_ACCUMULATE, TP_GEMM_NN, TP_GEMM_NT
     made = []
 
-    def gemm(op, A, B, m, n, k, C, epilogue=0):
+    def gemm(op, A, B, m, n, k, C, epilogue=0, ragged=False):
         if op not in (TP_GEMM_NT, TP_GEMM_NN):
             made.append("add" if epilogue == TP_EPI_ACCUMULATE else "dw")
         a, b = (A[:, :k], B.t()) if op == TP_GEMM_NT else (A[:, :k], B) if op == TP_GEMM_NN else (A[:, :m].t(), B)

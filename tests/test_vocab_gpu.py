@@ -98,3 +98,31 @@ def test_where_gradients_go(dtype, tied):
     handle.remove()
     assert_close(sum(seen), ws[0].grad, dtype, "what a hook sees")
     assert_close(params[0].grad, 3 * ws[0].grad, dtype, "backward with a hook")
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32], ids=str)
+@pytest.mark.parametrize("V", [1, 9, 50])
+def test_products_next_to_other_values(dtype, V):
+    """N of NT, k of NN and M of TN inside a chunk: a plain product refuses them, and one that says it may use the rest of
+    the chunk writes C's columns up to the next multiple of 8 and none beyond, and depends on nothing it reads there."""
+    from terapipe_amd import _lib, ops
+    from terapipe_amd._lib import TP_GEMM_NN, TP_GEMM_NT, TP_GEMM_TN
+    M, E, up = 40, 64, (V + 7) // 8 * 8
+    g = torch.Generator(device=DEV).manual_seed(V)
+    h, w = (torch.randn(n, E, generator=g, device=DEV).to(dtype) for n in (M, V))
+    wide = torch.full((M, up + 8), 7.0, dtype=dtype, device=DEV)
+    dl = torch.randn(M, up + 8, generator=g, device=DEV).to(dtype)
+    with pytest.raises(_lib.TeraPipeHipError, match="multiple of 8"):
+        ops.gemm(TP_GEMM_NT, h, w, M, V, E, C=wide)
+    for op, A, B, m, n, k in ((TP_GEMM_NN, dl, w, M, E, V), (TP_GEMM_TN, dl, h, V, E, M)):
+        with pytest.raises(_lib.TeraPipeHipError, match="must be multiples"):
+            ops.gemm(op, A, B, m, n, k, C=torch.empty(m, n, dtype=dtype, device=DEV))
+    ops.gemm(TP_GEMM_NT, h, w, M, V, E, C=wide, ragged=True)
+    assert_close(wide[:, :V], h.double() @ w.double().t(), dtype, "NT")
+    assert (wide[:, up:] == 7).all()
+    dh, dw = torch.empty(M, E, dtype=dtype, device=DEV), torch.full((V + 1, E), 7.0, dtype=dtype, device=DEV)
+    ops.gemm(TP_GEMM_NN, dl, w, M, E, V, C=dh, ragged=True)
+    ops.gemm(TP_GEMM_TN, dl, h, V, E, M, C=dw[:V], ragged=True)
+    assert_close(dh, dl[:, :V].double() @ w.double(), dtype, "NN")
+    assert_close(dw[:V], dl[:, :V].double().t() @ h.double(), dtype, "TN")
+    assert (dw[V:] == 7).all()
