@@ -217,11 +217,7 @@ def _flat_views(flat, layout):
     return [{n: flat[o:o + int(np.prod(s))].view(s) for n, (o, s) in d.items()} for d in layout]
 
 
-# Where a runner with slice_streams=1 merges too (rows of a slice on average, rows of all, hidden size): see merges.
-MERGE_ONE_STREAM_ROWS, MERGE_ONE_STREAM_TOTAL, MERGE_ONE_STREAM_HIDDEN = 256, 2048, 2048
-
-
-def merges(seq_slices, batch, hidden, slice_streams):
+def merges(slice_streams):
     """Whether a single-stage step runs the sequence in one piece.  slice_streams: what the caller set, None if nothing.
 
     Slices are the unit in which pipeline STAGES hand work to each other.  One runner holds every slice of its stage
@@ -230,19 +226,12 @@ def merges(seq_slices, batch, hidden, slice_streams):
     the query's own.  A slice costs a pass over the stack's weights and a chain of launches, so the fewer the better: a
     product of 64 rows is bound by reading its weight, one of 2048 by the matrix pipe.  Measured (16 bit, 2048 tokens):
     64 slices of 32 x 2 rows of hidden 6144: 104.8 ms -> 44.7; seven slices of 160-512 rows of hidden 5120: 25.9 ->
-    21.0.  Two pieces on two streams, which fill each other's last waves of tiles, are level or slower with the tiles
-    chosen for whole rounds of the chip (44.7 and 22.3; hidden 4096: 8.8 against 8.2).
+    21.0; eight of 256 rows of hidden 2048, five layers: 6.0 -> 4.6.  Two pieces on two streams, which fill each other's
+    last waves of tiles, are level or slower with the tiles chosen for whole rounds of the chip (44.7 and 22.3; hidden
+    4096: 8.8 against 8.2).
 
-    A caller that sets slice_streams asks for slices on that many streams.  The exception: one stream, slices of
-    MERGE_ONE_STREAM_ROWS rows and more, MERGE_ONE_STREAM_TOTAL together, on a hidden size up to MERGE_ONE_STREAM_HIDDEN.
-    A slice of that size fills a row of tiles but not the chip, which one stream leaves idle otherwise (8 x 256 rows of
-    hidden 2048 on three streams: 6.0 ms, in one piece 4.6), and a runner on one stream gives the same bits there as the
-    default one, whose launches it is the plain version of."""
-    if slice_streams is None:
-        return True
-    rows = sum(seq_slices) * batch
-    return (slice_streams == 1 and MERGE_ONE_STREAM_ROWS * len(seq_slices) <= rows <= MERGE_ONE_STREAM_TOTAL
-            and hidden <= MERGE_ONE_STREAM_HIDDEN)
+    A caller that sets slice_streams asks for slices on that many streams, whatever their size."""
+    return slice_streams is None
 
 
 def fused_backward_slices(seq_slices, n_lanes, window=None):
@@ -722,11 +711,12 @@ class TeraPipe(nn.Module):
     dK/dV kernel for the dQ kernels of the later slices; nothing else orders slices, so consecutive slices
     run through the stack side by side.  Same kernels, same arguments, same results; the overlap fills the
     chip where one chain of short kernels cannot, and GEMMs that stream the same weight at the same time
-    share its way through the caches.  Default 3 (1 under use_hip_graph).
+    share its way through the caches.  Default 3 (1 under use_hip_graph); a step that runs in one piece (merge_slices)
+    uses the calling stream only, whatever the attribute says.
     merge_slices: the step runs the sequence in one piece instead of slice by slice (merges says why and when), with
     the same results up to rounding.  None (the default): where the caller leaves the way the step runs to the runner.
     A caller that sets slice_streams asks for its slices on that many streams (1: one after the other, as on a stage
-    that gets them one by one; but see merges), suffix_dkdv=False and fp32_grad_cache=False for the hand-over of cache
+    that gets them one by one), suffix_dkdv=False and fp32_grad_cache=False for the hand-over of cache
     gradients from slice to slice, several batch slices for that grid: those run as they are cut, and so does a step
     whose slices are timed (slice_timing).
     launch_replay: the first step runs as written, the second also keeps every library call it makes (bound
@@ -757,8 +747,7 @@ class TeraPipe(nn.Module):
         self.suffix_dkdv = suffix_dkdv
         self.fused_attn_bwd = bool(fused_attn_bwd)
         self.merge_slices = bool(merge_slices) if merge_slices is not None else (
-            merges(self.seq_slices, batch_size, layers.embedding_dim, slice_streams)
-            and not use_hip_graph and suffix_dkdv and fp32_grad_cache and len(self.batch_slices) == 1)
+            merges(slice_streams) and not use_hip_graph and suffix_dkdv and fp32_grad_cache and len(self.batch_slices) == 1)
         # defaults: three slice streams and launch replay; one stream and no replay under use_hip_graph
         self.slice_streams = int(slice_streams) if slice_streams is not None else (1 if use_hip_graph else 3)
         self.launch_replay = bool(launch_replay) if launch_replay is not None else not use_hip_graph

@@ -4,8 +4,9 @@ layer count).  test_full_width_against_the_oracle runs configs 4 and 5 on a pref
 1024 of 2048 positions = 8 of 16 slices of 128 tokens; the first 512 = 16 of 64 slices of 32 tokens, batch 2)
 with the eager runner on one and on three streams; test_full_length_default_runner_against_the_oracle runs
 both at all 2048 positions, and configs 2 and 3 with all their layers (24 and 5: the workloads as the benchmark times
-them), through the runner as it is constructed by default (three slice streams, launch replay) and compares the first
-step (eager) and the third (re-issued from the recorded launches).
+them), through the runner as it is constructed by default (the sequence in one piece, launch replay), configs 4 and 5
+also slice by slice on three streams, and compares the first step (eager) and the third (re-issued from the recorded
+launches).
 
 Compared per tensor (max |got - ref| / max |ref| <= 2e-2): the output, the input gradient, the final K/V
 caches and all twelve parameter gradients of every layer.  The oracle computes in fp32 from the weights and
@@ -88,7 +89,7 @@ def _compare_step(name, tag, runner, layers, y, xd, yo, dxo, fco, leaf, dtype):
     print("  %s worst rel err: " % tag + ", ".join("%s %.2e" % kv for kv in worst.items()), flush=True)
 
 
-# every config on one stream; the three-stream runner (the default) also against the oracle on C3, C4 and C5: on three
+# every config on one stream; the three-stream runner also against the oracle on C3, C4 and C5: on three
 # streams C3 never fuses its attention backward, C5 always does, and C4's windows (384 positions, 256 and 128 at the
 # sequence end) are the ones a per-slice decision would mix (C2 has its own bit-equality test against the
 # single-stream runner)
@@ -159,12 +160,13 @@ def test_full_width_layer_surface_against_the_oracle(in_place, defer):
     assert all(not layer._grad_options.pending for layer in layers.layers), "a deferred sequence was left open"
 
 
-@pytest.mark.parametrize("name", ["C4-full", "C5-full", "C3-full", "C2-full"])
-def test_full_length_default_runner_against_the_oracle(name):
+@pytest.mark.parametrize("name,sliced", [("C4-full", False), ("C5-full", False), ("C3-full", False), ("C2-full", False),
+                                         ("C4-full", True), ("C5-full", True)])
+def test_full_length_default_runner_against_the_oracle(name, sliced):
     """All 2048 positions of configs 4 and 5 (one layer) and of configs 2 and 3 with all their layers (24 and 5) -- the
-    workloads as the benchmark times them -- through the runner as constructed by default (three slice streams,
-    launch replay): inside the runner this is what reaches the forward's key split (from 1024 keys on), the
-    one-pass dK/dV over a tail of up to 2016 positions, and (config 5) the fused attention backward on lanes.
+    workloads as the benchmark times them -- through the runner as constructed by default (one piece, launch replay).
+    sliced: three slice streams; inside the runner this is what reaches the forward's key split (from 1024 keys on),
+    the one-pass dK/dV over a tail of up to 2016 positions, and (config 5) the fused attention backward on lanes.
     Step 1 runs eagerly, step 2 records, step 3 is re-issued from the record; steps 1 and 3 are each compared
     with the oracle."""
     import terapipe_amd as ta
@@ -177,7 +179,7 @@ def test_full_length_default_runner_against_the_oracle(name):
     dy = torch.randn(L, B, E, generator=g).to(dtype)
     layers = ta.TransformerLayers(n_layers, E, Fd, H, dtype=dtype, device=DEV)
     load_params_into(layers, ps, dtype)
-    runner = ta.TeraPipe(layers, B, L, [B], ss)
+    runner = ta.TeraPipe(layers, B, L, [B], ss, merge_slices=False if sliced else None)
     assert runner.slice_streams == 3 and runner.launch_replay
     runner.keep_states = True
     steps = {}
@@ -194,6 +196,7 @@ def test_full_length_default_runner_against_the_oracle(name):
         if step != 2:
             steps[step] = (y.detach().cpu(), xd.grad.cpu(), [c.cpu() for c in runner.last_caches[0]],
                            [{n: t.grad.cpu() for n, t in layer.param_dict().items()} for layer in layers.layers])
+    assert runner._sbufs.pieces == (ss if sliced else [L])
     assert isinstance(runner._sbufs.fwd_program, list) and isinstance(runner._sbufs.bwd_program, list), \
         "the third step was not re-issued from recorded launches"
     leaf = [{k: v.clone().requires_grad_(True) for k, v in p.items()} for p in ps]

@@ -795,8 +795,8 @@ def test_replay_survives_a_larger_workspace_on_the_same_stream():
 @pytest.mark.parametrize("n_layers,steps", [(2, 5), (24, 4)])
 def test_default_runner_matches_single_stream_at_c2_shape(n_layers, steps):
     """benchmark config 2's geometry (hidden 2048, 16 heads, FFN 8192, sequence 2048 as 8 x 256, fp16) on two
-    layers and on all 24: the constructor's defaults (three slice streams, launch replay) against one stream
-    launched from Python, several steps -- the first as written, the second recorded, the rest re-issued.  Same
+    layers and on all 24: slice by slice on three streams with launch replay (the constructor's defaults for a step that
+    is not merged) against one stream launched from Python, several steps -- the first as written, the second recorded, the rest re-issued.  Same
     kernels on the same data: outputs and input gradients are bit-identical; the parameter gradients (fp32
     atomics for the vector parameters) agree to rounding."""
     ta = _mods()
@@ -818,7 +818,7 @@ def test_default_runner_matches_single_stream_at_c2_shape(n_layers, steps):
                         t.copy_(1.0 + 0.2 * torch.randn(t.shape, generator=gd, device=DEV))
                     else:
                         t.copy_(torch.randn(t.shape, generator=gd, device=DEV) * (0.1 if name.endswith("bias") else 0.02))
-    fast = ta.TeraPipe(layers, B, L, [B], ss)
+    fast = ta.TeraPipe(layers, B, L, [B], ss, merge_slices=False)
     plain = ta.TeraPipe(layers, B, L, [B], ss, slice_streams=1, launch_replay=False)
     assert fast.slice_streams == 3 and fast.launch_replay
 
@@ -837,6 +837,7 @@ def test_default_runner_matches_single_stream_at_c2_shape(n_layers, steps):
         y0, dx0, g0 = step(plain, x, dy)
         y1, dx1, g1 = step(fast, x, dy)
         torch.cuda.synchronize()
+        assert fast._sbufs.pieces == plain._sbufs.pieces == ss and len(fast._sbufs.lanes) == 2 and not plain._sbufs.lanes
         assert torch.equal(y1, y0), "step %d: y" % seed
         assert torch.equal(dx1, dx0), "step %d: dx" % seed
         for a, b in zip(g1, g0):

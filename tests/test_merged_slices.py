@@ -1,4 +1,4 @@
-"""The pieces a default runner's step runs in: the rule on the CPU, and merged steps against the CPU oracle."""
+"""The pieces a runner's step runs in: the rule on the CPU, and merged steps against the CPU oracle."""
 import pytest
 import torch
 
@@ -8,10 +8,7 @@ from tests.util import assert_close, load_params_into, make_params
 
 def test_rule():
     from terapipe_amd.terapipe import merges
-    for case in (([32] * 64, 1, 6144), ([16] * 8, 2, 256), ([256] * 8, 1, 2048), ([2048] * 2, 8, 8192)):
-        assert merges(*case, None) and not merges(*case, 3)
-    assert merges([256] * 8, 1, 2048, 1)                # long slices, small weights: on one stream too
-    assert not any(merges(*case, 1) for case in (([255] * 8, 1, 2048), ([256] * 8, 1, 2056), ([256] * 8, 2, 2048)))
+    assert merges(None) and not any(merges(n) for n in (1, 2, 3))
 
 
 def test_who_merges():
@@ -19,8 +16,21 @@ def test_who_merges():
     layers = ta.TransformerLayers(1, 64, 128, 1, dtype=torch.float16, device="cpu")
     make = lambda bs=(2,), **kw: ta.TeraPipe(layers, 2, 64, list(bs), [32, 32], **kw).merge_slices
     assert make() and make(launch_replay=False) and make(slice_streams=1, merge_slices=True)
-    assert not any(make(**kw) for kw in (dict(slice_streams=3), dict(use_hip_graph=True), dict(suffix_dkdv=False),
-                                         dict(fp32_grad_cache=False), dict(bs=(1, 1)), dict(merge_slices=False)))
+    assert not any(make(**kw) for kw in (dict(slice_streams=3), dict(slice_streams=1), dict(use_hip_graph=True),
+                                         dict(suffix_dkdv=False), dict(fp32_grad_cache=False), dict(bs=(1, 1)), dict(merge_slices=False)))
+
+
+@pytest.mark.gpu
+def test_one_stream_runs_the_slices():
+    """Slices that somebody asks for run one by one also where they are long and the weights small (eight of 256 rows of
+    hidden 2048)."""
+    import terapipe_amd as ta
+    layers = ta.TransformerLayers(1, 2048, 2048, 16, dtype=torch.float16)
+    x = torch.randn(2048, 1, 2048, device="cuda").half()
+    for kw, pieces in ((dict(slice_streams=1), [256] * 8), (dict(merge_slices=False), [256] * 8), (dict(), [2048])):
+        runner = ta.TeraPipe(layers, 1, 2048, [1], [256] * 8, **kw)
+        runner(x).sum().backward()
+        assert runner._sbufs.pieces == pieces and len(runner._sbufs.lanes) == (2 if kw.get("merge_slices") is False else 0)
 
 
 @pytest.mark.gpu
