@@ -618,9 +618,11 @@ static bool tile_serves(const TileCost& c, int op, int K) {
 // estimate's choice takes 0.61 to 1.0 of their time (1024 x 5120 x 20480: 284 -> 188 us; 4096 x 1600 x 6400: 117 -> 80).
 static void plan_large(const tp_gemm_desc* d, int& cfg, int& ns) {
     const float K = (float)d->K;
-    // an LM head's data gradient (k = vocabulary): 48 to 63 tiles of 256 x 256 on a long k, split to one round
+    // 48 to 63 tiles of 256 x 256 on a long k are split to one round: the estimate has too little for the 128 x 128 tiles it
+    // names there.  2048 x 1792 x 16384: 121 us against 141, 2048 x 1600 x 12800: 97 against 113; at k = 8192 the
+    // estimate is right (1536 x 2048: 65 against 55, 1700 x 2048: 67 against 54), from 24576 on it names the same.
     const long t256 = (long)((d->M + 255) / 256) * ((d->N + 255) / 256);
-    if (d->op != TP_GEMM_TN && d->K >= 8192 && t256 >= 48 && t256 < 64) {
+    if (d->op != TP_GEMM_TN && d->K >= 12288 && t256 >= 48 && t256 < 64) {
         cfg = kWideCfg;
         ns = (int)(kNumCU / t256);
         return;

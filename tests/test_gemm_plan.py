@@ -149,3 +149,10 @@ def test_extents_inside_a_chunk_are_asked_for(lib, op, M, N, K, ld, dtype):
     assert plan(ld=13) == 2                             # rows that do not hold the chunk
     if op == "NT":
         assert plan(epilogue=L.TP_EPI_BIAS) == plan(defer_reduce=1) == plan(colsum_acc=4096) == 2
+
+
+def test_few_large_tiles_on_a_long_k():
+    """48 to 63 tiles of 256 x 256: split to one round from k = 12288 on, the estimate's choice below."""
+    for M, N, splits in ((2048, 1792, 4), (1536, 2048, 5), (2000, 1600, 4)):
+        assert plan("NN", M, N, 12288) == plan("NT", M, N, 12288) == (44, splits)
+        assert plan("NN", M, N, 12224)[0] != 44
