@@ -296,7 +296,8 @@ __global__ __launch_bounds__(1024) void cross_entropy_loss_kernel(const T* __res
         for (int i = 0; i < U * CH; ++i) s += softmax_exp<T>(v[i] - base);
     }
     const float all = block_reduce(mx, scratch, true);
-    s = block_reduce(mx == -INFINITY ? 0.f : s * softmax_exp<T>(mx - all), scratch, false);
+    // (a thread without values, or with none above -infinity, has s = 0; one whose values are all NaN has no maximum but s = NaN)
+    s = block_reduce(s == 0.f ? 0.f : s * softmax_exp<T>(mx - all), scratch, false);
     if (threadIdx.x == 0) {
         const int64_t t = target[m];
         loss[m] = logf(s) + all - (t >= 0 && t < V ? Elem<T>::to_float(z[t]) : 0.f);

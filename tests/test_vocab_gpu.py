@@ -126,3 +126,37 @@ def test_products_next_to_other_values(dtype, V):
     assert_close(dh, dl[:, :V].double() @ w.double(), dtype, "NN")
     assert_close(dw[:V], dl[:, :V].double().t() @ h.double(), dtype, "TN")
     assert (dw[V:] == 7).all()
+
+
+@DTYPES
+@pytest.mark.parametrize("V,ld", [(5, 7), (40, 40), (1000, 1003), (2050, 2056), (33000, 33000)], ids=str)
+def test_loss_of_infinities_nan_and_masks(dtype, V, ld):
+    """Rows with +-infinity, NaN (one, a thread's whole share, all) and masks of the type's lowest value: loss and gradient as
+    the fp64 softmax has them, NaN where it has NaN.  (Vectors and scalars, one thread's share and several.)"""
+    from terapipe_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(V)
+    inf, nan, low = float("inf"), float("nan"), torch.finfo(dtype).min
+    share = slice(min(V - 1, 8), min(V, 16))
+    changes = [(slice(0, 0), 0.), (slice(1, 2), -inf), (slice(0, V - 1), -inf), (slice(0, V), -inf), (slice(2, 3), inf),
+               (slice(0, 2), inf), (slice(V - 1, V), nan), (share, nan), (slice(0, V), nan), (slice(0, V - 1), low),
+               (share, low)]
+    M = len(changes)
+    z = torch.randn(M, ld, generator=g, device=DEV).to(dtype)
+    for m, (where, value) in enumerate(changes):
+        z[m, where] = value
+    target = torch.full((M,), V - 1, device=DEV)
+    scale = torch.rand(M, generator=g, device=DEV) + 0.5
+    zd = z[:, :V].double()
+    ref = torch.logsumexp(zd, 1) - zd[:, V - 1]
+    p = (zd - zd.max(1, keepdim=True).values).exp()
+    grad = p / p.sum(1, keepdim=True)
+    grad[:, V - 1] -= 1
+    grad *= scale.double()[:, None]
+    bad = torch.isnan(grad).any(1)
+    assert bad.tolist() == [m in (3, 4, 5, 6, 7, 8) for m in range(M)]
+    loss, stats = ops.cross_entropy_loss(z, target, V)
+    ops.cross_entropy_grad_(z, target, stats, scale, V)
+    assert torch.isnan(loss[bad]).all() and torch.isnan(z[bad][:, :V]).all()
+    assert_close(loss[~bad], ref[~bad], torch.float32, "loss", 1.0 if dtype == torch.float32 else 10.0)
+    assert_close(z[~bad][:, :V], grad[~bad], dtype, "gradient")
+    assert not z[:, V:].any()
