@@ -253,13 +253,6 @@ __global__ __launch_bounds__(1024) void cross_entropy_reg_kernel(T* __restrict__
     }
 }
 
-// exp(x) of the softmax kernels below: the hardware's 2^x in 16 bit (its argument's rounding is 2^-18 of the result at the
-// far end of what a 16-bit probability can hold), the library's exp in fp32
-template <typename T> __device__ __forceinline__ float softmax_exp(float x) {
-    if constexpr (sizeof(T) == 2) return __builtin_amdgcn_exp2f(x * 1.44269504088896341f);
-    else return expf(x);
-}
-
 // Per-token loss without touching the logits: one read.  max_sum[m] = (row maximum, sum of exp(z - maximum)) for the
 // gradient kernel.  A workgroup per row; each thread keeps its own running maximum and sum (a maximum that moves
 // rescales the sum), and the workgroup combines them once.  VEC: 16-byte accesses.
@@ -288,16 +281,16 @@ __global__ __launch_bounds__(1024) void cross_entropy_loss_kernel(const T* __res
 #pragma unroll
         for (int i = 1; i < U * CH; ++i) top = fmaxf(top, v[i]);
         if (top > mx) {
-            s *= softmax_exp<T>(mx - top);
+            s *= expf(mx - top);
             mx = top;
         }
         const float base = mx == -INFINITY ? 0.f : mx;
 #pragma unroll
-        for (int i = 0; i < U * CH; ++i) s += softmax_exp<T>(v[i] - base);
+        for (int i = 0; i < U * CH; ++i) s += expf(v[i] - base);
     }
     const float all = block_reduce(mx, scratch, true);
     // (a thread without values, or with none above -infinity, has s = 0; one whose values are all NaN has no maximum but s = NaN)
-    s = block_reduce(s == 0.f ? 0.f : s * softmax_exp<T>(mx - all), scratch, false);
+    s = block_reduce(s == 0.f ? 0.f : s * expf(mx - all), scratch, false);
     if (threadIdx.x == 0) {
         const int64_t t = target[m];
         loss[m] = logf(s) + all - (t >= 0 && t < V ? Elem<T>::to_float(z[t]) : 0.f);
@@ -326,7 +319,7 @@ __global__ __launch_bounds__(256) void cross_entropy_grad_kernel(T* __restrict__
     for (int i = 0; i < CH; ++i) {
         const int v = c * CH + i;
         float g = 0.f;
-        if (v < V) g = softmax_exp<T>(Elem<T>::to_float(e[i]) - ms.x) * inv - (v == t ? sc : 0.f);
+        if (v < V) g = expf(Elem<T>::to_float(e[i]) - ms.x) * inv - (v == t ? sc : 0.f);
         e[i] = Elem<T>::from_float(g);
     }
     if constexpr (VEC) *reinterpret_cast<uint4*>(z) = *reinterpret_cast<const uint4*>(e);
