@@ -293,7 +293,8 @@ __global__ __launch_bounds__(1024) void cross_entropy_loss_kernel(const T* __res
     s = block_reduce(s == 0.f ? 0.f : s * expf(mx - all), scratch, false);
     if (threadIdx.x == 0) {
         const int64_t t = target[m];
-        loss[m] = logf(s) + all - (t >= 0 && t < V ? Elem<T>::to_float(z[t]) : 0.f);
+        // (the difference first: the logarithm must not be lost in a maximum of -65504, or of 1e38)
+        loss[m] = logf(s) + (all - (t >= 0 && t < V ? Elem<T>::to_float(z[t]) : 0.f));
         max_sum[m] = make_float2(all, s);
     }
 }

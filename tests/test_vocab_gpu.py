@@ -139,7 +139,7 @@ def test_loss_of_infinities_nan_and_masks(dtype, V, ld):
     share = slice(min(V - 1, 8), min(V, 16))
     changes = [(slice(0, 0), 0.), (slice(1, 2), -inf), (slice(0, V - 1), -inf), (slice(0, V), -inf), (slice(2, 3), inf),
                (slice(0, 2), inf), (slice(V - 1, V), nan), (share, nan), (slice(0, V), nan), (slice(0, V - 1), low),
-               (share, low)]
+               (share, low), (slice(0, V), low)]
     M = len(changes)
     z = torch.randn(M, ld, generator=g, device=DEV).to(dtype)
     for m, (where, value) in enumerate(changes):
@@ -147,8 +147,10 @@ def test_loss_of_infinities_nan_and_masks(dtype, V, ld):
     target = torch.full((M,), V - 1, device=DEV)
     scale = torch.rand(M, generator=g, device=DEV) + 0.5
     zd = z[:, :V].double()
-    ref = torch.logsumexp(zd, 1) - zd[:, V - 1]
-    p = (zd - zd.max(1, keepdim=True).values).exp()
+    top = zd.max(1, keepdim=True).values
+    p = (zd - top).exp()
+    # (the maximum and the target's logit first: beside 3.4e38 a logarithm is lost in fp64 as well)
+    ref = (top[:, 0] - zd[:, V - 1]) + p.sum(1).log()
     grad = p / p.sum(1, keepdim=True)
     grad[:, V - 1] -= 1
     grad *= scale.double()[:, None]
