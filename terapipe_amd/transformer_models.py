@@ -328,11 +328,9 @@ class _LayerFunction(torch.autograd.Function):
         base, off = buf.data_ptr(), geo.bwd.off
         p = {n: base + off[n] for n in off}
         fo, fbase = geo.fwd.off, arena.data_ptr()
-        # addresses of the four linears' inputs over the rows of the weight-gradient products
-        xs = {n: fbase + fo[n] for n in ("xn", "o", "hn", "a")}
         rows, dy = M, dout.data_ptr()
         pend, done, fresh = None, True, True
-        if opts.defer and ctx.has_cache and (seq is not None or cache_len == 0):
+        if seq is not None:         # (deferred when its forward ran, whatever the switch says by now)
             # rows [r0, r1) of the sequence's position-indexed gradient buffers
             r0, r1 = cache_len * B, (cache_len + T) * B
             key = k_cache.data_ptr()
@@ -378,7 +376,8 @@ class _LayerFunction(torch.autograd.Function):
                 wg = (pend.dqkv.data_ptr(), s.xn.data_ptr(), pend.dh.data_ptr(), s.o.data_ptr(), pend.dz1.data_ptr(),
                       s.hn.data_ptr(), pend.dout.data_ptr(), s.a.data_ptr())
             else:
-                wg = (p["dqkv"], xs["xn"], p["dh"], xs["o"], p["dz1"], xs["hn"], dy, xs["a"])
+                xn, o, hn, a = (fbase + fo[n] for n in ("xn", "o", "hn", "a"))
+                wg = (p["dqkv"], xn, p["dh"], o, p["dz1"], hn, dy, a)
         core._BWD_PACK.pack_into(ctx.image, core._FWD_PACK.size, dy, p["dz1"], p["dhn"], p["dh"], p["d_o"], p["dqkv"],
                                  p["dxn"], dx.data_ptr(), p["delta"], p["small"],
                                  0 if gk is None else gk.data_ptr(), 0 if gv is None else gv.data_ptr(),
