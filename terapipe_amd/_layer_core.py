@@ -216,6 +216,7 @@ def layer_bwd(w, st, dout, heads, gk, gv, accumulate_prefix, has_incoming, zero_
 _FWD_PACK = struct.Struct("8iq28Q4q")          # tp_layer_desc
 _BWD_PACK = struct.Struct("12Q4iq8Q4Q2i8Q2i")  # tp_layer_bwd_desc after its tp_layer_desc
 _ACTIVATIONS = {"relu": 0, "gelu": 1}
+LINEAR_INPUTS = ("xn", "o", "hn", "a")          # of in_proj, out_proj, fc1 and fc2
 
 
 def operands(params):
@@ -255,7 +256,7 @@ class _Arena:
 class LayerGeometry:
     """Sizes of one layer call and where its buffers lie.  Forward: what the backward reads again.  Backward: the
     intermediate gradients and the fp32 sums of the vector-parameter gradients."""
-    __slots__ = ("T", "B", "E", "F", "H", "dtype", "es", "M", "activation", "fwd", "bwd", "n_small", "dt")
+    __slots__ = ("T", "B", "E", "F", "H", "dtype", "es", "M", "activation", "fwd", "fwd_rest", "bwd", "n_small", "dt")
     _cache = {}
 
     def __init__(self, T, B, E, F, H, dtype, activation):
@@ -264,9 +265,11 @@ class LayerGeometry:
         M, es = self.M, self.es
         rows = lambda width: M * width * es
         self.n_small = small_acc_numel(E, F)
-        self.fwd = _Arena([("xn", rows(E)), ("mean1", 4 * M), ("rstd1", 4 * M), ("q", rows(E)), ("o", rows(E)),
-                           ("lse", 4 * M * H), ("h", rows(E)), ("mean2", 4 * M), ("rstd2", 4 * M), ("hn", rows(E)),
-                           ("a", rows(F)), ("z", rows(F) if activation == "gelu" else 0)])
+        fwd = ([("xn", rows(E)), ("mean1", 4 * M), ("rstd1", 4 * M), ("q", rows(E)), ("o", rows(E)),
+                ("lse", 4 * M * H), ("h", rows(E)), ("mean2", 4 * M), ("rstd2", 4 * M), ("hn", rows(E)),
+                ("a", rows(F)), ("z", rows(F) if activation == "gelu" else 0)])
+        # fwd_rest: without the inputs of the four linears, which a sequence with deferred weight gradients keeps
+        self.fwd, self.fwd_rest = _Arena(fwd), _Arena([f for f in fwd if f[0] not in LINEAR_INPUTS])
         self.bwd = _Arena([("dz1", rows(F)), ("dhn", rows(E)), ("dh", rows(E)), ("d_o", rows(E)), ("dqkv", rows(3 * E)),
                            ("dxn", rows(E)), ("delta", 4 * M * H), ("small", 4 * self.n_small)])
 
@@ -283,10 +286,10 @@ class LayerGeometry:
         return g
 
     def pack_fwd(self, image, at, cache_len, cache_rows, params, x, k, v, base, out, over=None):
-        """Writes a tp_layer_desc at byte `at` of `image`.  params: the layer's 12; base: address of the forward arena; over: addresses that take
-        the place of the arena's."""
+        """Writes a tp_layer_desc at byte `at` of `image`.  params: the layer's 12; base: address of the forward arena; over: the
+        addresses of LINEAR_INPUTS where they are not part of it (its layout is fwd_rest then)."""
         w_ptrs, ldw = operands(params)
-        o = self.fwd.off
+        o = (self.fwd_rest if over else self.fwd).off
         p = {n: base + o[n] for n in o}
         if over:
             p.update(over)

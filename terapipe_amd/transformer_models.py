@@ -273,7 +273,6 @@ class _LayerFunction(torch.autograd.Function):
             k_cache, v_cache = _temp_cache(B, heads, T, E // heads, x)
         x = x.contiguous()
         geo = core.LayerGeometry.of(T, B, E, F, heads, dt, activation)
-        arena = torch.empty(geo.fwd.total, dtype=torch.uint8, device=dev)
         out = torch.empty(T, B, E, dtype=dt, device=dev)
         seq, over = None, None
         if opts.defer and ctx.has_cache:
@@ -287,7 +286,8 @@ class _LayerFunction(torch.autograd.Function):
                     seq = opts.inputs[key] = _SequenceInputs(k_cache.shape[1] * B, E, F, dt, dev)
             if seq is not None:
                 seq.rows = r1
-                over = {n: getattr(seq, n)[r0:].data_ptr() for n in ("xn", "o", "hn", "a")}
+                over = {n: getattr(seq, n)[r0:].data_ptr() for n in core.LINEAR_INPUTS}
+        arena = torch.empty((geo.fwd_rest if over else geo.fwd).total, dtype=torch.uint8, device=dev)
         image = bytearray(core._FWD_PACK.size + core._BWD_PACK.size)
         geo.pack_fwd(image, 0, cache_len, k_cache.shape[1], params, x.data_ptr(), k_cache.data_ptr(), v_cache.data_ptr(),
                      arena.data_ptr(), out.data_ptr(), over)
@@ -376,7 +376,7 @@ class _LayerFunction(torch.autograd.Function):
                 wg = (pend.dqkv.data_ptr(), s.xn.data_ptr(), pend.dh.data_ptr(), s.o.data_ptr(), pend.dz1.data_ptr(),
                       s.hn.data_ptr(), pend.dout.data_ptr(), s.a.data_ptr())
             else:
-                xn, o, hn, a = (fbase + fo[n] for n in ("xn", "o", "hn", "a"))
+                xn, o, hn, a = (fbase + fo[n] for n in core.LINEAR_INPUTS)
                 wg = (p["dqkv"], xn, p["dh"], o, p["dz1"], hn, dy, a)
         core._BWD_PACK.pack_into(ctx.image, core._FWD_PACK.size, dy, p["dz1"], p["dhn"], p["dh"], p["d_o"], p["dqkv"],
                                  p["dxn"], dx.data_ptr(), p["delta"], p["small"],

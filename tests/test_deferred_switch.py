@@ -60,3 +60,14 @@ def test_two_slices(descriptors):
     assert b1.wg_rows == 0 and b0.wg_rows == 8
     for n, width in zip(INPUTS, (64, 64, 64, 128)):
         assert getattr(b0, "wg_" + n) == getattr(f0, n) and getattr(f1, n) == getattr(f0, n) + 4 * width * 4
+
+
+def test_the_linears_inputs_are_kept_once(descriptors):
+    """By the slice, or by the sequence with deferred weight gradients: not by both."""
+    import terapipe_amd as ta
+    layer = ta.ModelParallelTransformerLayer(64, 128, 1)
+    sizes = {}
+    for layer.defer_weight_grads in (False, True):
+        y, _, _ = _slice(layer, T=32, L=64)
+        sizes[layer.defer_weight_grads] = y.grad_fn.kept[3].numel()
+    assert sizes[False] - sizes[True] == 32 * (3 * 64 + 128) * 4
