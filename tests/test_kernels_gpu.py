@@ -160,15 +160,17 @@ def test_gemm_large_products_take_the_tall_tiles(dtype):
     C = torch.empty(1000, 12600, dtype=dtype, device=DEV)
     ops.gemm(L.TP_GEMM_NT, A, B, 1000, 12600, 192, C=C)
     assert_close(C, A.double() @ B.double().t(), dtype, "NT 1000x12600x192")
-    # NN, 4 x 13 tiles, k = 8256 split four ways
-    A, B = rnd(1000, 8256), rnd(8256, 3104, 0.02)
-    d = L.GemmDesc()
-    d.op, d.dtype, d.epilogue, d.M, d.N, d.K = L.TP_GEMM_NN, ops.tp_dtype(dtype), L.TP_EPI_STORE, 1000, 3104, 8256
-    d.A, d.lda, d.B, d.ldb, d.C, d.ldc = A.data_ptr(), 8256, B.data_ptr(), 3104, A.data_ptr(), 3104
-    assert L.load().tp_gemm_splits(d) == 4
-    C = torch.empty(1000, 3104, dtype=dtype, device=DEV)
-    ops.gemm(L.TP_GEMM_NN, A, B, 1000, 3104, 8256, C=C)
-    assert_close(C, A.double() @ B.double(), dtype, "NN 1000x3104x8256")
+    # NN, 4 x 13 tiles: k = 12352 is split four ways; at k = 8256 one round of smaller tiles is the faster plan (1000 x 3104:
+    # 60 us against 71) and the same product is checked without a split
+    for K, splits in ((12352, 4), (8256, 1)):
+        A, B = rnd(1000, K), rnd(K, 3104, 0.02)
+        d = L.GemmDesc()
+        d.op, d.dtype, d.epilogue, d.M, d.N, d.K = L.TP_GEMM_NN, ops.tp_dtype(dtype), L.TP_EPI_STORE, 1000, 3104, K
+        d.A, d.lda, d.B, d.ldb, d.C, d.ldc = A.data_ptr(), K, B.data_ptr(), 3104, A.data_ptr(), 3104
+        assert L.load().tp_gemm_splits(d) == splits
+        C = torch.empty(1000, 3104, dtype=dtype, device=DEV)
+        ops.gemm(L.TP_GEMM_NN, A, B, 1000, 3104, K, C=C)
+        assert_close(C, A.double() @ B.double(), dtype, "NN 1000x3104x%d" % K)
 
 
 def _group(ops, L, items, dtype, force_cfg=None):
