@@ -499,7 +499,6 @@ static bool tile_cfg(int id, TileCfg& c) {
     case 3: c = {128, 256, 64, 3}; return true;
     case 5: c = {128, 128, 64, 2}; return true;
     case 8: c = {64, 64, 64, 4}; return true;
-    case 10: c = {128, 128, 32, 4}; return true;
     case 11: c = {64, 256, 64, 3}; return true;
     case 12: c = {64, 64, 128, 4}; return true;
     case 13: c = {128, 128, 64, 3}; return true;
@@ -786,7 +785,6 @@ static void launch_cfg(const GemmPlan& p, const GemmArgs& a, hipStream_t s) {
         case 5: gemm_dma_kernel<T, AKM, BKM, 128, 128, 64, 2, 2, 2><<<grid, 256, 0, s>>>(a); break;
         case 8: gemm_dma_kernel<T, AKM, BKM, 64, 64, 64, 2, 2, 4><<<grid, 256, 0, s>>>(a); break;
         case 11: gemm_dma_kernel<T, AKM, BKM, 64, 256, 64, 2, 2, 3><<<grid, 256, 0, s>>>(a); break;
-        case 10: gemm_dma_kernel<T, AKM, BKM, 128, 128, 32, 2, 2, 4><<<grid, 256, 0, s>>>(a); break;
         case 12: gemm_dma_kernel<T, AKM, BKM, 64, 64, 128, 2, 2, 4><<<grid, 256, 0, s>>>(a); break;
         case 13: gemm_dma_kernel<T, AKM, BKM, 128, 128, 64, 2, 2, 3><<<grid, 256, 0, s>>>(a); break;
         case 17: if constexpr (BKM) gemm_tall_kernel<T, AKM, BKM, 256, 160, 64, 4, 1, 3><<<grid, 256, 0, s>>>(a); break;

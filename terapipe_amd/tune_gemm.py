@@ -31,7 +31,7 @@ DEFAULT_GEOMETRIES = [
     "12288:49152:128:2048",                                 # 175B shape, 128-token slices
     "6144:24576:64:4096",                                   # 44B shape, 32-token slices x batch 2
 ]
-DMA_CFGS = [2, 3, 5, 6, 7, 8, 10, 11, 12, 13, 14, 15, 16, 17, 18, 19, 20, 41, 42, 43]
+DMA_CFGS = [2, 3, 5, 6, 7, 8, 11, 12, 13, 14, 15, 16, 17, 18, 19, 20, 41, 42, 43]
 # the weight-streaming kernel's configurations (NT and NN only; 24 and 25 NT only): cfg -> rows of its row tile
 STREAM_CFGS = {21: 192, 22: 256, 24: 192, 25: 256, 26: 128, 29: 256, 30: 192, 31: 192, 32: 256, 33: 192, 34: 256,
                35: 128, 36: 64, 37: 128, 38: 64}
