@@ -165,9 +165,8 @@ size_t tp_gemm_workspace_bytes(const tp_gemm_desc* d);
 int tp_gemm(const tp_gemm_desc* d, void* workspace, size_t workspace_bytes, void* stream);
 /* n independent products as if by n tp_gemm calls in order on the stream (the four weight gradients of a layer,
    which autograd's backward of the four linears of transformer_models.py:273-285 produces one by one).  Up to four
-   16-bit TP_GEMM_TN products of one dtype, k a multiple of 64, whose largest plans to 256 x 256 tiles with unsplit
-   k share ONE launch, so that together they fill whole rounds of the chip's CUs; any other group runs member by
-   member.  workspace: the largest member's tp_gemm_workspace_bytes. */
+   16-bit TP_GEMM_TN products of one dtype and one k, a multiple of 64, share ONE launch on one tile shape, so that
+   together they fill whole rounds of the chip's CUs; any other group runs member by member.  workspace: the largest member's tp_gemm_workspace_bytes. */
 int tp_gemm_grouped(const tp_gemm_desc* descs, int n, void* workspace, size_t workspace_bytes, void* stream);
 /* the tile configuration of the single launch tp_gemm_grouped makes for this group; 0 = member by member */
 int tp_gemm_group_cfg(const tp_gemm_desc* descs, int n);
@@ -281,22 +280,23 @@ int tp_attn_bwd_fused(const tp_attn_desc* d, const tp_attn_suffix_desc* sd, cons
 int tp_embedding_fwd(const int64_t* ids, const void* weight, void* out, int M, int E, int V, int dtype, void* stream);
 /* dweight_acc[ids[m], :] += dout[m, :]   (fp32 accumulators; autograd's embedding backward) */
 int tp_embedding_bwd(const int64_t* ids, const void* dout, float* dweight_acc, int M, int E, int V, int dtype, void* stream);
-/* _VocabParallelCrossEntropy (mpu/cross_entropy.py:25-104) forward and backward in one pass over logits
- * [M, ld] whose first V columns are the vocabulary (columns [V, Vpad) are alignment padding of the LM-head
- * GEMM): loss[m] = logsumexp(logits[m, :V]) - logits[m, target[m]], and logits is overwritten IN PLACE with
- * its gradient (softmax - onehot(target)) * grad_scale (padding columns 0), the way the reference overwrites
- * its input with the softmax (:65-74) and returns it scaled as grad_input (:79-99). */
 /* dweight[ids[m], :] += dout[m, :] in `dtype`, every row's sum taken in fp32 and rounded once; no atomics.  M <= 8192, E whole
    16-byte chunks. */
 int tp_embedding_bwd_rows(const int64_t* ids, const void* dout, void* dweight, int M, int E, int V, int dtype, void* stream);
+/* _VocabParallelCrossEntropy (mpu/cross_entropy.py:25-104) forward and backward in one launch over logits
+ * [M, ld] whose first V columns are the vocabulary (columns [V, Vpad) are alignment padding of the LM-head
+ * GEMM): loss[m] = logsumexp(logits[m, :V]) - logits[m, target[m]], and logits is overwritten IN PLACE with
+ * its gradient (softmax - onehot(target)) * grad_scale (padding columns 0), the way the reference overwrites
+ * its input with the softmax (:65-74) and returns it scaled as grad_input (:79-99).  For callers that know the scale
+ * beforehand and hold no scratch memory; the package's autograd function uses the two halves below. */
+int tp_cross_entropy(void* logits, int64_t ld, const int64_t* target, float* loss, int M, int V, int Vpad,
+                     float grad_scale, int dtype, void* stream);
 /* The two halves of tp_cross_entropy.  Loss: logits are read only; max_sum[2m], [2m+1] = the row's maximum and
    sum exp(z - maximum).  Gradient, from those: logits[m, v] <- (softmax - onehot) * scale[m], padding columns <- 0. */
 int tp_cross_entropy_loss(const void* logits, int64_t ld, const int64_t* target, float* loss, float* max_sum, int M, int V,
                           int dtype, void* stream);
 int tp_cross_entropy_grad(void* logits, int64_t ld, const int64_t* target, const float* max_sum, const float* scale, int M,
                           int V, int Vpad, int dtype, void* stream);
-int tp_cross_entropy(void* logits, int64_t ld, const int64_t* target, float* loss, int M, int V, int Vpad,
-                     float grad_scale, int dtype, void* stream);
 /* x[m, :N] *= scale[m] in place: the per-token grad_output factor of the cross-entropy backward (:97) */
 int tp_scale_rows(void* x, int64_t ld, const float* scale, int M, int N, int dtype, void* stream);
 
@@ -354,10 +354,10 @@ int tp_adam_step(const tp_adam_desc* desc, void* stream);
 /* dst[n] (dtype) = (accumulate ? dst[n] : 0) + src[n] (fp32): folds the fp32 accumulators of the
  * LayerNorm / bias gradients into parameter .grad tensors (autograd's sum over slices). */
 int tp_accum_cast(void* dst, const float* src, int64_t n, int accumulate, int dtype, void* stream);
-/* acc[N] += column sums of x[M, N] (fp32 accumulators). */
 /* The same for n (at most 8) tensors whose fp32 sums lie one after the other in src, sizes[i] values each, in one launch. */
 int tp_accum_cast_parts(void* const* dst, const int32_t* sizes, int n, const float* src, int accumulate, int dtype,
                         void* stream);
+/* acc[N] += column sums of x[M, N] (fp32 accumulators). */
 int tp_colsum_acc(const void* x, int64_t ldx, float* acc, int M, int N, int dtype, void* stream);
 /* fills n 32-bit words with zero (a kernel, so it can be recorded into a HIP graph) */
 int tp_zero_words(void* dst, int64_t n_words, void* stream);
