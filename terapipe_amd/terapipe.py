@@ -17,7 +17,7 @@ from . import _layer_core as core
 from . import _lib
 from . import ops
 from ._lib import TP_EPI_ACCUMULATE, TP_EPI_STORE, TP_GEMM_TN
-from .transformer_models import ModelParallelTransformerLayer, _check_cache, grid_slice_batch_and_sequence, is_plain
+from .transformer_models import ModelParallelTransformerLayer, _check_cache, grid_slice_batch_and_sequence, is_followed, is_plain
 
 
 def loss_func(y):
@@ -64,7 +64,7 @@ class TransformerLayers(nn.Module):
         return cache
 
     def forward(self, x, cache, cache_len):
-        if not torch.is_grad_enabled() and self.n_layers and all(is_plain(layer) for layer in self.layers):
+        if not torch.is_grad_enabled() and self.n_layers and not is_followed() and all(is_plain(layer) for layer in self.layers):
             return self._forward_only(x, cache, cache_len), list(cache[:2 * self.n_layers])
         cache_outputs = []
         for layer_id in range(self.n_layers):

@@ -14,6 +14,7 @@ import weakref
 import numpy as np
 import torch
 import torch.nn as nn
+from torch.autograd import forward_ad
 from torch.nn.modules import module as _modules
 
 from . import _layer_core as core
@@ -550,7 +551,7 @@ class TransformerLayer(nn.Module):
         else:
             assert cache_len == 0
         params = self.param_list()
-        if not torch.is_grad_enabled():
+        if not torch.is_grad_enabled() and not is_followed():
             # nothing to keep for a backward
             kv = (k, v) if k is not None else _temp_cache(bsz, attn.num_heads, tgt_len, attn.head_dim, x)
             out = core.stack_forward_only([(params, attn.num_heads, self.activation)], x, [kv], cache_len)
@@ -561,6 +562,12 @@ class TransformerLayer(nn.Module):
         if full_cache is not None:
             return res[0], (res[1], res[2])
         return res, None
+
+
+def is_followed():
+    """Whether somebody follows the computation node by node also without gradients: a trace records the layer as an autograd
+    function, forward-mode differentiation has that function refuse."""
+    return torch._C._get_tracing_state() is not None or forward_ad._current_level >= 0
 
 
 def is_plain(layer):

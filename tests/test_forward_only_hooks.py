@@ -82,3 +82,24 @@ def test_other_forwards(stack):
     assert run() == [1, 1, 1] and seen == ["instance"]
     del plain.forward
     assert run() == [3]
+
+
+def test_traces_and_forward_mode_see_the_autograd_function(stack, monkeypatch):
+    """What follows a computation without gradients meets the layer as the node it is with gradients."""
+    from terapipe_amd import transformer_models as tm
+    layers, run = stack
+    seen = []
+
+    class Node:
+        @staticmethod
+        def apply(heads, cache_len, activation, opts, x, k, v, *params):
+            seen.append("node")
+            return (x + 1, k, v)
+
+    monkeypatch.setattr(tm, "_LayerFunction", Node)
+    assert run() == [3] and not seen
+    with torch.autograd.forward_ad.dual_level():
+        assert run() == [] and len(seen) == 3
+    seen.clear()
+    monkeypatch.setattr(torch._C, "_get_tracing_state", lambda: object())
+    assert run() == [] and len(seen) == 3
