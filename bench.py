@@ -83,16 +83,18 @@ def gemm_shape_name(meta):
     return " + ".join("%s %dx%dx%d" % (GEMM_OPS[op], M, N, K) for (op, M, N, K) in metas)
 
 
-def pmc_traffic(workload):
+def pmc_traffic(workload, launches):
     """Bytes per GEMM launch of a step between L2 and the fabric, from the committed summary of the two rocprofv3 --pmc
     runs (FETCH_SIZE, WRITE_SIZE, each scaled by its reading on kernels of known size) over one step of this workload;
-    None when no such summary is in the tree."""
+    None when no such summary is in the tree, or only one of a step with another number of GEMM launches."""
     path = os.path.join(ROOT, "profiles", "bench_%s_gemm_hbm_traffic.pmc.txt" % workload)
     try:
-        m = re.search(r"traffic_bytes_per_gemm_launch:\s*([0-9.eE+]+)", open(path).read())
+        text = open(path).read()
     except OSError:
         return None
-    return float(m.group(1)) if m else None
+    n = re.search(r"gemm_launches_per_step:\s*(\d+)", text)
+    m = re.search(r"traffic_bytes_per_gemm_launch:\s*([0-9.eE+]+)", text)
+    return float(m.group(1)) if m and n and int(n.group(1)) == launches else None
 
 
 def build_model(w, device):
@@ -453,10 +455,10 @@ def measure_workload(name, args, device, detail):
     bound_s = sum(max(f / peak, b / PEAK_HBM) for f, b in work)
     attainable = sum(f for f, _ in work) / bound_s
     roof = {
-        "kernel": "tp::gemm_pipe_kernel / tp::gemm_tall_kernel / tp::gemm_dma_kernel / tp::gemm_stream_kernel (all NT/NN/TN launches of one step, "
-                  "split-K reduce included)",
+        "kernel": "tp::gemm_wide_kernel / tp::gemm_pipe_kernel / tp::gemm_tall_kernel / tp::gemm_dma_kernel / tp::gemm_stream_kernel (all "
+                  "NT/NN/TN launches of one step, split-K reduce included)",
         "bound": "mfma", "achieved": achieved / 1e12, "peak": peak / 1e12, "unit": "TFLOP/s",
-        "frac": achieved / peak, "traffic": pmc_traffic(name),
+        "frac": achieved / peak, "traffic": pmc_traffic(name, len(gemm_calls)),
         "traffic_note": "bytes per launch that L2 exchanges with the fabric (the memory-side cache serves part of them): rocprofv3 "
                         "FETCH_SIZE / 0.500 + WRITE_SIZE / 1.000, the factors read off a plain copy and a fill of known size in "
                         "the same counter runs; from the committed profiles/ summary of one eager step",
@@ -794,7 +796,10 @@ def main():
                    "launch": "HIP-graph replay of forward and of backward" if args.graph else
                              ("eager, every kernel launched from the host" if args.no_launch_replay else
                               "eager, recorded launches re-issued from the host"),
-                   "pieces": res["pieces"], "slice_streams": res["slice_streams"]},
+                   "slices": len(w["slices"]), "pieces": res["pieces"], "slice_streams": res["slice_streams"],
+                   "timed_step": "the runner as constructed by default: the workload's slices in one piece; cut as the workload "
+                                 "says: tokens_per_s_sliced, tokens_per_s_one_stream" if res["pieces"] == 1 else
+                                 "slice by slice"},
     }
     for k in ("ms_per_step_sliced", "tokens_per_s_sliced", "sliced_slice_streams", "ms_per_step_one_stream", "tokens_per_s_one_stream", "layer_surface", "roofline", "kernel_time_ms_per_step"):
         if k in res:
