@@ -2,57 +2,81 @@
 import weakref
 
 import torch
+from torch.utils.hooks import RemovableHandle
 
 from . import ops
 
-_KNOWN = "terapipe_amd"     # in the metadata of an AccumulateGrad node: its _Leaf
+# In the metadata of an AccumulateGrad node: the stream it runs on, and how many handles of hooks had been made, on anything,
+# when nobody had one on the node or on its parameter.
+_KNOWN = "terapipe_amd"
 
 
-class _Leaf:
-    """What was seen of one AccumulateGrad node: the stream it runs on (None: it has not run yet) and where Python hooks on
-    the node itself are kept."""
-    __slots__ = ("stream", "pre", "post")
+def fresh_leaves(params):
+    """Indices of the parameters that no autograd graph alive leads to, and that have no hooks: the next forward makes their
+    AccumulateGrad nodes.  (Such a node holds its parameter: there is more than the Python object's reference to one that
+    has a node.)  Where the first parameter has a node none is looked for: the kernels add all gradients of a node or none."""
+    if params[0]._use_count() != 1:
+        return ()
+    return [i for i, p in enumerate(params) if p._use_count() == 1 and not _has_tensor_hooks(p)]
 
-    def __init__(self, node):
-        # The node's stream is that of the first forward that used the parameter while the graph was alive, which need
-        # not be one of ours: it is read off when the node runs, by a hook that takes itself off again.
-        self.stream = None
 
-        def on_run(*_):
-            self.stream = ops._stream()
-            pre.remove()
+def _has_tensor_hooks(p):
+    return bool(p._backward_hooks or getattr(p, "_post_accumulate_grad_hooks", None))
 
-        pre, post = node.register_prehook(on_run), node.register_hook(on_run)
-        post.remove()
-        self.pre, self.post = pre.hooks_dict_ref, post.hooks_dict_ref
+
+def note_leaves(node, first, fresh):
+    """After a forward: what is known of the AccumulateGrad nodes that it made.  They run on the stream they were made on
+    as long as they live, and nobody has put a hook on them yet.  node.next_functions[first:] are the parameters'."""
+    if node is None or not fresh:
+        return
+    made = (ops._stream(), RemovableHandle.next_id)
+    nodes = node.next_functions
+    for i in fresh:
+        leaf = nodes[first + i][0]
+        if leaf is not None and leaf.metadata.setdefault(_KNOWN, made)[0] != made[0]:
+            leaf.metadata[_KNOWN] = (None, 0)       # (two threads at once, on two streams)
+
+
+def _has_hooks(node):
+    """Python hooks on an autograd node, found by putting one beside them."""
+    for register in (node.register_prehook, node.register_hook):
+        handle = register(_has_hooks)
+        n = len(handle.hooks_dict_ref())
+        handle.remove()
+        if n > 1:
+            return True
+    return False
 
 
 def engine_adds_to_grad(ctx, params, first):
     """Whether the kernels of this node may add its gradients to the parameters' .grad (autograd gets None) in place of the
     engine.  ctx.next_functions[first:] are the parameters' AccumulateGrad nodes.  They have to run in the backward pass
     under way (under torch.autograd.grad they do not: the query raises for captured leaves), nobody may look at the
-    gradients on the way (hooks on a parameter or on its node, a graph of the backward itself), and they have to run on
-    THIS node's stream: what another node hands the engine for the same parameter is added there, and that stream is the
-    one the caller of backward() waits for.  A node seen for the first time is only watched, so the first backward through
-    a graph hands its gradients to the engine (which has nothing to add them to then, as a rule)."""
+    gradients on the way (hooks on a parameter or on its node, a graph of the backward itself), and they have to be known
+    to run on THIS node's stream (note_leaves): what another node hands the engine for the same parameter is added there,
+    and that stream is the one the caller of backward() waits for.  A node that a forward of ours did not make -- somebody
+    used the parameter first, or holds its node, as data-parallel wrappers do -- is not known."""
     if torch.is_grad_enabled():
         return False
-    stream = ops._stream()
-    ours = True
+    stream, handles = ops._stream(), RemovableHandle.next_id
+    unsure = []
     try:
         for p, (node, _) in zip(params, ctx.next_functions[first:]):
-            if getattr(node, "variable", None) is not p or not torch._C._will_engine_execute_node(node):
+            if getattr(node, "variable", None) is not p:
                 return False
             known = node.metadata.get(_KNOWN)
-            if known is None:
-                node.metadata[_KNOWN] = _Leaf(node)
-                ours = False
-            elif known.stream != stream or known.pre() or known.post() or p._backward_hooks \
-                    or getattr(p, "_post_accumulate_grad_hooks", None):
-                ours = False
+            if known is None or known[0] != stream or not torch._C._will_engine_execute_node(node):
+                return False
+            if known[1] != handles:         # somebody has put a hook on something since
+                unsure.append((p, node))
     except RuntimeError:
         return False
-    return ours
+    if unsure:
+        if any(_has_tensor_hooks(p) or _has_hooks(node) for p, node in unsure):
+            return False
+        for p, node in unsure:
+            node.metadata[_KNOWN] = (stream, RemovableHandle.next_id)
+    return True
 
 
 _LOOKUPS = "terapipe_amd lookups"       # in the metadata of the node a weight's gradient goes to: see note_lookup

@@ -219,27 +219,30 @@ _ACTIVATIONS = {"relu": 0, "gelu": 1}
 LINEAR_INPUTS = ("xn", "o", "hn", "a")          # of in_proj, out_proj, fc1 and fc2
 
 
-def operands(params):
-    """(addresses, ldw) of a layer's 12 parameters in PARAM_NAMES order, as tp_layer_desc has them.  A weight may be a
-    column range of a wider matrix; what no kernel can read is refused."""
+def operands(params, dtype):
+    """(addresses, ldw) of a layer's 12 parameters in PARAM_NAMES order, as tp_layer_desc has them.  The library gets
+    addresses only: what is not in GPU memory, not of the layer's type or not laid out as a kernel can read it is refused."""
+    ldw = (0, 0, 0, 0)
+    for p in params:
+        if not (p.is_cuda and p.dtype is dtype and p.is_contiguous()):
+            ldw = _row_pitches(params, dtype)
+            break
+    return [p.data_ptr() for p in params], ldw
+
+
+def _row_pitches(params, dtype):
+    """ldw where a weight may be a column range of a wider matrix."""
     ldw = [0, 0, 0, 0]
     for i, p in enumerate(params):
+        ops._require_cuda(p)
+        if p.dtype is not dtype:
+            raise _lib.TeraPipeHipError("%s is %s, the layer's input %s" % (PARAM_NAMES[i], p.dtype, dtype))
         if not p.is_contiguous():
             if p.dim() != 2 or p.stride(1) != 1 or p.stride(0) < p.shape[1]:
                 raise _lib.TeraPipeHipError("%s: strides %s; a vector, and each row of a weight, has to be contiguous"
                                             % (PARAM_NAMES[i], tuple(p.stride())))
             ldw[(2, 4, 8, 10).index(i)] = p.stride(0)
-    return [p.data_ptr() for p in params], ldw
-
-
-def require_operands(x, params, k_cache, v_cache):
-    """The library gets addresses only: everything a layer reads or writes is in GPU memory and of x's type."""
-    ops._require_cuda(x, k_cache, v_cache)
-    dtype = x.dtype
-    for i, p in enumerate(params):
-        if not p.is_cuda or p.dtype is not dtype:
-            ops._require_cuda(p)
-            raise _lib.TeraPipeHipError("%s is %s, the layer's input %s" % (PARAM_NAMES[i], p.dtype, dtype))
+    return ldw
 
 
 class _Arena:
@@ -288,7 +291,7 @@ class LayerGeometry:
     def pack_fwd(self, image, at, cache_len, cache_rows, params, x, k, v, base, out, over=None):
         """Writes a tp_layer_desc at byte `at` of `image`.  params: the layer's 12; base: address of the forward arena; over: the
         addresses of LINEAR_INPUTS where they are not part of it (its layout is fwd_rest then)."""
-        w_ptrs, ldw = operands(params)
+        w_ptrs, ldw = operands(params, self.dtype)
         o = (self.fwd_rest if over else self.fwd).off
         p = {n: base + o[n] for n in o}
         if over:
@@ -332,12 +335,17 @@ def stack_forward_only(layers, x, caches, cache_len):
     set of intermediate buffers.  layers: [(12 parameters in PARAM_NAMES order, heads, activation)], each with its own
     FFN width, heads and activation; caches: [(k, v)] per layer.  Returns the output [T, B, E]."""
     T, B, E = x.shape
-    for (params, _, _), (k, v) in zip(layers, caches):
-        require_operands(x, params, k, v)
+    ops._require_cuda(x, *(c for kv in caches for c in kv))
     x = x.contiguous()
     n = len(layers)
-    geos = [LayerGeometry.of(T, B, E, params[8].shape[0], heads, x.dtype, activation) for params, heads, activation in layers]
-    shared = max(g.fwd.total for g in geos)
+    known = {}
+    geos = []
+    for params, heads, activation in layers:
+        kind = (params[8].shape[0], heads, activation)
+        if kind not in known:
+            known[kind] = LayerGeometry.of(T, B, E, kind[0], heads, x.dtype, activation)
+        geos.append(known[kind])
+    shared = max(g.fwd.total for g in known.values())
     step = (T * B * E * geos[0].es + 255) // 256 * 256
     # one allocation: the arena and, from two layers on, the outputs between the layers in turn
     arena = torch.empty(shared + (2 if n > 2 else n - 1) * step, dtype=torch.uint8, device=x.device)

@@ -19,7 +19,7 @@ from torch.nn.modules import module as _modules
 
 from . import _layer_core as core
 from . import ops
-from ._autograd import engine_adds_to_grad
+from ._autograd import engine_adds_to_grad, fresh_leaves, note_leaves
 from ._lib import TP_EPI_ACCUMULATE, TP_EPI_BIAS, TP_EPI_STORE, TP_GEMM_NN, TP_GEMM_NT, TP_GEMM_TN
 
 # reference transformer_models.py:16 -- kept for callers that import it; the kernels mask by index.
@@ -184,13 +184,15 @@ def _temp_cache(B, H, T, Dh, like):
 
 
 def _grads_can_go_in_place(w):
-    """Every parameter of the layer already has a dense .grad of its own dtype to add to, where the kernels can write it."""
-    for n, p in w.items():
-        g = p.grad if p.is_leaf else None
-        if g is None or g.dtype != p.dtype or g.shape != p.shape or g.layout != torch.strided or not g.is_contiguous() \
-                or (n in core.BIG_PARAMS and g.data_ptr() % 16):
-            return False
-    return True
+    """Every parameter of the layer is a leaf with a dense .grad of its own dtype to add to, where the kernels can write it."""
+    try:
+        for p in w.values():
+            g = p.grad if p.is_leaf else None
+            if g is None or g.dtype is not p.dtype or g.shape != p.shape or not g.is_contiguous():
+                return False
+    except RuntimeError:        # (a sparse one is neither contiguous nor not)
+        return False
+    return not any(w[n].grad.data_ptr() % 16 for n in core.BIG_PARAMS)
 
 
 class _GradOptions:
@@ -257,16 +259,16 @@ class _LayerFunction(torch.autograd.Function):
     Forward and backward are one library call each (tp_layers_fwd, tp_layer_bwd).  The backward of a slice: the data
     gradients, the eight vector-parameter gradients as one launch, the four weight gradients as one grouped one.
     Where every parameter already has a .grad that the engine is going to add to on this node's stream
-    (_autograd.engine_adds_to_grad: a slice loop's second backward is the first that can know), or with opts.in_place, the
-    kernels add the gradients to it (the GEMM's accumulate epilogue, one rounding) and autograd gets None, instead of
-    twelve tensors that autograd adds one elementwise kernel each.  opts.defer -- keep the slice's dY / X
+    (_autograd.engine_adds_to_grad), or with opts.in_place, the kernels add the gradients to it (the GEMM's accumulate
+    epilogue, one rounding) and autograd gets None, instead of twelve tensors that autograd adds one elementwise kernel
+    each.  opts.defer -- keep the slice's dY / X
     rows and take the weight gradients once per sequence, over all its rows, in the backward of the slice at position 0
     (the last one the reverse-slice order reaches); the slices before it hand autograd None for the parameters."""
 
     @staticmethod
     def forward(ctx, heads, cache_len, activation, opts, x, k_cache, v_cache, *params):
         T, B, E = x.shape
-        core.require_operands(x, params, k_cache, v_cache)
+        ops._require_cuda(x, k_cache, v_cache)
         dt, dev = x.dtype, x.device
         F = params[8].shape[0]
         ctx.has_cache = k_cache is not None
@@ -358,8 +360,8 @@ class _LayerFunction(torch.autograd.Function):
                 if opts.inputs.get(key) is seq:
                     del opts.inputs[key]
                 rows = pend.rows
-        in_place = done and (opts.in_place or engine_adds_to_grad(ctx, ctx.w, 3 if ctx.has_cache else 1)) \
-            and _grads_can_go_in_place(w)
+        in_place = done and _grads_can_go_in_place(w) and \
+            (opts.in_place or engine_adds_to_grad(ctx, ctx.w, 3 if ctx.has_cache else 1))
         wg_out, small_out, wg = (0,) * 4, (0,) * 8, (0,) * 8
         grads = {}
         if done:
@@ -558,9 +560,12 @@ class TransformerLayer(nn.Module):
             return out, None if k is None else (k, v)
         opts = self._grad_options
         opts.in_place, opts.defer = bool(self.accumulate_grads_in_place), bool(self.defer_weight_grads)
+        fresh = fresh_leaves(params)
         res = _LayerFunction.apply(attn.num_heads, cache_len, self.activation, opts, x, k, v, *params)
         if full_cache is not None:
+            note_leaves(res[0].grad_fn, 3, fresh)
             return res[0], (res[1], res[2])
+        note_leaves(res.grad_fn, 1, fresh)
         return res, None
 
 

@@ -22,7 +22,7 @@ def descriptors(monkeypatch):
 
     monkeypatch.setattr(core, "layers_fwd", forward)
     monkeypatch.setattr(core, "layer_bwd_native", backward)
-    monkeypatch.setattr(core, "require_operands", lambda *a: None)
+    monkeypatch.setattr(ops, "_require_cuda", lambda *tensors: None)
     monkeypatch.setattr(ops, "_stream", lambda: 0)
     return made
 

@@ -21,11 +21,20 @@ class _Twice(torch.autograd.Function):
         ops._stream.now = ctx.stream
         ours = _autograd.engine_adds_to_grad(ctx, (ctx.p,), 1)
         ctx.log.append(ours)
-        ops._stream.now = ops._stream.leaf       # the stream the AccumulateGrad node is going to find
         if ours:
-            ctx.p.grad += (2 * x * dy).detach()
+            ctx.p.grad = (0 if ctx.p.grad is None else ctx.p.grad) + (2 * x * dy).detach()
             return None, None, None, None
         return None, 2 * x * dy, None, None
+
+
+def _twice(x, p, stream=0, log=None):
+    """As the layers call theirs, on a stream."""
+    from terapipe_amd import _autograd, ops
+    ops._stream.now = stream
+    fresh = _autograd.fresh_leaves([p])
+    y = _Twice.apply(x, p, stream, log)
+    _autograd.note_leaves(y.grad_fn, 1, fresh)
+    return y
 
 
 @pytest.fixture
@@ -35,40 +44,56 @@ def streams(monkeypatch):
     def current():
         return current.now
 
-    current.now = current.leaf = 0
+    current.now = 0
     monkeypatch.setattr(ops, "_stream", current)
     return current
 
 
-def _slices(p, n, log, stream=0):
-    return [_Twice.apply(torch.full((3,), float(i + 1)), p, stream, log).sum() for i in range(n)]
+def _slices(p, streams_of, log):
+    return [_twice(torch.full((3,), float(i + 1)), p, s, log).sum() for i, s in enumerate(streams_of)]
 
 
-@pytest.mark.parametrize("node,leaf,ours", [(0, 0, True), (7, 7, True), (7, 0, False), (0, 7, False)])
-def test_only_on_the_stream_of_the_engines_own_addition(streams, node, leaf, ours):
+def test_only_on_the_stream_of_the_engines_own_addition(streams):
+    """The AccumulateGrad node is the first forward's: slices on its stream add, others hand their gradients over."""
+    for on in ([0, 0, 0], [7, 7, 7], [7, 0, 7], [0, 7, 9]):
+        p, log = torch.nn.Parameter(torch.ones(3)), []
+        for y in _slices(p, on, log):
+            y.backward()
+        assert log == [s == on[0] for s in on]
+        assert torch.equal(p.grad, torch.full((3,), 12.0))
+
+
+def test_a_node_that_somebody_else_made(streams):
+    """By using the parameter first, by holding its node; a parameter that is used again by nobody is ours again."""
     p, log = torch.nn.Parameter(torch.ones(3)), []
-    streams.leaf = leaf
-    outs = _slices(p, 4, log, node)
-    for y in outs:
+    other = (p * 0.5).sum()
+    for y in _slices(p, [0, 0], log) + [other]:
         y.backward()
-    assert log == [False, ours, ours, ours]      # the first one has not seen the node run
-    assert torch.equal(p.grad, torch.full((3,), 20.0))
+    assert log == [False, False] and torch.equal(p.grad, torch.full((3,), 6.5))
+    node = torch.autograd.graph.get_gradient_edge(p).node
+    _slices(p, [0], log)[0].backward()
+    assert log.pop() is False and node.variable is p
+    del node, other, y
+    _slices(p, [0], log)[0].backward()
+    assert log.pop() is True and torch.equal(p.grad, torch.full((3,), 10.5))
 
 
-def test_other_streams_forward_in_one_graph(streams):
-    """One of the slices ran elsewhere: it hands its gradient to the engine, the others add theirs."""
+def test_two_threads_make_the_node_at_once(streams):
+    """Both found no node and both note their own stream: neither is believed."""
+    from terapipe_amd import _autograd
     p, log = torch.nn.Parameter(torch.ones(3)), []
-    outs = _slices(p, 2, log) + _slices(p, 1, log, 9)
-    outs[0].backward()
-    sum(outs[1:]).backward()
-    assert sorted(log) == [False, False, True] and torch.equal(p.grad, torch.full((3,), 8.0))
+    y0, y1 = _twice(torch.ones(3), p, 0, log), _twice(torch.ones(3), p, 5, log)
+    _autograd.note_leaves(y1.grad_fn, 1, [0])
+    y0.sum().backward()
+    y1.sum().backward()
+    assert log == [False, False]
 
 
 def test_who_looks_at_gradients(streams):
     """Hooks on the parameter or on its node, torch.autograd.grad and a graph of the backward get tensors; hooks that are
-    gone do not count."""
+    gone, or on something else, do not count."""
     p, log = torch.nn.Parameter(torch.ones(3)), []
-    outs = _slices(p, 9, log)
+    outs = _slices(p, [0] * 9, log)
     node = outs[0].grad_fn.next_functions[0][0].next_functions[1][0]
     one = torch.full((3,), 1.0)
     outs[0].backward()
@@ -81,9 +106,11 @@ def test_who_looks_at_gradients(streams):
         outs[i].backward()
         handle.remove()
         assert torch.equal(seen.pop(), 2 * (i + 1) * one) and not seen
-    assert log == [False] * 5 and torch.equal(p.grad, 30 * one)
+    assert log == [True] + [False] * 4 and torch.equal(p.grad, 30 * one)
     assert torch.equal(torch.autograd.grad(outs[5], p)[0], 12 * one)
+    elsewhere = torch.nn.Linear(1, 1).register_forward_hook(print)
     torch.autograd.backward([outs[6]], inputs=[p])
+    elsewhere.remove()
     outs[7].backward(create_graph=True)
     outs[8].backward()
     assert log[5:] == [False, True, False, True] and torch.equal(p.grad.detach(), (30 + 14 + 16 + 18) * one)
@@ -94,7 +121,7 @@ def test_parameters_that_are_no_leaves_or_frozen(streams):
     for q in (p * 1, torch.ones(3)):
         for _ in range(2):
             x = torch.ones(3, requires_grad=True)
-            (_Twice.apply(x, q, 0, log) + x).sum().backward(retain_graph=True)
+            (_twice(x, q, 0, log) + x).sum().backward(retain_graph=True)
     assert log == [False] * 4
 
 

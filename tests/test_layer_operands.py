@@ -40,23 +40,24 @@ def _forward_backward(layer, x, dy, P=3):
     return [y.detach(), y0, x.grad] + [c.grad for c in caches] + [p.grad for p in layer.param_list()]
 
 
-def test_addresses_and_row_pitches():
+def test_addresses_and_row_pitches(monkeypatch):
     from terapipe_amd import _layer_core as core
-    from terapipe_amd import _lib
+    from terapipe_amd import _lib, ops
+    monkeypatch.setattr(ops, "_require_cuda", lambda *tensors: None)
     layer = _layer(64, 1, 128, torch.float16, device="cpu")
-    ptrs, ldw = core.operands(layer.param_list())
-    assert ptrs == [p.data_ptr() for p in layer.param_list()] and ldw == [0] * 4
+    ptrs, ldw = core.operands(layer.param_list(), torch.float16)
+    assert ptrs == [p.data_ptr() for p in layer.param_list()] and list(ldw) == [0] * 4
     _replace_weights(layer, _column_range)
-    ptrs, ldw = core.operands(layer.param_list())
+    ptrs, ldw = core.operands(layer.param_list(), torch.float16)
     assert ptrs == [p.data_ptr() for p in layer.param_list()] and ldw == [64 + 24] * 3 + [128 + 24]
     for change in (lambda w: w.t().contiguous().t(), lambda w: w[:1].expand(w.shape), lambda w: torch.cat([w, w], 1)[:, ::2]):
         _replace_weights(layer, change)
         with pytest.raises(_lib.TeraPipeHipError, match="in_proj.weight: strides"):
-            core.operands(layer.param_list())
+            core.operands(layer.param_list(), torch.float16)
     layer = _layer(64, 1, 128, torch.float16, device="cpu")
     layer.fc1.bias = torch.nn.Parameter(torch.zeros(256, dtype=torch.float16)[::2])
     with pytest.raises(_lib.TeraPipeHipError, match="fc1.bias: strides"):
-        core.operands(layer.param_list())
+        core.operands(layer.param_list(), torch.float16)
 
 
 @pytest.mark.gpu
