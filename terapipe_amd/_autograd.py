@@ -85,7 +85,7 @@ _TAKEN = object()
 
 def note_lookup(node, index):
     """Remembers an autograd node whose backward adds a few rows to a dense gradient (an embedding): a product with the same
-    weight may hand it that gradient (take_on).  node.next_functions[index] is the weight's."""
+    weight may hand it that gradient (lookup_to_hand_to).  node.next_functions[index] is the weight's."""
     weight, _ = node.next_functions[index]
     if weight is not None:
         node.stream, node.task, node.handed = ops._stream(), None, None
@@ -120,6 +120,6 @@ def lookup_to_hand_to(ctx, index):
 def taken_on(ctx):
     """In the backward of a node (note_lookup): the gradient it was handed, its own from now on, or None."""
     task = torch._C._current_graph_task_id()
-    handed = ctx.handed if ctx.task == task else None
+    handed = ctx.handed if getattr(ctx, "task", None) == task else None
     ctx.task, ctx.handed = task, _TAKEN
     return handed

@@ -210,3 +210,12 @@ def test_nothing_is_kept_alive(calls):
     for _ in range(5):
         emb(IDS).sum().backward()
     assert len(node.metadata[_autograd._LOOKUPS]) == 1
+
+
+def test_a_lookup_nobody_noted(calls):
+    """The autograd function by itself, without the module."""
+    from terapipe_amd import vocab
+    emb, h = _embedding(), _hidden()
+    (vocab._EmbeddingFunction.apply(IDS, emb.weight).sum() + _head(h, emb.weight)).backward()
+    _same(emb.weight.grad, _expected(emb.weight, [1.0], [h]))
+    assert sorted(calls()) == ["dw", "zeros"]
