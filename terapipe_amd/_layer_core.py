@@ -213,7 +213,9 @@ def layer_bwd(w, st, dout, heads, gk, gv, accumulate_prefix, has_incoming, zero_
 # A layer is nine to fifteen launches; issued one by one through ops.py each costs about 11 us of Python, which bounds
 # short slices from the host.
 # ------------------------------------------------------------------------------------------------
-_FWD_PACK = struct.Struct("8iq28Q4q")          # tp_layer_desc
+_FWD_PACK = struct.Struct("8iq28Q4q")          # tp_layer_desc: sizes, w[12], x, k_cache, v_cache, ..., ldw[4]
+_FWD_READ, _FWD_LDW = struct.Struct("15Q"), struct.Struct("4q")
+_FWD_READ_AT, _FWD_LDW_AT = 8 * 4 + 8, 8 * 4 + 8 + 28 * 8
 _BWD_PACK = struct.Struct("12Q4iq8Q4Q2i8Q2i")  # tp_layer_bwd_desc after its tp_layer_desc
 _ACTIVATIONS = {"relu": 0, "gelu": 1}
 LINEAR_INPUTS = ("xn", "o", "hn", "a")          # of in_proj, out_proj, fc1 and fc2
@@ -300,6 +302,13 @@ class LayerGeometry:
                             cache_len, cache_rows, *w_ptrs, x, k, v, p["xn"], p["mean1"], p["rstd1"], p["q"], p["o"],
                             p["lse"], p["h"], p["mean2"], p["rstd2"], p["hn"], p["a"],
                             p["z"] if self.activation == "gelu" else 0, out, *ldw)
+
+
+def repack_operands(image, params, x, k, v):
+    """Writes into a packed tp_layer_desc where the parameters, the input and the caches are NOW."""
+    w_ptrs, ldw = operands(params, x.dtype)
+    _FWD_READ.pack_into(image, _FWD_READ_AT, *w_ptrs, x.data_ptr(), k.data_ptr(), v.data_ptr())
+    _FWD_LDW.pack_into(image, _FWD_LDW_AT, *ldw)
 
 
 def _address(image):

@@ -296,7 +296,7 @@ class _LayerFunction(torch.autograd.Function):
                      arena.data_ptr(), out.data_ptr(), over)
         core.layers_fwd(image, 1, dev)
         ctx.geo, ctx.cache_len, ctx.opts = geo, cache_len, opts
-        ctx.image = image               # the descriptor's addresses stay valid: what they point to is kept
+        ctx.image = image               # the descriptor, for the backward to go on from (repack_operands)
         ctx.kept = (x, k_cache, v_cache, arena, seq)
         ctx.st = _SliceKept(geo, arena, seq, cache_len)
         ctx.w = params
@@ -381,6 +381,7 @@ class _LayerFunction(torch.autograd.Function):
             else:
                 xn, o, hn, a = (fbase + fo[n] for n in core.LINEAR_INPUTS)
                 wg = (p["dqkv"], xn, p["dh"], o, p["dz1"], hn, dy, a)
+        core.repack_operands(ctx.image, ctx.w, x, k_cache, v_cache)     # (a parameter's storage may have been replaced)
         core._BWD_PACK.pack_into(ctx.image, core._FWD_PACK.size, dy, p["dz1"], p["dhn"], p["dh"], p["d_o"], p["dqkv"],
                                  p["dxn"], dx.data_ptr(), p["delta"], p["small"],
                                  0 if gk is None else gk.data_ptr(), 0 if gv is None else gv.data_ptr(),

@@ -133,3 +133,45 @@ def test_a_layer_can_be_copied_and_pickled():
         assert all(torch.equal(a, b) for a, b in zip(other.param_list(), layer.param_list()))
         assert not other._grad_options.pending and not other._grad_options.inputs
         assert other._grad_options is not layer._grad_options
+
+
+def test_the_backward_reads_the_parameters_where_they_are_then(monkeypatch):
+    """Not where they were when the forward ran: storage that was replaced in between may be anybody's."""
+    from terapipe_amd import _layer_core as core
+    from terapipe_amd import _lib, ops
+    made = []
+    monkeypatch.setattr(core, "layers_fwd", lambda images, n, device: made.append(_lib.LayerDesc.from_buffer_copy(images)))
+    monkeypatch.setattr(core, "layer_bwd_native", lambda image, device: made.append(_lib.LayerBwdDesc.from_buffer_copy(image).f))
+    monkeypatch.setattr(ops, "_require_cuda", lambda *tensors: None)
+    monkeypatch.setattr(ops, "_stream", lambda: 0)
+    layer = _layer(64, 1, 128, torch.float32, device="cpu")
+    y, _ = layer(torch.zeros(4, 1, 64, requires_grad=True))
+    kept = [p.data for p in layer.param_list()]         # (keeps the old memory from being handed out again)
+    for p in layer.param_list():
+        p.data = _column_range(p.data) if p.dim() == 2 else p.data.clone()
+    y.sum().backward()
+    forward, backward = made
+    assert list(forward.w) == [t.data_ptr() for t in kept] and list(forward.ldw) == [0] * 4
+    assert list(backward.w) == [p.data_ptr() for p in layer.param_list()] and list(backward.ldw) == [64 + 24] * 3 + [128 + 24]
+    same = [name for name, _ in _lib.LayerDesc._fields_ if name not in ("w", "ldw")]
+    assert [getattr(forward, n) for n in same] == [getattr(backward, n) for n in same]
+
+
+@pytest.mark.gpu
+def test_parameters_that_move_between_forward_and_backward():
+    layer = _layer(128, 2, 512, torch.float16)
+    x, dy = (torch.randn(9, 2, 128, device="cuda").half() for _ in range(2))
+    ref = _forward_backward(layer, x, dy)[5:]
+    layer.zero_grad()
+    g = torch.Generator(device="cuda").manual_seed(1)
+    caches = [torch.randn(4, 12, 64, generator=g, device="cuda").half().requires_grad_() for _ in range(2)]
+    y, _ = layer(x.clone().requires_grad_(), tuple(caches), 3)
+    for p in layer.param_list():
+        old, p.data = p.data, p.data.clone()
+        old.fill_(float("nan"))
+    del old
+    junk = [torch.full((128, 512), float("nan"), dtype=torch.float16, device="cuda") for _ in range(8)]
+    y.backward(dy)
+    for i, (p, r) in enumerate(zip(layer.param_list(), ref)):
+        assert_close(p.grad, r, torch.float16, "parameter %d" % i, 0.1)
+    assert all(t.isnan().all() for t in junk)
