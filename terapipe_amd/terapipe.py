@@ -17,7 +17,7 @@ from . import _layer_core as core
 from . import _lib
 from . import ops
 from ._lib import TP_EPI_ACCUMULATE, TP_EPI_STORE, TP_GEMM_TN
-from .transformer_models import ModelParallelTransformerLayer, _check_cache, grid_slice_batch_and_sequence, is_followed, is_plain
+from .transformer_models import ModelParallelTransformerLayer, _check_cache, all_plain, grid_slice_batch_and_sequence, is_followed
 
 
 def loss_func(y):
@@ -64,7 +64,7 @@ class TransformerLayers(nn.Module):
         return cache
 
     def forward(self, x, cache, cache_len):
-        if not torch.is_grad_enabled() and self.n_layers and not is_followed() and all(is_plain(layer) for layer in self.layers):
+        if not torch.is_grad_enabled() and self.n_layers and not is_followed() and all_plain(self.layers):
             return self._forward_only(x, cache, cache_len), list(cache[:2 * self.n_layers])
         cache_outputs = []
         for layer_id in range(self.n_layers):
@@ -78,8 +78,7 @@ class TransformerLayers(nn.Module):
         T, B, E = x.shape
         assert E == self.embedding_dim
         stack, caches = [], []
-        for i in range(self.n_layers):
-            layer = self.layers[i]
+        for i, layer in zip(range(self.n_layers), self.layers):     # (indexing a ModuleList costs 3 us)
             attn = layer._modules["attn"]
             caches.append(_check_cache((cache[2 * i], cache[2 * i + 1]), B, attn.num_heads, attn.head_dim, cache_len + T, x.dtype))
             stack.append((layer.param_list(), attn.num_heads, layer.activation))

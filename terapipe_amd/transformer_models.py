@@ -576,15 +576,18 @@ def is_followed():
     return torch._C._get_tracing_state() is not None or forward_ad._current_level >= 0
 
 
-def is_plain(layer):
-    """Whether calling the module is TransformerLayer.forward and nothing else: no subclass's or instance's own forward, no
-    wrapper in the layer's place, no forward hooks (on the module or for all modules), not compiled.  A stack of such layers
-    can run as one library call without anyone seeing the difference."""
-    kind = type(layer)
-    return (isinstance(layer, TransformerLayer) and kind.forward is TransformerLayer.forward
-            and kind.__call__ is nn.Module.__call__ and "forward" not in layer.__dict__
-            and not (layer._forward_hooks or layer._forward_pre_hooks or _modules._global_forward_hooks
-                     or _modules._global_forward_pre_hooks) and layer._compiled_call_impl is None)
+def all_plain(layers):
+    """Whether calling each of the modules is TransformerLayer.forward and nothing else: no subclass's or instance's own
+    forward, no wrapper in a layer's place, no forward hooks (on a module or for all modules), not compiled.  A stack of such
+    layers can run as one library call without anyone seeing the difference."""
+    if _modules._global_forward_hooks or _modules._global_forward_pre_hooks:
+        return False
+    for layer in layers:
+        kind, own = type(layer), layer.__dict__
+        if (kind.forward is not TransformerLayer.forward or kind.__call__ is not nn.Module.__call__ or "forward" in own
+                or own["_forward_hooks"] or own["_forward_pre_hooks"] or layer._compiled_call_impl is not None):
+            return False
+    return True
 
 
 class ModelParallelMultiheadLMAttentionWithCache(MultiheadLMAttentionWithCache):
