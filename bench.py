@@ -408,8 +408,9 @@ def measure_workload(name, args, device, detail):
             "tokens_per_s_deferred_weight_grads": w["L"] * w["B"] / (msd * 1e-3),
             "what": "ModelParallelTransformerLayer.forward per slice under the reference's own loop and autograd "
                     "(terapipe.py:249-264, :182-191): per-slice parameter-gradient GEMMs, gradient caches, one stream, "
-                    "every launch issued from Python; grads_in_place: with accumulate_grads_in_place=True, the "
-                    "slices after the first add their parameter gradients to .grad inside the gradient kernels; "
+                    "one library call per layer and direction; the slices after the first add their parameter gradients to "
+                    ".grad inside the gradient kernels; grads_in_place: with accumulate_grads_in_place=True, which asks for "
+                    "that whoever looks at the gradients; "
                     "deferred_weight_grads: with defer_weight_grads=True, a sequence's weight gradients are taken once, "
                     "in the backward of its first slice, over all its rows"}
     if args.no_roofline:
