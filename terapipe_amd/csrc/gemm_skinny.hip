@@ -11,8 +11,9 @@ namespace tp {
 // registers the MFMA takes (lane l: row l & 15, k 8 * (l >> 4) .. + 7 of each 32), the activation rows the same way
 // (they stay in the caches; NT weight tiles share one read of them).  No LDS and no barrier until the eight partial
 // tiles are added at the end.
-// Measured (4 rows, weights from HBM): 6144 x 2048 10.3 -> 8.4 us, 2048 x 2048 8.5 -> 5.3, 2048 x 8192 (four k splits)
-// 14.6 -> 8.2 (4.1 TB/s), 2304 x 768 6.1 -> 3.7.
+// Measured (4 rows, weights from HBM, the same launch back to back): 6144 x 2048 10.3 -> 8.4 us, 2048 x 2048 8.5 -> 5.3,
+// 2048 x 8192 (four k splits) 14.6 -> 8.2 (4.1 TB/s), 2304 x 768 6.1 -> 3.7.  In a decoding step's chain of dependent
+// launches: 9.9 (2.6 TB/s), 6.0 (1.4), 9.8 (3.4), 8192 x 2048 11.6 (2.9).
 // ---------------------------------------------------------------------------------------------
 template <typename T, int MB, int NT>
 __global__ __launch_bounds__(512) void gemm_skinny_kernel(GemmArgs a) {
