@@ -163,6 +163,9 @@ int tp_gemm_splits(const tp_gemm_desc* d);
 /* The plan tp_gemm would run the product with: the tile configuration's number (the kernel and tile shape, as listed
  * in csrc/gemm.hip) and the number of k splits.  Host code only; for tuning, tests and logs. */
 int tp_gemm_plan(const tp_gemm_desc* d, int* tile_cfg, int* nsplit);
+/* Rows and columns of the tile (0: the kernel of few rows has none) and the k splits of the launch that tp_gemm makes, with
+ * static_ws of that of tp_gemm_static_ws.  Host code only; for tuning, tests and logs. */
+int tp_gemm_tile(const tp_gemm_desc* d, int static_ws, int* rows, int* columns, int* nsplit);
 size_t tp_gemm_workspace_bytes(const tp_gemm_desc* d);
 int tp_gemm(const tp_gemm_desc* d, void* workspace, size_t workspace_bytes, void* stream);
 /* n independent products as if by n tp_gemm calls in order on the stream (the four weight gradients of a layer,
@@ -178,7 +181,7 @@ int tp_gemm_group_cfg(const tp_gemm_desc* descs, int n);
  * callers only.  The k-split partial sums go to a TP_GEMM_STATIC_WS_BYTES array that the library holds in every
  * GPU's memory from load to process exit; the call allocates and frees nothing.  Same kernels, same plan, same
  * result bits as tp_gemm with a caller workspace, but for a plan of the library's own whose splits need more than the array
- * holds: that is cut to the splits that fit.  With forced splits that need more the call is refused with TP_ERR_WORKSPACE,
+ * holds: that is cut to the splits that fit, on the same tile.  With forced splits that need more the call is refused with TP_ERR_WORKSPACE,
  * defer_reduce with TP_ERR_ARG.  Every call on a GPU shares that GPU's array: calls that overlap on one GPU (two streams, two
  * threads) race on the partial sums; nothing in it needs to start at zero.  The array's address on a device is
  * looked up once, by the first call of either function with that device current (a module and symbol lookup):

@@ -172,7 +172,7 @@ static const TunedPlan* find_tuned(const tp_gemm_desc* d) {
 struct GemmPlan {
     int cfg;
     int nsplit;
-    int kper;
+    int kper, bk;   // k per split, and the k-tile it is a multiple of
     int gx, gy;
     int deep;       // columns of the deep-ring tile (gemm_deep.hip) that runs configuration 12, 0: none
     int wide;       // columns of the eight-wave tile (gemm_wide.hip) that runs configuration 44: 256 or 192
@@ -183,6 +183,7 @@ static void finish_plan(const tp_gemm_desc* d, GemmPlan& p, int bk, int nsplit) 
     if (nsplit > kt) nsplit = (int)kt;
     if (nsplit < 1) nsplit = 1;
     long per = (kt + nsplit - 1) / nsplit;
+    p.bk = bk;
     p.kper = (int)(per * bk);
     p.nsplit = (int)((d->K + p.kper - 1) / p.kper);
 }
@@ -477,6 +478,19 @@ static GemmPlan plan_gemm(const tp_gemm_desc* d) {
     return p;
 }
 
+static size_t plan_bytes(const tp_gemm_desc* d, const GemmPlan& p) {
+    return p.nsplit > 1 ? (size_t)p.nsplit * d->M * d->N * sizeof(float) : 0;
+}
+
+// The plan of tp_gemm_static_ws: splits of the library's own that need more than the built-in workspace are cut to what fits,
+// on the same tile, so that what fits it does not hang on how the plan weighs splits.
+static GemmPlan plan_static_ws(const tp_gemm_desc* d) {
+    GemmPlan p = plan_gemm(d);
+    if (plan_bytes(d, p) > (size_t)TP_GEMM_STATIC_WS_BYTES && !((d->reserved >> 8) & 0xff))
+        finish_plan(d, p, p.bk, (int)((size_t)TP_GEMM_STATIC_WS_BYTES / ((size_t)d->M * d->N * sizeof(float))));
+    return p;
+}
+
 // the tile configurations of gemm_pipe.hip
 static inline bool is_pipe_cfg(int cfg) { return cfg == 6 || cfg == 7 || (cfg >= 14 && cfg <= 16) || (cfg >= 41 && cfg <= 43); }
 
@@ -589,10 +603,22 @@ extern "C" int tp_gemm_plan(const tp_gemm_desc* d, int* tile_cfg, int* nsplit) {
     return TP_OK;
 }
 
+extern "C" int tp_gemm_tile(const tp_gemm_desc* d, int static_ws, int* rows, int* columns, int* nsplit) {
+    int rc = tp::validate_gemm(d);
+    if (rc != TP_OK) return rc;
+    const tp::GemmPlan p = static_ws ? tp::plan_static_ws(d) : tp::plan_gemm(d);
+    tp::TileCfg tc = {};
+    if (tp::runs_f32_small(d)) tc = {32, 32, 0, 0};
+    else if (!tp::runs_skinny(d)) tp::tile_cfg(p.cfg, tc);
+    if (rows) *rows = tc.bm;
+    if (columns) *columns = p.deep ? p.deep : p.wide ? p.wide : tc.bn;
+    if (nsplit) *nsplit = p.nsplit;
+    return TP_OK;
+}
+
 extern "C" size_t tp_gemm_workspace_bytes(const tp_gemm_desc* d) {
     if (tp::validate_gemm(d) != TP_OK) return 0;
-    tp::GemmPlan p = tp::plan_gemm(d);
-    return p.nsplit > 1 ? (size_t)p.nsplit * d->M * d->N * sizeof(float) : 0;
+    return tp::plan_bytes(d, tp::plan_gemm(d));
 }
 
 namespace tp {
@@ -612,6 +638,24 @@ static GemmArgs fill_args(const tp_gemm_desc* d, const GemmPlan& p, void* worksp
     a.P = d->cache_len; a.cache_rows = d->cache_rows; a.qscale = d->q_scale;
     a.kper = p.kper; a.nsplit = p.nsplit; a.partial = reinterpret_cast<float*>(workspace);
     return a;
+}
+
+static int run_gemm(const tp_gemm_desc* d, const GemmPlan& p, void* workspace, void* stream) {
+    const GemmArgs a = fill_args(d, p, workspace);
+    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
+    bool launched;
+    switch (d->dtype) {
+    case TP_F32: launched = launch_gemm<float>(d, p, a, s); break;
+    case TP_F16: launched = launch_gemm<f16>(d, p, a, s); break;
+    default: launched = launch_gemm<bf16>(d, p, a, s); break;
+    }
+    if (!launched) {
+        set_error("tp_gemm: no kernel for tile configuration %d with op %d, dtype %d", p.cfg, d->op, d->dtype);
+        return TP_ERR_UNSUPPORTED;
+    }
+    hipError_t e = hipGetLastError();
+    if (e != hipSuccess) { set_error("tp_gemm: launch failed: %s", hipGetErrorString(e)); return TP_ERR_LAUNCH; }
+    return TP_OK;
 }
 
 // One launch for the whole group when every member is a 16-bit TN product (parameter gradients) of the same dtype and
@@ -755,18 +799,8 @@ extern "C" int tp_gemm_static_ws(const tp_gemm_desc* d, void* stream) {
         tp::set_error("tp_gemm_static_ws: defer_reduce hands the workspace to a later call; use tp_gemm");
         return TP_ERR_ARG;
     }
-    tp::GemmPlan p = tp::plan_gemm(d);
-    size_t need = p.nsplit > 1 ? (size_t)p.nsplit * d->M * d->N * sizeof(float) : 0;
-    // a plan of the library's own takes the splits that the built-in workspace holds, so that what fits it does not hang on how
-    // the plan weighs splits
-    tp_gemm_desc fit = *d;
-    if (need > (size_t)TP_GEMM_STATIC_WS_BYTES && !((d->reserved >> 8) & 0xff)) {
-        const size_t n = (size_t)TP_GEMM_STATIC_WS_BYTES / ((size_t)d->M * d->N * sizeof(float));
-        fit.reserved = (p.cfg + 1) | (int)(n < 1 ? 1 : n) << 8;
-        d = &fit;
-        p = tp::plan_gemm(d);
-        need = p.nsplit > 1 ? (size_t)p.nsplit * d->M * d->N * sizeof(float) : 0;
-    }
+    const tp::GemmPlan p = tp::plan_static_ws(d);
+    const size_t need = tp::plan_bytes(d, p);
     if (need > (size_t)TP_GEMM_STATIC_WS_BYTES) {
         tp::set_error("tp_gemm_static_ws: this product needs %zu bytes of k-split workspace, the built-in one holds %zu "
                       "(M=%d N=%d K=%d, %d splits); use tp_gemm with a caller workspace",
@@ -778,33 +812,19 @@ extern "C" int tp_gemm_static_ws(const tp_gemm_desc* d, void* stream) {
         ws = tp::scratch_on_current_device();
         if (!ws) return TP_ERR_LAUNCH;
     }
-    return tp_gemm(d, ws, need, stream);
+    return tp::run_gemm(d, p, ws, stream);
 }
 
 extern "C" int tp_gemm(const tp_gemm_desc* d, void* workspace, size_t workspace_bytes, void* stream) {
     int rc = tp::validate_gemm(d);
     if (rc != TP_OK) return rc;
-    tp::GemmPlan p = tp::plan_gemm(d);
-    size_t need = p.nsplit > 1 ? (size_t)p.nsplit * d->M * d->N * sizeof(float) : 0;
+    const tp::GemmPlan p = tp::plan_gemm(d);
+    const size_t need = tp::plan_bytes(d, p);
     if (need > 0 && (!workspace || workspace_bytes < need)) {
         tp::set_error("tp_gemm: workspace of %zu bytes needed, %zu given", need, workspace_bytes);
         return TP_ERR_WORKSPACE;
     }
-    tp::GemmArgs a = tp::fill_args(d, p, workspace);
-    hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    bool launched;
-    switch (d->dtype) {
-    case TP_F32: launched = tp::launch_gemm<float>(d, p, a, s); break;
-    case TP_F16: launched = tp::launch_gemm<tp::f16>(d, p, a, s); break;
-    default: launched = tp::launch_gemm<tp::bf16>(d, p, a, s); break;
-    }
-    if (!launched) {
-        tp::set_error("tp_gemm: no kernel for tile configuration %d with op %d, dtype %d", p.cfg, d->op, d->dtype);
-        return TP_ERR_UNSUPPORTED;
-    }
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) { tp::set_error("tp_gemm: launch failed: %s", hipGetErrorString(e)); return TP_ERR_LAUNCH; }
-    return TP_OK;
+    return tp::run_gemm(d, p, workspace, stream);
 }
 
 extern "C" int tp_gemm_group_cfg(const tp_gemm_desc* descs, int n) {
