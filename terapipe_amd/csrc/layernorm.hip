@@ -23,6 +23,7 @@ __device__ __forceinline__ void block_sum(float (&v)[NREDUCE], float* scratch /*
     }
 }
 
+// (fp32 chunks change type by value: taken apart through a pointer some are put into scratch memory)
 template <typename T> __device__ __forceinline__ void load_chunk(const T* p, float* out) {
     constexpr int CH = 16 / sizeof(T);
     uint4 raw = *reinterpret_cast<const uint4*>(p);
@@ -31,7 +32,7 @@ template <typename T> __device__ __forceinline__ void load_chunk(const T* p, flo
 #pragma unroll
         for (int e = 0; e < CH; ++e) out[e] = Elem<T>::to_float(h[e]);
     } else {
-        const float* f = reinterpret_cast<const float*>(&raw);
+        const float4v f = __builtin_bit_cast(float4v, raw);
 #pragma unroll
         for (int e = 0; e < CH; ++e) out[e] = f[e];
     }
@@ -45,9 +46,10 @@ template <typename T> __device__ __forceinline__ void store_chunk(T* p, const fl
 #pragma unroll
         for (int e = 0; e < CH; ++e) h[e] = Elem<T>::from_float(v[e]);
     } else {
-        float* f = reinterpret_cast<float*>(&raw);
+        float4v f;
 #pragma unroll
         for (int e = 0; e < CH; ++e) f[e] = v[e];
+        raw = __builtin_bit_cast(uint4, f);
     }
     *reinterpret_cast<uint4*>(p) = raw;
 }
@@ -228,7 +230,7 @@ __global__ __launch_bounds__(1024) void ln_bwd_kernel(LnPartialSrc ps, const T* 
 // dx alone (what the layer calls and the runner ask for: the parameter gradients are reductions of their own): one workgroup
 // per row, everything the row needs asked for before the first reduction.  Without the sums that ln_bwd_kernel keeps beside
 // (it spills from two chunks a thread on) a row is bound by its bytes: 2048 x 5120 35 -> 19.6 us (4.3 TB/s), 4096 x 6144 74 -> 39
-// (5.2), 2048 x 2048 11.6 -> 8.5, 256 x 1600 5.2 -> 4.1.
+// (5.2), 2048 x 2048 11.6 -> 8.5, 256 x 1600 5.2 -> 4.1; fp32 2512 x 1528 15.5 -> 11.8, 6602 x 1624 35 -> 27.7.
 template <typename T, int MAXC>
 __global__ __launch_bounds__(1024) void ln_bwd_rows_kernel(LnPartialSrc ps, const T* __restrict__ dy, const T* __restrict__ x,
                                                       const float* __restrict__ mean, const float* __restrict__ rstd,
@@ -271,7 +273,13 @@ __global__ __launch_bounds__(1024) void ln_bwd_rows_kernel(LnPartialSrc ps, cons
             for (int e = 0; e < CH; ++e) o[e] = rs * (g[i][e] - m1 - xh[i][e] * m2);
             if (dres) {
                 float r[CH];
-                load_chunk<T>(reinterpret_cast<const T*>(&res[i]), r);
+                if constexpr (sizeof(T) == 2) {
+                    load_chunk<T>(reinterpret_cast<const T*>(&res[i]), r);
+                } else {
+                    const float4v f = __builtin_bit_cast(float4v, res[i]);
+#pragma unroll
+                    for (int e = 0; e < CH; ++e) r[e] = f[e];
+                }
 #pragma unroll
                 for (int e = 0; e < CH; ++e) o[e] += r[e];
             }
