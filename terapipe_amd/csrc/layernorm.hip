@@ -474,19 +474,22 @@ __global__ __launch_bounds__(512) void vec_param_sums_kernel(VecSumArgs args) {
 // Threads of a row's workgroup and chunks of 16 bytes each holds.  Few rows: a thread per chunk, the row's latency is what
 // counts.  Many: two or three chunks a thread, so that a CU holds more rows under way: 2048 x 5120 forward 17.9 -> 12.4 us (a
 // workgroup of 1024 threads, 384 of them without a chunk, before), 4096 x 6144 31 -> 21; a few hundred rows lose 3 to 10 %
-// by it.
+// by it.  A thread per chunk means a power of two of them: 5 to 7 or 13 to 15 waves take 4 to 7 % longer than 8 or 16 (50 x 2952
+// 4.42 against 4.19 us).  Rows of more than 1536 chunks keep workgroups of 1024: two or three chunks a thread are level at best
+// there (fp32 forward 0.96 to 1.02).
 static int ln_geometry(int M, int E, int dtype, bool accumulates, int* threads, int* maxc) {
     const int ch = dtype == TP_F32 ? 4 : 8;
     if (E <= 0 || E % ch) { set_error("layernorm: E=%d must be a positive multiple of %d", E, ch); return TP_ERR_UNSUPPORTED; }
     const int nch = E / ch;
     if (nch > 4096) { set_error("layernorm: E=%d too large (max %d)", E, 1024 * 4 * ch); return TP_ERR_UNSUPPORTED; }
     int c = 1;
-    if (!accumulates) {
+    if (!accumulates && nch <= 1536) {
         if (nch >= 512) c = M >= 1024 ? 3 : M >= 512 ? 2 : 1;
         else if (nch >= 128) c = M >= 2048 ? 2 : 1;
     }
-    int nt = ((nch + c - 1) / c + 63) / 64 * 64;
-    if (nt > 1024) nt = 1024;
+    int nt = 64;
+    if (c == 1) while (nt < nch && nt < 1024) nt *= 2;
+    else nt = ((nch + c - 1) / c + 63) / 64 * 64;
     const int mc = (nch + nt - 1) / nt;
     *threads = nt;
     *maxc = mc <= 1 ? 1 : (mc <= 2 ? 2 : 4);

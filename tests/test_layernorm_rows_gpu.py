@@ -11,7 +11,8 @@ DEV = "cuda"
 @pytest.mark.gpu
 @pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16, torch.float32], ids=str)
 @pytest.mark.parametrize("M,chunks", [(1, 1), (3, 65), (2047, 127), (2048, 128), (2049, 203), (2048, 511), (511, 512), (512, 513),
-                                      (1023, 640), (1024, 769), (1025, 512), (5, 4096), (1024, 4095)], ids=str)
+                                      (1023, 640), (1024, 769), (1025, 512), (5, 4096), (1024, 4095),
+                                      (7, 257), (300, 448), (40, 769), (2048, 1536), (2048, 1537)], ids=str)
 def test_rows(M, chunks, dtype):
     from terapipe_amd import ops
     E = chunks * (4 if dtype == torch.float32 else 8)
