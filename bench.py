@@ -248,20 +248,13 @@ def fill_path(device):
 
 
 def in_step_picks():
-    """{(op, M, N, K)} of the measured plan table's entries that were chosen by timing whole steps on the slice
-    streams rather than the launch alone (their comments in gemm_tuned.inc say so): alone on the chip, as the
-    per-GEMM roofline times them, they are not the fastest plan of their shape."""
-    path = os.path.join(ROOT, "terapipe_amd", "csrc", "gemm_tuned.inc")
+    """{(op, M, N, K)} of the products whose plan beside other streams' launches is one of its own, chosen by timing
+    whole steps on the slice streams (gemm_tuned_beside.inc): alone on the chip, as the per-GEMM roofline times them,
+    it is not the fastest plan of their shape."""
     ops_ = {"NT": 0, "NN": 1, "TN": 2}
-    out = set()
-    try:
-        for line in open(path):
-            m = re.match(r"\{TP_GEMM_(\w+), (\d+), (\d+), (\d+), (\d+), (\d+)\},\s*//(.*)", line)
-            if m and ("in-step" in m.group(7) or "inside the step" in m.group(7)):
-                out.add((ops_[m.group(1)], int(m.group(2)), int(m.group(3)), int(m.group(4))))
-    except OSError:
-        pass
-    return out
+    with open(os.path.join(ROOT, "terapipe_amd", "csrc", "gemm_tuned_beside.inc")) as f:
+        rows = re.findall(r"^\{TP_GEMM_(\w+), (\d+), (\d+), (\d+),", f.read(), re.M)
+    return {(ops_[op],) + tuple(int(v) for v in extents) for op, *extents in rows}
 
 
 def cpu_baseline(w, sample_layers=None):
@@ -470,9 +463,9 @@ def measure_workload(name, args, device, detail):
         "achieved_over_attainable": achieved / attainable,
         "attainable_note": "per launch min(MFMA peak, (A + B + C bytes) / 8 TB/s), summed over the step's launches",
         "method": "graph replay of the step's GEMM calls between two HIP events, one after the other on one stream: each "
-                  "launch has the chip to itself, with the tile and k splits the step uses (several of those were "
-                  "chosen by timing whole steps on the slice streams and are not the fastest alone; shared_chip times "
-                  "the same launches as the step overlaps them)",
+                  "launch has the chip to itself, with the tile and k splits the step uses (on several slice streams some of "
+                  "those were chosen by timing such steps and are not the fastest alone; shared_chip times the same "
+                  "launches as the step overlaps them)",
     }
     if detail:
         groups = {}
@@ -480,7 +473,7 @@ def measure_workload(name, args, device, detail):
             groups.setdefault(c[1], []).append(c[2])
         groups = dict(sorted(groups.items(), key=lambda kv: str(kv[0])))
         per = []
-        picks = in_step_picks()
+        picks = in_step_picks() if args.slice_streams > 1 and not merge else set()
         for meta, fns in groups.items():
             ms = _graph_ms(fns)
             f, b = gemm_shape_work(meta, es)
@@ -506,8 +499,9 @@ def measure_workload(name, args, device, detail):
         per.sort(key=lambda r: -r["avg_us"] * r["calls"])
         roof["per_gemm"] = per
         roof["per_gemm_note"] = ("avg_us is the launch alone on the chip with the plan the step uses; in_step_pick marks "
-                                 "the shapes whose plan was chosen by timing whole steps on the slice streams (fewer k "
-                                 "splits than the fastest plan alone), so vendor_us may be below avg_us there")
+                                 "the shapes that a step on several slice streams runs with a plan chosen by timing such "
+                                 "steps (it takes less of the chip than the fastest plan alone), so vendor_us may be "
+                                 "below avg_us there")
     if args.slice_streams > 1 and not merge:
         # the same GEMM calls as the step issues them: spread over the slice streams, so that a launch
         # which fills part of the chip runs beside its neighbours'.  Launched from the host (closures

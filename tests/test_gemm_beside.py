@@ -31,3 +31,8 @@ def test_plans_beside_other_streams():
         assert _plan(*key, 1 << 24) == beside.get(key, want)
     for key in ((L.TP_GEMM_NT, 300, 1000, 3000), (L.TP_GEMM_NN, 2048, 4096, 4096), (L.TP_GEMM_NT, 16, 2048, 2048)):
         assert _plan(*key, 1 << 24) == _plan(*key, 0)
+
+
+def test_the_benchmark_names_the_products_of_the_table():
+    import bench
+    assert bench.in_step_picks() == set(_entries("gemm_tuned_beside.inc"))
