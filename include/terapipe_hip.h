@@ -243,6 +243,9 @@ size_t tp_attn_fwd_workspace_bytes(const tp_attn_desc* d);
 int tp_attn_prefix_fwd(const tp_attn_desc* d, void* workspace, size_t workspace_bytes, void* stream);
 size_t tp_attn_bwd_workspace_bytes(const tp_attn_desc* d);
 int tp_attn_prefix_bwd(const tp_attn_desc* d, void* workspace, size_t workspace_bytes, void* stream);
+/* Whether that call takes dQ by workgroups of 128 queries, and dK / dV by workgroups of 128 keys, that share the tiles they
+ * stream.  Host code only; for tuning, tests and logs. */
+int tp_attn_bwd_forms(const tp_attn_desc* d, int* shared_queries, int* shared_keys);
 
 /* dK / dV of one slice's keys against EVERY query that can see them, in one pass: the sum that
  * _AssignCache.backward (transformer_models.py:186-190) builds up slice by slice in the gradient caches

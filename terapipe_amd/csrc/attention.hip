@@ -1851,15 +1851,19 @@ static bool shares_queries(const tp_attn_desc* d) {
     return shares_bwd(d->batch, d->heads, d->head_dim, d->T);
 }
 // dK / dV with gradient caches: the other form gives 32 keys to ONE wave, which walks over all queries alone.  Above head
-// dimension 64 the shared form is faster throughout (2 to 128 pairs, 1 to 1024 queries, up to 2048 keys): 1.11 to 3.1 times, 40 pairs
-// of 128, 256 queries after 768 47.7 -> 29 us.  At 64 in one round of an XCD's 32 CUs from 32 queries on (1.17 to 1.7; fewer
+// dimension 64 the shared form is faster (2 to 1152 pairs, 1 to 1024 queries, up to 2048 keys): 0.96 to 3.1 times, 40 pairs
+// of 128, 256 queries after 768 47.7 -> 29 us; but not where its one workgroup per CU makes a second, part-filled round of
+// calls so short that two of the other form's fit a CU: 257 to 511 pairs with up to 32 positions (0.84 to 1.02; 384 pairs of 128, one
+// position 22.5 against 18.6 us with dQ), and up to 384 with up to 64 (16 queries and fewer 0.89 to 1.06, more 0.96 to 1.09).
+// At 64 in one round of an XCD's 32 CUs from 32 queries on (1.17 to 1.7; fewer
 // queries 0.3 to 1.18), and beyond it for 512 queries and more in up to three (0.98 to 1.6; fewer queries 0.8 to 1.1).
 static bool shares_keys(const tp_attn_desc* d) {
     if (d->dtype == TP_F32 || !tiled16(d->head_dim)) return false;
     if (d->reserved2 & (32 | 64)) return d->reserved2 & 32;
-    const long pairs = (long)d->batch * d->heads, blocks = (d->cache_len + d->T + 127) / 128;
+    const long pairs = (long)d->batch * d->heads, S = d->cache_len + d->T, blocks = (S + 127) / 128;
     if (pairs * d->head_dim > (1L << 24)) return false;
-    if (d->head_dim > 64) return true;
+    if (d->head_dim > 64)
+        return pairs <= kNumCU || !((S <= 32 && pairs < 2 * kNumCU) || (S <= 64 && d->T <= 16 && 2 * pairs <= 3 * kNumCU));
     return d->T >= 32 && ((pairs + 7) / 8 * blocks <= kNumCU / 8 || (d->T >= 512 && pairs * blocks <= 3 * kNumCU));
 }
 
@@ -2065,6 +2069,15 @@ extern "C" int tp_attn_prefix_fwd(const tp_attn_desc* d, void* workspace, size_t
 }
 
 extern "C" size_t tp_attn_bwd_workspace_bytes(const tp_attn_desc* d) { (void)d; return 0; }
+
+extern "C" int tp_attn_bwd_forms(const tp_attn_desc* d, int* shared_queries, int* shared_keys) {
+    using namespace tp;
+    const int rc = validate_attn(d, true);
+    if (rc != TP_OK) return rc;
+    if (shared_queries) *shared_queries = shares_queries(d);
+    if (shared_keys) *shared_keys = !d->dq_only && d->grad_cache_dtype == d->dtype && shares_keys(d);
+    return TP_OK;
+}
 
 extern "C" int tp_attn_prefix_bwd(const tp_attn_desc* d, void* workspace, size_t workspace_bytes, void* stream) {
     using namespace tp;

@@ -1,5 +1,7 @@
 """The attention kernels for whole sequences and long slices (workgroups of 128 queries) forced at their edges against fp32:
 rows, blocks and key tiles that end inside a workgroup's, prefixes of every alignment, references that move on most tiles."""
+import ctypes
+
 import pytest
 import torch
 
@@ -45,7 +47,8 @@ def test_forward(B, H, T, P, drift, D, dtype):
 @pytest.mark.parametrize("B,H,D,T,P,acc,incoming,zero", [
     (2, 128, 64, 129, 0, 0, 0, 0), (1, 256, 64, 130, 67, 1, 1, 1), (4, 48, 80, 128, 1, 0, 1, 0), (1, 110, 96, 200, 131, 1, 0, 1),
     (2, 56, 128, 193, 63, 1, 1, 0), (1, 96, 128, 255, 0, 0, 0, 0),
-    (1, 3, 96, 1, 70, 1, 1, 1), (2, 2, 128, 33, 95, 0, 1, 0), (1, 2, 64, 40, 0, 0, 0, 0)], ids=str)
+    (1, 3, 96, 1, 70, 1, 1, 1), (2, 2, 128, 33, 95, 0, 1, 0), (1, 2, 64, 40, 0, 0, 0, 0),
+    (1, 257, 80, 1, 0, 0, 0, 0), (1, 300, 96, 7, 25, 1, 1, 1), (1, 384, 128, 16, 48, 1, 0, 1)], ids=str)
 def test_backward(B, H, D, T, P, acc, incoming, zero, dtype):
     """Both backward forms: with gradient caches, and dQ with the one-pass dK / dV (the last rows: the first of them alone, for which
     few workgroups are enough)."""
@@ -89,3 +92,19 @@ def test_backward(B, H, D, T, P, acc, incoming, zero, dtype):
     assert_close(part[:, :, 1], rows(dk[:, :T]), dtype, "suffix dk")
     assert_close(part[:, :, 2], rows(dv[:, :T]), dtype, "suffix dv")
     assert part[:, :, 0].isnan().all()
+
+
+# (B * H, head dim, T, P) -> whether the gradient-cache dK / dV takes the shared form
+@pytest.mark.parametrize("pairs,D,T,P,want", [
+    (256, 128, 1, 0, 1), (257, 80, 1, 0, 0), (511, 96, 32, 0, 0), (512, 128, 1, 31, 1), (257, 128, 33, 0, 1), (384, 80, 16, 48, 0),
+    (385, 80, 16, 48, 1), (384, 96, 17, 47, 1), (384, 128, 16, 49, 1), (768, 128, 1, 0, 1), (40, 128, 256, 768, 1), (300, 64, 8, 8, 0)], ids=str)
+def test_short_calls_of_a_second_round_keep_the_form_with_a_wave_per_key_block(pairs, D, T, P, want):
+    from terapipe_amd import _lib as L
+    d = L.AttnDesc()
+    d.dtype = d.grad_cache_dtype = L.TP_F16
+    d.batch, d.heads, d.head_dim, d.T, d.cache_len, d.cache_rows = 1, pairs, D, T, P, T + P
+    for name in ("q", "k_cache", "v_cache", "o", "lse", "d_o", "delta", "dqkv", "dk_cache", "dv_cache"):
+        setattr(d, name, 4096)
+    keys = ctypes.c_int(-1)
+    assert L.load().tp_attn_bwd_forms(ctypes.byref(d), None, ctypes.byref(keys)) == 0
+    assert keys.value == want
