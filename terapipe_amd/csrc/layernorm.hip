@@ -74,13 +74,24 @@ __device__ __forceinline__ void load_input_chunk(const LnPartialSrc& ps, const T
     }
 #pragma unroll
     for (int e = 0; e < CH; ++e) out[e] = 0.f;
-    for (int z = 0; z < ps.nsplit; ++z) {
-        const float* pp = ps.partial + (long)z * ps.zstride + off;
+    // four splits' loads under way at a time, added in the order of the splits
+    for (int z = 0; z < ps.nsplit; z += 4) {
+        float4 v[4][CH / 4];
 #pragma unroll
-        for (int q = 0; q < CH / 4; ++q) {
-            const float4 v = *reinterpret_cast<const float4*>(pp + 4 * q);
-            out[4 * q] += v.x; out[4 * q + 1] += v.y; out[4 * q + 2] += v.z; out[4 * q + 3] += v.w;
-        }
+        for (int u = 0; u < 4; ++u)
+            if (z + u < ps.nsplit) {
+#pragma unroll
+                for (int q = 0; q < CH / 4; ++q)
+                    v[u][q] = *reinterpret_cast<const float4*>(ps.partial + (long)(z + u) * ps.zstride + off + 4 * q);
+            }
+#pragma unroll
+        for (int u = 0; u < 4; ++u)
+            if (z + u < ps.nsplit) {
+#pragma unroll
+                for (int q = 0; q < CH / 4; ++q) {
+                    out[4 * q] += v[u][q].x; out[4 * q + 1] += v[u][q].y; out[4 * q + 2] += v[u][q].z; out[4 * q + 3] += v[u][q].w;
+                }
+            }
     }
     if (ps.bias) {
         float b[CH];
