@@ -191,16 +191,16 @@ static void finish_plan(const tp_gemm_desc* d, GemmPlan& p, int bk, int nsplit) 
 // The time (us) of `tiles` workgroups of a tile configuration over k: rounds of one workgroup per CU, each a fixed part
 // (prologue, epilogue) and a part per k; a partly filled round runs somewhat faster per k (less traffic, higher clocks).
 // Where the operands outgrow the memory-side cache (`spill`) a tile that reads them more often falls behind.  NT and NN: fitted to
-// 147 products (512 to 8192 rows, hidden 512 to 12800, both alone on the chip), rms 4 to 8 %; the plan's choice takes 1.006 times the
-// fastest of 64 x 64 to 256 x 256 tiles and up to four splits in the mean.  TN: fitted to 66 (hidden 1024 to 6144; k of 1024, 2048
-// and 4096).
+// 1300 products (520 to 8192 rows, hidden 512 to 12288, alone on the chip, weights from memory), rms 5 to 9 %, then moved to
+// where the choice is best: 1.006 times the fastest of 64 x 64 to 256 x 256 tiles and their splits in the mean.  TN: fitted to 66
+// (hidden 1024 to 6144; k of 1024, 2048 and 4096).
 struct TileCost { int cfg, bm, bn; float fixed, per_k, per_k_spill, partial; };
 static const TileCost kTileCost[] = {
-    {16, 128, 128, 3.3f, 0.00834f, 0.00880f, 0.64f},
-    {14, 192, 128, 5.3f, 0.00967f, 0.01067f, 0.68f},
-    {15, 256, 128, 6.6f, 0.01278f, 0.01286f, 0.69f},
-    {kWideCfg, 256, 256, 7.9f, 0.02432f, 0.02432f, 0.65f},
-    {kWideCfg, 256, 192, 5.4f, 0.02002f, 0.02089f, 0.70f},
+    {16, 128, 128, 3.86f, 0.00845f, 0.00950f, 0.927f},
+    {14, 192, 128, 5.74f, 0.01031f, 0.01179f, 0.982f},
+    {15, 256, 128, 6.60f, 0.01257f, 0.01245f, 0.920f},
+    {kWideCfg, 256, 256, 6.70f, 0.02276f, 0.02220f, 0.832f},
+    {kWideCfg, 256, 192, 5.62f, 0.01992f, 0.02102f, 0.970f},
 };
 static const TileCost kTileCostTN[] = {
     {16, 128, 128, 4.8f, 0.0068f, 0.0084f, 0.72f},
@@ -216,19 +216,28 @@ static bool tile_serves(const TileCost& c, int K) { return c.cfg != kWideCfg || 
 
 // Products on weights of up to 4096 x 4096, NT and NN.  The time (us) of `tiles` workgroups, one round per 256: a fixed part
 // and a part per k, which grows from `lo` for a few workgroups to `hi` for a full round (they share the caches' and the
-// memory's bandwidth).  Fitted to a sweep of 640 products (hidden 256 to 4096, 32 to 1024 rows, up to 8 splits; each weight
-// used once in a pass over a model of 24 layers, so from hidden 1024 on they come from memory): rms error 10 to 15 %.  The
-// rules it replaces named 64 x 64 tiles without a split from 96 of them on, the 128 x 128 tile beyond two per CU.
+// memory's bandwidth).  64 x 64 tiles fit a CU twice: theirs is a round per 512, `lo` to `mid` while each has a CU to itself, `two`
+// to `hi` when a second one comes beside.  Fitted to 1300 products (hidden 512 to 2816, 33 to 512 rows, up to 4 splits, no weight used
+// twice within 400 MB): rms error 6 to 11 %, then moved to where the choice is best: 1.004 times the fastest of these tiles in the
+// mean, 1.11 at most.  (With a round per 256 of the 64 x 64 tiles the estimate gave up to 512 of them to the 128 x 128 tile: 640 x 2304 x
+// 768 8.2 us, 11.0 with it; 1500 x 1024 x 1024 9.7 and 11.8.)
 struct SliceCost { float fixed, round, lo, hi; };
-static const SliceCost kSlice64[2] = {{3.69f, 0.85f, 0.00380f, 0.00457f}, {3.41f, 0.42f, 0.00437f, 0.00539f}};    // cfg 8: NT, NN
-static const SliceCost kSlice128[2] = {{4.52f, 4.43f, 0.00721f, 0.01134f}, {4.29f, 4.27f, 0.00701f, 0.01128f}};   // cfg 16
-static const SliceCost kDeep32[2] = {{4.27f, 2.61f, 0.00266f, 0.00280f}, {4.46f, 2.41f, 0.00360f, 0.00370f}};
-static const SliceCost kDeep64[2] = {{4.55f, 2.84f, 0.00360f, 0.00448f}, {4.44f, 2.40f, 0.00428f, 0.00524f}};
-static const SliceCost kDeep128[2] = {{5.03f, 3.65f, 0.00475f, 0.00822f}, {4.85f, 2.89f, 0.00524f, 0.00917f}};
+struct PairCost { float fixed, round, lo, mid, two, hi; };
+static const PairCost kSlice64[2] = {{3.14f, 1.12f, 0.00402f, 0.00448f, 0.00630f, 0.00811f},     // cfg 8: NT, NN
+                                     {3.12f, 0.66f, 0.00438f, 0.00450f, 0.00682f, 0.00936f}};
+static const SliceCost kSlice128[2] = {{3.83f, 2.19f, 0.00909f, 0.00922f}, {3.96f, 2.10f, 0.00742f, 0.00802f}};   // cfg 16
+static const SliceCost kDeep32[2] = {{4.18f, 2.47f, 0.00237f, 0.00264f}, {4.06f, 1.87f, 0.00359f, 0.00399f}};
+static const SliceCost kDeep64[2] = {{4.29f, 2.40f, 0.00341f, 0.00383f}, {4.05f, 1.93f, 0.00422f, 0.00422f}};
+static const SliceCost kDeep128[2] = {{4.76f, 2.31f, 0.00608f, 0.00611f}, {4.50f, 1.88f, 0.00690f, 0.00690f}};
 static float slice_time(const SliceCost& c, long tiles, float k) {
     const long full = (tiles - 1) / kNumCU;
     const float part = (float)(tiles - full * kNumCU) / kNumCU;
     return c.fixed + full * (c.round + k * c.hi) + k * (c.lo + (c.hi - c.lo) * part);
+}
+static float slice_time(const PairCost& c, long tiles, float k) {
+    const long full = (tiles - 1) / (2 * kNumCU);
+    const float part = (float)(tiles - full * 2 * kNumCU) / kNumCU;
+    return c.fixed + full * (c.round + k * c.hi) + k * (part <= 1.f ? c.lo + (c.mid - c.lo) * part : c.two + (c.hi - c.two) * (part - 1.f));
 }
 static bool small_weight(const tp_gemm_desc* d) { return (long)d->N * d->K <= (16L << 20); }
 // (the deep rings have no column sums, and no tiles for weights that stream from HBM beside other launches)
@@ -248,8 +257,19 @@ static float deep_time(const tp_gemm_desc* d, int ns, int* columns) {
     take(128, kDeep128[op]);
     return best;
 }
-// A split's partial sums and the launch that adds them (or the LayerNorm's reads of them).
-static float reduce_time(const tp_gemm_desc* d, int ns) { return ns > 1 ? 3.01f + 0.152e-6f * ns * 4.f * d->M * d->N : 0.f; }
+// Products whose sums of k splits the layer calls and the runner leave to the LayerNorm behind them: the two with a residual,
+// and the data gradients of the widening linears.
+static bool feeds_layernorm(const tp_gemm_desc* d) {
+    return d->epilogue == TP_EPI_BIAS_RESIDUAL || (d->op == TP_GEMM_NN && d->epilogue == TP_EPI_STORE && d->K >= 3L * d->N);
+}
+// A split's partial sums and the launch that adds them, or the LayerNorm's reads of them (264 products with the LayerNorm behind,
+// 96 to 3072 rows, hidden 768 to 2560: the choice takes 1.011 times the fastest in the mean; priced like the launch the splits went
+// unused, 768 x 1024 x 4096 NN with the LayerNorm 22.2 us in four splits, 27.6 in one piece).
+static float reduce_time(const tp_gemm_desc* d, int ns) {
+    if (ns == 1) return 0.f;
+    const float sums = 4.f * ns * d->M * d->N;
+    return feeds_layernorm(d) ? 1.5f + 0.15e-6f * sums : 3.19f + 0.21e-6f * sums;
+}
 static void plan_slice(const tp_gemm_desc* d, int& cfg, int& ns) {
     const int op = d->op == TP_GEMM_NN;
     const long t64 = (long)((d->M + 63) / 64) * ((d->N + 63) / 64), t128 = (long)((d->M + 127) / 128) * ((d->N + 127) / 128);
@@ -282,7 +302,8 @@ static int wide_columns(const tp_gemm_desc* d, int ns) {
 }
 
 // Products of more than 512 rows and parameter gradients: the tile and the k split with the smallest estimate.  A split
-// costs its fp32 partial sums (written and read once at 5.5 TB/s) and the launch that adds them.  The rules this replaces
+// costs its fp32 partial sums (written and read once at 5.5 TB/s) and the launch that adds them, and has to be 4 % ahead (NT, NN:
+// part of the same fit); less where a LayerNorm takes them.  The rules this replaces
 // named 256 x 256 tiles from 192 of them on and split or shrank them otherwise, without regard for the last round: the
 // estimate's choice takes 0.61 to 1.0 of their time (1024 x 5120 x 20480: 284 -> 188 us; 4096 x 1600 x 6400: 117 -> 80).
 static void plan_large(const tp_gemm_desc* d, int& cfg, int& ns) {
@@ -308,14 +329,16 @@ static void plan_large(const tp_gemm_desc* d, int& cfg, int& ns) {
         const float t = deep_time(d, 1, &columns);
         if (t < best) { best = t; cfg = 12; }
     }
+    const bool layernorm = feeds_layernorm(d);
     auto consider = [&](const TileCost& c) {
         if (!tile_serves(c, d->K)) return;
         const long tiles = (long)((d->M + c.bm - 1) / c.bm) * ((d->N + c.bn - 1) / c.bn);
         for (int n = 1; n <= 8; ++n) {
             if (n > 1 && (d->N % 8 || d->K / n < 512 || tiles * n > 2 * kNumCU)) break;
             float t = tile_time(c, tiles * n, K / n, spill);
-            if (n > 1) t += 4.f + (float)((double)n * d->M * d->N * 8 / 5.5e6);
-            if (t < best) { best = t; cfg = c.cfg; ns = n; }
+            if (n > 1 && layernorm) t += 2.5f + 1.2e-6f * n * d->M * d->N;
+            else if (n > 1) t = (t + 4.f + (float)((double)n * d->M * d->N * 8 / 5.5e6)) * (d->op == TP_GEMM_TN ? 1.f : 1.044f);
+            if (t < best * (n > 1 && layernorm ? 0.98f : 1.f)) { best = t; cfg = c.cfg; ns = n; }       // (a tie goes to fewer splits)
         }
     };
     if (d->op == TP_GEMM_TN) for (const TileCost& c : kTileCostTN) consider(c);
