@@ -138,7 +138,8 @@ static constexpr int kSkinnyRows = 32;
 
 // Measured plans: for NT / NN the weight extents (N, K) match exactly and M (tokens of the slice) picks the
 // nearest measured M at or above it (at least half of it, so that a much shorter slice falls through to the
-// heuristics); TN (parameter gradients) matches all three extents.
+// heuristics); on weights of up to 4096 x 4096, which have an estimate of their own, M itself (128 rows on 8192 x 2048 with the entry
+// of 256, 128 x 128 tiles, 22.8 us; 64 x 64 as the estimate has it 13.9).  TN (parameter gradients) matches all three extents.
 struct TunedPlan { int op, M, N, K, cfg, nsplit; };
 static const TunedPlan kTuned[] = {
 #include "gemm_tuned.inc"
@@ -153,6 +154,7 @@ static const TunedPlan kTunedBeside[] = {
 };
 constexpr int kBeside = 1 << 24, kForced = 0xffffff;        // of tp_gemm_desc.reserved
 
+static bool small_weight(const tp_gemm_desc* d) { return (long)d->N * d->K <= (16L << 20); }
 static const TunedPlan* find_tuned(const tp_gemm_desc* d) {
     const TunedPlan* best = nullptr;
     for (const TunedPlan* t = kTuned; t->op >= 0; ++t) {
@@ -161,7 +163,7 @@ static const TunedPlan* find_tuned(const tp_gemm_desc* d) {
             if (t->M == d->M) return t;
             continue;
         }
-        if (t->M >= d->M && t->M <= 2 * d->M && (!best || t->M < best->M)) best = t;
+        if (t->M >= d->M && t->M <= (small_weight(d) ? 1 : 2) * d->M && (!best || t->M < best->M)) best = t;
     }
     if (best && (d->reserved & kBeside))
         for (const TunedPlan* t = kTunedBeside; t->op >= 0; ++t)
@@ -239,7 +241,6 @@ static float slice_time(const PairCost& c, long tiles, float k) {
     const float part = (float)(tiles - full * 2 * kNumCU) / kNumCU;
     return c.fixed + full * (c.round + k * c.hi) + k * (part <= 1.f ? c.lo + (c.mid - c.lo) * part : c.two + (c.hi - c.two) * (part - 1.f));
 }
-static bool small_weight(const tp_gemm_desc* d) { return (long)d->N * d->K <= (16L << 20); }
 // (the deep rings have no column sums, and no tiles for weights that stream from HBM beside other launches)
 static bool deep_serves(const tp_gemm_desc* d) { return d->op != TP_GEMM_TN && d->dtype != TP_F32 && small_weight(d) && !d->colsum_acc; }
 // The deep ring's time at `ns` splits and its tile's columns.
@@ -464,7 +465,17 @@ static GemmPlan plan_gemm(const tp_gemm_desc* d) {
             if (ns > 1 && ns > cap) ns = cap < 1 ? 1 : cap;
         }
     }
-    if (const TunedPlan* t = find_tuned(d)) { cfg = t->cfg; ns = t->nsplit; }
+    if (const TunedPlan* t = find_tuned(d)) {
+        cfg = t->cfg;
+        ns = t->nsplit;
+        // An entry that fewer rows take with fewer row tiles keeps its number of workgroups (NN 80 to 128 x 5120 x 5120 with the 160-row
+        // entry's three splits 25.1 to 27.2 us, with six 20.0 to 22.6), unless other streams' launches are to have the rest of the chip.
+        TileCfg tt;
+        if (ns > 1 && !(d->reserved & kBeside) && tile_cfg(cfg, tt)) {
+            const int more = ns * ((t->M + tt.bm - 1) / tt.bm) / ((d->M + tt.bm - 1) / tt.bm);
+            if (d->K / more >= 768) ns = more;
+        }
+    }
     if (ns < 1) ns = 1;
     if (ns > 16) ns = 16;
     TileCfg tc;

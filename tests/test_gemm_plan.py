@@ -100,6 +100,22 @@ def test_rule_examples():
     assert plan("NT", 128, 4096, 4096, _lib.TP_F32)[0] == 0
 
 
+def test_entries_between_their_row_counts():
+    """Small weights take an entry at its own row count only; on larger ones fewer row tiles mean more k splits."""
+    assert plan("NT", 256, 6144, 2048) == (8, 1) and plan("NT", 256, 8192, 2048) == (16, 1)
+    for M in (128, 160, 192):
+        assert plan("NT", M, 6144, 2048)[0] in (8, 12) and plan("NT", M, 8192, 2048)[0] in (8, 12), M      # the estimate
+    assert plan("NN", 160, 5120, 5120) == (16, 3)
+    for M in (80, 112, 128):
+        assert plan("NN", M, 5120, 5120) == (16, 6), M
+    assert plan("NN", 129, 5120, 5120) == (16, 3)           # the same row tiles as 160
+    d = _lib.GemmDesc()
+    d.op, d.dtype, d.epilogue, d.M, d.N, d.K, d.reserved = OPS["NN"], _lib.TP_F16, _lib.TP_EPI_STORE, 128, 5120, 5120, 1 << 24
+    d.A = d.B = d.C = 4096
+    d.lda = d.ldb = d.ldc = 5120
+    assert _lib.load().tp_gemm_splits(ctypes.byref(d)) == 4         # beside other streams: its own entry, as it is
+
+
 def test_the_estimate_keeps_narrow_tiles_where_two_fit_a_cu():
     """64 x 64 tiles up to two per CU, not a third as many of 128 x 128 (8.2 to 9.7 us against 11.0 to 11.8)."""
     for op, M, N, K in (("NT", 640, 2304, 768), ("NT", 768, 2304, 768), ("NT", 1500, 1024, 1024), ("NN", 1500, 1024, 1024),
