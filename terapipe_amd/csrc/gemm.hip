@@ -138,8 +138,8 @@ static constexpr int kSkinnyRows = 32;
 
 // Measured plans: for NT / NN the weight extents (N, K) match exactly and M (tokens of the slice) picks the
 // nearest measured M at or above it (at least half of it, so that a much shorter slice falls through to the
-// heuristics); on weights of up to 4096 x 4096, which have an estimate of their own, M itself (128 rows on 8192 x 2048 with the entry
-// of 256, 128 x 128 tiles, 22.8 us; 64 x 64 as the estimate has it 13.9).  TN (parameter gradients) matches all three extents.
+// heuristics); on weights of up to 4096 x 4096, which have an estimate of their own, rows that end in the same 16 as M (128 rows on
+// 8192 x 2048 with the entry of 256, 128 x 128 tiles, 22.8 us; 64 x 64 as the estimate has it 13.9).  TN (parameter gradients) matches all three extents.
 struct TunedPlan { int op, M, N, K, cfg, nsplit; };
 static const TunedPlan kTuned[] = {
 #include "gemm_tuned.inc"
@@ -163,7 +163,7 @@ static const TunedPlan* find_tuned(const tp_gemm_desc* d) {
             if (t->M == d->M) return t;
             continue;
         }
-        if (t->M >= d->M && t->M <= (small_weight(d) ? 1 : 2) * d->M && (!best || t->M < best->M)) best = t;
+        if (t->M >= d->M && (small_weight(d) ? (t->M + 15) / 16 == (d->M + 15) / 16 : t->M <= 2 * d->M) && (!best || t->M < best->M)) best = t;
     }
     if (best && (d->reserved & kBeside))
         for (const TunedPlan* t = kTunedBeside; t->op >= 0; ++t)

@@ -101,7 +101,7 @@ def test_rule_examples():
 
 
 def test_entries_between_their_row_counts():
-    """Small weights take an entry at its own row count only; on larger ones fewer row tiles mean more k splits."""
+    """Small weights take an entry near its own row count only; on larger ones fewer row tiles mean more k splits."""
     assert plan("NT", 256, 6144, 2048) == (8, 1) and plan("NT", 256, 8192, 2048) == (16, 1)
     for M in (128, 160, 192):
         assert plan("NT", M, 6144, 2048)[0] in (8, 12) and plan("NT", M, 8192, 2048)[0] in (8, 12), M      # the estimate
