@@ -175,6 +175,8 @@ int tp_gemm(const tp_gemm_desc* d, void* workspace, size_t workspace_bytes, void
 int tp_gemm_grouped(const tp_gemm_desc* descs, int n, void* workspace, size_t workspace_bytes, void* stream);
 /* the tile configuration of the single launch tp_gemm_grouped makes for this group; 0 = member by member */
 int tp_gemm_group_cfg(const tp_gemm_desc* descs, int n);
+/* Rows and columns of that launch's tile (0, 0: member by member).  Host code only; for tuning, tests and logs. */
+int tp_gemm_group_tile(const tp_gemm_desc* descs, int n, int* rows, int* columns);
 
 /* tp_gemm for callers that cannot allocate device memory or pass a workspace (code under HIP-graph capture,
  * tight serving loops, harnesses that forbid hipMalloc).  No counterpart in the reference: it exists for those

@@ -135,6 +135,7 @@ SYMBOLS = {
     "tp_gemm_grouped": (c_int, [ctypes.POINTER(GemmDesc), c_int, c_void_p, c_size_t, c_void_p]),
     "tp_gemm_tile": (c_int, [ctypes.POINTER(GemmDesc), c_int, ctypes.POINTER(c_int), ctypes.POINTER(c_int), ctypes.POINTER(c_int)]),
     "tp_gemm_group_cfg": (c_int, [ctypes.POINTER(GemmDesc), c_int]),
+    "tp_gemm_group_tile": (c_int, [ctypes.POINTER(GemmDesc), c_int, ctypes.POINTER(c_int), ctypes.POINTER(c_int)]),
     "tp_attn_fwd_workspace_bytes": (c_size_t, [ctypes.POINTER(AttnDesc)]),
     "tp_attn_prefix_fwd": (c_int, [ctypes.POINTER(AttnDesc), c_void_p, c_size_t, c_void_p]),
     "tp_attn_bwd_workspace_bytes": (c_size_t, [ctypes.POINTER(AttnDesc)]),

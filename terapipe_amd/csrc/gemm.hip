@@ -8,12 +8,10 @@ namespace tp {
 
 // The tiles of gemm_dma.hip (configurations 0, 3, 5, 8, 11, 12, 13; fp32: 0) and of gemm_tall.hip (2, 17 to 20; a grouped
 // launch, TN, of 2, 19 or 20): launch `cfg` on `grid` = (column tiles, row tiles, k splits); false when there is no such
-// kernel.  Deep rings of tiles 64 rows by `columns` (gemm_deep.hip; NT and NN, 16-bit).
+// kernel.
 bool launch_gemm_dma(int cfg, int op, int dtype, dim3 grid, const GemmArgs& a, hipStream_t s);
 bool launch_gemm_tall(int cfg, int op, int dtype, dim3 grid, const GemmArgs& a, hipStream_t s);
 bool launch_gemm_tall_group(int cfg, int dtype, int tiles, const GemmGroupArgs& ga, hipStream_t s);
-bool launch_gemm_deep(int columns, int op, int dtype, dim3 grid, const GemmArgs& a, hipStream_t s);
-
 
 // Sums the split-K partials and applies the epilogue.  A block of 256 threads covers 256 columns
 // (32 threads x 8 columns) by 8 rows, one vector of 8 columns a thread; column sums are combined across the
@@ -356,8 +354,9 @@ static inline bool runs_skinny(const tp_gemm_desc* d) {
 
 // fp32 products that run on tiles of 32 x 32 whose waves share k, in one launch (gemm_f32.hip): where the tiles come to at
 // most two workgroups per CU and eight waves take all of k at once.  Against 64 x 64 tiles with splits: k = 256 1.9 (up to 128
-// tiles) to 1.4 (512) times as fast, k = 64 1.25 to 1.05 up to 256 tiles, less beyond; k = 512, in two turns, 1.45 to 1.15,
-// k = 1024 1.1 to 0.8.  (A forced tile or split, and column sums, take the tile kernel.)
+// tiles) to 1.4 (512) times as fast, k = 64 1.25 to 1.05 up to 256 tiles, less beyond.  The rule ends with the first turn: k = 512, in
+// two, was measured on products alone only (1.45 to 1.15), k = 1024 at 1.1 to 0.8.  (A forced tile or split, and column sums, take
+// the tile kernel.)
 void launch_gemm_f32_small(int op, const GemmArgs& a, hipStream_t s);
 static bool runs_f32_small(const tp_gemm_desc* d) {
     if (d->dtype != TP_F32 || d->colsum_acc || (d->reserved & kForced)) return false;
@@ -382,7 +381,7 @@ static GemmPlan plan_gemm(const tp_gemm_desc* d) {
             long kt = (d->K + 15) / 16;
             long maxs = kt / 8 > 0 ? kt / 8 : 1;
             nsplit = (int)(want < maxs ? want : maxs);
-            if (nsplit > 32) nsplit = 32;
+            if (nsplit > 32) nsplit = 32;       // (16 at most: 8 rows on 1024 x 4096 18.0 -> 16.6 us alone, 20.9 -> 16.6 with the LayerNorm)
         }
         if (d->N % 8) nsplit = 1;       // (partial sums are rows of N)
         finish_plan(d, p, 16, nsplit);
@@ -866,6 +865,16 @@ extern "C" int tp_gemm_group_cfg(const tp_gemm_desc* descs, int n) {
     for (int i = 0; i < n; ++i)
         if (tp::validate_gemm(&descs[i]) != TP_OK) return 0;
     return tp::group_cfg(descs, n);
+}
+
+extern "C" int tp_gemm_group_tile(const tp_gemm_desc* descs, int n, int* rows, int* columns) {
+    const int cfg = tp_gemm_group_cfg(descs, n);
+    tp::TileCfg tc = {};
+    if (cfg) tp::tile_cfg(cfg, tc);
+    if (cfg == 2 && tp::runs_short(descs, n)) tc.bm = tc.bn = 128;
+    if (rows) *rows = tc.bm;
+    if (columns) *columns = tc.bn;
+    return TP_OK;
 }
 
 extern "C" int tp_gemm_grouped(const tp_gemm_desc* descs, int n, void* workspace, size_t workspace_bytes, void* stream) {

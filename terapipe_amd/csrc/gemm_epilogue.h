@@ -192,8 +192,8 @@ bool launch_gemm_pipe(int cfg, int op, int dtype, dim3 grid, const GemmArgs& a, 
 bool launch_gemm_pipe_group(int cfg, int dtype, int tiles, const GemmGroupArgs& ga, hipStream_t s);
 // Products of up to 32 rows (gemm_skinny.hip; NT, 16-bit): whole k ranges per workgroup, k splits as the arguments say.
 void launch_gemm_skinny(int dtype, const GemmArgs& a, hipStream_t s);
-// Deep rings of 64 x 32 or 64 x 64 tiles (gemm_deep.hip; NT and NN, 16-bit): grid = (column tiles of `columns`, row tiles,
-// k splits).
+// Deep rings of 64 x 32, 64 x 64 and 64 x 128 tiles (gemm_deep.hip; NT and NN, 16-bit): grid = (column tiles of `columns`, row
+// tiles, k splits).
 bool launch_gemm_deep(int columns, int op, int dtype, dim3 grid, const GemmArgs& a, hipStream_t s);
 // The eight-wave tiles of 256 rows x 256 or 192 columns of gemm_wide.hip (tile configuration 44; NT and NN).
 bool launch_gemm_wide(int columns, int op, int dtype, dim3 grid, const GemmArgs& a, hipStream_t s);
