@@ -7,14 +7,14 @@ namespace tp {
 // 32 x 32 tile, eight waves that share its k (v_mfma_f32_32x32x2_f32).  A product of a few hundred rows and columns has
 // about a hundred such tiles and is over in the time of its launches: gemm_kernel brings it to 512 workgroups of 64 x 64
 // with k splits, each a chain of 16-wide k-tiles that wait for memory, and a second launch adds the splits.  Here a wave asks
-// for all of its share of k at once (64 positions of both operands per turn), no LDS and no barrier stand between, and the
-// eight partial tiles are added through LDS, in pairs.
+// for all of its share of k at once (32 positions of both operands; products of up to 256 of k come here), no LDS and no barrier
+// stand between, and the eight partial tiles are added through LDS, in pairs.
 // A lane (row or column lane & 31 of its operand, g = lane >> 5) takes k-positions 4 g .. 4 g + 3 of every 8 from a
 // k-contiguous operand as one 16-byte load, position by position from the other kind: MFMA j of 4 sees k = 4 g + j from both.
 // ---------------------------------------------------------------------------------------------
-template <bool AKM, bool BKM, int STEP>
+template <bool AKM, bool BKM>
 __global__ __launch_bounds__(512) void gemm_f32_small_kernel(GemmArgs a) {
-    constexpr int WAVES = 8, NV = STEP / 8, PITCH = 36;
+    constexpr int WAVES = 8, STEP = 32, NV = STEP / 8, PITCH = 36;
     __shared__ float part[WAVES][32][PITCH];
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, li = lane & 31, g = lane >> 5;
     const int m0 = blockIdx.y * 32, n0 = blockIdx.x * 32;
@@ -68,14 +68,11 @@ __global__ __launch_bounds__(512) void gemm_f32_small_kernel(GemmArgs a) {
     epilogue_vec8<float>(a, m0 + row, n0 + c, v);
 }
 
-template <int STEP> static void launch_f32_small(int op, const GemmArgs& a, hipStream_t s) {
-    const dim3 grid((a.N + 31) / 32, (a.M + 31) / 32);
-    if (op == TP_GEMM_NT) gemm_f32_small_kernel<true, true, STEP><<<grid, 512, 0, s>>>(a);
-    else if (op == TP_GEMM_NN) gemm_f32_small_kernel<true, false, STEP><<<grid, 512, 0, s>>>(a);
-    else gemm_f32_small_kernel<false, false, STEP><<<grid, 512, 0, s>>>(a);
-}
 void launch_gemm_f32_small(int op, const GemmArgs& a, hipStream_t s) {
-    launch_f32_small<32>(op, a, s);
+    const dim3 grid((a.N + 31) / 32, (a.M + 31) / 32);
+    if (op == TP_GEMM_NT) gemm_f32_small_kernel<true, true><<<grid, 512, 0, s>>>(a);
+    else if (op == TP_GEMM_NN) gemm_f32_small_kernel<true, false><<<grid, 512, 0, s>>>(a);
+    else gemm_f32_small_kernel<false, false><<<grid, 512, 0, s>>>(a);
 }
 
 }  // namespace tp

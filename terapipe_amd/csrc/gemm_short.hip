@@ -11,7 +11,7 @@ namespace tp {
 // 1600-wide layer's 532 tiles are 2.08 rounds of them.  Here C (32 KB) is asked for right behind the first k-tiles and lands in
 // LDS while the k loop runs, and two workgroups share a CU (80 KB each): one's stores go out under the other's loop.
 // Four products of a 1600-wide layer added over 256 rows 51.3 -> 40.9 us (3.0 TB/s of C), over 64 37.4 -> 29.8; stored 36.5 -> 32.2.
-// From k of about 512 on the smaller tile's operands cost more than that saves.
+// The smaller tile's operands eat the gain as k grows: added over 768 rows 86 -> 75, over 1024 level at best.
 // ---------------------------------------------------------------------------------------------
 template <typename T, bool ADD>
 __global__ __launch_bounds__(256, 2)

@@ -5,8 +5,8 @@ the winners to ``csrc/gemm_tuned.inc``, the table ``plan_gemm`` consults before 
 
 A geometry is ``hidden:ffn:slice_tokens[,slice_tokens...]:step_tokens``: the forward GEMMs (NT) and data-gradient
 GEMMs (NN) are measured at every ``slice_tokens`` (tokens of a slice x batch), the parameter-gradient GEMMs
-(TN) at ``step_tokens`` (all tokens of a step).  Weights rotate through a set larger than the caches so that
-they stream from HBM as they do in a step.  Needs the GPU, and a library built with an empty table (the
+(TN) at ``step_tokens`` (all tokens of a step).  Weights rotate through a set larger than the caches (600 MB, each
+used once in a timed pass) so that they stream from HBM as they do in a step.  Needs the GPU, and a library built with an empty table (the
 heuristic plan is the yardstick); rebuild the library afterwards.
 
     python -m terapipe_amd.tune_gemm --in-step 2048:8192:16:24:1:256,256,256,256,256,256,256,256
@@ -35,8 +35,8 @@ DEFAULT_GEOMETRIES = [
 DMA_CFGS = [2, 3, 5, 6, 7, 8, 11, 12, 13, 14, 15, 16, 17, 18, 19, 20, 41, 42, 43]
 # the weight-streaming kernel's configurations (NT and NN only; 24 and 25 NT only): cfg -> rows of its row tile
 STREAM_CFGS = {21: 192, 22: 256, 24: 192, 25: 256, 26: 128, 29: 256, 30: 192, 31: 192, 32: 256, 33: 192, 34: 256,
-               35: 128, 36: 64, 37: 128, 38: 64}
-SPLITS = [1, 2, 3, 4, 6, 8]
+               35: 128, 36: 64, 37: 128, 38: 64, 39: 128, 40: 64}
+SPLITS = [1, 2, 3, 4, 5, 6, 8]
 # k splits the in-step search tries (the library deals whole k-tiles to the splits, evenly to within one).  Inside a step the slice streams share the
 # chip, and fewer splits than are fastest for a launch alone often win: fewer, larger workgroups and fewer partial sums.
 IN_STEP_SPLITS = (1, 2, 3, 4, 5, 6, 8)
@@ -114,16 +114,16 @@ def sweep(op, M, N, K, dtype, device, log, pair=False):
     """Returns (best_us, cfg, nsplit, automatic_us) for one shape."""
     a_shape = (K, M) if op == "TN" else (M, K)
     b_shape = (N, K) if op == "NT" else (K, N)
-    nb = max(2, min(8, int(1.0e9 // (N * K * 2))))
+    nb = max(2, -(-int(6e8) // (N * K * 2)))
     A = torch.randn(a_shape, device=device, dtype=dtype)
     Bs = [torch.randn(b_shape, device=device, dtype=dtype) for _ in range(nb)]
     C = torch.empty(M, N, device=device, dtype=dtype)
     code = OPS[op]
     if pair:
         Cs = [C, torch.empty_like(C)]
-        time_it = lambda **kw: _time_pair_us(lambda i, lane: ops.gemm(code, A, Bs[i % nb], M, N, K, C=Cs[lane], **kw))
+        time_it = lambda **kw: _time_pair_us(lambda i, lane: ops.gemm(code, A, Bs[i % nb], M, N, K, C=Cs[lane], **kw), max(6, nb))
     else:
-        time_it = lambda **kw: _time_us(lambda i: ops.gemm(code, A, Bs[i % nb], M, N, K, C=C, **kw))
+        time_it = lambda **kw: _time_us(lambda i: ops.gemm(code, A, Bs[i % nb], M, N, K, C=C, **kw), max(6, nb))
     auto = time_it()
     results = []
     for cfg in DMA_CFGS + (sorted(STREAM_CFGS) if op != "TN" and K % 64 == 0 else []):
