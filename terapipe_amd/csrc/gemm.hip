@@ -257,9 +257,9 @@ static float deep_time(const tp_gemm_desc* d, int ns, int* columns) {
     return best;
 }
 // Products whose sums of k splits the layer calls and the runner leave to the LayerNorm behind them: the two with a residual,
-// and the data gradients of the widening linears.
+// and the data gradients of the widening linears (the LM head's, which has no LayerNorm behind it, comes as `ragged`).
 static bool feeds_layernorm(const tp_gemm_desc* d) {
-    return d->epilogue == TP_EPI_BIAS_RESIDUAL || (d->op == TP_GEMM_NN && d->epilogue == TP_EPI_STORE && d->K >= 3L * d->N);
+    return d->epilogue == TP_EPI_BIAS_RESIDUAL || (d->op == TP_GEMM_NN && d->epilogue == TP_EPI_STORE && !d->ragged && d->K >= 3L * d->N);
 }
 // A split's partial sums and the launch that adds them, or the LayerNorm's reads of them (264 products with the LayerNorm behind,
 // 96 to 3072 rows, hidden 768 to 2560: the choice takes 1.011 times the fastest in the mean; priced like the launch the splits went
