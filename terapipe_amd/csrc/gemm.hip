@@ -346,10 +346,14 @@ static void plan_large(const tp_gemm_desc* d, int& cfg, int& ns) {
 
 // Forward products of up to kSkinnyRows rows on a weight of up to 4096 x 4096 run without LDS tiles: the plan's k splits,
 // whatever its tile.  (Beyond, both are bound by the weight stream and the tile kernels read the activation less often:
-// 16 rows on 20480 x 5120 37 us against 45.  A forced tile, and column sums, take the tile kernels.)
+// 16 rows on 20480 x 5120 58 us against 49.  A forced tile, and column sums, take the tile kernels.)  Up to 8 rows they take larger
+// weights too, where no k split is called for: us, 4 rows, tile kernels / these: 5120 x 5120 17.8 / 15.0, 8192 x 8192 37 / 31.6,
+// 20480 x 5120 46.6 / 37.8, 12288 x 4096 23.2 / 24.0 and without the LayerNorm before, 4096 x 16384 35.2 / 32.8; but 5120 x 20480, 1.25
+// workgroups of 16 rows to a CU, 40 / 48.
+static inline bool skinny_unsplit(const tp_gemm_desc* d) { return d->M <= 8 && (d->K <= 8192 || d->N % 4096 == 0); }
 static inline bool runs_skinny(const tp_gemm_desc* d) {
-    return d->op == TP_GEMM_NT && d->dtype != TP_F32 && d->M <= kSkinnyRows && (long)d->N * d->K <= (16L << 20) &&
-           (d->reserved & 0xff) == 0 && !d->colsum_acc;
+    return d->op == TP_GEMM_NT && d->dtype != TP_F32 && d->M <= kSkinnyRows && (d->reserved & 0xff) == 0 && !d->colsum_acc &&
+           (long)d->N * d->K <= (skinny_unsplit(d) ? 256L << 20 : 16L << 20);
 }
 
 // fp32 products that run on tiles of 32 x 32 whose waves share k, in one launch (gemm_f32.hip): where the tiles come to at
@@ -415,7 +419,7 @@ static GemmPlan plan_gemm(const tp_gemm_desc* d) {
         const long t3 = (long)((d->M + 127) / 128) * t256n;          // 128 x 256 tiles
         if (runs_skinny(d)) {
             cfg = 8;                // (its k splits are what counts)
-            ns = splits_for(t64, 2048);
+            ns = skinny_unsplit(d) ? 1 : splits_for(t64, 2048);
         } else if (small_weight(d)) {
             plan_slice(d, cfg, ns);
         } else if (d->M <= 64) {
@@ -529,9 +533,9 @@ static inline bool is_pipe_cfg(int cfg) { return cfg == 6 || cfg == 7 || (cfg >=
 
 // false: the plan names a (tile configuration, op, dtype) that no kernel is built for -- nothing was launched
 template <typename T>
-static bool launch_gemm(const tp_gemm_desc* d, const GemmPlan& p, const GemmArgs& a, hipStream_t s) {
+static bool launch_gemm(const tp_gemm_desc* d, const GemmPlan& p, const GemmArgs& a, hipStream_t s, const SkinnyLn* ln) {
     if (runs_skinny(d)) {
-        launch_gemm_skinny(d->dtype, a, s);
+        launch_gemm_skinny(d->dtype, a, ln, s);
     } else if (runs_f32_small(d)) {
         launch_gemm_f32_small(d->op, a, s);
     } else if (p.deep) {
@@ -673,14 +677,15 @@ static GemmArgs fill_args(const tp_gemm_desc* d, const GemmPlan& p, void* worksp
     return a;
 }
 
-static int run_gemm(const tp_gemm_desc* d, const GemmPlan& p, void* workspace, void* stream) {
-    const GemmArgs a = fill_args(d, p, workspace);
+static int run_gemm(const tp_gemm_desc* d, const GemmPlan& p, void* workspace, void* stream, const SkinnyLn* ln = nullptr, const void* ln_x = nullptr) {
+    GemmArgs a = fill_args(d, p, workspace);
+    if (ln) { a.A = ln_x; a.lda = d->K; }
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     bool launched;
     switch (d->dtype) {
-    case TP_F32: launched = launch_gemm<float>(d, p, a, s); break;
-    case TP_F16: launched = launch_gemm<f16>(d, p, a, s); break;
-    default: launched = launch_gemm<bf16>(d, p, a, s); break;
+    case TP_F32: launched = launch_gemm<float>(d, p, a, s, ln); break;
+    case TP_F16: launched = launch_gemm<f16>(d, p, a, s, ln); break;
+    default: launched = launch_gemm<bf16>(d, p, a, s, ln); break;
     }
     if (!launched) {
         set_error("tp_gemm: no kernel for tile configuration %d with op %d, dtype %d", p.cfg, d->op, d->dtype);
@@ -689,6 +694,20 @@ static int run_gemm(const tp_gemm_desc* d, const GemmPlan& p, void* workspace, v
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) { set_error("tp_gemm: launch failed: %s", hipGetErrorString(e)); return TP_ERR_LAUNCH; }
     return TP_OK;
+}
+
+int gemm_of_layernorm(const tp_gemm_desc& d, const void* x, const void* gamma, const void* beta, float* mean, float* rstd, float eps,
+                      void* stream, bool* taken) {
+    *taken = false;
+    const int rc = validate_gemm(&d);
+    if (rc != TP_OK) return rc;
+    if (!runs_skinny(&d) || !skinny_takes_ln(d.M, d.K) || d.lda != d.K || !x || !gamma || !beta || !mean || !rstd ||
+        (((uintptr_t)x | (uintptr_t)gamma | (uintptr_t)beta) & 15)) return TP_OK;
+    const GemmPlan p = plan_gemm(&d);
+    if (p.nsplit > 1) return TP_OK;
+    const SkinnyLn ln = {gamma, beta, const_cast<void*>(d.A), mean, rstd, eps};
+    *taken = true;
+    return run_gemm(&d, p, nullptr, stream, &ln, x);
 }
 
 // One launch for the whole group when every member is a 16-bit TN product (parameter gradients) of the same dtype and

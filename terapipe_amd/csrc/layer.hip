@@ -57,6 +57,16 @@ static int gemm_deferred(tp_gemm_desc d, void* ws, size_t bytes, void* stream, i
     return tp_gemm(&d, ws, bytes, stream);
 }
 
+// A = LayerNorm(x), then the product d that reads it: one launch where the product takes the rows itself.
+static int layernorm_then(const tp_gemm_desc& d, const tp_layer_desc& l, const void* x, const void* gamma, const void* beta, float* mean,
+                          float* rstd, void* ws, size_t bytes, void* stream) {
+    bool taken;
+    int rc = gemm_of_layernorm(d, x, gamma, beta, mean, rstd, 1e-5f, stream, &taken);
+    if (rc != TP_OK || taken) return rc;
+    rc = tp_layernorm_fwd(x, gamma, beta, const_cast<void*>(d.A), mean, rstd, d.M, d.K, 1e-5f, l.dtype, stream);
+    return rc != TP_OK ? rc : tp_gemm(&d, ws, bytes, stream);
+}
+
 struct ForwardPlan { tp_gemm_desc qkv, out, fc1, fc2; tp_attn_desc attn; };
 static ForwardPlan forward_plan(const tp_layer_desc& l) {
     const int M = l.T * l.batch, E = l.hidden, F = l.ffn;
@@ -131,23 +141,25 @@ extern "C" int tp_layers_fwd(const tp_layer_desc* layers, int n, void* ws, size_
         const tp_layer_desc& l = layers[i];
         const int M = l.T * l.batch, E = l.hidden;
         const ForwardPlan p = forward_plan(l);
-        if (pending > 1)
+        if (pending > 1) {
             rc = tp_layernorm_fwd_partials((const float*)ws, pending, layers[i - 1].w[B_FC2], layers[i - 1].h, layers[i - 1].out,
                                            l.w[W_LN1_G], l.w[W_LN1_B], l.xn, l.mean1, l.rstd1, M, E, 1e-5f, l.dtype, stream);
-        else
-            rc = tp_layernorm_fwd(l.x, l.w[W_LN1_G], l.w[W_LN1_B], l.xn, l.mean1, l.rstd1, M, E, 1e-5f, l.dtype, stream);
+            if (rc == TP_OK) rc = tp_gemm(&p.qkv, ws, bytes, stream);
+        } else {
+            rc = layernorm_then(p.qkv, l, l.x, l.w[W_LN1_G], l.w[W_LN1_B], l.mean1, l.rstd1, ws, bytes, stream);
+        }
         if (rc != TP_OK) return rc;
-        if ((rc = tp_gemm(&p.qkv, ws, bytes, stream)) != TP_OK) return rc;
         if ((rc = tp_attn_prefix_fwd(&p.attn, ws, bytes, stream)) != TP_OK) return rc;
         int splits;
         if ((rc = gemm_deferred(p.out, ws, bytes, stream, &splits)) != TP_OK) return rc;
-        if (splits > 1)
+        if (splits > 1) {
             rc = tp_layernorm_fwd_partials((const float*)ws, splits, l.w[B_OUT], l.x, l.h, l.w[W_LN2_G], l.w[W_LN2_B], l.hn, l.mean2,
                                            l.rstd2, M, E, 1e-5f, l.dtype, stream);
-        else
-            rc = tp_layernorm_fwd(l.h, l.w[W_LN2_G], l.w[W_LN2_B], l.hn, l.mean2, l.rstd2, M, E, 1e-5f, l.dtype, stream);
+            if (rc == TP_OK) rc = tp_gemm(&p.fc1, ws, bytes, stream);
+        } else {
+            rc = layernorm_then(p.fc1, l, l.h, l.w[W_LN2_G], l.w[W_LN2_B], l.mean2, l.rstd2, ws, bytes, stream);
+        }
         if (rc != TP_OK) return rc;
-        if ((rc = tp_gemm(&p.fc1, ws, bytes, stream)) != TP_OK) return rc;
         if (i + 1 < n) rc = gemm_deferred(p.fc2, ws, bytes, stream, &pending);
         else rc = tp_gemm(&p.fc2, ws, bytes, stream);
         if (rc != TP_OK) return rc;
