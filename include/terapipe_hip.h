@@ -236,7 +236,11 @@ typedef struct tp_attn_desc {
     int64_t stat_bh_rows;               /* entries per (b,h) block of lse and delta: 0 = T */
     int32_t dq_only;                    /* backward: 1 = compute delta and the q part of dqkv only; dK/dV of the
                                            slice are left to tp_attn_suffix_dkdv and no gradient cache is touched */
-    int32_t reserved3;
+    int32_t whole_grad_caches;          /* backward: 1 = dk_cache / dv_cache are written whole, [0, L_max), from the
+                                           gradient of the cache outputs in dk_in / dv_in: rows [0,P) = dk_in + dK, rows
+                                           [P,P+T) = 0 (theirs go to dqkv with dK added), the others = dk_in.  The three
+                                           flags above are then taken as 1.  0: dk_in and dv_in are not read */
+    const void* dk_in; const void* dv_in; /* [B*H, L_max, Dh] in grad_cache_dtype; both NULL: zeros */
 } tp_attn_desc;
 
 /* A forward call with few (batch, head) x 32-query blocks and a long key range spreads each block's keys over
@@ -434,7 +438,8 @@ typedef struct tp_layer_bwd_desc {
     int32_t small_zero;                 /* 1: small_acc starts from zero */
     void* small_out[8];                 /* where the sums go, cast (small_out[0] NULL: nowhere) */
     int32_t small_accumulate;           /* 1: += */
-    int32_t reserved;
+    int32_t whole_grad_caches;          /* with dk_in, dv_in: see tp_attn_desc */
+    const void* dk_in; const void* dv_in;
 } tp_layer_bwd_desc;
 size_t tp_layer_bwd_workspace_bytes(const tp_layer_bwd_desc* d);
 int tp_layer_bwd(const tp_layer_bwd_desc* d, void* workspace, size_t workspace_bytes, void* stream);

@@ -217,7 +217,7 @@ def layer_bwd(w, st, dout, heads, gk, gv, accumulate_prefix, has_incoming, zero_
 _FWD_PACK = struct.Struct("8iq28Q4q")          # tp_layer_desc: sizes, w[12], x, k_cache, v_cache, ..., ldw[4]
 _FWD_READ, _FWD_LDW = struct.Struct("15Q"), struct.Struct("4q")
 _FWD_READ_AT, _FWD_LDW_AT = 8 * 4 + 8, 8 * 4 + 8 + 28 * 8
-_BWD_PACK = struct.Struct("12Q4iq8Q4Q2i8Q2i")  # tp_layer_bwd_desc after its tp_layer_desc
+_BWD_PACK = struct.Struct("12Q4iq8Q4Q2i8Q2i2Q")  # tp_layer_bwd_desc after its tp_layer_desc
 _ACTIVATIONS = {"relu": 0, "gelu": 1}
 LINEAR_INPUTS = ("xn", "o", "hn", "a")          # of in_proj, out_proj, fc1 and fc2
 

@@ -56,7 +56,8 @@ class AttnDesc(ctypes.Structure):
         ("colsum_dqkv_acc", c_void_p),
         ("reserved", c_int32), ("reserved2", c_int32),
         ("q_bh_rows", c_int64), ("stat_bh_rows", c_int64),
-        ("dq_only", c_int32), ("reserved3", c_int32),
+        ("dq_only", c_int32), ("whole_grad_caches", c_int32),
+        ("dk_in", c_void_p), ("dv_in", c_void_p),
     ]
 
 
@@ -113,7 +114,7 @@ class LayerBwdDesc(ctypes.Structure):
         ("wg_rows", c_int64)] + [
         (n, c_void_p) for n in ("wg_dqkv", "wg_xn", "wg_dh", "wg_o", "wg_dz1", "wg_hn", "wg_dout", "wg_a")] + [
         ("wg_out", c_void_p * 4), ("wg_accumulate", c_int32), ("small_zero", c_int32), ("small_out", c_void_p * 8),
-        ("small_accumulate", c_int32), ("reserved", c_int32)]
+        ("small_accumulate", c_int32), ("whole_grad_caches", c_int32), ("dk_in", c_void_p), ("dv_in", c_void_p)]
 
 
 # every symbol include/terapipe_hip.h declares: name -> (restype, argtypes)

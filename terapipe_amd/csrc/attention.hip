@@ -257,6 +257,7 @@ __global__ __launch_bounds__(NW * 64) void attn_bwd_dkdv_kernel(AttnArgs a) {
     const int T_ = a.T, P = a.P, S = a.P + a.T;
     const long EE = (long)a.H * DH;
     const int key0wg = blockIdx.x * NW * 32;
+    if (a.grad_rows > S && !grad_rows_beyond<GT, DH, NW * 32, NT>(a, bh, key0wg, S, tid)) return;
     const int key0w = key0wg + wave * 32;
     const int key = key0w + li;
 
@@ -323,6 +324,8 @@ __global__ __launch_bounds__(NW * 64) void attn_bwd_dkdv_kernel(AttnArgs a) {
     if (key < S) {
         GT* gK = reinterpret_cast<GT*>(a.gk) + ((long)bh * a.cache_rows + key) * DH;
         GT* gV = reinterpret_cast<GT*>(a.gv) + ((long)bh * a.cache_rows + key) * DH;
+        const GT* iK = reinterpret_cast<const GT*>(a.gk_in) + ((long)bh * a.cache_rows + key) * DH;
+        const GT* iV = reinterpret_cast<const GT*>(a.gv_in) + ((long)bh * a.cache_rows + key) * DH;
         if (key < P) {
 #pragma unroll
             for (int db = 0; db < NDB; ++db)
@@ -331,7 +334,7 @@ __global__ __launch_bounds__(NW * 64) void attn_bwd_dkdv_kernel(AttnArgs a) {
                     int dh = db * 32 + 8 * jq + 4 * g;
                     if (DP != DH && dh >= DH) continue;
                     float ok[4] = {0.f, 0.f, 0.f, 0.f}, ov[4] = {0.f, 0.f, 0.f, 0.f};
-                    if (a.accumulate_prefix) { load4<GT>(gK + dh, ok); load4<GT>(gV + dh, ov); }
+                    if (a.accumulate_prefix) { load4<GT>(iK + dh, ok); load4<GT>(iV + dh, ov); }
                     store4<GT>(gK + dh, ok[0] + dk[db][4 * jq], ok[1] + dk[db][4 * jq + 1],
                                ok[2] + dk[db][4 * jq + 2], ok[3] + dk[db][4 * jq + 3]);
                     store4<GT>(gV + dh, ov[0] + dv[db][4 * jq], ov[1] + dv[db][4 * jq + 1],
@@ -347,7 +350,7 @@ __global__ __launch_bounds__(NW * 64) void attn_bwd_dkdv_kernel(AttnArgs a) {
                     int dh = db * 32 + 8 * jq + 4 * g;
                     if (DP != DH && dh >= DH) continue;
                     float ok[4] = {0.f, 0.f, 0.f, 0.f}, ov[4] = {0.f, 0.f, 0.f, 0.f};
-                    if (a.has_incoming) { load4<GT>(gK + dh, ok); load4<GT>(gV + dh, ov); }
+                    if (a.has_incoming) { load4<GT>(iK + dh, ok); load4<GT>(iV + dh, ov); }
                     store4<T>(dst + DH + dh, ok[0] + dk[db][4 * jq], ok[1] + dk[db][4 * jq + 1],
                               ok[2] + dk[db][4 * jq + 2], ok[3] + dk[db][4 * jq + 3]);
                     store4<T>(dst + 2 * DH + dh, ov[0] + dv[db][4 * jq], ov[1] + dv[db][4 * jq + 1],
@@ -506,6 +509,7 @@ __global__ __launch_bounds__(NW * 64) void attn_bwd_dkdv2_kernel(AttnArgs a) {
     const int T_ = a.T, P = a.P, S = a.P + a.T;
     const long EE = (long)a.H * DH;
     const int key0wg = kblk * NW * 32;
+    if (a.grad_rows > S && !grad_rows_beyond<GT, DH, NW * 32, NW * 64>(a, bh, key0wg, S, tid)) return;
     const int key0w = key0wg + wave * 32;
     const int key = key0w + li;
     const int nqb = (T_ + 31) / 32;
@@ -689,10 +693,13 @@ __global__ __launch_bounds__(NW * 64) void attn_bwd_dkdv2_kernel(AttnArgs a) {
     float* ebuf = reinterpret_cast<float*>(smem) + wave * 32 * EPI_LD;
     GT* gKb = reinterpret_cast<GT*>(a.gk) + ((long)bh * a.cache_rows + key0w) * DH;
     GT* gVb = reinterpret_cast<GT*>(a.gv) + ((long)bh * a.cache_rows + key0w) * DH;
+    const GT* iKb = reinterpret_cast<const GT*>(a.gk_in) + ((long)bh * a.cache_rows + key0w) * DH;
+    const GT* iVb = reinterpret_cast<const GT*>(a.gv_in) + ((long)bh * a.cache_rows + key0w) * DH;
 #pragma unroll
     for (int which = 0; which < 2; ++which) {
         acc_to_lds_rows<DH>(which == 0 ? dk : dv, ebuf, lane);
         GT* gb = which == 0 ? gKb : gVb;
+        const GT* ib = which == 0 ? iKb : iVb;
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         constexpr int NP = 32 * DH / 256;
         float4 val[NP];
@@ -712,7 +719,7 @@ __global__ __launch_bounds__(NW * 64) void attn_bwd_dkdv2_kernel(AttnArgs a) {
             const int kk = key0w + row;
             old[i][0] = old[i][1] = old[i][2] = old[i][3] = 0.f;
             const bool rd = kk < S && (kk < P ? a.accumulate_prefix != 0 : a.has_incoming != 0);
-            if (rd) load4<GT>(gb + (long)row * DH + col, old[i]);
+            if (rd) load4<GT>(ib + (long)row * DH + col, old[i]);
         }
 #pragma unroll
         for (int i = 0; i < NP; ++i) {
@@ -1522,6 +1529,13 @@ static int validate_attn(const tp_attn_desc* d, bool bwd) {
         if (!d->d_o || !d->delta || !d->dqkv) { set_error("%s: null gradient tensor", who); return TP_ERR_ARG; }
         if (((uintptr_t)d->d_o | (uintptr_t)d->dqkv | (uintptr_t)d->dk_cache | (uintptr_t)d->dv_cache) & 15) { set_error("%s: tensors must be 16-byte aligned", who); return TP_ERR_ARG; }
         if (!d->dq_only && (d->cache_len > 0 || d->has_incoming || d->zero_slice_rows) && (!d->dk_cache || !d->dv_cache)) { set_error("%s: gradient caches required", who); return TP_ERR_ARG; }
+        if (d->whole_grad_caches) {
+            if (d->dq_only || !d->dk_cache || !d->dv_cache || !d->dk_in != !d->dv_in || d->cache_rows > INT32_MAX - 256) {
+                set_error("%s: whole_grad_caches takes both gradient caches, dk_in and dv_in both or neither, and not dq_only", who);
+                return TP_ERR_ARG;
+            }
+            if (((uintptr_t)d->dk_in | (uintptr_t)d->dv_in) & 15) { set_error("%s: tensors must be 16-byte aligned", who); return TP_ERR_ARG; }
+        }
         if (d->grad_cache_dtype != d->dtype && d->grad_cache_dtype != TP_F32) { set_error("%s: grad_cache_dtype must be dtype or fp32", who); return TP_ERR_ARG; }
     }
     return TP_OK;
@@ -1654,6 +1668,12 @@ static AttnArgs make_args(const tp_attn_desc* d) {
     a.nsplit = 1; a.part_o = nullptr; a.part_lse = nullptr;
     a.accumulate_prefix = d->accumulate_prefix; a.has_incoming = d->has_incoming;
     a.zero_slice_rows = d->zero_slice_rows; a.qscale = d->q_scale;
+    a.gk_in = a.gk; a.gv_in = a.gv; a.grad_rows = a.P + a.T;
+    if (d->whole_grad_caches) {
+        a.gk_in = d->dk_in; a.gv_in = d->dv_in; a.grad_rows = (int)d->cache_rows;
+        a.accumulate_prefix = a.has_incoming = d->dk_in != nullptr;
+        a.zero_slice_rows = 1;
+    }
     a.dq_only = d->dq_only;
     a.shared_queries = shares_queries(d);
     a.shared_keys = shares_keys(d);
@@ -1697,7 +1717,7 @@ static void launch_bwd(const AttnArgs& a, hipStream_t s) {
     if constexpr (kTiled16 && std::is_same<T, GT>::value) {
         if (!keys_done && a.shared_keys) {
             const AttnKeysArgs k = {a.kc, a.vc, a.q, a.d_o, a.lse, a.delta, a.dqkv, a.gk, a.gv, a.B, a.H, 0, S, a.P, a.T, a.P,
-                                    a.accumulate_prefix, a.has_incoming, a.zero_slice_rows, a.cache_rows, a.q_bhs, a.st_bhs};
+                                    a.accumulate_prefix, a.has_incoming, a.zero_slice_rows, a.gk_in, a.gv_in, a.grad_rows, a.cache_rows, a.q_bhs, a.st_bhs};
             launch_attn_dkdv_long(std::is_same<T, f16>::value ? TP_F16 : TP_BF16, DH, false, k, s);
             keys_done = true;
         }
@@ -1708,7 +1728,7 @@ static void launch_bwd(const AttnArgs& a, hipStream_t s) {
         int nw = 4;
         if (((S + 127) / 128) * bh < 2L * kNumCU) nw = 2;
         if (((S + 63) / 64) * bh < 2L * kNumCU) nw = 1;
-        dim3 grid((S + 32 * nw - 1) / (32 * nw), (unsigned)bh);
+        dim3 grid((a.grad_rows + 32 * nw - 1) / (32 * nw), (unsigned)bh);
         if (kTiled16 && a.T <= kMaxTLds) {
             if constexpr (kTiled16) {
                 const size_t dyn = (size_t)2 * ((a.T + 31) / 32) * 32 * sizeof(float);
@@ -1833,7 +1853,7 @@ extern "C" int tp_attn_suffix_dkdv(const tp_attn_suffix_desc* d, void* stream) {
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     if (shares_bwd(d->batch, d->heads, d->head_dim, d->key_count)) {
         const AttnKeysArgs k = {a.kc, a.vc, a.q, a.d_o, a.lse, a.delta, a.dqkv, nullptr, nullptr, a.B, a.H, a.P, a.P + a.T, a.P, a.Lq, 0,
-                                0, 0, 0, a.cache_rows, a.q_bhs, a.st_bhs};
+                                0, 0, 0, nullptr, nullptr, a.P + a.T, a.cache_rows, a.q_bhs, a.st_bhs};
         launch_attn_dkdv_long(d->dtype, d->head_dim, true, k, s);
     } else {
         const unsigned grid = xcd_grid(d->batch * d->heads, (d->key_count + 31) / 32);

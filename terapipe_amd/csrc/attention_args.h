@@ -12,6 +12,8 @@ struct AttnArgs {
     int nsplit;
     float* part_o; float* part_lse;
     int accumulate_prefix, has_incoming, zero_slice_rows;
+    const void* gk_in; const void* gv_in;   // where the incoming gradients lie: gk, gv, or caches of their own
+    int grad_rows;                          // rows of the gradient caches that the call writes: P + T, or all
     int dq_only;
     int shared_queries, shared_keys;    // dQ / dK and dV by workgroups of 128 rows (attention_long.hip)
     float qscale;
@@ -87,6 +89,29 @@ __device__ __forceinline__ void acc_to_lds_rows(const float16v* acc, float* buf,
             *reinterpret_cast<float4*>(buf + li * LD + db * 32 + 8 * jq + 4 * g) =
                 make_float4(acc[db][4 * jq], acc[db][4 * jq + 1], acc[db][4 * jq + 2], acc[db][4 * jq + 3]);
 }
+
+// The part of a key block's rows [first, first + BLK) that lies past the call's positions, in both gradient caches: the incoming
+// gradient, or zeros.  False: the block has no other rows.  (uniform over the workgroup of NT threads)
+// Copying both caches before the call read and wrote them once more than the call itself does, in two launches: 2 x 5.8 us for 25
+// heads of 64 at 2048 positions, 2 x 9.8 for 40 of 128; here the rows below P cost nothing that the in-place form does not read.
+template <typename GT, int DH, int BLK, int NT, typename Args>
+__device__ __forceinline__ bool grad_rows_beyond(const Args& a, int bh, int first, int S, int tid) {
+    const int lo = max(first, S), n = (min(first + BLK, a.grad_rows) - lo) * (DH * (int)sizeof(GT) / 16);
+    const long off = ((long)bh * a.cache_rows + lo) * (DH * (int)sizeof(GT) / 16);
+    uint4 *k = reinterpret_cast<uint4*>(a.gk) + off, *v = reinterpret_cast<uint4*>(a.gv) + off;
+    if (a.gk_in) {
+        const uint4 *ki = reinterpret_cast<const uint4*>(a.gk_in) + off, *vi = reinterpret_cast<const uint4*>(a.gv_in) + off;
+        for (int i = tid; i < n; i += NT) {
+            const uint4 x = ki[i], y = vi[i];
+            k[i] = x;
+            v[i] = y;
+        }
+    } else {
+        for (int i = tid; i < n; i += NT) k[i] = v[i] = make_uint4(0, 0, 0, 0);
+    }
+    return first < S;
+}
+
 // piece i of the row-major read-back: row and first column of the four floats this lane gets
 template <int DH> __device__ __forceinline__ void row_piece(int i, int lane, int& row, int& col) {
     constexpr int LPR = DH / 4;            // lanes per row
@@ -105,6 +130,8 @@ struct AttnKeysArgs {
     const float* lse; const float* delta; void* dqkv; void* gk; void* gv;
     int B, H, key0, key_end, slice0, nq, q_pos;
     int accumulate_prefix, has_incoming, zero_slice_rows;
+    const void* gk_in; const void* gv_in;
+    int grad_rows;
     long cache_rows, q_bhs, st_bhs;
 };
 void launch_attn_dkdv_long(int dtype, int head_dim, bool suffix, const AttnKeysArgs& a, hipStream_t s);

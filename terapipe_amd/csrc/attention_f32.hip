@@ -222,6 +222,7 @@ __global__ __launch_bounds__(256) void attn_f32_dkdv_kernel(AttnArgs a) {
     const int T_ = a.T, P = a.P, S = a.P + a.T;
     const long EE = (long)a.H * DH;
     const int key0 = blockIdx.x * 32, key = key0 + li;                  // (the first keys have the most queries)
+    if (a.grad_rows > S && !grad_rows_beyond<float, DH, 32, 256>(a, bh, key0, S, tid)) return;
     float* sQ = smem + wave * 2 * TILE;
     float* sdO = sQ + TILE;
     const float* Qb = reinterpret_cast<const float*>(a.q) + (long)bh * a.q_bhs;
@@ -290,12 +291,14 @@ __global__ __launch_bounds__(256) void attn_f32_dkdv_kernel(AttnArgs a) {
         const long goff = ((long)bh * a.cache_rows + k) * DH + col;
         float4v* gK = reinterpret_cast<float4v*>(reinterpret_cast<float*>(a.gk) + goff);
         float4v* gV = reinterpret_cast<float4v*>(reinterpret_cast<float*>(a.gv) + goff);
+        const float4v* iK = reinterpret_cast<const float4v*>(reinterpret_cast<const float*>(a.gk_in) + goff);
+        const float4v* iV = reinterpret_cast<const float4v*>(reinterpret_cast<const float*>(a.gv_in) + goff);
         if (k < P) {
-            if (a.accumulate_prefix) { vk += *gK; vv += *gV; }
+            if (a.accumulate_prefix) { vk += *iK; vv += *iV; }
             *gK = vk;
             *gV = vv;
         } else {
-            if (a.has_incoming) { vk += *gK; vv += *gV; }
+            if (a.has_incoming) { vk += *iK; vv += *iV; }
             float* dst = reinterpret_cast<float*>(a.dqkv) + ((long)(k - P) * a.B + b) * (3 * EE) + (long)h * 3 * DH + col;
             *reinterpret_cast<float4v*>(dst + DH) = vk;
             *reinterpret_cast<float4v*>(dst + 2 * DH) = vv;
@@ -312,7 +315,7 @@ template <int DH> static void fwd_f32(const AttnArgs& a, hipStream_t s) {
 }
 template <int DH> static void bwd_f32(const AttnArgs& a, hipStream_t s) {
     attn_f32_dq_kernel<DH><<<dim3((a.T + 31) / 32, a.B * a.H), 256, 0, s>>>(a);
-    if (!a.dq_only) attn_f32_dkdv_kernel<DH><<<dim3((a.P + a.T + 31) / 32, a.B * a.H), 256, 0, s>>>(a);
+    if (!a.dq_only) attn_f32_dkdv_kernel<DH><<<dim3((a.grad_rows + 31) / 32, a.B * a.H), 256, 0, s>>>(a);
 }
 void launch_attn_f32(bool backward, int head_dim, const AttnArgs& a, hipStream_t s) {
     switch (head_dim) {

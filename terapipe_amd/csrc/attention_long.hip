@@ -541,6 +541,8 @@ __global__ __launch_bounds__(512) void attn_dkdv_long_kernel(AttnKeysArgs a) {
     const int b = bh / a.H, h = bh - b * a.H;
     const long EE = (long)a.H * DH;
     // the first keys, which the most queries see, start first
+    if constexpr (!SUFFIX)
+        if (a.grad_rows > a.key_end && !grad_rows_beyond<T, DH, 128, 512>(a, bh, a.key0 + blk * 128, a.key_end, tid)) return;
     const int key0 = a.key0 + blk * 128, kw = key0 + 32 * kb, key = kw + li, last_key = a.key_end - 1;
     const int q_beg = max(0, key0 - a.q_pos), nt = max(0, (a.nq - q_beg + QT - 1) / QT);
 
@@ -724,6 +726,7 @@ __global__ __launch_bounds__(512) void attn_dkdv_long_kernel(AttnKeysArgs a) {
         acc_to_lds_rows<DH>(x, mine, lane);             // the wave's own block: LDS operations of one wave complete in order
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         T* gcache = reinterpret_cast<T*>(qh ? a.gv : a.gk);
+        const T* gin = reinterpret_cast<const T*>(qh ? a.gv_in : a.gk_in);
 #pragma unroll
         for (int p = lane; p < 32 * DH / 8; p += 64) {
             const int row = p / (DH / 8), col = (p % (DH / 8)) * 8, k = kw + row;
@@ -733,9 +736,10 @@ __global__ __launch_bounds__(512) void attn_dkdv_long_kernel(AttnKeysArgs a) {
             *reinterpret_cast<float4*>(v + 4) = *reinterpret_cast<const float4*>(mine + row * EPI_LD + col + 4);
             uint4* dst = reinterpret_cast<uint4*>(reinterpret_cast<T*>(a.dqkv) + ((long)(k - a.slice0) * a.B + b) * (3 * EE) + (long)h * 3 * DH + (1 + qh) * DH + col);
             if constexpr (!SUFFIX) {
-                uint4* gp = reinterpret_cast<uint4*>(gcache + ((long)bh * a.cache_rows + k) * DH + col);
+                const long at = ((long)bh * a.cache_rows + k) * DH + col;
+                uint4* gp = reinterpret_cast<uint4*>(gcache + at);
                 if (k < a.slice0 ? a.accumulate_prefix : a.has_incoming) {
-                    const float8v old = __builtin_convertvector(__builtin_bit_cast(vec8_t<T>, *gp), float8v);
+                    const float8v old = __builtin_convertvector(__builtin_bit_cast(vec8_t<T>, *reinterpret_cast<const uint4*>(gin + at)), float8v);
 #pragma unroll
                     for (int e = 0; e < 8; ++e) v[e] += old[e];
                 }
@@ -750,7 +754,7 @@ __global__ __launch_bounds__(512) void attn_dkdv_long_kernel(AttnKeysArgs a) {
 }
 
 template <typename T, bool SUFFIX> static void dkdv_long(int hd, const AttnKeysArgs& a, hipStream_t s) {
-    const unsigned grid = xcd_grid(a.B * a.H, (a.key_end - a.key0 + 127) / 128);
+    const unsigned grid = xcd_grid(a.B * a.H, (a.grad_rows - a.key0 + 127) / 128);
     switch (hd) {
     case 64: attn_dkdv_long_kernel<T, 64, SUFFIX><<<grid, 512, 0, s>>>(a); break;
     case 80: attn_dkdv_long_kernel<T, 80, SUFFIX><<<grid, 512, 0, s>>>(a); break;

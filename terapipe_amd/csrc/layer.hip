@@ -204,6 +204,8 @@ extern "C" int tp_layer_bwd(const tp_layer_bwd_desc* b, void* ws, size_t bytes, 
     at.dk_cache = b->dk_cache; at.dv_cache = b->dv_cache;
     at.grad_cache_dtype = b->dk_cache ? b->grad_cache_dtype : l.dtype;
     at.accumulate_prefix = b->accumulate_prefix; at.has_incoming = b->has_incoming; at.zero_slice_rows = b->zero_slice_rows;
+    at.whole_grad_caches = b->whole_grad_caches;
+    if (b->whole_grad_caches) { at.dk_in = b->dk_in; at.dv_in = b->dv_in; }
     if ((rc = tp_attn_prefix_bwd(&at, nullptr, 0, stream)) != TP_OK) return rc;
     if ((rc = gemm_deferred(p.dxn, ws, bytes, stream, &splits)) != TP_OK) return rc;
     if (splits > 1)

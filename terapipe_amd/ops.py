@@ -305,8 +305,9 @@ def attn_prefix_fwd(q, k_cache, v_cache, batch, heads, head_dim, T, cache_len, q
 
 def attn_prefix_bwd(q, k_cache, v_cache, o, lse, d_o, dqkv, dk_cache, dv_cache, batch, heads, head_dim, T,
                     cache_len, q_scale, accumulate_prefix, has_incoming, zero_slice_rows, colsum_dqkv_acc=None,
-                    delta=None, q_bh_rows=0, stat_bh_rows=0, dq_only=False):
-    """Writes dqkv [T*B, 3*H*Dh]; updates rows [0, cache_len) of the gradient caches.  dq_only: delta and
+                    delta=None, q_bh_rows=0, stat_bh_rows=0, dq_only=False, whole_caches=False, dk_in=None, dv_in=None):
+    """Writes dqkv [T*B, 3*H*Dh]; updates rows [0, cache_len) of the gradient caches.  whole_caches: all of their rows are
+    written, from the cache outputs' gradients dk_in and dv_in (None: zeros).  dq_only: delta and
     the q part of dqkv only (the k and v parts are then attn_suffix_dkdv's; no gradient cache is touched)."""
     _require_cuda(q, k_cache, v_cache, d_o, dqkv)
     if delta is None:
@@ -318,6 +319,7 @@ def attn_prefix_bwd(q, k_cache, v_cache, o, lse, d_o, dqkv, dk_cache, dv_cache, 
     d.grad_cache_dtype = tp_dtype(dk_cache.dtype) if dk_cache is not None else d.dtype
     d.accumulate_prefix, d.has_incoming, d.zero_slice_rows = int(accumulate_prefix), int(has_incoming), int(zero_slice_rows)
     d.colsum_dqkv_acc = _p(colsum_dqkv_acc)
+    d.whole_grad_caches, d.dk_in, d.dv_in = int(whole_caches), _p(dk_in), _p(dv_in)
     lib = _lib.load()
     _lib.check(lib.tp_attn_prefix_bwd(ctypes.byref(d), None, 0, _stream()), "tp_attn_prefix_bwd")
     _record("attn_bwd", (batch, heads, head_dim, T, cache_len),

@@ -316,16 +316,7 @@ class _LayerFunction(torch.autograd.Function):
         if dout is None:
             dout = torch.zeros(T, B, E, dtype=dt, device=dev)
         dout = dout.contiguous()
-        gk = gv = None
-        has_incoming = False
-        if ctx.has_cache:
-            if dk_out is not None:
-                # grad_cache_output.clone(), reference transformer_models.py:188
-                gk, gv = dk_out.clone(), (dv_out.clone() if dv_out is not None else torch.zeros_like(dk_out))
-                has_incoming = True
-            else:
-                both = torch.zeros((2,) + k_cache.shape, dtype=dt, device=dev)
-                gk, gv = both[0], both[1]
+        gk, gv, gk_in, gv_in = _cache_grads(k_cache, dk_out, dv_out) if ctx.has_cache else (None,) * 4
         buf = torch.empty(geo.bwd.total, dtype=torch.uint8, device=dev)
         dx = torch.empty(T, B, E, dtype=dt, device=dev)
         base, off = buf.data_ptr(), geo.bwd.off
@@ -385,13 +376,28 @@ class _LayerFunction(torch.autograd.Function):
         core._BWD_PACK.pack_into(ctx.image, core._FWD_PACK.size, dy, p["dz1"], p["dhn"], p["dh"], p["d_o"], p["dqkv"],
                                  p["dxn"], dx.data_ptr(), p["delta"], p["small"],
                                  0 if gk is None else gk.data_ptr(), 0 if gv is None else gv.data_ptr(),
-                                 geo.dt, 1, int(has_incoming), int(has_incoming), rows if done else 0, *wg, *wg_out,
-                                 int(in_place), int(fresh), *small_out, int(in_place), 0)
+                                 geo.dt, 0, 0, 0, rows if done else 0, *wg, *wg_out,
+                                 int(in_place), int(fresh), *small_out, int(in_place), int(ctx.has_cache),
+                                 0 if gk_in is None else gk_in.data_ptr(), 0 if gv_in is None else gv_in.data_ptr())
         core.layer_bwd_native(ctx.image, dev)
         ctx.kept = ctx.image = ctx.w = ctx.st = None
         if not done or in_place:
             return (None, None, None, None, dx, gk, gv) + (None,) * len(core.PARAM_NAMES)
         return (None, None, None, None, dx, gk, gv) + tuple(grads[n] for n in core.PARAM_NAMES)
+
+
+def _cache_grads(cache, dk_out, dv_out):
+    """Gradients for the two cache inputs, not yet written, and those of the cache outputs as the kernel can read them (None
+    where there are none).  The kernel leaves the latter as they are (grad_cache_output.clone(), reference
+    transformer_models.py:188): it copies the rows that it does not add to."""
+    gk, gv = (torch.empty_like(cache, memory_format=torch.contiguous_format) for _ in range(2))
+    if dk_out is None:
+        return gk, gv, None, None
+    if dv_out is None:
+        dv_out = torch.zeros_like(dk_out)
+    # (the kernel's rows are contiguous and read 16 bytes at a time)
+    return (gk, gv) + tuple(g if g.is_contiguous() and g.data_ptr() % 16 == 0 else
+                            g.clone(memory_format=torch.contiguous_format) for g in (dk_out, dv_out))
 
 
 class _AttentionFunction(torch.autograd.Function):
@@ -424,14 +430,7 @@ class _AttentionFunction(torch.autograd.Function):
         if dy is None:
             dy = torch.zeros(T, B, E, dtype=x2d.dtype, device=x2d.device)
         dy2d = dy.contiguous().view(M, E)
-        gk = gv = None
-        has_incoming = False
-        if ctx.has_cache:
-            if dk_out is not None:
-                gk, gv = dk_out.clone(), (dv_out.clone() if dv_out is not None else torch.zeros_like(dk_out))
-                has_incoming = True
-            else:
-                gk, gv = torch.zeros_like(k_cache), torch.zeros_like(v_cache)
+        gk, gv, gk_in, gv_in = _cache_grads(k_cache, dk_out, dv_out) if ctx.has_cache else (None,) * 4
         acc = torch.zeros(4 * E, dtype=torch.float32, device=dy.device)
         acc_in, acc_out = acc[:3 * E], acc[3 * E:]
         d_o = torch.empty(M, E, dtype=dy.dtype, device=dy.device)
@@ -441,7 +440,8 @@ class _AttentionFunction(torch.autograd.Function):
         ops.colsum_acc(dy2d, acc_out)
         dqkv = torch.empty(M, 3 * E, dtype=dy.dtype, device=dy.device)
         ops.attn_prefix_bwd(q, k_cache, v_cache, o, lse, d_o, dqkv, gk, gv, B, heads, Dh, T, cache_len,
-                            float(Dh) ** -0.5, True, has_incoming, has_incoming, colsum_dqkv_acc=acc_in)
+                            float(Dh) ** -0.5, False, False, False, colsum_dqkv_acc=acc_in, whole_caches=ctx.has_cache,
+                            dk_in=gk_in, dv_in=gv_in)
         dx = torch.empty(M, E, dtype=dy.dtype, device=dy.device)
         ops.gemm(TP_GEMM_NN, dqkv, w_in, M, E, 3 * E, C=dx)
         dw_in = torch.empty_like(w_in)
