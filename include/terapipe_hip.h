@@ -226,11 +226,10 @@ typedef struct tp_attn_desc {
     int32_t reserved;                   /* 0 = automatic; bits 0-7: number of workgroups (fp32: splits) that share the key
                                            range of a query block in the forward (tuning, tests) */
     int32_t reserved2;                  /* tuning, tests.  bit 1 / bit 2: force the eight-wave / the four-wave form of the
-                                           16-bit forward kernel; bit 3 / bit 4: force workgroups of 32 queries / of 64 that
-                                           share their key tiles (from T >= 64 on, without a forced number of
-                                           workgroups); bit 5: force those of 128 queries that share them, bit 6:
-                                           forbid both; in the backward 5 / 6: force / forbid the workgroups of
-                                           128 queries and of 128 keys.  bit 7: fp32 without the workgroups of 32 rows whose
+                                           16-bit forward kernel; bit 3 / bit 4: force its workgroups of 32 / of 64 queries
+                                           (64 needs T >= 64); bit 5 / bit 6: force / forbid those of 128 queries that
+                                           share their key tiles, in the backward those of 128 queries and
+                                           of 128 keys.  bit 7: fp32 without the workgroups of 32 rows whose
                                            waves share the other axis */
     int64_t q_bh_rows;                  /* rows per (b,h) block of q: 0 = T; see tp_gemm_desc.q_bh_rows */
     int64_t stat_bh_rows;               /* entries per (b,h) block of lse and delta: 0 = T */

@@ -50,16 +50,6 @@ __device__ __forceinline__ bool xcd_map(int BH, int& bh, int& blk, int id = bloc
     blk = slot / nbh8;
     return bh < BH;
 }
-// The same for causal blocks that get shorter with blk, two workgroups to a CU: where all of an XCD's fit its 32 CUs at once, the
-// second half of them runs backwards, so that the longest shares its CU with the shortest.
-__device__ __forceinline__ bool xcd_map_causal(int BH, int nblocks, int& bh, int& blk) {
-    const int id = blockIdx.x, nbh8 = (BH + 7) >> 3, n = nbh8 * nblocks;
-    int slot = id >> 3;
-    if (n <= 64 && slot >= 32) slot = n + 31 - slot;
-    bh = (id & 7) + 8 * (slot % nbh8);
-    blk = slot / nbh8;
-    return bh < BH;
-}
 static inline unsigned xcd_grid(int BH, int nblocks) { return 8u * ((BH + 7) / 8) * nblocks; }
 
 // ---- shared pieces of the second-generation 16-bit attention kernels -------------------------------
@@ -121,7 +111,7 @@ template <int DH> __device__ __forceinline__ void row_piece(int i, int lane, int
 }
 
 // Calls of 128 queries and more against shared K / V tiles (attention_long.hip; 16-bit, head dimensions 64 to 128).
-void launch_attn_fwd_long(int dtype, int head_dim, int query_blocks, const AttnArgs& a, hipStream_t s);
+void launch_attn_fwd_long(int dtype, int head_dim, const AttnArgs& a, hipStream_t s);
 void launch_attn_dq_long(int dtype, int head_dim, const AttnArgs& a, hipStream_t s);       // (leaves delta too)
 // dK / dV of the keys [key0, key_end) against queries 0 .. nq - 1, which lie at the positions q_pos + i (attention_long.hip).  Row
 // k - slice0 of dqkv takes key k from slice0 on; without `suffix` the gradient caches are as in AttnArgs.

@@ -8,306 +8,241 @@ template <typename T> using vec8_t = T __attribute__((ext_vector_type(8)));
 template <typename T> __device__ __forceinline__ uint4 pack8v(float8v v) {
     return __builtin_bit_cast(uint4, __builtin_convertvector(v, vec8_t<T>));
 }
-template <typename T> using vec2_t = T __attribute__((ext_vector_type(2)));
-typedef float float2v __attribute__((ext_vector_type(2)));
-template <typename T> __device__ __forceinline__ unsigned pack2(float a, float b) {
-    const float2v two = {a, b};
-    return __builtin_bit_cast(unsigned, __builtin_convertvector(two, vec2_t<T>));
-}
-
-// A [DH x 32] accumulator set (as in acc_to_lds_rows) rounded to T, turned to rows in the wave's own 32 x (DH + 8) elements of LDS
-// and handed to store(row, column, 8 elements): the LDS operations of one wave complete in order.
-template <typename T, int DH, typename F>
-__device__ __forceinline__ void rows_out(const float16v* acc, T* buf, int lane, F store) {
-    constexpr int NDB = (DH + 31) / 32, LD = NDB * 32 + 8;
-    const int g = lane >> 5, li = lane & 31;
-#pragma unroll
-    for (int db = 0; db < NDB; ++db)
-#pragma unroll
-        for (int jq = 0; jq < 4; ++jq)
-            *reinterpret_cast<uint2*>(buf + li * LD + db * 32 + 8 * jq + 4 * g) =
-                make_uint2(pack2<T>(acc[db][4 * jq], acc[db][4 * jq + 1]), pack2<T>(acc[db][4 * jq + 2], acc[db][4 * jq + 3]));
-    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-    for (int i = 0; i < 32 * DH / 512; ++i) {
-        const int p = i * 64 + lane, row = p / (DH / 8), col = (p % (DH / 8)) * 8;
-        store(row, col, *reinterpret_cast<const uint4*>(buf + row * LD + col));
-    }
-}
 
 // ------------------------------------------------------------------------------------------------
-// Forward.  A workgroup of four waves owns 32 * QB queries of one (batch, head): blocks of 32, each by one wave (QB = 4) or by
-// two that take one half of every key tile and merge at the end (QB = 2).  K and V tiles are loaded once for all four waves, into
-// rings of 64 KB at most, so that two workgroups (three at head dimension 64) share a CU: the two waves of a SIMD belong to
-// different workgroups, and no barrier keeps them in step.  A wave works on three tiles at once, in one straight line: the
-// exponentials of one tile stand between the score MFMAs of the next and the output MFMAs of the last.
+// Forward.  A workgroup of eight waves owns 128 queries of one (batch, head): four blocks of 32, each by two waves that
+// take one half of every key tile and merge at the end.  A tile of 128 keys of K and V is loaded once for all of them, into
+// a ring of two stages in which K runs one tile ahead of V.
 //
-// What bounds it: the vector ALU, whose issue slots an MFMA takes too (a 32 x 32 x 16 one about four): per 32 x 32 block 70
-// operations, 16 of them exponentials, beside 8 to 16 MFMAs; MFMAs 0.41 and vector ALU 0.42 of the SIMD clocks at 96 heads of
-// 128.  Without the LDS reads 10 to 17 % of the time would go, without the exponentials 9 %.
-// Measured (fp16, causal, 2048 positions, us; before: eight waves on one ring of 128 KB, phases in step): 40 heads of 128
-// 70 -> 56, 96 of 128 149 -> 118 (870 TFLOP/s), 16 of 128 41 -> 32 (blocks of 64), 32 of 80 39 -> 38; 64 of 64 at 1024 20.7 -> 19;
-// 40 of 128, 512 after 1536 51 -> 32.  The tile's four slots with a barrier per tile instead of per two: 2 to 10 % slower at 64.
+// What bounds it: the vector ALU (16 exponentials at a quarter of its rate, and about as many cycles of the rest, per 32 x 32
+// block) and the MFMAs (as long again), two waves a SIMD.  The forms that give every wave its own ring (attn_fwd2_kernel,
+// attn_fwd3_kernel) take 128 KB of LDS for one wave a SIMD, which waits for memory a third of its time, and pull every K / V
+// byte through the global -> LDS path once per 32 or 64 queries; here it is once per 128.
+// Measured (fp16, causal, 2048 positions): 40 heads of 128 98 -> 70 us, 96 of 128 228 -> 152 (677 TFLOP/s), 32 of 80 69 -> 41;
+// 64 heads of 64 at 1024 27 -> 23.  Raising one of a SIMD's waves over the other (s_setprio), and score MFMAs interleaved
+// with the exponentials by the compiler (its LDS reads then sit in front of each MFMA), change nothing.
 // ------------------------------------------------------------------------------------------------
-
-template <typename T, int DH, int QB>
-__global__ __launch_bounds__(256, 2) void attn_fwd_long_kernel(AttnArgs a) {
+template <typename T, int DH>
+__global__ __launch_bounds__(512) void attn_fwd_long_kernel(AttnArgs a) {
     typedef Elem<T> E;
-    constexpr int KH = 4 / QB, SS = 2 / KH, R = 2 * SS;     // waves that share a query block's keys (a tile: 32 each); tiles between two barriers; slots of the rings
     constexpr int NDB = (DH + 31) / 32, NKS = DH / 16, PITCH = tile_pitch<DH>(), CPR = PITCH / 8;
-    constexpr int KT = 32 * KH, TILE = KT * PITCH;
-    constexpr int NLD = KT * CPR / 256;                     // loads per K or V tile and lane
+    constexpr int NB = 2;                                   // 32-key blocks of a tile per wave
+    constexpr int KT = 64 * NB, TILE = KT * PITCH, STAGE = 2 * TILE;
+    constexpr int NLD = KT * CPR / 512;                     // loads per K or V tile and lane
+    constexpr int NLOAD = 2 * NLD;
     constexpr int EPI_LD = NDB * 32 + 4;
-    constexpr int RING_BYTES = 2 * R * TILE * 2, EPI_BYTES = (KH > 1 ? QB * 64 * 4 : 0) + QB * 32 * EPI_LD * 4;
+    constexpr int RING_BYTES = 2 * STAGE * 2, EPI_BYTES = (4 * 2 * 32 + 4 * 32 * EPI_LD) * 4;
     __shared__ __attribute__((aligned(16))) unsigned char smem[RING_BYTES > EPI_BYTES ? RING_BYTES : EPI_BYTES];
     T* ring = reinterpret_cast<T*>(smem);
 
     const int tid = threadIdx.x, lane = tid & 63, g = lane >> 5, li = lane & 31;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), qb = wave % QB, kh = wave / QB;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), qb = wave & 3, kh = wave >> 2;
     int bh, blk;
-    if (!xcd_map_causal(a.B * a.H, (a.T + 32 * QB - 1) / (32 * QB), bh, blk)) return;
+    if (!xcd_map(a.B * a.H, bh, blk)) return;
     const int b = bh / a.H, h = bh - b * a.H;
     const int T_ = a.T, P = a.P, S = a.P + a.T;
-    const int q0 = ((T_ + 32 * QB - 1) / (32 * QB) - 1 - blk) * (32 * QB);      // the blocks with the longest key range start first
+    const int q0 = ((T_ + 127) / 128 - 1 - blk) * 128;      // the blocks with the longest key range start first
     const int qw = q0 + 32 * qb, tq = qw + li;
     const bool qok = tq < T_;
-    const int nt = (P + min(T_, q0 + 32 * QB) + KT - 1) / KT;   // tiles of the workgroup
-    const int key_end = qw < T_ ? P + min(T_, qw + 32) : 0;     // keys this wave's queries see
-    const int nt_w = max(0, (key_end - kh * 32 + KT - 1) / KT); // tiles that hold some of them for this wave
+    const int nt = (P + min(T_, q0 + 128) + KT - 1) / KT;   // tiles of the workgroup
+    const int key_end = qw < T_ ? P + min(T_, qw + 32) : 0; // keys this wave's queries see
 
-    // the lane's chunk of a tile's first rows and that of row S - 1 (the swizzle repeats every 16 rows: the same column in each load)
-    const int lr = tid / CPR, lc = (tid % CPR) ^ swz16<PITCH>(lr);
-    const unsigned koff = (unsigned)(lr * DH * 2 + lc * 16), klast = (unsigned)((S - 1) * DH * 2 + lc * 16);
-    const bool chunk = DH == PITCH || lc < DH / 8;
+    unsigned koff[NLD];
+#pragma unroll
+    for (int i = 0; i < NLD; ++i) {
+        const int p = i * 512 + tid, r = p / CPR, lc = (p % CPR) ^ swz16<PITCH>(r);
+        koff[i] = lc < DH / 8 ? (unsigned)(r * DH * 2 + lc * 16) : kNoChunk;
+    }
     const char* Kb = uniform_ptr(reinterpret_cast<const char*>(reinterpret_cast<const T*>(a.kc) + (long)bh * a.cache_rows * DH));
     const char* Vb = uniform_ptr(reinterpret_cast<const char*>(reinterpret_cast<const T*>(a.vc) + (long)bh * a.cache_rows * DH));
     const unsigned lds0 = lds_addr(smem) + wave * 1024;
-    // tile t of K (which = 0) or V (1) into a slot of its ring; rows at or past S are clamped to row S - 1: finite data, and
-    // every such key is masked
-    auto issue = [&](int slot, int which, int tile) __attribute__((always_inline)) {
-        const unsigned dst = lds0 + (unsigned)((which * R + slot) * TILE * 2), row = (unsigned)(tile * KT) * (DH * 2);
+    // tile t of K (which = 0) or V (1) into its half of a stage; rows at or past S are clamped to row S - 1: finite data,
+    // and every such key is masked
+    auto issue = [&](int stage, int which, int tile) {
+        const unsigned dst = lds0 + (unsigned)((stage * STAGE + which * TILE) * 2);
+        const char* base = which ? Vb : Kb;
+        const int row0 = tile * KT;
+        if (row0 + KT <= S) {
+            const char* sb = base + (long)row0 * (DH * 2);
 #pragma unroll
-        for (int i = 0; i < NLD; ++i)
-            if (chunk) dma16_saddr_lds(min(row + (unsigned)(i * (256 / CPR) * DH * 2) + koff, klast), which ? Vb : Kb, dst + i * 4096);
+            for (int i = 0; i < NLD; ++i) load_chunk_lds<DH>(koff[i], sb, dst + i * 8192);
+        } else {
+#pragma unroll
+            for (int i = 0; i < NLD; ++i) {
+                const int p = i * 512 + tid, r = p / CPR, lc = (p % CPR) ^ swz16<PITCH>(r);
+                const unsigned off = lc < DH / 8 ? (unsigned)(min(row0 + r, S - 1) * DH * 2 + lc * 16) : kNoChunk;
+                load_chunk_lds<DH>(off, base, dst + i * 8192);
+            }
+        }
     };
+    issue(0, 0, 0);
+    issue(0, 1, 0);
+    if (nt > 1) issue(1, 0, 1);
+
     typename E::opnd_t qreg[NKS];
     load_row_operands<T, DH>(qreg, reinterpret_cast<const T*>(a.q) + (long)bh * a.q_bhs + (long)(qok ? tq : 0) * DH, qok, g);
 
+    int okm[NKS], otr[NDB][2];          // element offsets of the lane's fetches inside a stage, its first block
 #pragma unroll
-    for (int i = 0; i < R; ++i) issue(i, 0, i);
-    if constexpr (SS == 2) issue(0, 1, 0);
+    for (int ks = 0; ks < NKS; ++ks) okm[ks] = km_offset<T, PITCH>(kh * 32 * NB + li, ks * 16, lane);
 #pragma unroll
-    for (int i = 0; i < TILE / 2048; ++i)               // the V of the tile before the first, whose P is zero
-        *reinterpret_cast<uint4*>(smem + (2 * R - 1) * TILE * 2 + (i * 256 + tid) * 16) = make_uint4(0, 0, 0, 0);
+    for (int db = 0; db < NDB; ++db) {
+        tr_offsets<T, PITCH, true>(kh * 32 * NB, db * 32, lane, otr[db][0], otr[db][1]);
+        otr[db][0] += TILE;
+        otr[db][1] += TILE;
+    }
 
-    int okm[NKS], otr[NDB][2];          // element offsets of the lane's fetches inside a tile
+    float16v oacc[NDB];
 #pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) okm[ks] = km_offset<T, PITCH>(kh * 32 + li, ks * 16, lane);
+    for (int db = 0; db < NDB; ++db)
 #pragma unroll
-    for (int db = 0; db < NDB; ++db) tr_offsets<T, PITCH, true>(kh * 32, db * 32, lane, otr[db][0], otr[db][1]);
+        for (int r = 0; r < 16; ++r) oacc[db][r] = 0.f;
+    float m = -INFINITY, lsum = 0.f;
 
-    float16v oacc[NDB], s[2];
-    const float16v zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
+    // the scores of the wave's keys of the tile in stage `so`
+    auto scores = [&](int so, float16v* s) __attribute__((always_inline)) {
 #pragma unroll
-    for (int db = 0; db < NDB; ++db) oacc[db] = zero;
-    float lsum = 0.f;
-    typename E::opnd_t kf[NKS], vf[2 * NDB];
-    uint4 p[2] = {make_uint4(0, 0, 0, 0), make_uint4(0, 0, 0, 0)};
+        for (int n = 0; n < NB; ++n)
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[n][r] = 0.f;
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks)
+#pragma unroll
+            for (int n = 0; n < NB; ++n) s[n] = E::mfma(load_km<T>(ring + so + okm[ks] + n * 32 * PITCH), qreg[ks], s[n]);
+    };
+    float16v s[NB];
+    wait_vmcnt<0>();
+    __builtin_amdgcn_s_barrier();
+    asm volatile("" ::: "memory");
+    scores(0, s);
 
-    auto barrier = [&]() __attribute__((always_inline)) {
+    auto step = [&](auto sc, int t) __attribute__((always_inline)) {
+        constexpr int st = decltype(sc)::value;
+        // this wave's loads of K(t + 1) and V(t) have landed and its reads of K(t) and V(t - 1) are back
         wait_vmcnt<0>();
         asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-    };
-    auto row_max = [&](const float16v& x) __attribute__((always_inline)) {
-        float v = x[0];
+        if (t + 1 < nt) issue(st ^ 1, 1, t + 1);
+        if (t + 2 < nt) issue(st, 0, t + 2);
+        const int key0 = t * KT + kh * NB * 32;
+        if (key0 >= key_end) return;        // wave-uniform: this tile and all after it lie beyond the wave's queries
+        if (key0 + 32 * NB - 1 > P + qw) {  // wave-uniform: the tile touches the causal boundary
 #pragma unroll
-        for (int j = 1; j < 16; ++j) v = fmaxf(v, x[j]);
-        return v;
-    };
-    barrier();
-    s[0] = zero;
-    s[1] = zero;
+            for (int n = 0; n < NB; ++n)
 #pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) s[0] = E::mfma(load_km<T>(ring + okm[ks]), qreg[ks], s[0]);
-#pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) kf[ks] = load_km<T>(ring + TILE + okm[ks]);
-    auto mask = [&](float16v& x, int key0) __attribute__((always_inline)) {
-#pragma unroll
-        for (int j = 0; j < 16; ++j)
-            if (key0 + acc_row(j, g) > P + tq) x[j] = -INFINITY;
-    };
-    // The first reference is the maximum of two tiles: of one, the largest P of a row is less often exactly 1, and the result
-    // 2 % further from fp64.
-#pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) s[1] = E::mfma(kf[ks], qreg[ks], s[1]);
-    mask(s[0], kh * 32);
-    mask(s[1], KT + kh * 32);
-    float smax = fmaxf(row_max(s[0]), row_max(s[1])), m = fmaxf(smax, __shfl_xor(smax, 32, 64));
-    smax = m;
-    if constexpr (SS == 1) {
-        barrier();
-        issue(0, 0, 2);
-    }
-
-    // Tile t: the exponentials of its scores (s[t & 1]) run between the MFMAs of its neighbours -- the scores of the next tile
-    // (K fragments in kf), then the output of the one before (its P in p).  A fragment's registers are free when its MFMA has
-    // gone: V fragments take the place of K's, and K's of the tile after next that of V's.
-    auto stage = [&](auto slc, int t) __attribute__((always_inline)) {
-        constexpr int sl = decltype(slc)::value, cur = sl & 1, nxt = cur ^ 1, NPV = 2 * NDB, NM = NKS + NPV;
-        const int key0 = t * KT + kh * 32;
-        const T* kafter = ring + (sl + 2) % R * TILE;
-        const T* vbefore = ring + (R + (sl + R - 1) % R) * TILE;
-        if (key0 + 31 > P + qw) {               // wave-uniform: the block touches the causal boundary
-            mask(s[cur], key0);
-            smax = row_max(s[cur]);
+                for (int j = 0; j < 16; ++j)
+                    if (key0 + n * 32 + acc_row(j, g) > P + tq) s[n][j] = -INFINITY;
         }
+        float mt = -INFINITY;
+#pragma unroll
+        for (int n = 0; n < NB; ++n)
+#pragma unroll
+            for (int j = 0; j < 16; ++j) mt = fmaxf(mt, s[n][j]);
+        mt = fmaxf(mt, __shfl_xor(mt, 32, 64));
         // m is the row's REFERENCE value of the exponentials, not its running maximum (as in attn_fwd2_kernel): it moves
         // only when a row outgrows it by kSlack, exponentials stay below e^kSlack = 148.
         constexpr float kSlack = 5.0f;
-        float alpha = 1.f;
-        unsigned long moved = __builtin_amdgcn_ballot_w64(smax > m + kSlack);
-        if (moved) {
-            const float m_new = fmaxf(m, fmaxf(smax, __shfl_xor(smax, 32, 64)));
-            alpha = m_new == -INFINITY ? 1.0f : fast_exp2((m - m_new) * kLog2e);
+        if (__builtin_amdgcn_ballot_w64(mt > m + kSlack) != 0) {
+            const float m_new = fmaxf(m, mt);
+            const float alpha = m_new == -INFINITY ? 1.0f : fast_exp2((m - m_new) * kLog2e);
             m = m_new;
             lsum *= alpha;
-        }
-        asm volatile("" : "+s"(moved));         // (one straight line between the two branches)
-        const float mneg = m == -INFINITY ? 0.f : -m * kLog2e;
-        __builtin_amdgcn_sched_barrier(0);
-        unsigned pw[8];
-        float e[16];
-        float psum = 0.f;
-#pragma unroll
-        for (int k = 0; k < NM; ++k) {
-            if (k < NKS) {
-                s[nxt] = E::mfma(kf[k], qreg[k], k == 0 ? zero : s[nxt]);
-#pragma unroll
-                for (int i = k; i < (k == NKS - 1 ? NPV : k + 1); ++i) {
-                    if (i >= NPV) break;
-                    const T* v = vbefore + i / NDB * 16 * PITCH;
-                    vf[i] = load_tr<T>(v + otr[i % NDB][0], v + otr[i % NDB][1]);
-                }
-            } else {
-                const int i = k - NKS;
-                oacc[i % NDB] = E::mfma(vf[i], p[i / NDB], oacc[i % NDB]);
-#pragma unroll
-                for (int ks = i; ks < (i == NPV - 1 ? NKS : i + 1); ++ks)
-                    if (ks < NKS) kf[ks] = load_km<T>(kafter + okm[ks]);
-            }
-#pragma unroll
-            for (int j = k * 16 / NM; j < (k + 1) * 16 / NM; ++j) {
-                e[j] = fast_exp2(fmaf(s[cur][j], kLog2e, mneg));        // -inf -> 0
-                psum += e[j];
-                if (j & 1) {
-                    pw[j / 2] = pack2<T>(e[j - 1], e[j]);
-                    asm volatile("" : "+v"(pw[j / 2]), "+v"(psum)); // (here, not where the next tile wants them)
-                }
-            }
-            if (k == NM - 2) {
-                smax = row_max(s[nxt]);
-                asm volatile("" : "+v"(smax));
-            }
-            __builtin_amdgcn_sched_barrier(0);
-        }
-        if (moved) {            // (what is added here was taken against the old reference)
 #pragma unroll
             for (int db = 0; db < NDB; ++db)
 #pragma unroll
                 for (int r = 0; r < 16; ++r) oacc[db][r] *= alpha;
         }
-        lsum += psum;
-        p[0] = make_uint4(pw[0], pw[1], pw[2], pw[3]);
-        p[1] = make_uint4(pw[4], pw[5], pw[6], pw[7]);
-    };
-    // before the first of SS tiles: this wave's loads of V(t - 1 .. t + SS - 2) and K(t + 2 .. t + SS + 1) have landed, and its
-    // reads of the tiles before them are back
-    auto advance = [&](int sl, int t) __attribute__((always_inline)) {
-        barrier();
+        const float mneg = m == -INFINITY ? 0.f : -m * kLog2e;
+        // Block by block: the next tile's K and this tile's V fragments are asked for, the exponentials run while they come,
+        // then the MFMAs, the next tile's scores in place of this one's.  (Behind the last tile the scores are those of
+        // whatever the other stage holds: nothing reads them.)
 #pragma unroll
-        for (int i = 0; i < SS; ++i) {
-            issue((sl + SS - 1 + i) % R, 1, t + SS - 1 + i);
-            issue((sl + SS + 2 + i) % R, 0, t + SS + 2 + i);
+        for (int n = 0; n < NB; ++n) {
+            typename E::opnd_t kf[NKS];
+            uint4 vf[2][NDB];
+#pragma unroll
+            for (int ks = 0; ks < NKS; ++ks) kf[ks] = load_km<T>(ring + (st ^ 1) * STAGE + okm[ks] + n * 32 * PITCH);
+#pragma unroll
+            for (int hs = 0; hs < 2; ++hs)
+#pragma unroll
+                for (int db = 0; db < NDB; ++db) {
+                    const int o = st * STAGE + (n * 32 + hs * 16) * PITCH;
+                    vf[hs][db] = load_tr<T>(ring + o + otr[db][0], ring + o + otr[db][1]);
+                }
+            __builtin_amdgcn_sched_barrier(0);
+            float8v e0, e1;
+            float psum = 0.f;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                e0[j] = fast_exp2(fmaf(s[n][j], kLog2e, mneg));        // -inf -> 0
+                e1[j] = fast_exp2(fmaf(s[n][j + 8], kLog2e, mneg));
+                psum += e0[j] + e1[j];
+            }
+            lsum += psum;
+            const uint4 p[2] = {pack8v<T>(e0), pack8v<T>(e1)};
+            __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+            for (int r = 0; r < 16; ++r) s[n][r] = 0.f;
+#pragma unroll
+            for (int ks = 0; ks < NKS; ++ks) s[n] = E::mfma(kf[ks], qreg[ks], s[n]);
+#pragma unroll
+            for (int hs = 0; hs < 2; ++hs)
+#pragma unroll
+                for (int db = 0; db < NDB; ++db) oacc[db] = E::mfma(vf[hs][db], p[hs], oacc[db]);
+            __builtin_amdgcn_sched_barrier(0);
         }
     };
-    auto step = [&](auto slc, int t) __attribute__((always_inline)) {
-        constexpr int sl = decltype(slc)::value;
-        if constexpr (sl % SS == 0) advance(sl, t);
-        stage(slc, t);
-    };
-    int t = 0;
-    while (t < nt_w) {
+    for (int t = 0; t < nt; t += 2) {
         step(std::integral_constant<int, 0>(), t);
-        if (++t >= nt_w) break;
-        step(std::integral_constant<int, 1>(), t);
-        if (++t >= nt_w) break;
-        if constexpr (R == 4) {
-            step(std::integral_constant<int, 2>(), t);
-            if (++t >= nt_w) break;
-            step(std::integral_constant<int, 3>(), t);
-            ++t;
-        }
+        if (t + 1 < nt) step(std::integral_constant<int, 1>(), t + 1);
     }
-    // the output of the wave's last tile, then the tiles of the waves with later queries
-    if (t % SS == 0) advance(t % R, t);
-    {
-        const T* vbefore = ring + (R + (t + R - 1) % R) * TILE;
-#pragma unroll
-        for (int i = 0; i < 2 * NDB; ++i) {
-            const T* v = vbefore + i / NDB * 16 * PITCH;
-            oacc[i % NDB] = E::mfma(load_tr<T>(v + otr[i % NDB][0], v + otr[i % NDB][1]), p[i / NDB], oacc[i % NDB]);
-        }
-    }
-    for (++t; t <= nt; ++t)
-        if (t % SS == 0) advance(t % R, t);
-    wait_vmcnt<0>();
-    __syncthreads();            // every wave is done with the ring: the space is reused
+    __syncthreads();            // every wave is done with the ring: the space is reused for the merge
 
-    float* sM = reinterpret_cast<float*>(smem);         // [QB][2][32]: the second halves' references and sums
-    float* ebuf = sM + (KH > 1 ? QB * 64 : 0) + qb * 32 * EPI_LD;
-    float lw = lsum + __shfl_xor(lsum, 32, 64);
-    float f0 = 1.f;
-    if constexpr (KH > 1) {
-        if (kh == 1) {
-            if (g == 0) { sM[qb * 64 + li] = m; sM[qb * 64 + 32 + li] = lw; }
-#pragma unroll
-            for (int db = 0; db < NDB; ++db)
-#pragma unroll
-                for (int jq = 0; jq < 4; ++jq)
-                    *reinterpret_cast<float4*>(ebuf + (db * 4 + jq) * 256 + lane * 4) =
-                        make_float4(oacc[db][4 * jq], oacc[db][4 * jq + 1], oacc[db][4 * jq + 2], oacc[db][4 * jq + 3]);
-        }
-        __syncthreads();
-        if (kh == 1) return;
-        const float m1 = sM[qb * 64 + li], l1 = sM[qb * 64 + 32 + li];
-        const float mt = fmaxf(m, m1), ms = mt == -INFINITY ? 0.f : mt;
-        f0 = fast_exp2((m - ms) * kLog2e);
-        const float f1 = fast_exp2((m1 - ms) * kLog2e);
-        lw = lw * f0 + l1 * f1;
-        m = mt;
+    float* sM = reinterpret_cast<float*>(smem);         // [4][2][32]: the second halves' references and sums
+    float* ebuf = sM + 4 * 2 * 32 + qb * 32 * EPI_LD;
+    const float lw = lsum + __shfl_xor(lsum, 32, 64);
+    if (kh == 1) {
+        if (g == 0) { sM[qb * 64 + li] = m; sM[qb * 64 + 32 + li] = lw; }
 #pragma unroll
         for (int db = 0; db < NDB; ++db)
 #pragma unroll
-            for (int jq = 0; jq < 4; ++jq) {
-                const float4 o = *reinterpret_cast<const float4*>(ebuf + (db * 4 + jq) * 256 + lane * 4);
-                oacc[db][4 * jq] = oacc[db][4 * jq] * f0 + o.x * f1;
-                oacc[db][4 * jq + 1] = oacc[db][4 * jq + 1] * f0 + o.y * f1;
-                oacc[db][4 * jq + 2] = oacc[db][4 * jq + 2] * f0 + o.z * f1;
-                oacc[db][4 * jq + 3] = oacc[db][4 * jq + 3] * f0 + o.w * f1;
-            }
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+            for (int jq = 0; jq < 4; ++jq)
+                *reinterpret_cast<float4*>(ebuf + (db * 4 + jq) * 256 + lane * 4) =
+                    make_float4(oacc[db][4 * jq], oacc[db][4 * jq + 1], oacc[db][4 * jq + 2], oacc[db][4 * jq + 3]);
     }
-    const float inv = lw > 0.f ? 1.0f / lw : 0.f;
+    __syncthreads();
+    if (kh == 1) return;
+    const float m1 = sM[qb * 64 + li], l1 = sM[qb * 64 + 32 + li];
+    const float mt = fmaxf(m, m1), ms = mt == -INFINITY ? 0.f : mt;
+    float f0 = fast_exp2((m - ms) * kLog2e), f1 = fast_exp2((m1 - ms) * kLog2e);
+    const float L = lw * f0 + l1 * f1, inv = L > 0.f ? 1.0f / L : 0.f;
+    f0 *= inv;
+    f1 *= inv;
 #pragma unroll
     for (int db = 0; db < NDB; ++db)
 #pragma unroll
-        for (int r = 0; r < 16; ++r) oacc[db][r] *= inv;
-    if (g == 0 && qok) a.lse[(long)bh * a.st_bhs + tq] = lw > 0.f ? m + logf(lw) : -INFINITY;
-    rows_out<T, DH>(oacc, reinterpret_cast<T*>(ebuf), lane, [&](int row, int col, uint4 v) __attribute__((always_inline)) {
-        if (qw + row < T_) *reinterpret_cast<uint4*>(reinterpret_cast<T*>(a.o) + ((long)(qw + row) * a.B + b) * ((long)a.H * DH) + (long)h * DH + col) = v;
-    });
+        for (int jq = 0; jq < 4; ++jq) {
+            const float4 o = *reinterpret_cast<const float4*>(ebuf + (db * 4 + jq) * 256 + lane * 4);
+            oacc[db][4 * jq] = oacc[db][4 * jq] * f0 + o.x * f1;
+            oacc[db][4 * jq + 1] = oacc[db][4 * jq + 1] * f0 + o.y * f1;
+            oacc[db][4 * jq + 2] = oacc[db][4 * jq + 2] * f0 + o.z * f1;
+            oacc[db][4 * jq + 3] = oacc[db][4 * jq + 3] * f0 + o.w * f1;
+        }
+    if (g == 0 && qok) a.lse[(long)bh * a.st_bhs + tq] = L > 0.f ? mt + logf(L) : -INFINITY;
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    acc_to_lds_rows<DH>(oacc, ebuf, lane);              // the wave's own block: LDS operations of one wave complete in order
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    const long EE = (long)a.H * DH;
+#pragma unroll
+    for (int p = lane; p < 32 * DH / 8; p += 64) {
+        const int row = p / (DH / 8), col = (p % (DH / 8)) * 8;
+        if (qw + row >= T_) break;
+        float v[8];
+        *reinterpret_cast<float4*>(v) = *reinterpret_cast<const float4*>(ebuf + row * EPI_LD + col);
+        *reinterpret_cast<float4*>(v + 4) = *reinterpret_cast<const float4*>(ebuf + row * EPI_LD + col + 4);
+        *reinterpret_cast<uint4*>(reinterpret_cast<T*>(a.o) + ((long)(qw + row) * a.B + b) * EE + (long)h * DH + col) = pack8<T>(v);
+    }
 }
 
 // ------------------------------------------------------------------------------------------------
@@ -767,18 +702,18 @@ void launch_attn_dkdv_long(int dtype, int head_dim, bool suffix, const AttnKeysA
     else suffix ? dkdv_long<bf16, true>(head_dim, a, s) : dkdv_long<bf16, false>(head_dim, a, s);
 }
 
-template <typename T, int QB> static void fwd_long(int hd, const AttnArgs& a, hipStream_t s) {
-    const unsigned grid = xcd_grid(a.B * a.H, (a.T + 32 * QB - 1) / (32 * QB));
+template <typename T> static void fwd_long(int hd, const AttnArgs& a, hipStream_t s) {
+    const unsigned grid = xcd_grid(a.B * a.H, (a.T + 127) / 128);
     switch (hd) {
-    case 64: attn_fwd_long_kernel<T, 64, QB><<<grid, 256, 0, s>>>(a); break;
-    case 80: attn_fwd_long_kernel<T, 80, QB><<<grid, 256, 0, s>>>(a); break;
-    case 96: attn_fwd_long_kernel<T, 96, QB><<<grid, 256, 0, s>>>(a); break;
-    default: attn_fwd_long_kernel<T, 128, QB><<<grid, 256, 0, s>>>(a); break;
+    case 64: attn_fwd_long_kernel<T, 64><<<grid, 512, 0, s>>>(a); break;
+    case 80: attn_fwd_long_kernel<T, 80><<<grid, 512, 0, s>>>(a); break;
+    case 96: attn_fwd_long_kernel<T, 96><<<grid, 512, 0, s>>>(a); break;
+    default: attn_fwd_long_kernel<T, 128><<<grid, 512, 0, s>>>(a); break;
     }
 }
-void launch_attn_fwd_long(int dtype, int head_dim, int query_blocks, const AttnArgs& a, hipStream_t s) {
-    if (dtype == TP_F16) query_blocks == 4 ? fwd_long<f16, 4>(head_dim, a, s) : fwd_long<f16, 2>(head_dim, a, s);
-    else query_blocks == 4 ? fwd_long<bf16, 4>(head_dim, a, s) : fwd_long<bf16, 2>(head_dim, a, s);
+void launch_attn_fwd_long(int dtype, int head_dim, const AttnArgs& a, hipStream_t s) {
+    if (dtype == TP_F16) fwd_long<f16>(head_dim, a, s);
+    else fwd_long<bf16>(head_dim, a, s);
 }
 
 }  // namespace tp
