@@ -141,7 +141,8 @@ typedef struct tp_gemm_desc {
     float q_scale;
     int32_t reserved;                   /* 0 = automatic; bits 0-7: tile configuration + 1, bits 8-15: k splits, bits 16-23: columns
                                            of configurations 12 and 44 (tuning, tests); bit 24: other streams' launches run beside
-                                           this one (measured plans that take less of the chip) */
+                                           this one (measured plans that take less of the chip); bit 25: no
+                                           backward follows (forms of a few rows that sum in another order) */
     int64_t q_bh_rows;                  /* rows per (b,h) block of q: 0 = T (compact [B*H,T,Dh]); a runner that
                                            keeps the queries of every slice passes L_max and q offset to row P */
     int32_t defer_reduce;               /* 1 (STORE / BIAS_RESIDUAL epilogues only): when the plan splits k
@@ -414,7 +415,8 @@ typedef struct tp_layer_desc {
                                            0: the rows lie one after the other */
 } tp_layer_desc;
 
-/* n layers in a chain (layers[i].x == layers[i-1].out).  Layers may share every buffer but x and out (forward only). */
+/* n layers in a chain (layers[i].x == layers[i-1].out).  Layers may share every buffer but x and out (forward only).  Where a
+   layer's xn and hn are one buffer no backward can follow it, and products of a few rows take forms that sum in another order. */
 size_t tp_layers_fwd_workspace_bytes(const tp_layer_desc* layers, int n);
 int tp_layers_fwd(const tp_layer_desc* layers, int n, void* workspace, size_t workspace_bytes, void* stream);
 

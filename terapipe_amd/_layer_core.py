@@ -291,14 +291,17 @@ class LayerGeometry:
             g = cls._cache[key] = cls(*key)
         return g
 
-    def pack_fwd(self, image, at, cache_len, cache_rows, params, x, k, v, base, out, over=None):
+    def pack_fwd(self, image, at, cache_len, cache_rows, params, x, k, v, base, out, over=None, forward_only=False):
         """Writes a tp_layer_desc at byte `at` of `image`.  params: the layer's 12; base: address of the forward arena; over: the
-        addresses of LINEAR_INPUTS where they are not part of it (its layout is fwd_rest then)."""
+        addresses of LINEAR_INPUTS where they are not part of it (its layout is fwd_rest then).  forward_only: both
+        LayerNorms write one buffer, which tells the library that no backward follows."""
         w_ptrs, ldw = operands(params, self.dtype)
         o = (self.fwd_rest if over else self.fwd).off
         p = {n: base + o[n] for n in o}
         if over:
             p.update(over)
+        if forward_only:
+            p["hn"] = p["xn"]
         _FWD_PACK.pack_into(image, at, self.dt, self.T, self.B, self.H, self.E, self.F, _ACTIVATIONS[self.activation],
                             cache_len, cache_rows, *w_ptrs, x, k, v, p["xn"], p["mean1"], p["rstd1"], p["q"], p["o"],
                             p["lse"], p["h"], p["mean2"], p["rstd2"], p["hn"], p["a"],
@@ -366,7 +369,8 @@ def stack_forward_only(layers, x, caches, cache_len):
     for i, (params, _, _) in enumerate(layers):
         k, v = caches[i]
         dst = out.data_ptr() if i == n - 1 else base + shared + (i & 1) * step
-        geos[i].pack_fwd(image, i * _FWD_PACK.size, cache_len, k.shape[1], params, src, k.data_ptr(), v.data_ptr(), base, dst)
+        geos[i].pack_fwd(image, i * _FWD_PACK.size, cache_len, k.shape[1], params, src, k.data_ptr(), v.data_ptr(), base, dst,
+                         forward_only=True)
         src = dst
     layers_fwd(image, n, x.device)
     return out

@@ -150,7 +150,7 @@ static const TunedPlan kTunedBeside[] = {
 #include "gemm_tuned_beside.inc"
     {-1, 0, 0, 0, 0, 0},
 };
-constexpr int kBeside = 1 << 24, kForced = 0xffffff;        // of tp_gemm_desc.reserved
+constexpr int kBeside = 1 << 24, kForced = 0xffffff;        // of tp_gemm_desc.reserved (and kNoBackward, gemm_epilogue.h)
 
 static bool small_weight(const tp_gemm_desc* d) { return (long)d->N * d->K <= (16L << 20); }
 static const TunedPlan* find_tuned(const tp_gemm_desc* d) {
@@ -349,8 +349,11 @@ static void plan_large(const tp_gemm_desc* d, int& cfg, int& ns) {
 // 16 rows on 20480 x 5120 58 us against 49.  A forced tile, and column sums, take the tile kernels.)  Up to 8 rows they take larger
 // weights too, where no k split is called for: us, 4 rows, tile kernels / these: 5120 x 5120 17.8 / 15.0, 8192 x 8192 37 / 31.6,
 // 20480 x 5120 46.6 / 37.8, 12288 x 4096 23.2 / 24.0 and without the LayerNorm before, 4096 x 16384 35.2 / 32.8; but 5120 x 20480, 1.25
-// workgroups of 16 rows to a CU, 40 / 48.
-static inline bool skinny_unsplit(const tp_gemm_desc* d) { return d->M <= 8 && (d->K <= 8192 || d->N % 4096 == 0); }
+// workgroups of 16 rows to a CU, 40 / 48.  Only where no backward follows: another order of the sums turns ReLU units near zero on or
+// off, and the weight gradients behind them move by 2e-2 in fp16.
+static inline bool skinny_unsplit(const tp_gemm_desc* d) {
+    return (d->reserved & kNoBackward) && d->M <= 8 && (d->K <= 8192 || d->N % 4096 == 0);
+}
 static inline bool runs_skinny(const tp_gemm_desc* d) {
     return d->op == TP_GEMM_NT && d->dtype != TP_F32 && d->M <= kSkinnyRows && (d->reserved & 0xff) == 0 && !d->colsum_acc &&
            (long)d->N * d->K <= (skinny_unsplit(d) ? 256L << 20 : 16L << 20);
@@ -535,7 +538,7 @@ static inline bool is_pipe_cfg(int cfg) { return cfg == 6 || cfg == 7 || (cfg >=
 template <typename T>
 static bool launch_gemm(const tp_gemm_desc* d, const GemmPlan& p, const GemmArgs& a, hipStream_t s, const SkinnyLn* ln) {
     if (runs_skinny(d)) {
-        launch_gemm_skinny(d->dtype, a, ln, s);
+        launch_gemm_skinny(d->dtype, a, d->reserved & kNoBackward, ln, s);
     } else if (runs_f32_small(d)) {
         launch_gemm_f32_small(d->op, a, s);
     } else if (p.deep) {
@@ -701,7 +704,7 @@ int gemm_of_layernorm(const tp_gemm_desc& d, const void* x, const void* gamma, c
     *taken = false;
     const int rc = validate_gemm(&d);
     if (rc != TP_OK) return rc;
-    if (!runs_skinny(&d) || !skinny_takes_ln(d.M, d.K) || d.lda != d.K || !x || !gamma || !beta || !mean || !rstd ||
+    if (!(d.reserved & kNoBackward) || !runs_skinny(&d) || !skinny_takes_ln(d.M, d.K) || d.lda != d.K || !x || !gamma || !beta || !mean || !rstd ||
         (((uintptr_t)x | (uintptr_t)gamma | (uintptr_t)beta) & 15)) return TP_OK;
     const GemmPlan p = plan_gemm(&d);
     if (p.nsplit > 1) return TP_OK;

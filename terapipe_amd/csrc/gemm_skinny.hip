@@ -89,7 +89,9 @@ __global__ __launch_bounds__(512, MB == 1 && !HALF ? 4 : 2) void gemm_skinny_ker
                 for (int m = 0; m < MB; ++m) acc[n][m] = Mfma16x16x32<T>::run(t.w[n][u], t.x[m][u], acc[n][m]);
     };
     Turn t, t1;
-    int k = kbeg + wave * STEP;
+    // a wave's turns: two beside each other with one tile of 16 rows, else a turn of all waves apart
+    constexpr int FROM = NT == 1 && !HALF ? 2 * STEP : STEP, APART = NT == 1 && !HALF ? STEP : WAVES * STEP;
+    int k = kbeg + wave * FROM;
     if constexpr (LN) {
         // 8, 4, 2 or 1 waves to a row; everything is asked for at once, the wave's first weights too
         const int share = a.M > 4 ? 1 : a.M > 2 ? 2 : a.M > 1 ? 4 : 8, row = min(wave / share, a.M - 1), part_of = wave % share;
@@ -147,11 +149,11 @@ __global__ __launch_bounds__(512, MB == 1 && !HALF ? 4 : 2) void gemm_skinny_ker
     // the next turn's loads are under way while this one's MFMAs wait for theirs
     if (!LN && k < kend) load(t, k);
     for (; k < kend; k += 2 * WAVES * STEP) {
-        const int k1 = k + WAVES * STEP;
+        const int k1 = k + APART;
         if (k1 < kend) load(t1, k1);
         use(t, k);
         if (k1 < kend) {
-            if (k1 + WAVES * STEP < kend) load(t, k1 + WAVES * STEP);
+            if (k + 2 * WAVES * STEP < kend) load(t, k + 2 * WAVES * STEP);
             use(t1, k1);
         }
     }
@@ -218,9 +220,9 @@ template <typename T, int MB, int NT, bool HALF> static void launch_tile(const G
         }
     gemm_skinny_kernel<T, MB, NT, HALF, false><<<grid, 512, 0, s>>>(a, SkinnyLn{});
 }
-template <typename T, int MB> static void launch_skinny(const GemmArgs& a, const SkinnyLn* ln, hipStream_t s) {
+template <typename T, int MB> static void launch_skinny(const GemmArgs& a, bool half, const SkinnyLn* ln, hipStream_t s) {
     const int nt = skinny_tiles(a);
-    if (MB == 1 && skinny_half(a.M, a.N)) launch_tile<T, 1, 1, true>(a, ln, s);
+    if (MB == 1 && half && skinny_half(a.M, a.N)) launch_tile<T, 1, 1, true>(a, ln, s);
     else if (nt == 4) launch_tile<T, MB, 4, false>(a, ln, s);
     else if (nt == 2) launch_tile<T, MB, 2, false>(a, ln, s);
     else launch_tile<T, MB, 1, false>(a, ln, s);
@@ -229,9 +231,9 @@ template <typename T, int MB> static void launch_skinny(const GemmArgs& a, const
 // (five chunks of 8 per lane, 64 * (8 / rows) lanes to a row)
 bool skinny_takes_ln(int M, int K) { return M <= 8 && K <= (M > 4 ? 2560 : M > 2 ? 5120 : M > 1 ? 10240 : 20480); }
 
-void launch_gemm_skinny(int dtype, const GemmArgs& a, const SkinnyLn* ln, hipStream_t s) {
-    if (dtype == TP_F16) { if (a.M <= 16) launch_skinny<f16, 1>(a, ln, s); else launch_skinny<f16, 2>(a, ln, s); }
-    else { if (a.M <= 16) launch_skinny<bf16, 1>(a, ln, s); else launch_skinny<bf16, 2>(a, ln, s); }
+void launch_gemm_skinny(int dtype, const GemmArgs& a, bool half, const SkinnyLn* ln, hipStream_t s) {
+    if (dtype == TP_F16) { if (a.M <= 16) launch_skinny<f16, 1>(a, half, ln, s); else launch_skinny<f16, 2>(a, half, ln, s); }
+    else { if (a.M <= 16) launch_skinny<bf16, 1>(a, half, ln, s); else launch_skinny<bf16, 2>(a, half, ln, s); }
 }
 
 }  // namespace tp

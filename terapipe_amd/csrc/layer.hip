@@ -1,7 +1,7 @@
 // Whole layers per call (host code only: every launch goes through the entry points of the other files).  A layer is nine
 // to fifteen launches; issued one by one from Python each costs about 11 us of host time, more than most of them run for
 // a short slice, so the chain is built here from one descriptor per layer.
-#include "common.h"
+#include "gemm_epilogue.h"
 
 #include <cmath>
 
@@ -84,6 +84,8 @@ static ForwardPlan forward_plan(const tp_layer_desc& l) {
     if (l.activation) { p.fc1.aux_out = l.z; p.fc1.ldauxo = F; }
     p.fc2 = gemm_desc(l, TP_GEMM_NT, TP_EPI_BIAS_RESIDUAL, M, E, F, l.a, l.w[W_FC2], l.out, LD_FC2);
     p.fc2.bias = l.w[B_FC2]; p.fc2.residual = l.h; p.fc2.ldr = E;
+    if (l.xn == l.hn)
+        for (tp_gemm_desc* d : {&p.qkv, &p.out, &p.fc1, &p.fc2}) d->reserved = kNoBackward;
     return p;
 }
 

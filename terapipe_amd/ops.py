@@ -174,13 +174,14 @@ def layernorm_bwd(dy, x2d, mean, rstd, gamma, dres, dgamma_acc, dbeta_acc, colsu
 
 
 def gemm(op, A, B, M, N, K, C=None, epilogue=TP_EPI_STORE, bias=None, residual=None, aux=None, aux_out=None,
-         colsum_acc=None, qkv=None, tile_cfg=None, ksplit=None, defer_reduce=False, desc_sink=None, ragged=False, beside=False):
+         colsum_acc=None, qkv=None, tile_cfg=None, ksplit=None, defer_reduce=False, desc_sink=None, ragged=False, beside=False,
+         no_backward=False):
     """Runs one GEMM.  A, B, C, residual, aux are 2-D row-major tensors (stride(1) == 1).
     qkv = dict(q, k_cache, v_cache, batch, heads, head_dim, cache_len, cache_rows, q_scale).
     tile_cfg / ksplit force a tile configuration / k-split count (tuning and tests); default automatic.
     defer_reduce (STORE / BIAS_RESIDUAL epilogues): if the plan splits k, C is left unwritten and a
     PendingReduce is returned for the LayerNorm call that consumes C; otherwise C as usual.
-    beside: launches of other streams run beside this one (tp_gemm_desc.reserved bit 24).
+    beside: launches of other streams run beside this one (tp_gemm_desc.reserved bit 24); no_backward: none follows (bit 25).
     desc_sink: a list that receives the call's descriptor (the one a recorded replay re-issues), for callers
     that re-point C before a replay.
     ragged: N of NT, k of NN and M of TN may be no multiple of 8; what lies in C's (NT) or A's rows from there to the
@@ -213,6 +214,8 @@ def gemm(op, A, B, M, N, K, C=None, epilogue=TP_EPI_STORE, bias=None, residual=N
         d.reserved = ((tile_cfg + 1) if tile_cfg is not None else 0) | ((ksplit or 0) << 8)
     if beside:
         d.reserved |= 1 << 24
+    if no_backward:
+        d.reserved |= 1 << 25
     if desc_sink is not None:
         desc_sink.append(d)
     lib = _lib.load()

@@ -15,17 +15,19 @@ DEV = "cuda"
     (1, 8, 8), (8, 24, 72), (5, 1000, 40), (3, 2048, 2048), (8, 2048, 4104), (7, 2056, 1032), (1, 520, 8200), (8, 1024, 16384),
     (4, 6144, 2056), (2, 8200, 520), (6, 20488, 968), (8, 4096, 8200), (1, 7680, 2560), (9, 2048, 2056), (16, 1000, 1032), (17, 264, 2048),
     (32, 4104, 264)], ids=str)
-def test_products(M, N, K, dtype):
+@pytest.mark.parametrize("no_backward", [False, True])
+def test_products(M, N, K, no_backward, dtype):
     from terapipe_amd import ops
     g = torch.Generator(device=DEV).manual_seed(M + N + K)
     rnd = lambda *s: torch.randn(*s, generator=g, device=DEV).to(dtype)
     A, B, bias, res = rnd(M, K), rnd(N, K) * K ** -0.5, rnd(N), rnd(M, N)
     want = A.double() @ B.double().t() + bias.double()
     C = torch.full((M + 1, N), 7.0, device=DEV, dtype=dtype)
-    ops.gemm(ops.TP_GEMM_NT, A, B, M, N, K, C=C[:M], epilogue=ops.TP_EPI_BIAS, bias=bias)
+    ops.gemm(ops.TP_GEMM_NT, A, B, M, N, K, C=C[:M], epilogue=ops.TP_EPI_BIAS, bias=bias, no_backward=no_backward)
     assert_close(C[:M], want, dtype, "bias")
     assert (C[M] == 7).all()
-    ops.gemm(ops.TP_GEMM_NT, A, B, M, N, K, C=C[:M], epilogue=ops.TP_EPI_BIAS_RESIDUAL, bias=bias, residual=res)
+    ops.gemm(ops.TP_GEMM_NT, A, B, M, N, K, C=C[:M], epilogue=ops.TP_EPI_BIAS_RESIDUAL, bias=bias, residual=res,
+             no_backward=no_backward)
     assert_close(C[:M], want + res.double(), dtype, "bias and residual")
 
 
