@@ -229,7 +229,7 @@ typedef struct tp_attn_desc {
     int32_t reserved2;                  /* tuning, tests.  bit 1 / bit 2: force the eight-wave / the four-wave form of the
                                            16-bit forward kernel; bit 3 / bit 4: force its workgroups of 32 / of 64 queries
                                            (64 needs T >= 64); bit 5 / bit 6: force / forbid those of 128 queries that
-                                           share their key tiles, in the backward those of 128 queries and
+                                           share their key tiles, in the backward those of 64 or 128 queries and
                                            of 128 keys.  bit 7: fp32 without the workgroups of 32 rows whose
                                            waves share the other axis */
     int64_t q_bh_rows;                  /* rows per (b,h) block of q: 0 = T; see tp_gemm_desc.q_bh_rows */
@@ -250,7 +250,7 @@ size_t tp_attn_fwd_workspace_bytes(const tp_attn_desc* d);
 int tp_attn_prefix_fwd(const tp_attn_desc* d, void* workspace, size_t workspace_bytes, void* stream);
 size_t tp_attn_bwd_workspace_bytes(const tp_attn_desc* d);
 int tp_attn_prefix_bwd(const tp_attn_desc* d, void* workspace, size_t workspace_bytes, void* stream);
-/* Whether that call takes dQ by workgroups of 128 queries, and dK / dV by workgroups of 128 keys, that share the tiles they
+/* Whether that call takes dQ by workgroups of 64 or 128 queries, and dK / dV by workgroups of 128 keys, that share the tiles they
  * stream.  Host code only; for tuning, tests and logs. */
 int tp_attn_bwd_forms(const tp_attn_desc* d, int* shared_queries, int* shared_keys);
 

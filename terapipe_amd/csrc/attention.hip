@@ -1851,18 +1851,25 @@ static bool shares_tiles(const tp_attn_desc* d) {
     return d->T >= 128 && enough;
 }
 
-// dQ by workgroups of 128 queries, dK / dV of a slice's keys by those of 128, eight waves on shared tiles.  The forms for slices take 32
-// rows a workgroup and one fits a CU, so what counts is the number of their rounds: three full ones and more go to the shared form.
-// Head dimensions 64 / 80 / 128, 8 to 160 (batch, head) pairs, rows 128 to 2048 of up to 2048 positions, against those: calls taken
-// gain 1.20 / 1.66 / 1.52 in the mean for dQ and 1.44 / 1.52 / 1.53 for dK / dV, 0.97 to 2.0 each; between two rounds and three 0.7 to 1.8, up
-// to two mostly 0.5 to 1.0.  The offsets of 64 rows of dO are 32-bit.
+// dK / dV of a slice's keys by workgroups of 128 keys, eight waves on shared tiles.  The form for slices takes 32 keys a
+// workgroup and one fits a CU, so what counts is the number of its rounds: three full ones and more go to the shared form.
+// Head dimensions 64 / 80 / 128, 8 to 160 (batch, head) pairs, rows 128 to 2048 of up to 2048 positions, against it: calls taken
+// gain 1.44 / 1.52 / 1.53 in the mean, 0.97 to 2.0 each; between two rounds and three 0.7 to 1.8, up to two mostly 0.5 to 1.0.  The
+// offsets of 64 rows of dO are 32-bit.
 static bool shares_bwd(int batch, int heads, int head_dim, int rows) {
     return rows >= 128 && (long)batch * heads * ((rows + 31) / 32) >= 3 * kNumCU && (long)batch * heads * head_dim <= (1L << 24);
 }
+// dQ by workgroups of 64 or 128 queries on shared tiles, from 160 of 64 on (256 at head dimension 64); where the longest of a sequence's
+// own rows sees more than 1024 keys and no context evens them out, from twice as many.  us, the form with 32 queries a workgroup / these, fp16:
+// 40 pairs of 128, 256 queries after 768 (160 workgroups) 26 / 20; 20 of 128, 512 after 512 (160) 24 / 21; 16 of 128, 640 after 1400
+// (160) 36 / 33; 200 of 128, 64 (200) 13 / 9; 40 of 128, 512 after 1536 (320) 59 / 44; 10 of 128, 2048 (320) 56 / 40; 100 of 64, 192 after 320
+// (300) 16 / 12; 12 of 64, 2048 (384) 26 / 23; not taken: 8 of 128, 1280 (160) 17 / 22; 40 of 128, 192 after 1728 (120) 22 / 30; 64 of
+// 128, 128 after 128 (128) 9.0 / 10.8; 25 of 64, 512 after 512 (200) 12.0 / 12.6.
 static bool shares_queries(const tp_attn_desc* d) {
     if (d->dtype == TP_F32 || !tiled16(d->head_dim)) return false;
     if (d->reserved2 & (32 | 64)) return d->reserved2 & 32;
-    return shares_bwd(d->batch, d->heads, d->head_dim, d->T);
+    const long w = (long)d->batch * d->heads * ((d->T + 63) / 64), least = d->head_dim > 64 ? 160 : 256;
+    return d->T >= 64 && w >= (d->cache_len >= d->T || d->cache_len + d->T <= 1024 ? least : 2 * least);
 }
 // dK / dV with gradient caches: the other form gives 32 keys to ONE wave, which walks over all queries alone.  Above head
 // dimension 64 the shared form is faster (2 to 1152 pairs, 1 to 1024 queries, up to 2048 keys): 0.96 to 3.1 times, 40 pairs

@@ -9,6 +9,24 @@ template <typename T> __device__ __forceinline__ uint4 pack8v(float8v v) {
     return __builtin_bit_cast(uint4, __builtin_convertvector(v, vec8_t<T>));
 }
 
+template <typename T> using vec2_t = T __attribute__((ext_vector_type(2)));
+typedef float float2v __attribute__((ext_vector_type(2)));
+template <typename T> __device__ __forceinline__ unsigned pack2(float a, float b) {
+    const float2v two = {a, b};
+    return __builtin_bit_cast(unsigned, __builtin_convertvector(two, vec2_t<T>));
+}
+
+// As xcd_map, for nblocks blocks that start longest first: where all of an XCD's workgroups fit its 32 CUs in twos, the second of a
+// CU is as short as the first is long.
+__device__ __forceinline__ bool xcd_map_causal(int BH, int nblocks, int& bh, int& blk) {
+    const int id = blockIdx.x, nbh8 = (BH + 7) >> 3, n = nbh8 * nblocks;
+    int slot = id >> 3;
+    if (n <= 64 && slot >= 32) slot = n + 31 - slot;
+    bh = (id & 7) + 8 * (slot % nbh8);
+    blk = slot / nbh8;
+    return bh < BH;
+}
+
 // ------------------------------------------------------------------------------------------------
 // Forward.  A workgroup of eight waves owns 128 queries of one (batch, head): four blocks of 32, each by two waves that
 // take one half of every key tile and merge at the end.  A tile of 128 keys of K and V is loaded once for all of them, into
@@ -246,70 +264,68 @@ __global__ __launch_bounds__(512) void attn_fwd_long_kernel(AttnArgs a) {
 }
 
 // ------------------------------------------------------------------------------------------------
-// dQ of 128 queries, and their delta = rowsum(dO * O) for the dK / dV kernel that follows on the stream: the partition of the
-// forward.  Per 32 x 32 block three products (K Q^T, V dO^T, K^T dS^T) and three fetches of 8 KB out of LDS against about 600
-// cycles of vector ALU.  Causal, 2048 positions: 40 heads of 128 151 -> 95 us, 96 of 128 365 -> 212, 32 of 80 108 -> 54; 64 heads
-// of 64 at 1024 39 -> 29.
+// dQ of 32 * QB queries, and their delta = rowsum(dO * O) for the dK / dV kernel that follows on the stream: blocks of 32
+// queries, each by one of four waves (QB = 4) or by two that take one half of every key tile and add their sums at the end (QB = 2).
+// K and V tiles lie in rings of 72 or 80 KB at most, so that two workgroups (three at head dimension 64) share a CU: the waves of a
+// SIMD belong to different workgroups, and no barrier keeps them in step.
+// A wave's work on a tile is one straight line of three rows of MFMAs, each beside the vector operations that it leaves the issue slots
+// for and the LDS fetches of those a few MFMAs later: V dO^T | exponentials; the NEXT tile's K Q^T | dS; dQ += K^T dS.
+// What bounds it: the waits between a tile's loads, LDS fetches and MFMAs that two waves a SIMD cover only in part (24 MFMAs of 32
+// clocks and about 900 clocks of issue in 1750 per block of 32 x 32, 96 heads of 128); QB = 4 has three tiles of 32 keys under way where QB = 2
+// has one of 64, and pulls half the bytes.
+// Measured (fp16, causal, 2048 positions, us; before: eight waves on one ring of 128 KB, phases in step): 40 heads of 128 91 -> 76, 96 of
+// 128 205 -> 170, 16 of 128 51 -> 43 (blocks of 64), 12 of 64 28 -> 23, 32 of 80 49 -> 50; 64 of 64 at 1024 24.4 -> 23.4, 300 of 64 at 256
+// 22.6 -> 17.7; 40 of 128, 512 after 1536 59 -> 44.  Two of the old workgroups on a CU at 64 (128 registers, spills): 24 -> 38.
 // ------------------------------------------------------------------------------------------------
-template <typename T, int DH>
-__global__ __launch_bounds__(512) void attn_dq_long_kernel(AttnArgs a) {
+template <typename T, int DH, int QB>
+__global__ __launch_bounds__(256, DH <= 64 ? 3 : 2) void attn_dq_long_kernel(AttnArgs a) {
     typedef Elem<T> E;
-    constexpr int NDB = (DH + 31) / 32, NKS = DH / 16, PITCH = tile_pitch<DH>(), CPR = PITCH / 8;
-    constexpr int NB = 2;                                   // 32-key blocks of a tile per wave
-    constexpr int KT = 64 * NB, TILE = KT * PITCH, STAGE = 2 * TILE;
-    constexpr int NLD = KT * CPR / 512;                     // loads per K or V tile and lane
+    constexpr int NDB = (DH + 31) / 32, NKS = DH / 16, NPV = 2 * NDB, PITCH = tile_pitch<DH>(), CPR = PITCH / 8;
+    constexpr int KH = 4 / QB, KT = 32 * KH, TILE = KT * PITCH * 2;     // waves that share a query block's keys; (bytes)
+    constexpr int AHEAD = QB == 4 ? 3 : 1, RK = AHEAD + 2, RV = AHEAD + 1, VRING = RK * TILE;      // tiles under way; slots
+    constexpr int NLD = KT * CPR / 256;                     // loads per K or V tile and lane
+    constexpr int W = DH == 128 || DH == 64 ? 6 : 9;        // fragments under way
+    constexpr bool FOLD = DH > 64;                          // V dO^T starts at -delta (16 registers, which 64 does not have)
     constexpr int EPI_LD = NDB * 32 + 4;
-    constexpr int RING_BYTES = 2 * STAGE * 2, EPI_BYTES = 4 * 32 * EPI_LD * 4;
+    constexpr int RING_BYTES = (RK + RV) * TILE, EPI_BYTES = QB * 32 * EPI_LD * 4;
     __shared__ __attribute__((aligned(16))) unsigned char smem[RING_BYTES > EPI_BYTES ? RING_BYTES : EPI_BYTES];
-    T* ring = reinterpret_cast<T*>(smem);
 
     const int tid = threadIdx.x, lane = tid & 63, g = lane >> 5, li = lane & 31;
-    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), qb = wave & 3, kh = wave >> 2;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), qb = wave % QB, kh = wave / QB;
     int bh, blk;
-    if (!xcd_map(a.B * a.H, bh, blk)) return;
+    if (!xcd_map_causal(a.B * a.H, (a.T + 32 * QB - 1) / (32 * QB), bh, blk)) return;
     const int b = bh / a.H, h = bh - b * a.H;
     const int T_ = a.T, P = a.P, S = a.P + a.T;
     const long EE = (long)a.H * DH;
-    const int q0 = ((T_ + 127) / 128 - 1 - blk) * 128;      // the blocks with the longest key range start first
-    const int qw = q0 + 32 * qb, tq = qw + li, tr = min(tq, T_ - 1);
+    const int q0 = ((T_ + 32 * QB - 1) / (32 * QB) - 1 - blk) * (32 * QB);      // the blocks with the longest key range start first
+    const int qw = q0 + 32 * qb, tq = qw + li, tr_row = min(tq, T_ - 1);
     const bool qok = tq < T_;
-    const int nt = (P + min(T_, q0 + 128) + KT - 1) / KT;   // tiles of the workgroup
-    const int key_end = qw < T_ ? P + min(T_, qw + 32) : 0; // keys this wave's queries see
+    const int nt = (P + min(T_, q0 + 32 * QB) + KT - 1) / KT;    // tiles of the workgroup
 
-    unsigned koff[NLD];
-#pragma unroll
-    for (int i = 0; i < NLD; ++i) {
-        const int p = i * 512 + tid, r = p / CPR, lc = (p % CPR) ^ swz16<PITCH>(r);
-        koff[i] = lc < DH / 8 ? (unsigned)(r * DH * 2 + lc * 16) : kNoChunk;
-    }
+    // the lane's chunk of a tile's first rows and that of row S - 1 (the swizzle repeats every 16 rows: the same column in each load)
+    const int lr = tid / CPR, lc = (tid % CPR) ^ swz16<PITCH>(lr);
+    const unsigned koff = (unsigned)(lr * DH * 2 + lc * 16), klast = (unsigned)((S - 1) * DH * 2 + lc * 16);
+    const bool chunk = DH == PITCH || lc < DH / 8;
     const char* Kb = uniform_ptr(reinterpret_cast<const char*>(reinterpret_cast<const T*>(a.kc) + (long)bh * a.cache_rows * DH));
     const char* Vb = uniform_ptr(reinterpret_cast<const char*>(reinterpret_cast<const T*>(a.vc) + (long)bh * a.cache_rows * DH));
     const unsigned lds0 = lds_addr(smem) + wave * 1024;
-    auto issue = [&](int stage, int tile) {                 // (rows at or past S as in the forward)
-        const unsigned dst = lds0 + (unsigned)(stage * STAGE * 2);
-        const int row0 = tile * KT;
+    // tile t of K or V to where it belongs; rows at or past S are clamped to row S - 1: finite data, and every such key is masked
+    auto issue = [&](const char* base, unsigned dst, int tile) __attribute__((always_inline)) {
+        const unsigned row = (unsigned)(tile * KT) * (DH * 2);
 #pragma unroll
-        for (int which = 0; which < 2; ++which) {
-            const char* base = which ? Vb : Kb;
-            if (row0 + KT <= S) {
-                const char* sb = base + (long)row0 * (DH * 2);
-#pragma unroll
-                for (int i = 0; i < NLD; ++i) load_chunk_lds<DH>(koff[i], sb, dst + which * TILE * 2 + i * 8192);
-            } else {
-#pragma unroll
-                for (int i = 0; i < NLD; ++i) {
-                    const int p = i * 512 + tid, r = p / CPR, lc = (p % CPR) ^ swz16<PITCH>(r);
-                    const unsigned off = lc < DH / 8 ? (unsigned)(min(row0 + r, S - 1) * DH * 2 + lc * 16) : kNoChunk;
-                    load_chunk_lds<DH>(off, base, dst + which * TILE * 2 + i * 8192);
-                }
-            }
-        }
+        for (int i = 0; i < NLD; ++i)
+            if (chunk) dma16_saddr_lds(min(row + (unsigned)(i * (256 / CPR) * DH * 2) + koff, klast), base, lds0 + dst + i * 4096);
     };
-    issue(0, 0);
+    issue(Kb, 0, 0);
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) {
+        issue(Vb, VRING + i * TILE, i);
+        issue(Kb, (i + 1) * TILE, i + 1);
+    }
 
     typename E::opnd_t qreg[NKS], doreg[NKS];
-    const long orow = ((long)tr * a.B + b) * EE + (long)h * DH;
-    load_row_operands<T, DH>(qreg, reinterpret_cast<const T*>(a.q) + (long)bh * a.q_bhs + (long)tr * DH, qok, g);
+    const long orow = ((long)tr_row * a.B + b) * EE + (long)h * DH;
+    load_row_operands<T, DH>(qreg, reinterpret_cast<const T*>(a.q) + (long)bh * a.q_bhs + (long)tr_row * DH, qok, g);
     load_row_operands<T, DH>(doreg, reinterpret_cast<const T*>(a.d_o) + orow, qok, g);
     float delta = 0.f;
     {
@@ -327,96 +343,140 @@ __global__ __launch_bounds__(512) void attn_dq_long_kernel(AttnArgs a) {
     }
     const float lneg = qok ? -a.lse[(long)bh * a.st_bhs + tq] * kLog2e : 0.f;
 
-    int okm[NKS], otr[NDB][2];          // element offsets of the lane's fetches inside a K tile, its first block
+    // LDS addresses of the lane's fetches, which go round the rings: km in the next tile's K, vm in this one's V, tr in this one's K
+    unsigned km[NKS], tr[NDB][2];
 #pragma unroll
-    for (int ks = 0; ks < NKS; ++ks) okm[ks] = km_offset<T, PITCH>(kh * 32 * NB + li, ks * 16, lane);
+    for (int ks = 0; ks < NKS; ++ks) km[ks] = lds_addr(smem) + km_offset<T, PITCH>(kh * 32 + li, ks * 16, lane) * 2;
 #pragma unroll
-    for (int db = 0; db < NDB; ++db) tr_offsets<T, PITCH, true>(kh * 32 * NB, db * 32, lane, otr[db][0], otr[db][1]);
+    for (int db = 0; db < NDB; ++db) {
+        int o0, o1;
+        tr_offsets<T, PITCH, true>(kh * 32, db * 32, lane, o0, o1);
+        tr[db][0] = lds_addr(smem) + o0 * 2;
+        tr[db][1] = lds_addr(smem) + o1 * 2;
+    }
+    auto km_from = [&](unsigned off, int ks) __attribute__((always_inline)) {
+        typedef unsigned uint4v __attribute__((ext_vector_type(4)));
+        return __builtin_bit_cast(uint4, *(__attribute__((address_space(3))) const uint4v*)(km[ks] + off));
+    };
+    auto transposed = [&](unsigned off, int i) __attribute__((always_inline)) {
+        typedef __attribute__((address_space(3))) short4v* P3;
+        const unsigned o = off + i / NDB * 16 * PITCH * 2;
+        const uint2 lo = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((P3)(tr[i % NDB][0] + o)));
+        const uint2 hi = __builtin_bit_cast(uint2, __builtin_amdgcn_ds_read_tr16_b64_v4i16((P3)(tr[i % NDB][1] + o)));
+        return make_uint4(lo.x, lo.y, hi.x, hi.y);
+    };
 
-    float16v dq[NDB];
+    float16v dq[NDB], s, x, d, minus_delta;     // s: scores of the next tile; x: those of this one, then P and dS
 #pragma unroll
-    for (int db = 0; db < NDB; ++db)
+    for (int r = 0; r < 16; ++r) minus_delta[r] = -delta;
+    const float16v zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int r = 0; r < 16; ++r) dq[db][r] = 0.f;
-
-    auto step = [&](auto sc, int t) __attribute__((always_inline)) {
-        constexpr int st = decltype(sc)::value;
-        wait_vmcnt<0>();                    // this wave's part of tile t has landed
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // and its reads of tile t - 1 are back
+    for (int db = 0; db < NDB; ++db) dq[db] = zero;
+    auto barrier = [&](auto n) __attribute__((always_inline)) {
+        wait_vmcnt<decltype(n)::value>();
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
-        if (t + 1 < nt) issue(st ^ 1, t + 1);
+    };
+    barrier(std::integral_constant<int, 0>());
+    s = zero;
 #pragma unroll
-        for (int n = 0; n < NB; ++n) {
-            const int key0 = t * KT + (kh * NB + n) * 32, so = st * STAGE + n * 32 * PITCH;
-            if (key0 >= key_end) break;     // wave-uniform
-            typename E::opnd_t kf[NKS], vf[NKS];
+    for (int ks = 0; ks < NKS; ++ks) s = E::mfma(km_from(0, ks), qreg[ks], s);
+
+    unsigned kslot = 0, vslot = 0;      // byte offsets of tile t's slots
+    for (int t = 0; t < nt; ++t) {
+        // this wave's loads of K(t + 1) and V(t) have landed, and its reads of the tiles before t are back
+        if (t) barrier(std::integral_constant<int, (AHEAD - 1) * 2 * NLD>());
+        const unsigned knext = kslot == (RK - 1) * TILE ? 0 : kslot + TILE;
+        issue(Vb, VRING + (vslot ? vslot : RV * TILE) - TILE, t + AHEAD);
+        issue(Kb, (kslot ? kslot : RK * TILE) - TILE, t + AHEAD + 1);
+        const int key0 = t * KT + kh * 32;
+        x = s;
+        if (key0 + 31 > P + qw) {       // wave-uniform: the block touches the causal boundary, or lies beyond it
+            const int end = P + tq - key0 - acc_row(0, g);
 #pragma unroll
-            for (int ks = 0; ks < NKS; ++ks) kf[ks] = load_km<T>(ring + so + okm[ks]);
+            for (int j = 0; j < 16; ++j)
+                if (acc_row(j, 0) > end) x[j] = -INFINITY;
+        }
+        // the fragments of the tile's NKS + NKS + NPV MFMAs in their order, W of them under way
+        constexpr int NF = 2 * NKS + NPV;
+        uint4 f[NF];
+        auto fetch = [&](int i) __attribute__((always_inline)) {
+            if (i < NKS) f[i] = km_from(VRING + vslot, i);
+            else if (i < 2 * NKS) f[i] = km_from(knext, i - NKS);
+            else if (i < NF) f[i] = transposed(kslot, i - 2 * NKS);
+        };
 #pragma unroll
-            for (int ks = 0; ks < NKS; ++ks) vf[ks] = load_km<T>(ring + so + TILE + okm[ks]);
-            __builtin_amdgcn_sched_barrier(0);
-            float16v s, d;
+        for (int i = 0; i < W; ++i) fetch(i);
+        unsigned dw[8];
+        __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-            for (int r = 0; r < 16; ++r) { s[r] = 0.f; d[r] = 0.f; }
+        for (int k = 0; k < NKS; ++k) {
+            d = E::mfma(f[k], doreg[k], k == 0 ? (FOLD ? minus_delta : zero) : d);
+            fetch(k + W);
 #pragma unroll
-            for (int ks = 0; ks < NKS; ++ks) s = E::mfma(kf[ks], qreg[ks], s);
-#pragma unroll
-            for (int ks = 0; ks < NKS; ++ks) d = E::mfma(vf[ks], doreg[ks], d);
-            __builtin_amdgcn_sched_barrier(0);
-            uint4 kt[2][NDB];
-#pragma unroll
-            for (int hs = 0; hs < 2; ++hs)
-#pragma unroll
-                for (int db = 0; db < NDB; ++db)
-                    kt[hs][db] = load_tr<T>(ring + so + otr[db][0] + hs * 16 * PITCH, ring + so + otr[db][1] + hs * 16 * PITCH);
-            __builtin_amdgcn_sched_barrier(0);
-            if (key0 + 31 > P + qw) {       // wave-uniform: the block touches the causal boundary
-#pragma unroll
-                for (int j = 0; j < 16; ++j)
-                    if (key0 + acc_row(j, g) > P + tq) s[j] = -INFINITY;
+            for (int j = k * 16 / NKS; j < (k + 1) * 16 / NKS; ++j) {
+                x[j] = fast_exp2(fmaf(x[j], kLog2e, lneg));
+                asm volatile("" : "+v"(x[j]));
             }
-            float8v e0, e1;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                e0[j] = fast_exp2(fmaf(s[j], kLog2e, lneg)) * (d[j] - delta);
-                e1[j] = fast_exp2(fmaf(s[j + 8], kLog2e, lneg)) * (d[j + 8] - delta);
-            }
-            const uint4 p[2] = {pack8v<T>(e0), pack8v<T>(e1)};
-#pragma unroll
-            for (int hs = 0; hs < 2; ++hs)
-#pragma unroll
-                for (int db = 0; db < NDB; ++db) dq[db] = E::mfma(kt[hs][db], p[hs], dq[db]);
             __builtin_amdgcn_sched_barrier(0);
         }
-    };
-    for (int t = 0; t < nt; t += 2) {
-        step(std::integral_constant<int, 0>(), t);
-        if (t + 1 < nt) step(std::integral_constant<int, 1>(), t + 1);
+#pragma unroll
+        for (int k = 0; k < NKS; ++k) {
+            s = E::mfma(f[NKS + k], qreg[k], k == 0 ? zero : s);
+            fetch(NKS + k + W);
+            if (k > 0) {                // (the last of V dO^T is under way beside the first)
+#pragma unroll
+                for (int j = (k - 1) * 16 / (NKS - 1); j < k * 16 / (NKS - 1); ++j) {
+                    x[j] *= FOLD ? d[j] : d[j] - delta;
+                    if (j & 1) {
+                        dw[j / 2] = pack2<T>(x[j - 1], x[j]);
+                        asm volatile("" : "+v"(dw[j / 2]));
+                    }
+                }
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        const uint4 ds[2] = {make_uint4(dw[0], dw[1], dw[2], dw[3]), make_uint4(dw[4], dw[5], dw[6], dw[7])};
+#pragma unroll
+        for (int i = 0; i < NPV; ++i) {
+            dq[i % NDB] = E::mfma(f[2 * NKS + i], ds[i / NDB], dq[i % NDB]);
+            fetch(2 * NKS + i + W);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        kslot = knext;
+        vslot = vslot == (RV - 1) * TILE ? 0 : vslot + TILE;
     }
-    __syncthreads();            // every wave is done with the ring
+    wait_vmcnt<0>();            // (the loads past the last tile)
+    __syncthreads();            // every wave is done with the rings
 
     float* ebuf = reinterpret_cast<float*>(smem) + qb * 32 * EPI_LD;
-    if (kh == 1) {
+    if constexpr (KH > 1) {
+        if (kh == 1) {
+#pragma unroll
+            for (int db = 0; db < NDB; ++db)
+#pragma unroll
+                for (int jq = 0; jq < 4; ++jq)
+                    *reinterpret_cast<float4*>(ebuf + (db * 4 + jq) * 256 + lane * 4) =
+                        make_float4(dq[db][4 * jq], dq[db][4 * jq + 1], dq[db][4 * jq + 2], dq[db][4 * jq + 3]);
+        }
+        __syncthreads();
+        if (kh == 1) return;
 #pragma unroll
         for (int db = 0; db < NDB; ++db)
 #pragma unroll
-            for (int jq = 0; jq < 4; ++jq)
-                *reinterpret_cast<float4*>(ebuf + (db * 4 + jq) * 256 + lane * 4) =
-                    make_float4(dq[db][4 * jq], dq[db][4 * jq + 1], dq[db][4 * jq + 2], dq[db][4 * jq + 3]);
+            for (int jq = 0; jq < 4; ++jq) {
+                const float4 o = *reinterpret_cast<const float4*>(ebuf + (db * 4 + jq) * 256 + lane * 4);
+                dq[db][4 * jq] += o.x;
+                dq[db][4 * jq + 1] += o.y;
+                dq[db][4 * jq + 2] += o.z;
+                dq[db][4 * jq + 3] += o.w;
+            }
     }
-    __syncthreads();
-    if (kh == 1) return;
 #pragma unroll
     for (int db = 0; db < NDB; ++db)
 #pragma unroll
-        for (int jq = 0; jq < 4; ++jq) {
-            const float4 o = *reinterpret_cast<const float4*>(ebuf + (db * 4 + jq) * 256 + lane * 4);
-            dq[db][4 * jq] = (dq[db][4 * jq] + o.x) * a.qscale;
-            dq[db][4 * jq + 1] = (dq[db][4 * jq + 1] + o.y) * a.qscale;
-            dq[db][4 * jq + 2] = (dq[db][4 * jq + 2] + o.z) * a.qscale;
-            dq[db][4 * jq + 3] = (dq[db][4 * jq + 3] + o.w) * a.qscale;
-        }
+        for (int r = 0; r < 16; ++r) dq[db][r] *= a.qscale;
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
     acc_to_lds_rows<DH>(dq, ebuf, lane);                // the wave's own block: LDS operations of one wave complete in order
     asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
@@ -431,18 +491,24 @@ __global__ __launch_bounds__(512) void attn_dq_long_kernel(AttnArgs a) {
     }
 }
 
-template <typename T> static void dq_long(int hd, const AttnArgs& a, hipStream_t s) {
-    const unsigned grid = xcd_grid(a.B * a.H, (a.T + 127) / 128);
+template <typename T, int QB> static void dq_long(int hd, const AttnArgs& a, hipStream_t s) {
+    const unsigned grid = xcd_grid(a.B * a.H, (a.T + 32 * QB - 1) / (32 * QB));
     switch (hd) {
-    case 64: attn_dq_long_kernel<T, 64><<<grid, 512, 0, s>>>(a); break;
-    case 80: attn_dq_long_kernel<T, 80><<<grid, 512, 0, s>>>(a); break;
-    case 96: attn_dq_long_kernel<T, 96><<<grid, 512, 0, s>>>(a); break;
-    default: attn_dq_long_kernel<T, 128><<<grid, 512, 0, s>>>(a); break;
+    case 64: attn_dq_long_kernel<T, 64, QB><<<grid, 256, 0, s>>>(a); break;
+    case 80: attn_dq_long_kernel<T, 80, QB><<<grid, 256, 0, s>>>(a); break;
+    case 96: attn_dq_long_kernel<T, 96, QB><<<grid, 256, 0, s>>>(a); break;
+    default: attn_dq_long_kernel<T, 128, QB><<<grid, 256, 0, s>>>(a); break;
     }
 }
 void launch_attn_dq_long(int dtype, int head_dim, const AttnArgs& a, hipStream_t s) {
-    if (dtype == TP_F16) dq_long<f16>(head_dim, a, s);
-    else dq_long<bf16>(head_dim, a, s);
+    // Blocks of 128 queries once they give every CU one and some a second (at head dimension 64, with three to a CU, two each); below,
+    // blocks of 64 spread the longest rows of keys over more CUs.  us, 64 / 128 queries: 48 heads of 128 at 1024 (384 blocks of 128)
+    // 40 / 36, 40 of 128, 512 after 1536 (160) 44 / 49, 16 of 128 at 2048 (256) 43 / 55; 64 of 64 at 1024 (512) 24.5 / 23.4, 25 of 64 at
+    // 2048 (400) 35 / 39.
+    const long w = (long)a.B * a.H * ((a.T + 127) / 128);
+    const bool wide = head_dim > 64 ? w > 256 : w >= 512;
+    if (dtype == TP_F16) wide ? dq_long<f16, 4>(head_dim, a, s) : dq_long<f16, 2>(head_dim, a, s);
+    else wide ? dq_long<bf16, 4>(head_dim, a, s) : dq_long<bf16, 2>(head_dim, a, s);
 }
 
 // ------------------------------------------------------------------------------------------------

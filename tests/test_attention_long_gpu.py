@@ -108,3 +108,54 @@ def test_short_calls_of_a_second_round_keep_the_form_with_a_wave_per_key_block(p
     keys = ctypes.c_int(-1)
     assert L.load().tp_attn_bwd_forms(ctypes.byref(d), None, ctypes.byref(keys)) == 0
     assert keys.value == want
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=str)
+@pytest.mark.parametrize("D", [64, 80, 96, 128])
+@pytest.mark.parametrize("B,H,T,P", [(1, 3, 1, 0), (2, 1, 63, 2), (1, 2, 64, 31), (1, 2, 65, 95), (1, 1, 193, 500), (3, 13, 128, 0), (2, 300, 33, 5),
+                                     (1, 520, 65, 0), (2, 260, 97, 70)], ids=str)
+def test_dq(B, H, T, P, D, dtype):
+    """Blocks of 64 and (the last three) of 128 queries: those that end inside a block, key tiles that end inside or that only one of
+    two waves sees, fewer tiles than the rings have slots; 39 pairs of two blocks go in the paired order of one round."""
+    from terapipe_amd import _lib as L
+    from terapipe_amd import ops
+    S, BH, sc = P + T, B * H, D ** -0.5
+    g = torch.Generator(device=DEV).manual_seed(T + 7 * P + D)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    q, k, v, do = (rnd(BH, T, D) * sc).to(dtype), rnd(BH, S + 3, D).to(dtype), rnd(BH, S + 3, D).to(dtype), rnd(T, B, H * D).to(dtype)
+    k[:, S:], v[:, S:] = float("nan"), float("nan")       # rows past the slice are never used
+    qd, kd, vd = (t.double() for t in (q, k[:, :S].contiguous(), v[:, :S].contiguous()))
+    s = torch.bmm(qd, kd.transpose(1, 2).contiguous())
+    s = s.masked_fill(torch.arange(S, device=DEV)[None] > P + torch.arange(T, device=DEV)[:, None], float("-inf"))
+    p, o, lse = torch.softmax(s, -1), torch.bmm(torch.softmax(s, -1), vd), torch.logsumexp(s, -1)
+    dod = do.double().view(T, B, H, D).permute(1, 2, 0, 3).reshape(BH, T, D)
+    delta = (o * dod).sum(-1)
+    want = torch.bmm(p * (torch.bmm(dod, vd.transpose(1, 2).contiguous()) - delta[..., None]), kd) * sc
+    o16 = o.view(B, H, T, D).permute(2, 0, 1, 3).reshape(T, B, H * D).to(dtype).contiguous()
+    got_delta, lse32 = torch.full((BH, T), float("nan"), device=DEV), lse.float()
+    dqkv = torch.full((T * B, 3 * H * D), float("nan"), device=DEV, dtype=dtype)
+    d = ops._attn_desc(q, k, v, o16, lse32, B, H, D, T, P, sc)
+    d.dq_only, d.reserved2, d.grad_cache_dtype = 1, 32, d.dtype
+    d.d_o, d.delta, d.dqkv = do.data_ptr(), got_delta.data_ptr(), dqkv.data_ptr()
+    L.check(L.load().tp_attn_prefix_bwd(ctypes.byref(d), None, 0, ops._stream()), "tp_attn_prefix_bwd")
+    part = dqkv.view(T * B, H, 3, D)
+    assert_close(part[:, :, 0], want.view(B, H, T, D).permute(2, 0, 1, 3).reshape(-1, H, D), dtype, "dq")
+    assert part[:, :, 1:].isnan().all()
+    rounded = (o16.double().view(T, B, H, D).permute(1, 2, 0, 3).reshape(BH, T, D) * dod).sum(-1)
+    assert_close(got_delta, rounded, torch.float32, "delta")
+
+
+@pytest.mark.parametrize("pairs,D,T,P,want", [
+    (160, 128, 64, 0, 1), (159, 128, 64, 0, 0), (400, 128, 63, 0, 0), (40, 80, 256, 768, 1), (8, 96, 1280, 0, 0), (16, 128, 640, 1400, 1),
+    (10, 128, 2048, 0, 1), (256, 64, 64, 0, 1), (255, 64, 64, 0, 0), (16, 64, 2048, 0, 1), (8, 64, 2048, 0, 0)], ids=str)
+def test_who_shares_the_tiles_of_dq(pairs, D, T, P, want):
+    from terapipe_amd import _lib as L
+    d = L.AttnDesc()
+    d.dtype = d.grad_cache_dtype = L.TP_F16
+    d.batch, d.heads, d.head_dim, d.T, d.cache_len, d.cache_rows = 1, pairs, D, T, P, T + P
+    for name in ("q", "k_cache", "v_cache", "o", "lse", "d_o", "delta", "dqkv", "dk_cache", "dv_cache"):
+        setattr(d, name, 4096)
+    queries = ctypes.c_int(-1)
+    assert L.load().tp_attn_bwd_forms(ctypes.byref(d), ctypes.byref(queries), None) == 0
+    assert queries.value == want
