@@ -174,6 +174,10 @@ int tp_gemm(const tp_gemm_desc* d, void* workspace, size_t workspace_bytes, void
    16-bit TP_GEMM_TN products of one dtype and one k, a multiple of 64, share ONE launch on one tile shape, so that
    together they fill whole rounds of the chip's CUs; any other group runs member by member.  workspace: the largest member's tp_gemm_workspace_bytes. */
 int tp_gemm_grouped(const tp_gemm_desc* descs, int n, void* workspace, size_t workspace_bytes, void* stream);
+/* The same and, as if by tp_vec_param_grads on the same stream, n_vecs reductions of the members' type: in the group's launch where that
+   runs on tiles of 256 x 256, else in a launch of their own.  The products may not change what the reductions read. */
+int tp_gemm_grouped_vec(const tp_gemm_desc* descs, int n, const tp_vecgrad_desc* vecs, int n_vecs, void* workspace,
+                        size_t workspace_bytes, void* stream);
 /* the tile configuration of the single launch tp_gemm_grouped makes for this group; 0 = member by member */
 int tp_gemm_group_cfg(const tp_gemm_desc* descs, int n);
 /* Rows and columns of that launch's tile (0, 0: member by member).  Host code only; for tuning, tests and logs. */

@@ -134,6 +134,7 @@ SYMBOLS = {
     "tp_gemm_static_ws_capacity": (c_size_t, []),
     "tp_gemm_static_ws": (c_int, [ctypes.POINTER(GemmDesc), c_void_p]),
     "tp_gemm_grouped": (c_int, [ctypes.POINTER(GemmDesc), c_int, c_void_p, c_size_t, c_void_p]),
+    "tp_gemm_grouped_vec": (c_int, [ctypes.POINTER(GemmDesc), c_int, ctypes.POINTER(VecGradDesc), c_int, c_void_p, c_size_t, c_void_p]),
     "tp_gemm_tile": (c_int, [ctypes.POINTER(GemmDesc), c_int, ctypes.POINTER(c_int), ctypes.POINTER(c_int), ctypes.POINTER(c_int)]),
     "tp_gemm_group_cfg": (c_int, [ctypes.POINTER(GemmDesc), c_int]),
     "tp_gemm_group_tile": (c_int, [ctypes.POINTER(GemmDesc), c_int, ctypes.POINTER(c_int), ctypes.POINTER(c_int)]),

@@ -35,7 +35,7 @@ def _stale(src_path, obj):
     """True unless obj is newer than its source and every header the sources share."""
     if not os.path.exists(obj):
         return True
-    deps = [src_path, os.path.join(CSRC, "common.h"), os.path.join(CSRC, "gemm_args.h"), os.path.join(CSRC, "attention_args.h"), os.path.join(CSRC, "gemm_epilogue.h"), os.path.join(CSRC, "gemm_tuned.inc"), os.path.join(CSRC, "gemm_tuned_beside.inc"),
+    deps = [src_path, os.path.join(CSRC, "common.h"), os.path.join(CSRC, "gemm_args.h"), os.path.join(CSRC, "attention_args.h"), os.path.join(CSRC, "gemm_epilogue.h"), os.path.join(CSRC, "vec_grads.h"), os.path.join(CSRC, "gemm_tuned.inc"), os.path.join(CSRC, "gemm_tuned_beside.inc"),
             os.path.join(os.path.dirname(HERE), "include", "terapipe_hip.h")]
     t = os.path.getmtime(obj)
     return any(os.path.getmtime(d) > t for d in deps if os.path.exists(d))

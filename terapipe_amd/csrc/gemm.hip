@@ -1,6 +1,7 @@
 // MFMA GEMMs (NT / NN / TN) with fused epilogues for the linears of the GPT layer at tensor-parallel size 1: which kernel
 // runs a product (the plan), the sums of k splits, and the C entry points.  The kernels are in the gemm_*.hip beside.
 #include "gemm_epilogue.h"
+#include "vec_grads.h"
 
 #include <mutex>
 
@@ -11,7 +12,7 @@ namespace tp {
 // kernel.
 bool launch_gemm_dma(int cfg, int op, int dtype, dim3 grid, const GemmArgs& a, hipStream_t s);
 bool launch_gemm_tall(int cfg, int op, int dtype, dim3 grid, const GemmArgs& a, hipStream_t s);
-bool launch_gemm_tall_group(int cfg, int dtype, int tiles, const GemmGroupArgs& ga, hipStream_t s);
+bool launch_gemm_tall_group(int cfg, int dtype, int tiles, const GemmGroupArgs& ga, const VecGradArgs* vec, hipStream_t s);
 
 // Sums the split-K partials and applies the epilogue.  A block of 256 threads covers 256 columns
 // (32 threads x 8 columns) by 8 rows, one vector of 8 columns a thread; column sums are combined across the
@@ -771,7 +772,8 @@ static bool runs_short(const tp_gemm_desc* descs, int n) {
     return group_time(kShort[add], t128, 2 * kNumCU, K) < 0.95f * group_time(kWide[add], t256, kNumCU, K);
 }
 
-static bool launch_group(const tp_gemm_desc* descs, int n, int cfg, hipStream_t s) {
+// vec: blocks behind the tiles (takes_vec_grads)
+static bool launch_group(const tp_gemm_desc* descs, int n, int cfg, const VecGradArgs* vec, hipStream_t s) {
     GemmGroupArgs ga;
     int tiles = 0;
     for (int i = 0; i < n; ++i) {
@@ -801,7 +803,15 @@ static bool launch_group(const tp_gemm_desc* descs, int n, int cfg, hipStream_t 
         return launch_gemm_short_group(descs[0].epilogue == TP_EPI_ACCUMULATE, descs[0].dtype, tiles, ga, s);
     }
     if (cfg == 15 || cfg == 16) return launch_gemm_pipe_group(cfg, descs[0].dtype, tiles, ga, s);
-    return launch_gemm_tall_group(cfg, descs[0].dtype, tiles, ga, s);
+    return launch_gemm_tall_group(cfg, descs[0].dtype, tiles, ga, vec, s);
+}
+// Vector-parameter gradients, `columns` blocks of 256 columns of them, behind the group's tiles: where those are of 256 x 256 and the last
+// round leaves CUs to take most of them by its end (a tile's time and that of a column of blocks both go with the rows).
+static bool takes_vec_grads(const tp_gemm_desc* descs, int n, int cfg, int columns) {
+    if (!((cfg == 2 && !runs_short(descs, n)) || cfg == 19 || cfg == 20)) return false;
+    long tiles = 0;
+    for (int i = 0; i < n; ++i) tiles += (long)((descs[i].M + 255) / 256) * ((descs[i].N + 255) / 256);
+    return tiles % kNumCU && 3 * (kNumCU - tiles % kNumCU) >= 2 * columns;
 }
 }  // namespace tp
 
@@ -900,14 +910,32 @@ extern "C" int tp_gemm_group_tile(const tp_gemm_desc* descs, int n, int* rows, i
 }
 
 extern "C" int tp_gemm_grouped(const tp_gemm_desc* descs, int n, void* workspace, size_t workspace_bytes, void* stream) {
+    return tp_gemm_grouped_vec(descs, n, nullptr, 0, workspace, workspace_bytes, stream);
+}
+
+extern "C" int tp_gemm_grouped_vec(const tp_gemm_desc* descs, int n, const tp_vecgrad_desc* vecs, int n_vecs, void* workspace,
+                                   size_t workspace_bytes, void* stream) {
     if (!descs || n < 1) { tp::set_error("tp_gemm_grouped: bad argument"); return TP_ERR_ARG; }
     for (int i = 0; i < n; ++i) {
         int rc = tp::validate_gemm(&descs[i]);
         if (rc != TP_OK) return rc;
     }
+    tp::VecGradArgs vec;
+    int blocks = 0, columns = 0;
+    if (n_vecs) {
+        const int rc = tp::fill_vec_grads(vecs, n_vecs, descs[0].dtype, vec, blocks);
+        if (rc != TP_OK) return rc;
+        for (int i = 0; i < n_vecs; ++i) columns += (vecs[i].N + 255) / 256;
+    }
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
-    if (const int cfg = tp::group_cfg(descs, n)) {
-        if (!tp::launch_group(descs, n, cfg, s)) {
+    const int cfg = tp::group_cfg(descs, n);
+    const bool together = n_vecs && tp::takes_vec_grads(descs, n, cfg, columns);
+    if (n_vecs && !together) {
+        const int rc = tp_vec_param_grads(vecs, n_vecs, descs[0].dtype, stream);
+        if (rc != TP_OK) return rc;
+    }
+    if (cfg) {
+        if (!tp::launch_group(descs, n, cfg, together ? &vec : nullptr, s)) {
             tp::set_error("tp_gemm_grouped: no kernel for tile configuration %d, dtype %d", cfg, descs[0].dtype);
             return TP_ERR_UNSUPPORTED;
         }

@@ -1,5 +1,6 @@
 // The 256-row GEMM tiles for long activations and parameter gradients, all operand orders (16-bit).
 #include "gemm_epilogue.h"
+#include "vec_grads.h"
 
 namespace tp {
 
@@ -13,10 +14,14 @@ namespace tp {
 // before the MFMAs of k-step s.
 // MI16: 16 x 16 x 32 MFMA blocks and ONE set of operand registers per wave (two waves share a SIMD: one computes
 // while the other fetches; two sets of the twice as many operand registers do not fit beside the accumulators).
+// GROUPED: behind the tiles, the blocks of the same rows' vector-parameter gradients: they run on the CUs that the last, part-filled round
+// of tiles leaves, where in a launch of their own they wait for its end.
+struct GemmTallGroupArgs : GemmGroupArgs { VecGradArgs vec; int tiles; };
+
 template <typename T, bool AKM, bool BKM, int BM, int BN, int BK, int WM, int WN, int STAGES, bool GROUPED = false,
           bool MI16 = false>
 __global__ __launch_bounds__(WM * WN * 64)
-void gemm_tall_kernel(typename std::conditional<GROUPED, GemmGroupArgs, GemmArgs>::type args) {
+void gemm_tall_kernel(typename std::conditional<GROUPED, GemmTallGroupArgs, GemmArgs>::type args) {
     // which problem and which of its tiles (wave-uniform)
     int prob = 0, tile_x = blockIdx.x, tile_y = blockIdx.y;
     if constexpr (GROUPED) {
@@ -60,6 +65,15 @@ void gemm_tall_kernel(typename std::conditional<GROUPED, GemmGroupArgs, GemmArgs
     constexpr int SMEM_BYTES = TILE_BYTES > EPI_BYTES ? TILE_BYTES : EPI_BYTES;
     __shared__ __attribute__((aligned(16))) unsigned char smem[SMEM_BYTES];
     T* tiles = reinterpret_cast<T*>(smem);
+    if constexpr (GROUPED) {
+        static_assert(NT == kVecGradLanes * 32 && SMEM_BYTES >= kVecGradLds, "a block of vec_param_grads_block");
+        if ((int)blockIdx.x >= args.tiles) {
+            const int block = (int)blockIdx.x - args.tiles;
+            VEC_GRAD_PICK(args.vec, block, pr, first)
+            vec_param_grads_block<T, 8>(pr, block - first, smem);
+            return;
+        }
+    }
 
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const int wm = wave % WM, wn = wave / WM;
@@ -227,7 +241,14 @@ bool launch_gemm_tall(int cfg, int op, int dtype, dim3 grid, const GemmArgs& a, 
     return false;
 }
 
-template <typename T> static bool launch_tall_group(int cfg, int tiles, const GemmGroupArgs& ga, hipStream_t s) {
+template <typename T> static bool launch_tall_group(int cfg, int tiles, const GemmGroupArgs& group, const VecGradArgs* vec, hipStream_t s) {
+    GemmTallGroupArgs ga = {};
+    static_cast<GemmGroupArgs&>(ga) = group;
+    ga.tiles = tiles;
+    if (vec) {
+        ga.vec = *vec;
+        tiles += vec->first_block[kVecGradMax];
+    }
     if (cfg == 2) gemm_tall_kernel<T, false, false, 256, 256, 32, 4, 2, 4, true, true><<<dim3(tiles), 512, 0, s>>>(ga);
     else if (cfg == 19) gemm_tall_kernel<T, false, false, 256, 256, 64, 4, 2, 2, true><<<dim3(tiles), 512, 0, s>>>(ga);
     else if (cfg == 20) gemm_tall_kernel<T, false, false, 256, 256, 32, 4, 2, 4, true><<<dim3(tiles), 512, 0, s>>>(ga);
@@ -235,9 +256,9 @@ template <typename T> static bool launch_tall_group(int cfg, int tiles, const Ge
     return true;
 }
 
-bool launch_gemm_tall_group(int cfg, int dtype, int tiles, const GemmGroupArgs& ga, hipStream_t s) {
-    if (dtype == TP_F16) return launch_tall_group<f16>(cfg, tiles, ga, s);
-    if (dtype == TP_BF16) return launch_tall_group<bf16>(cfg, tiles, ga, s);
+bool launch_gemm_tall_group(int cfg, int dtype, int tiles, const GemmGroupArgs& ga, const VecGradArgs* vec, hipStream_t s) {
+    if (dtype == TP_F16) return launch_tall_group<f16>(cfg, tiles, ga, vec, s);
+    if (dtype == TP_BF16) return launch_tall_group<bf16>(cfg, tiles, ga, vec, s);
     return false;
 }
 

@@ -249,8 +249,8 @@ extern "C" int tp_layer_bwd(const tp_layer_bwd_desc* b, void* ws, size_t bytes, 
         {b->dxn, l.x, l.mean1, l.rstd1, acc[0], acc[1], E, M, E},
         {b->dhn, l.h, l.mean2, l.rstd2, acc[4], acc[5], E, M, E},
     };
-    if ((rc = tp_vec_param_grads(vg, 6, l.dtype, stream)) != TP_OK) return rc;
-    if (b->wg_rows && (rc = tp_gemm_grouped(p.wg, 4, ws, bytes, stream)) != TP_OK) return rc;
+    rc = b->wg_rows ? tp_gemm_grouped_vec(p.wg, 4, vg, 6, ws, bytes, stream) : tp_vec_param_grads(vg, 6, l.dtype, stream);
+    if (rc != TP_OK) return rc;
     if (b->small_out[0]) rc = tp_accum_cast_parts(b->small_out, sizes, 8, b->small_acc, b->small_accumulate, l.dtype, stream);
     return rc;
 }

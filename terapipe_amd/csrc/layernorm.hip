@@ -1,6 +1,6 @@
 // Fused LayerNorm forward / backward: one workgroup per row, the row cached in registers, 16-byte
 // coalesced accesses, fp32 statistics, wave64 shuffle + LDS block reductions.
-#include "common.h"
+#include "vec_grads.h"
 
 namespace tp {
 
@@ -20,21 +20,6 @@ __device__ __forceinline__ void block_sum(float (&v)[NREDUCE], float* scratch /*
         float s = 0.f;
         for (int w = 0; w < nw; ++w) s += scratch[i * 16 + w];
         v[i] = s;
-    }
-}
-
-// (fp32 chunks change type by value: taken apart through a pointer some are put into scratch memory)
-template <typename T> __device__ __forceinline__ void load_chunk(const T* p, float* out) {
-    constexpr int CH = 16 / sizeof(T);
-    uint4 raw = *reinterpret_cast<const uint4*>(p);
-    if constexpr (sizeof(T) == 2) {
-        const T* h = reinterpret_cast<const T*>(&raw);
-#pragma unroll
-        for (int e = 0; e < CH; ++e) out[e] = Elem<T>::to_float(h[e]);
-    } else {
-        const float4v f = __builtin_bit_cast(float4v, raw);
-#pragma unroll
-        for (int e = 0; e < CH; ++e) out[e] = f[e];
     }
 }
 
@@ -346,80 +331,11 @@ __global__ __launch_bounds__(256) void ln_param_grads_kernel(const T* __restrict
     }
 }
 
-// The vector-parameter gradients of a layer in ONE launch: up to kVecGradMax reductions over the rows of a step,
-// each either column sums of dy (a bias gradient) or the LayerNorm pair (dgamma += sum dy * xhat, dbeta += sum dy).
-// A block of 256 threads = 32 column chunks (8 columns, 16-byte loads for 16-bit types) x 8 row lanes covers
-// 256 columns x kVecGradRows rows of one problem; the row lanes are combined in LDS and every column then costs one
-// atomic per block.  Blocks are numbered problem by problem (first_block[]).
-constexpr int kVecGradMax = 8;
-constexpr int kVecGradLanes = 16, kVecGradRows = 256;
-struct VecGradProblem {
-    const void* dy; const void* x; const float* mean; const float* rstd;
-    float* acc0; float* acc1;
-    long ld; int M, N;
-};
-struct VecGradArgs {
-    VecGradProblem p[kVecGradMax];
-    int first_block[kVecGradMax + 1];
-    int n;
-};
-
 template <typename T>
 __global__ __launch_bounds__(kVecGradLanes * 32) void vec_param_grads_kernel(VecGradArgs args) {
-    __shared__ float sg[kVecGradLanes][256], sb[kVecGradLanes][256];
-    int pi = 0;
-#pragma unroll
-    for (int i = 1; i < kVecGradMax; ++i)
-        if (i < args.n && (int)blockIdx.x >= args.first_block[i]) pi = i;
-    // (constant indices only: a dynamically indexed kernel argument would be copied to scratch memory)
-    VecGradProblem pr = args.p[0];
-    int first = args.first_block[0];
-#pragma unroll
-    for (int i = 1; i < kVecGradMax; ++i)
-        if (pi == i) { pr = args.p[i]; first = args.first_block[i]; }
-    const int ncb = (pr.N + 255) / 256;
-    const int local = (int)blockIdx.x - first;
-    const int cb = local % ncb, rb = local / ncb;
-    const int cl = threadIdx.x & 31, rl = threadIdx.x >> 5;
-    const int col0 = (cb * 32 + cl) * 8;
-    const int r0 = rb * kVecGradRows, r1 = min(pr.M, r0 + kVecGradRows);
-    const T* dy = reinterpret_cast<const T*>(pr.dy);
-    const T* x = reinterpret_cast<const T*>(pr.x);
-    float ag[8], ab[8];
-#pragma unroll
-    for (int e = 0; e < 8; ++e) { ag[e] = 0.f; ab[e] = 0.f; }
-    if (col0 < pr.N) {
-        for (int row = r0 + rl; row < r1; row += kVecGradLanes) {
-            float d[8];
-            load_chunk<T>(dy + (long)row * pr.ld + col0, d);
-            if constexpr (sizeof(T) == 4) load_chunk<T>(dy + (long)row * pr.ld + col0 + 4, d + 4);
-            if (x) {
-                const float mu = pr.mean[row], rs = pr.rstd[row];
-                float xv[8];
-                load_chunk<T>(x + (long)row * pr.ld + col0, xv);
-                if constexpr (sizeof(T) == 4) load_chunk<T>(x + (long)row * pr.ld + col0 + 4, xv + 4);
-#pragma unroll
-                for (int e = 0; e < 8; ++e) ag[e] += d[e] * (xv[e] - mu) * rs;
-            }
-#pragma unroll
-            for (int e = 0; e < 8; ++e) ab[e] += d[e];
-        }
-    }
-#pragma unroll
-    for (int e = 0; e < 8; ++e) { sg[rl][cl * 8 + e] = ag[e]; sb[rl][cl * 8 + e] = ab[e]; }
-    __syncthreads();
-    const int c = threadIdx.x, col = cb * 256 + c;
-    if (c < 256 && col < pr.N) {
-        float tg = 0.f, tb = 0.f;
-#pragma unroll
-        for (int r = 0; r < kVecGradLanes; ++r) { tg += sg[r][c]; tb += sb[r][c]; }
-        if (x) {
-            atomicAdd(pr.acc0 + col, tg);
-            atomicAdd(pr.acc1 + col, tb);
-        } else {
-            atomicAdd(pr.acc0 + col, tb);
-        }
-    }
+    __shared__ __attribute__((aligned(16))) unsigned char lds[kVecGradLds];
+    VEC_GRAD_PICK(args, (int)blockIdx.x, pr, first)
+    vec_param_grads_block<T, 1>(pr, (int)blockIdx.x - first, lds);
 }
 
 // The same sums where one workgroup can take all rows of its columns: no fp32 atomics, so nothing has to be zeroed before and
@@ -666,12 +582,10 @@ extern "C" int tp_ln_param_grads(const void* dy, const void* x, const float* mea
     return check_launch("tp_ln_param_grads");
 }
 
-extern "C" int tp_vec_param_grads(const tp_vecgrad_desc* descs, int n, int dtype, void* stream) {
-    using namespace tp;
+int tp::fill_vec_grads(const tp_vecgrad_desc* descs, int n, int dtype, VecGradArgs& args, int& blocks) {
     if (!descs || n < 1 || n > kVecGradMax) { set_error("tp_vec_param_grads: 1 to %d problems (n=%d)", kVecGradMax, n); return TP_ERR_ARG; }
     if (dtype < TP_F32 || dtype > TP_BF16) { set_error("tp_vec_param_grads: bad dtype %d", dtype); return TP_ERR_ARG; }
-    VecGradArgs args;
-    int blocks = 0;
+    blocks = 0;
     for (int i = 0; i < n; ++i) {
         const tp_vecgrad_desc& d = descs[i];
         if (!d.dy || !d.acc0 || d.M <= 0 || d.N <= 0 || d.N % 8 || d.ld < d.N || d.ld % 8) {
@@ -687,6 +601,15 @@ extern "C" int tp_vec_param_grads(const tp_vecgrad_desc* descs, int n, int dtype
     for (int i = n; i < kVecGradMax; ++i) { args.p[i] = args.p[0]; args.first_block[i] = blocks; }
     args.first_block[kVecGradMax] = blocks;
     args.n = n;
+    return TP_OK;
+}
+
+extern "C" int tp_vec_param_grads(const tp_vecgrad_desc* descs, int n, int dtype, void* stream) {
+    using namespace tp;
+    VecGradArgs args;
+    int blocks;
+    const int rc = fill_vec_grads(descs, n, dtype, args, blocks);
+    if (rc != TP_OK) return rc;
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     switch (dtype) {
     case TP_F32: vec_param_grads_kernel<float><<<blocks, kVecGradLanes * 32, 0, s>>>(args); break;

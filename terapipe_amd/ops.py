@@ -237,11 +237,12 @@ def gemm(op, A, B, M, N, K, C=None, epilogue=TP_EPI_STORE, bias=None, residual=N
     return C
 
 
-def gemm_grouped(items, desc_sinks=None):
+def gemm_grouped(items, desc_sinks=None, vec_problems=()):
     """Plain products (epilogue STORE or ACCUMULATE) as one library call: items is a list of
     (op, A, B, M, N, K, C, epilogue).  The library runs the group as one launch when its members allow it and
     one after the other otherwise; the result is that of ``gemm`` on every item in order.
-    desc_sinks: per item a list (or None) that receives the item's descriptor, as ``gemm``'s desc_sink."""
+    desc_sinks: per item a list (or None) that receives the item's descriptor, as ``gemm``'s desc_sink.
+    vec_problems: ``vec_param_grads``' reductions, in the same call."""
     n = len(items)
     descs = (GemmDesc * n)()
     lib = _lib.load()
@@ -263,8 +264,9 @@ def gemm_grouped(items, desc_sinks=None):
     ws = Workspace.get(need, items[0][1].device) if need else None
     wsp, wsn = _p(ws), (ws.numel() if ws is not None else 0)
     meta = tuple((op, M, N, K) for (op, _, _, M, N, K, _, _) in items)
-    _lib.check(lib.tp_gemm_grouped(descs, n, wsp, wsn, _stream()), "tp_gemm_grouped")
-    _record("gemm", meta, lambda s=None, ws=ws: lib.tp_gemm_grouped(descs, n, _p(ws), wsn, _on(s)))
+    vecs, nv = _vec_descs(vec_problems), len(vec_problems)
+    _lib.check(lib.tp_gemm_grouped_vec(descs, n, vecs, nv, wsp, wsn, _stream()), "tp_gemm_grouped")
+    _record("gemm", meta, lambda s=None, ws=ws: lib.tp_gemm_grouped_vec(descs, n, vecs, nv, _p(ws), wsn, _on(s)))
 
 
 def _attn_desc(q, k_cache, v_cache, o, lse, batch, heads, head_dim, T, cache_len, q_scale, q_bh_rows=0,
@@ -400,12 +402,8 @@ def ln_param_grads(dy, x2d, mean, rstd, dgamma_acc, dbeta_acc):
         _record("ln_param_grads", (M, E), lambda s=None: lib.tp_ln_param_grads(*a, _on(s)))
 
 
-def vec_param_grads(problems):
-    """Up to 8 reductions over the rows of a step in one launch.  problems: (dy, acc) for a column sum
-    (acc[N] += sum_m dy[m]) or (dy, x, mean, rstd, dgamma_acc, dbeta_acc) for a LayerNorm pair; every dy / x is a
-    2-D row-major tensor of one dtype, the accumulators are fp32."""
-    n = len(problems)
-    descs = (_lib.VecGradDesc * n)()
+def _vec_descs(problems):
+    descs = (_lib.VecGradDesc * len(problems))()
     for d, pr in zip(descs, problems):
         dy = pr[0]
         _require_cuda(*pr)
@@ -416,6 +414,14 @@ def vec_param_grads(problems):
             _, x, mean, rstd, dg, db = pr
             assert x.stride(0) == dy.stride(0)
             d.x, d.mean, d.rstd, d.acc0, d.acc1 = x.data_ptr(), mean.data_ptr(), rstd.data_ptr(), dg.data_ptr(), db.data_ptr()
+    return descs
+
+
+def vec_param_grads(problems):
+    """Up to 8 reductions over the rows of a step in one launch.  problems: (dy, acc) for a column sum
+    (acc[N] += sum_m dy[m]) or (dy, x, mean, rstd, dgamma_acc, dbeta_acc) for a LayerNorm pair; every dy / x is a
+    2-D row-major tensor of one dtype, the accumulators are fp32."""
+    n, descs = len(problems), _vec_descs(problems)
     lib = _lib.load()
     dt = tp_dtype(problems[0][0].dtype)
     _lib.check(lib.tp_vec_param_grads(descs, n, dt, _stream()), "tp_vec_param_grads")
