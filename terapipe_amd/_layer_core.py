@@ -346,7 +346,8 @@ def layer_bwd_native(image, device):
 def stack_forward_only(layers, x, caches, cache_len):
     """The forward of a chain of layers without anything kept for a backward, as one library call: all layers share one
     set of intermediate buffers.  layers: [(12 parameters in PARAM_NAMES order, heads, activation)], each with its own
-    FFN width, heads and activation; caches: [(k, v)] per layer.  Returns the output [T, B, E]."""
+    FFN width, heads and activation; caches: [(k, v)] per layer.  Returns the output [T, B, E]: one layer's
+    has the bits that it has under autograd, from two on products of a few rows take their forward-only forms."""
     T, B, E = x.shape
     ops._require_cuda(x, *(c for kv in caches for c in kv))
     x = x.contiguous()
@@ -370,7 +371,7 @@ def stack_forward_only(layers, x, caches, cache_len):
         k, v = caches[i]
         dst = out.data_ptr() if i == n - 1 else base + shared + (i & 1) * step
         geos[i].pack_fwd(image, i * _FWD_PACK.size, cache_len, k.shape[1], params, src, k.data_ptr(), v.data_ptr(), base, dst,
-                         forward_only=True)
+                         forward_only=n > 1)
         src = dst
     layers_fwd(image, n, x.device)
     return out
