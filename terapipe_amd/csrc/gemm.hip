@@ -805,13 +805,11 @@ static bool launch_group(const tp_gemm_desc* descs, int n, int cfg, const VecGra
     if (cfg == 15 || cfg == 16) return launch_gemm_pipe_group(cfg, descs[0].dtype, tiles, ga, s);
     return launch_gemm_tall_group(cfg, descs[0].dtype, tiles, ga, vec, s);
 }
-// Vector-parameter gradients, `columns` blocks of 256 columns of them, behind the group's tiles: where those are of 256 x 256 and the last
-// round leaves CUs to take most of them by its end (a tile's time and that of a column of blocks both go with the rows).
-static bool takes_vec_grads(const tp_gemm_desc* descs, int n, int cfg, int columns) {
-    if (!((cfg == 2 && !runs_short(descs, n)) || cfg == 19 || cfg == 20)) return false;
-    long tiles = 0;
-    for (int i = 0; i < n; ++i) tiles += (long)((descs[i].M + 255) / 256) * ((descs[i].N + 255) / 256);
-    return tiles % kNumCU && 3 * (kNumCU - tiles % kNumCU) >= 2 * columns;
+// Vector-parameter gradients behind the group's tiles, where those are of 256 x 256: their blocks run on the CUs that the last round
+// leaves, and what is left when it ends spreads over all of them.  Four layers' four products of 1024 over 4096 rows (64 CUs left): 108 us
+// and 23 for a launch of its own, 108 so; five layers of 2048 over 2048 (three full rounds, none left) a pass of 4013 us, 3953 so.
+static bool takes_vec_grads(const tp_gemm_desc* descs, int n, int cfg) {
+    return (cfg == 2 && !runs_short(descs, n)) || cfg == 19 || cfg == 20;
 }
 }  // namespace tp
 
@@ -921,15 +919,14 @@ extern "C" int tp_gemm_grouped_vec(const tp_gemm_desc* descs, int n, const tp_ve
         if (rc != TP_OK) return rc;
     }
     tp::VecGradArgs vec;
-    int blocks = 0, columns = 0;
+    int blocks = 0;
     if (n_vecs) {
         const int rc = tp::fill_vec_grads(vecs, n_vecs, descs[0].dtype, vec, blocks);
         if (rc != TP_OK) return rc;
-        for (int i = 0; i < n_vecs; ++i) columns += (vecs[i].N + 255) / 256;
     }
     hipStream_t s = reinterpret_cast<hipStream_t>(stream);
     const int cfg = tp::group_cfg(descs, n);
-    const bool together = n_vecs && tp::takes_vec_grads(descs, n, cfg, columns);
+    const bool together = n_vecs && tp::takes_vec_grads(descs, n, cfg);
     if (n_vecs && !together) {
         const int rc = tp_vec_param_grads(vecs, n_vecs, descs[0].dtype, stream);
         if (rc != TP_OK) return rc;
