@@ -417,10 +417,13 @@ typedef struct tp_layer_desc {
     void* out;                          /* [T*B, E] */
     int64_t ldw[4];                     /* elements from row to row of the in_proj, out_proj, fc1 and fc2 weight;
                                            0: the rows lie one after the other */
+    int32_t no_backward;                /* 1: nothing is differentiated through this call, now or in a later recomputation: products
+                                           of a few rows may take forms that sum in another order, and only out and the
+                                           cache rows are results.  tp_layer_bwd refuses it */
+    int32_t reserved;
 } tp_layer_desc;
 
-/* n layers in a chain (layers[i].x == layers[i-1].out).  Layers may share every buffer but x and out (forward only).  Where a
-   layer's xn and hn are one buffer no backward can follow it, and products of a few rows take forms that sum in another order. */
+/* n layers in a chain (layers[i].x == layers[i-1].out).  Layers may share every buffer but x and out (forward only). */
 size_t tp_layers_fwd_workspace_bytes(const tp_layer_desc* layers, int n);
 int tp_layers_fwd(const tp_layer_desc* layers, int n, void* workspace, size_t workspace_bytes, void* stream);
 

@@ -214,7 +214,7 @@ def layer_bwd(w, st, dout, heads, gk, gv, accumulate_prefix, has_incoming, zero_
 # A layer is nine to fifteen launches; issued one by one through ops.py each costs about 11 us of Python, which bounds
 # short slices from the host.
 # ------------------------------------------------------------------------------------------------
-_FWD_PACK = struct.Struct("8iq28Q4q")          # tp_layer_desc: sizes, w[12], x, k_cache, v_cache, ..., ldw[4]
+_FWD_PACK = struct.Struct("8iq28Q4q2i")        # tp_layer_desc: sizes, w[12], x, k_cache, v_cache, ..., ldw[4], no_backward
 _FWD_READ, _FWD_LDW = struct.Struct("15Q"), struct.Struct("4q")
 _FWD_READ_AT, _FWD_LDW_AT = 8 * 4 + 8, 8 * 4 + 8 + 28 * 8
 _BWD_PACK = struct.Struct("12Q4iq8Q4Q2i8Q2i2Q")  # tp_layer_bwd_desc after its tp_layer_desc
@@ -291,21 +291,22 @@ class LayerGeometry:
             g = cls._cache[key] = cls(*key)
         return g
 
-    def pack_fwd(self, image, at, cache_len, cache_rows, params, x, k, v, base, out, over=None, forward_only=False):
+    def pack_fwd(self, image, at, cache_len, cache_rows, params, x, k, v, base, out, over=None, one_buffer=False,
+                 no_backward=False):
         """Writes a tp_layer_desc at byte `at` of `image`.  params: the layer's 12; base: address of the forward arena; over: the
-        addresses of LINEAR_INPUTS where they are not part of it (its layout is fwd_rest then).  forward_only: both
-        LayerNorms write one buffer, which tells the library that no backward follows."""
+        addresses of LINEAR_INPUTS where they are not part of it (its layout is fwd_rest then).  one_buffer: for
+        the rows of both LayerNorms.  no_backward: see tp_layer_desc."""
         w_ptrs, ldw = operands(params, self.dtype)
         o = (self.fwd_rest if over else self.fwd).off
         p = {n: base + o[n] for n in o}
         if over:
             p.update(over)
-        if forward_only:
+        if one_buffer:
             p["hn"] = p["xn"]
         _FWD_PACK.pack_into(image, at, self.dt, self.T, self.B, self.H, self.E, self.F, _ACTIVATIONS[self.activation],
                             cache_len, cache_rows, *w_ptrs, x, k, v, p["xn"], p["mean1"], p["rstd1"], p["q"], p["o"],
                             p["lse"], p["h"], p["mean2"], p["rstd2"], p["hn"], p["a"],
-                            p["z"] if self.activation == "gelu" else 0, out, *ldw)
+                            p["z"] if self.activation == "gelu" else 0, out, *ldw, int(no_backward), 0)
 
 
 def repack_operands(image, params, x, k, v):
@@ -346,8 +347,10 @@ def layer_bwd_native(image, device):
 def stack_forward_only(layers, x, caches, cache_len):
     """The forward of a chain of layers without anything kept for a backward, as one library call: all layers share one
     set of intermediate buffers.  layers: [(12 parameters in PARAM_NAMES order, heads, activation)], each with its own
-    FFN width, heads and activation; caches: [(k, v)] per layer.  Returns the output [T, B, E]: one layer's
-    has the bits that it has under autograd, from two on products of a few rows take their forward-only forms."""
+    FFN width, heads and activation; caches: [(k, v)] per layer.  Returns the output [T, B, E], the bits that the layers
+    give under autograd: a forward without gradients may be recomputed with them (activation checkpointing), and half a
+    rounding more or less turns ReLU units near zero on or off.  Only in inference mode, whose tensors autograd
+    refuses, do products of a few rows take the forms that sum in another order."""
     T, B, E = x.shape
     ops._require_cuda(x, *(c for kv in caches for c in kv))
     x = x.contiguous()
@@ -371,7 +374,7 @@ def stack_forward_only(layers, x, caches, cache_len):
         k, v = caches[i]
         dst = out.data_ptr() if i == n - 1 else base + shared + (i & 1) * step
         geos[i].pack_fwd(image, i * _FWD_PACK.size, cache_len, k.shape[1], params, src, k.data_ptr(), v.data_ptr(), base, dst,
-                         forward_only=n > 1)
+                         one_buffer=n > 1, no_backward=torch.is_inference_mode_enabled())
         src = dst
     layers_fwd(image, n, x.device)
     return out

@@ -102,7 +102,7 @@ class LayerDesc(ctypes.Structure):
     _fields_ = [(n, c_int32) for n in ("dtype", "T", "batch", "heads", "hidden", "ffn", "activation", "cache_len")] + [
         ("cache_rows", c_int64), ("w", c_void_p * 12)] + [
         (n, c_void_p) for n in ("x", "k_cache", "v_cache", "xn", "mean1", "rstd1", "q", "o", "lse", "h", "mean2", "rstd2",
-                                "hn", "a", "z", "out")] + [("ldw", c_int64 * 4)]
+                                "hn", "a", "z", "out")] + [("ldw", c_int64 * 4), ("no_backward", c_int32), ("reserved", c_int32)]
 
 
 class LayerBwdDesc(ctypes.Structure):

@@ -439,10 +439,11 @@ struct VecSum {
 constexpr int kVecSums = 6;
 int vec_param_sums(const VecSum (&sums)[kVecSums], bool acc_add, bool dst_add, int dtype, void* stream);
 
-// d, whose A are the rows LayerNorm(x) that nobody has taken yet (gemm.hip): where d runs on gemm_skinny_kernel and the rows fit its
-// LDS, one launch takes them, leaves them in A, their statistics in mean and rstd, and runs d; *taken = false: nothing was launched.
-int gemm_of_layernorm(const tp_gemm_desc& d, const void* x, const void* gamma, const void* beta, float* mean, float* rstd, float eps,
-                      void* stream, bool* taken);
+// d, whose A are the rows LayerNorm(x) that nobody has taken yet (gemm.hip): whether one launch can take them and run d (d runs on
+// gemm_skinny_kernel and the rows fit its LDS), and that launch, which leaves the rows in A, their statistics in mean and rstd.
+struct LayerNormOf { const void* x; const void* gamma; const void* beta; float* mean; float* rstd; };
+bool gemm_takes_layernorm(const tp_gemm_desc& d, const LayerNormOf& ln);
+int gemm_of_layernorm(const tp_gemm_desc& d, const LayerNormOf& ln, float eps, void* stream);
 
 // error plumbing shared by the host-side entry points
 void set_error(const char* fmt, ...);

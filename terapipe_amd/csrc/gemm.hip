@@ -700,18 +700,15 @@ static int run_gemm(const tp_gemm_desc* d, const GemmPlan& p, void* workspace, v
     return TP_OK;
 }
 
-int gemm_of_layernorm(const tp_gemm_desc& d, const void* x, const void* gamma, const void* beta, float* mean, float* rstd, float eps,
-                      void* stream, bool* taken) {
-    *taken = false;
+bool gemm_takes_layernorm(const tp_gemm_desc& d, const LayerNormOf& l) {
+    return (d.reserved & kNoBackward) && runs_skinny(&d) && skinny_takes_ln(d.M, d.K) && d.lda == d.K && l.x && l.gamma && l.beta &&
+           l.mean && l.rstd && !(((uintptr_t)l.x | (uintptr_t)l.gamma | (uintptr_t)l.beta) & 15) && plan_gemm(&d).nsplit <= 1;
+}
+int gemm_of_layernorm(const tp_gemm_desc& d, const LayerNormOf& l, float eps, void* stream) {
     const int rc = validate_gemm(&d);
     if (rc != TP_OK) return rc;
-    if (!(d.reserved & kNoBackward) || !runs_skinny(&d) || !skinny_takes_ln(d.M, d.K) || d.lda != d.K || !x || !gamma || !beta || !mean || !rstd ||
-        (((uintptr_t)x | (uintptr_t)gamma | (uintptr_t)beta) & 15)) return TP_OK;
-    const GemmPlan p = plan_gemm(&d);
-    if (p.nsplit > 1) return TP_OK;
-    const SkinnyLn ln = {gamma, beta, const_cast<void*>(d.A), mean, rstd, eps};
-    *taken = true;
-    return run_gemm(&d, p, nullptr, stream, &ln, x);
+    const SkinnyLn ln = {l.gamma, l.beta, const_cast<void*>(d.A), l.mean, l.rstd, eps};
+    return run_gemm(&d, plan_gemm(&d), nullptr, stream, &ln, l.x);
 }
 
 // One launch for the whole group when every member is a 16-bit TN product (parameter gradients) of the same dtype and

@@ -196,7 +196,7 @@ struct SkinnyLn { const void* gamma; const void* beta; void* y; float* mean; flo
 bool skinny_takes_ln(int M, int K);
 // half: tiles of 8 weight rows where those of 16 come to at most half of the 256 CUs (their sums are in another order).
 void launch_gemm_skinny(int dtype, const GemmArgs& a, bool half, const SkinnyLn* ln, hipStream_t s);
-constexpr int kNoBackward = 1 << 25;        // of tp_gemm_desc.reserved
+constexpr int kNoBackward = 1 << 25;        // of tp_gemm_desc.reserved; set where tp_layer_desc.no_backward is
 static inline bool skinny_half(int M, int N) { return M <= 8 && (N + 15) / 16 <= 128; }
 // Deep rings of 64 x 32, 64 x 64 and 64 x 128 tiles (gemm_deep.hip; NT and NN, 16-bit): grid = (column tiles of `columns`, row
 // tiles, k splits).

@@ -58,14 +58,12 @@ static int gemm_deferred(tp_gemm_desc d, void* ws, size_t bytes, void* stream, i
 }
 
 // A = LayerNorm(x), then the product d that reads it: one launch where the product takes the rows itself.
-static int layernorm_then(const tp_gemm_desc& d, const tp_layer_desc& l, const void* x, const void* gamma, const void* beta, float* mean,
-                          float* rstd, void* ws, size_t bytes, void* stream) {
-    bool taken;
-    int rc = gemm_of_layernorm(d, x, gamma, beta, mean, rstd, 1e-5f, stream, &taken);
-    if (rc != TP_OK || taken) return rc;
-    rc = tp_layernorm_fwd(x, gamma, beta, const_cast<void*>(d.A), mean, rstd, d.M, d.K, 1e-5f, l.dtype, stream);
+static int layernorm_then(const tp_gemm_desc& d, const LayerNormOf& ln, void* ws, size_t bytes, void* stream) {
+    if (gemm_takes_layernorm(d, ln)) return gemm_of_layernorm(d, ln, 1e-5f, stream);
+    const int rc = tp_layernorm_fwd(ln.x, ln.gamma, ln.beta, const_cast<void*>(d.A), ln.mean, ln.rstd, d.M, d.K, 1e-5f, d.dtype, stream);
     return rc != TP_OK ? rc : tp_gemm(&d, ws, bytes, stream);
 }
+static LayerNormOf first_layernorm(const tp_layer_desc& l) { return {l.x, l.w[W_LN1_G], l.w[W_LN1_B], l.mean1, l.rstd1}; }
 
 struct ForwardPlan { tp_gemm_desc qkv, out, fc1, fc2; tp_attn_desc attn; };
 static ForwardPlan forward_plan(const tp_layer_desc& l) {
@@ -84,7 +82,7 @@ static ForwardPlan forward_plan(const tp_layer_desc& l) {
     if (l.activation) { p.fc1.aux_out = l.z; p.fc1.ldauxo = F; }
     p.fc2 = gemm_desc(l, TP_GEMM_NT, TP_EPI_BIAS_RESIDUAL, M, E, F, l.a, l.w[W_FC2], l.out, LD_FC2);
     p.fc2.bias = l.w[B_FC2]; p.fc2.residual = l.h; p.fc2.ldr = E;
-    if (l.xn == l.hn)
+    if (l.no_backward)
         for (tp_gemm_desc* d : {&p.qkv, &p.out, &p.fc1, &p.fc2}) d->reserved = kNoBackward;
     return p;
 }
@@ -148,7 +146,7 @@ extern "C" int tp_layers_fwd(const tp_layer_desc* layers, int n, void* ws, size_
                                            l.w[W_LN1_G], l.w[W_LN1_B], l.xn, l.mean1, l.rstd1, M, E, 1e-5f, l.dtype, stream);
             if (rc == TP_OK) rc = tp_gemm(&p.qkv, ws, bytes, stream);
         } else {
-            rc = layernorm_then(p.qkv, l, l.x, l.w[W_LN1_G], l.w[W_LN1_B], l.mean1, l.rstd1, ws, bytes, stream);
+            rc = layernorm_then(p.qkv, first_layernorm(l), ws, bytes, stream);
         }
         if (rc != TP_OK) return rc;
         if ((rc = tp_attn_prefix_fwd(&p.attn, ws, bytes, stream)) != TP_OK) return rc;
@@ -159,11 +157,15 @@ extern "C" int tp_layers_fwd(const tp_layer_desc* layers, int n, void* ws, size_
                                            l.rstd2, M, E, 1e-5f, l.dtype, stream);
             if (rc == TP_OK) rc = tp_gemm(&p.fc1, ws, bytes, stream);
         } else {
-            rc = layernorm_then(p.fc1, l, l.h, l.w[W_LN2_G], l.w[W_LN2_B], l.mean2, l.rstd2, ws, bytes, stream);
+            rc = layernorm_then(p.fc1, {l.h, l.w[W_LN2_G], l.w[W_LN2_B], l.mean2, l.rstd2}, ws, bytes, stream);
         }
         if (rc != TP_OK) return rc;
-        if (i + 1 < n) rc = gemm_deferred(p.fc2, ws, bytes, stream, &pending);
-        else rc = tp_gemm(&p.fc2, ws, bytes, stream);
+        // (a LayerNorm that its product takes has its sums in its own order: the layers of a chain take it as one alone does)
+        pending = 1;
+        if (i + 1 < n && !gemm_takes_layernorm(forward_plan(layers[i + 1]).qkv, first_layernorm(layers[i + 1])))
+            rc = gemm_deferred(p.fc2, ws, bytes, stream, &pending);
+        else
+            rc = tp_gemm(&p.fc2, ws, bytes, stream);
         if (rc != TP_OK) return rc;
     }
     return TP_OK;
@@ -187,6 +189,7 @@ extern "C" int tp_layer_bwd(const tp_layer_bwd_desc* b, void* ws, size_t bytes, 
         set_error("tp_layer_bwd: null buffer");
         return TP_ERR_ARG;
     }
+    if (b->f.no_backward) { set_error("tp_layer_bwd: the forward was asked for as one that no backward follows"); return TP_ERR_ARG; }
     const tp_layer_desc& l = b->f;
     const int M = l.T * l.batch, E = l.hidden, F = l.ffn;
     const BackwardPlan p = backward_plan(*b);

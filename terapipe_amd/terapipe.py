@@ -74,7 +74,7 @@ class TransformerLayers(nn.Module):
         return x, cache_outputs
 
     def _forward_only(self, x, cache, cache_len):
-        """All layers as one library call (evaluation, generation: no backward follows)."""
+        """All layers as one library call (evaluation, generation)."""
         T, B, E = x.shape
         assert E == self.embedding_dim
         stack, caches = [], []
