@@ -301,6 +301,8 @@ __global__ __launch_bounds__(256, DH <= 64 ? 3 : 2) void attn_dq_long_kernel(Att
     const int qw = q0 + 32 * qb, tq = qw + li, tr_row = min(tq, T_ - 1);
     const bool qok = tq < T_;
     const int nt = (P + min(T_, q0 + 32 * QB) + KT - 1) / KT;    // tiles of the workgroup
+    // those in which the wave's block of 32 keys has one that its queries see: what lies beyond is not multiplied, not even by zero
+    const int nw = qw < T_ ? max(0, P + min(T_, qw + 32) - kh * 32 + KT - 1) / KT : 0;
 
     // the lane's chunk of a tile's first rows and that of row S - 1 (the swizzle repeats every 16 rows: the same column in each load)
     const int lr = tid / CPR, lc = (tid % CPR) ^ swz16<PITCH>(lr);
@@ -384,15 +386,19 @@ __global__ __launch_bounds__(256, DH <= 64 ? 3 : 2) void attn_dq_long_kernel(Att
     for (int ks = 0; ks < NKS; ++ks) s = E::mfma(km_from(0, ks), qreg[ks], s);
 
     unsigned kslot = 0, vslot = 0;      // byte offsets of tile t's slots
-    for (int t = 0; t < nt; ++t) {
+    auto next_slot = [&](unsigned slot, unsigned n) __attribute__((always_inline)) { return slot == (n - 1) * TILE ? 0 : slot + TILE; };
+    auto next_loads = [&](int t) __attribute__((always_inline)) {
         // this wave's loads of K(t + 1) and V(t) have landed, and its reads of the tiles before t are back
         if (t) barrier(std::integral_constant<int, (AHEAD - 1) * 2 * NLD>());
-        const unsigned knext = kslot == (RK - 1) * TILE ? 0 : kslot + TILE;
         issue(Vb, VRING + (vslot ? vslot : RV * TILE) - TILE, t + AHEAD);
         issue(Kb, (kslot ? kslot : RK * TILE) - TILE, t + AHEAD + 1);
+    };
+    for (int t = 0; t < nw; ++t) {
+        next_loads(t);
+        const unsigned knext = next_slot(kslot, RK);
         const int key0 = t * KT + kh * 32;
         x = s;
-        if (key0 + 31 > P + qw) {       // wave-uniform: the block touches the causal boundary, or lies beyond it
+        if (key0 + 31 > P + qw) {       // wave-uniform: the block touches the causal boundary
             const int end = P + tq - key0 - acc_row(0, g);
 #pragma unroll
             for (int j = 0; j < 16; ++j)
@@ -445,7 +451,12 @@ __global__ __launch_bounds__(256, DH <= 64 ? 3 : 2) void attn_dq_long_kernel(Att
             __builtin_amdgcn_sched_barrier(0);
         }
         kslot = knext;
-        vslot = vslot == (RV - 1) * TILE ? 0 : vslot + TILE;
+        vslot = next_slot(vslot, RV);
+    }
+    for (int t = nw; t < nt; ++t) {     // the other waves' tiles: this one's share of their loads
+        next_loads(t);
+        kslot = next_slot(kslot, RK);
+        vslot = next_slot(vslot, RV);
     }
     wait_vmcnt<0>();            // (the loads past the last tile)
     __syncthreads();            // every wave is done with the rings
