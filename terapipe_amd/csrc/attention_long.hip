@@ -273,9 +273,9 @@ __global__ __launch_bounds__(512) void attn_fwd_long_kernel(AttnArgs a) {
 // What bounds it: the waits between a tile's loads, LDS fetches and MFMAs that two waves a SIMD cover only in part (24 MFMAs of 32
 // clocks and about 900 clocks of issue in 1750 per block of 32 x 32, 96 heads of 128); QB = 4 has three tiles of 32 keys under way where QB = 2
 // has one of 64, and pulls half the bytes.
-// Measured (fp16, causal, 2048 positions, us; before: eight waves on one ring of 128 KB, phases in step): 40 heads of 128 91 -> 76, 96 of
-// 128 205 -> 170, 16 of 128 51 -> 43 (blocks of 64), 12 of 64 28 -> 23, 32 of 80 49 -> 50; 64 of 64 at 1024 24.4 -> 23.4, 300 of 64 at 256
-// 22.6 -> 17.7; 40 of 128, 512 after 1536 59 -> 44.  Two of the old workgroups on a CU at 64 (128 registers, spills): 24 -> 38.
+// Measured (fp16, causal, 2048 positions, us; before: eight waves on one ring of 128 KB, phases in step): 40 heads of 128 90 -> 76, 96 of
+// 128 206 -> 168, 16 of 128 49 -> 41 (blocks of 64), 12 of 64 30 -> 25, 40 of 80 66 -> 58, 40 of 96 72 -> 63; 64 of 64 at 1024 24.1 -> 23.8, 300 of
+// 64 at 256 22.2 -> 16.7; 40 of 128, 512 after 1536 60 -> 47 (32 queries a workgroup).  Two of the old workgroups on a CU at 64 (128 registers, spills): 24 -> 38.
 // ------------------------------------------------------------------------------------------------
 template <typename T, int DH, int QB>
 __global__ __launch_bounds__(256, DH <= 64 ? 3 : 2) void attn_dq_long_kernel(AttnArgs a) {
@@ -502,6 +502,202 @@ __global__ __launch_bounds__(256, DH <= 64 ? 3 : 2) void attn_dq_long_kernel(Att
     }
 }
 
+// ------------------------------------------------------------------------------------------------
+// The same by eight waves for 128 queries: four blocks of 32, each by two waves that take one half of every key tile, tiles of 128
+// keys, one workgroup to a CU above head dimension 64.  For 289 to 512 workgroups of long sequences (dq_form): the longest block then sets the
+// time, and here two waves share its walk over the keys, with a CU to themselves.  us, this form / the better of the two above, causal,
+// 2048 positions: 32 heads of 64 35.2 / 37.8, 25 of 80 44.6 / 46.1, 32 of 80 48.6 / 51.0, 32 of 96 51.6 / 54.1, 20 of 128 52.3 / 53.3;
+// 24 of 96 at 1536 (288) 32.0 / 32.9; outside: 36 of 80 64.7 / 56.2, 16 of 128 48.7 / 40.9, 64 of 80 at 1024 33.5 / 31.6.
+// ------------------------------------------------------------------------------------------------
+template <typename T, int DH>
+__global__ __launch_bounds__(512) void attn_dq_pairs_kernel(AttnArgs a) {
+    typedef Elem<T> E;
+    constexpr int NDB = (DH + 31) / 32, NKS = DH / 16, PITCH = tile_pitch<DH>(), CPR = PITCH / 8;
+    constexpr int NB = 2;                                   // 32-key blocks of a tile per wave
+    constexpr int KT = 64 * NB, TILE = KT * PITCH, STAGE = 2 * TILE;
+    constexpr int NLD = KT * CPR / 512;                     // loads per K or V tile and lane
+    constexpr int EPI_LD = NDB * 32 + 4;
+    constexpr int RING_BYTES = 2 * STAGE * 2, EPI_BYTES = 4 * 32 * EPI_LD * 4;
+    __shared__ __attribute__((aligned(16))) unsigned char smem[RING_BYTES > EPI_BYTES ? RING_BYTES : EPI_BYTES];
+    T* ring = reinterpret_cast<T*>(smem);
+
+    const int tid = threadIdx.x, lane = tid & 63, g = lane >> 5, li = lane & 31;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), qb = wave & 3, kh = wave >> 2;
+    int bh, blk;
+    if (!xcd_map(a.B * a.H, bh, blk)) return;
+    const int b = bh / a.H, h = bh - b * a.H;
+    const int T_ = a.T, P = a.P, S = a.P + a.T;
+    const long EE = (long)a.H * DH;
+    const int q0 = ((T_ + 127) / 128 - 1 - blk) * 128;      // the blocks with the longest key range start first
+    const int qw = q0 + 32 * qb, tq = qw + li, tr = min(tq, T_ - 1);
+    const bool qok = tq < T_;
+    const int nt = (P + min(T_, q0 + 128) + KT - 1) / KT;   // tiles of the workgroup
+    const int key_end = qw < T_ ? P + min(T_, qw + 32) : 0; // keys this wave's queries see
+
+    unsigned koff[NLD];
+#pragma unroll
+    for (int i = 0; i < NLD; ++i) {
+        const int p = i * 512 + tid, r = p / CPR, lc = (p % CPR) ^ swz16<PITCH>(r);
+        koff[i] = lc < DH / 8 ? (unsigned)(r * DH * 2 + lc * 16) : kNoChunk;
+    }
+    const char* Kb = uniform_ptr(reinterpret_cast<const char*>(reinterpret_cast<const T*>(a.kc) + (long)bh * a.cache_rows * DH));
+    const char* Vb = uniform_ptr(reinterpret_cast<const char*>(reinterpret_cast<const T*>(a.vc) + (long)bh * a.cache_rows * DH));
+    const unsigned lds0 = lds_addr(smem) + wave * 1024;
+    auto issue = [&](int stage, int tile) {                 // (rows at or past S as in the forward)
+        const unsigned dst = lds0 + (unsigned)(stage * STAGE * 2);
+        const int row0 = tile * KT;
+#pragma unroll
+        for (int which = 0; which < 2; ++which) {
+            const char* base = which ? Vb : Kb;
+            if (row0 + KT <= S) {
+                const char* sb = base + (long)row0 * (DH * 2);
+#pragma unroll
+                for (int i = 0; i < NLD; ++i) load_chunk_lds<DH>(koff[i], sb, dst + which * TILE * 2 + i * 8192);
+            } else {
+#pragma unroll
+                for (int i = 0; i < NLD; ++i) {
+                    const int p = i * 512 + tid, r = p / CPR, lc = (p % CPR) ^ swz16<PITCH>(r);
+                    const unsigned off = lc < DH / 8 ? (unsigned)(min(row0 + r, S - 1) * DH * 2 + lc * 16) : kNoChunk;
+                    load_chunk_lds<DH>(off, base, dst + which * TILE * 2 + i * 8192);
+                }
+            }
+        }
+    };
+    issue(0, 0);
+
+    typename E::opnd_t qreg[NKS], doreg[NKS];
+    const long orow = ((long)tr * a.B + b) * EE + (long)h * DH;
+    load_row_operands<T, DH>(qreg, reinterpret_cast<const T*>(a.q) + (long)bh * a.q_bhs + (long)tr * DH, qok, g);
+    load_row_operands<T, DH>(doreg, reinterpret_cast<const T*>(a.d_o) + orow, qok, g);
+    float delta = 0.f;
+    {
+        typename E::opnd_t oreg[NKS];
+        load_row_operands<T, DH>(oreg, reinterpret_cast<const T*>(a.o) + orow, qok, g);
+#pragma unroll
+        for (int ks = 0; ks < NKS; ++ks) {
+            const float8v x = __builtin_convertvector(__builtin_bit_cast(vec8_t<T>, oreg[ks]), float8v) *
+                              __builtin_convertvector(__builtin_bit_cast(vec8_t<T>, doreg[ks]), float8v);
+#pragma unroll
+            for (int e = 0; e < 8; ++e) delta += x[e];
+        }
+        delta += __shfl_xor(delta, 32, 64);
+        if (kh == 0 && g == 0 && qok) a.delta[(long)bh * a.st_bhs + tq] = delta;
+    }
+    const float lneg = qok ? -a.lse[(long)bh * a.st_bhs + tq] * kLog2e : 0.f;
+
+    int okm[NKS], otr[NDB][2];          // element offsets of the lane's fetches inside a K tile, its first block
+#pragma unroll
+    for (int ks = 0; ks < NKS; ++ks) okm[ks] = km_offset<T, PITCH>(kh * 32 * NB + li, ks * 16, lane);
+#pragma unroll
+    for (int db = 0; db < NDB; ++db) tr_offsets<T, PITCH, true>(kh * 32 * NB, db * 32, lane, otr[db][0], otr[db][1]);
+
+    float16v dq[NDB];
+#pragma unroll
+    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) dq[db][r] = 0.f;
+
+    auto step = [&](auto sc, int t) __attribute__((always_inline)) {
+        constexpr int st = decltype(sc)::value;
+        wait_vmcnt<0>();                    // this wave's part of tile t has landed
+        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");      // and its reads of tile t - 1 are back
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+        if (t + 1 < nt) issue(st ^ 1, t + 1);
+#pragma unroll
+        for (int n = 0; n < NB; ++n) {
+            const int key0 = t * KT + (kh * NB + n) * 32, so = st * STAGE + n * 32 * PITCH;
+            if (key0 >= key_end) break;     // wave-uniform
+            typename E::opnd_t kf[NKS], vf[NKS];
+#pragma unroll
+            for (int ks = 0; ks < NKS; ++ks) kf[ks] = load_km<T>(ring + so + okm[ks]);
+#pragma unroll
+            for (int ks = 0; ks < NKS; ++ks) vf[ks] = load_km<T>(ring + so + TILE + okm[ks]);
+            __builtin_amdgcn_sched_barrier(0);
+            float16v s, d;
+#pragma unroll
+            for (int r = 0; r < 16; ++r) { s[r] = 0.f; d[r] = 0.f; }
+#pragma unroll
+            for (int ks = 0; ks < NKS; ++ks) s = E::mfma(kf[ks], qreg[ks], s);
+#pragma unroll
+            for (int ks = 0; ks < NKS; ++ks) d = E::mfma(vf[ks], doreg[ks], d);
+            __builtin_amdgcn_sched_barrier(0);
+            uint4 kt[2][NDB];
+#pragma unroll
+            for (int hs = 0; hs < 2; ++hs)
+#pragma unroll
+                for (int db = 0; db < NDB; ++db)
+                    kt[hs][db] = load_tr<T>(ring + so + otr[db][0] + hs * 16 * PITCH, ring + so + otr[db][1] + hs * 16 * PITCH);
+            __builtin_amdgcn_sched_barrier(0);
+            if (key0 + 31 > P + qw) {       // wave-uniform: the block touches the causal boundary
+#pragma unroll
+                for (int j = 0; j < 16; ++j)
+                    if (key0 + acc_row(j, g) > P + tq) s[j] = -INFINITY;
+            }
+            float8v e0, e1;
+#pragma unroll
+            for (int j = 0; j < 8; ++j) {
+                e0[j] = fast_exp2(fmaf(s[j], kLog2e, lneg)) * (d[j] - delta);
+                e1[j] = fast_exp2(fmaf(s[j + 8], kLog2e, lneg)) * (d[j + 8] - delta);
+            }
+            const uint4 p[2] = {pack8v<T>(e0), pack8v<T>(e1)};
+#pragma unroll
+            for (int hs = 0; hs < 2; ++hs)
+#pragma unroll
+                for (int db = 0; db < NDB; ++db) dq[db] = E::mfma(kt[hs][db], p[hs], dq[db]);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    for (int t = 0; t < nt; t += 2) {
+        step(std::integral_constant<int, 0>(), t);
+        if (t + 1 < nt) step(std::integral_constant<int, 1>(), t + 1);
+    }
+    __syncthreads();            // every wave is done with the ring
+
+    float* ebuf = reinterpret_cast<float*>(smem) + qb * 32 * EPI_LD;
+    if (kh == 1) {
+#pragma unroll
+        for (int db = 0; db < NDB; ++db)
+#pragma unroll
+            for (int jq = 0; jq < 4; ++jq)
+                *reinterpret_cast<float4*>(ebuf + (db * 4 + jq) * 256 + lane * 4) =
+                    make_float4(dq[db][4 * jq], dq[db][4 * jq + 1], dq[db][4 * jq + 2], dq[db][4 * jq + 3]);
+    }
+    __syncthreads();
+    if (kh == 1) return;
+#pragma unroll
+    for (int db = 0; db < NDB; ++db)
+#pragma unroll
+        for (int jq = 0; jq < 4; ++jq) {
+            const float4 o = *reinterpret_cast<const float4*>(ebuf + (db * 4 + jq) * 256 + lane * 4);
+            dq[db][4 * jq] = (dq[db][4 * jq] + o.x) * a.qscale;
+            dq[db][4 * jq + 1] = (dq[db][4 * jq + 1] + o.y) * a.qscale;
+            dq[db][4 * jq + 2] = (dq[db][4 * jq + 2] + o.z) * a.qscale;
+            dq[db][4 * jq + 3] = (dq[db][4 * jq + 3] + o.w) * a.qscale;
+        }
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+    acc_to_lds_rows<DH>(dq, ebuf, lane);                // the wave's own block: LDS operations of one wave complete in order
+    asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
+#pragma unroll
+    for (int p = lane; p < 32 * DH / 8; p += 64) {
+        const int row = p / (DH / 8), col = (p % (DH / 8)) * 8;
+        if (qw + row >= T_) break;
+        float v[8];
+        *reinterpret_cast<float4*>(v) = *reinterpret_cast<const float4*>(ebuf + row * EPI_LD + col);
+        *reinterpret_cast<float4*>(v + 4) = *reinterpret_cast<const float4*>(ebuf + row * EPI_LD + col + 4);
+        *reinterpret_cast<uint4*>(reinterpret_cast<T*>(a.dqkv) + ((long)(qw + row) * a.B + b) * (3 * EE) + (long)h * 3 * DH + col) = pack8<T>(v);
+    }
+}
+
+template <typename T> static void dq_pairs(int hd, const AttnArgs& a, hipStream_t s) {
+    const unsigned grid = xcd_grid(a.B * a.H, (a.T + 127) / 128);
+    switch (hd) {
+    case 64: attn_dq_pairs_kernel<T, 64><<<grid, 512, 0, s>>>(a); break;
+    case 80: attn_dq_pairs_kernel<T, 80><<<grid, 512, 0, s>>>(a); break;
+    case 96: attn_dq_pairs_kernel<T, 96><<<grid, 512, 0, s>>>(a); break;
+    default: attn_dq_pairs_kernel<T, 128><<<grid, 512, 0, s>>>(a); break;
+    }
+}
 template <typename T, int QB> static void dq_long(int hd, const AttnArgs& a, hipStream_t s) {
     const unsigned grid = xcd_grid(a.B * a.H, (a.T + 32 * QB - 1) / (32 * QB));
     switch (hd) {
@@ -511,15 +707,29 @@ template <typename T, int QB> static void dq_long(int hd, const AttnArgs& a, hip
     default: attn_dq_long_kernel<T, 128, QB><<<grid, 256, 0, s>>>(a); break;
     }
 }
+// Blocks of 64 queries, of 128 or, eight waves each, of 128.  With w blocks of 128 that a chip of two (three at head dimension 64)
+// to a CU runs at once, what counts is whether the longest one's walk over the keys ends after all others' work: then two waves to a
+// block of 32 queries are better than one, by blocks of 64 or, for long sequences, by the eight-wave form.  Few heads, 512 to 3072 positions, 0
+// to 1024 of context, 270 to 900 blocks: the form taken is within 0.7 % of the best of the three in the mean, 14 % at worst (120 of 64 at
+// 512: 18.5 / 16.2); us, 64 / 128 / eight waves: 16 of 128 at 2048 (w = 256) 41 / 52 / 49, 20 of 80 (320) 39.5 / 45.5 / 39.0, 36 of 80
+// (576) 62 / 56 / 65; 40 of 96 at 1024 (320) 26.0 / 29.0 / 26.4, 60 (480) 35.6 / 32.8 / 34.2, 40 after 512 43.5 / 41.0 / 41.9; 160 of 128 at 256 (320)
+// 25.6 / 19.4 / 26.1; 48 of 64 at 2048 (768) 50.8 / 52.0 / 54.2, at 512 less to share: 120 (480) 18.5 / 16.2 / 18.8.
+// Short calls of many heads take blocks of 128 that no second row fills: 600 of 128, 64 queries 20.9 / 19.2, 96 queries 33.4 / 25.0.
+enum DqForm { kDq64, kDq128, kDqPairs };
+static DqForm dq_form(int head_dim, long pairs, int T, int P) {
+    const long w = pairs * ((T + 127) / 128);
+    const bool uneven = T >= 1400 && 2L * P <= T;
+    if (uneven && w > 288 && w <= (head_dim < 128 ? 512 : 384)) return kDqPairs;
+    if (head_dim == 64) return w >= (uneven ? 800 : 512) ? kDq128 : kDq64;
+    const bool longest = T >= 700 && w * (2L * P + T) <= (head_dim < 128 ? 384L : 340L) * ((long)P + T);
+    return w > 256 && !longest ? kDq128 : kDq64;
+}
 void launch_attn_dq_long(int dtype, int head_dim, const AttnArgs& a, hipStream_t s) {
-    // Blocks of 128 queries once they give every CU one and some a second (at head dimension 64, with three to a CU, two each); below,
-    // blocks of 64 spread the longest rows of keys over more CUs.  us, 64 / 128 queries: 48 heads of 128 at 1024 (384 blocks of 128)
-    // 40 / 36, 40 of 128, 512 after 1536 (160) 44 / 49, 16 of 128 at 2048 (256) 43 / 55; 64 of 64 at 1024 (512) 24.5 / 23.4, 25 of 64 at
-    // 2048 (400) 35 / 39.
-    const long w = (long)a.B * a.H * ((a.T + 127) / 128);
-    const bool wide = head_dim > 64 ? w > 256 : w >= 512;
-    if (dtype == TP_F16) wide ? dq_long<f16, 4>(head_dim, a, s) : dq_long<f16, 2>(head_dim, a, s);
-    else wide ? dq_long<bf16, 4>(head_dim, a, s) : dq_long<bf16, 2>(head_dim, a, s);
+    switch (dq_form(head_dim, (long)a.B * a.H, a.T, a.P)) {
+    case kDqPairs: dtype == TP_F16 ? dq_pairs<f16>(head_dim, a, s) : dq_pairs<bf16>(head_dim, a, s); break;
+    case kDq128: dtype == TP_F16 ? dq_long<f16, 4>(head_dim, a, s) : dq_long<bf16, 4>(head_dim, a, s); break;
+    default: dtype == TP_F16 ? dq_long<f16, 2>(head_dim, a, s) : dq_long<bf16, 2>(head_dim, a, s); break;
+    }
 }
 
 // ------------------------------------------------------------------------------------------------

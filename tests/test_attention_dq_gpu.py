@@ -4,6 +4,8 @@ import ctypes
 import pytest
 import torch
 
+from tests.util import assert_close
+
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
@@ -23,7 +25,7 @@ def _dq(q, k, v, o, lse, do, P):
 
 @pytest.mark.parametrize("value", [float("inf"), float("nan")])
 @pytest.mark.parametrize("D", [64, 80, 96, 128])
-@pytest.mark.parametrize("BH,T,P", [(3, 256, 0), (300, 256, 0), (5, 200, 37), (270, 200, 101), (2, 33, 0)], ids=str)
+@pytest.mark.parametrize("BH,T,P", [(3, 256, 0), (300, 256, 0), (5, 200, 37), (270, 200, 101), (2, 33, 0), (27, 1411, 0)], ids=str)
 def test_values_that_a_query_cannot_see(BH, T, P, D, value):
     """An infinite or undefined value in K or V reaches, of the queries before it, at most those of its own block of 32 x 32."""
     from terapipe_amd import ops
@@ -45,3 +47,24 @@ def test_values_that_a_query_cannot_see(BH, T, P, D, value):
             got = _dq(q, k, v, o, lse, do, P)
             poisoned[:, at] = kept
             assert torch.equal(got[:, :before], want[:, :before]), (at, before)
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16], ids=str)
+@pytest.mark.parametrize("D", [64, 80, 96, 128])
+@pytest.mark.parametrize("BH,T,P", [(25, 1400, 0), (27, 1411, 705), (32, 1473, 100), (24, 1536, 0), (33, 1399, 0), (43, 1500, 13)], ids=str)
+def test_long_sequences_of_few_heads(BH, T, P, D, dtype):
+    """Both sides of the lines between the eight-wave form and the two others, with key tiles and query blocks that end inside."""
+    from terapipe_amd import ops
+    g = torch.Generator(device=DEV).manual_seed(T + P + D)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV).to(dtype)
+    S, sc = P + T, D ** -0.5
+    q, k, v, do = rnd(BH, T, D) * sc, rnd(BH, S + 3, D), rnd(BH, S + 3, D), rnd(T, 1, BH * D)
+    k[:, S:], v[:, S:] = float("nan"), float("nan")         # rows past the slice are never used
+    o, lse = ops.attn_prefix_fwd(q, k, v, 1, BH, D, T, P, sc)
+    got = _dq(q, k, v, o, lse, do, P).double()
+    unseen = torch.arange(S, device=DEV)[None] > P + torch.arange(T, device=DEV)[:, None]
+    for h in range(BH):
+        kd, vd, dod, od = k[h, :S].double(), v[h, :S].double(), do[:, 0, h * D:(h + 1) * D].double(), o[:, 0, h * D:(h + 1) * D].double()
+        p = torch.softmax((q[h].double() @ kd.t()).masked_fill(unseen, float("-inf")), -1)
+        want = (p * (dod @ vd.t() - (od * dod).sum(-1, keepdim=True))) @ kd * sc
+        assert_close(got[h], want, dtype, "dq of head %d" % h)
