@@ -1864,12 +1864,14 @@ static bool shares_bwd(int batch, int heads, int head_dim, int rows) {
 // 40 pairs of 128, 256 queries after 768 (160 workgroups) 26 / 20; 20 of 128, 512 after 512 (160) 24 / 21; 16 of 128, 640 after 1400
 // (160) 36 / 33; 200 of 128, 64 (200) 13 / 9; 40 of 128, 512 after 1536 (320) 59 / 44; 10 of 128, 2048 (320) 56 / 40; 100 of 64, 192 after 320
 // (300) 16 / 12; 12 of 64, 2048 (384) 26 / 23; not taken: 8 of 128, 1280 (160) 17 / 22; 40 of 128, 192 after 1728 (120) 22 / 30; 64 of
-// 128, 128 after 128 (128) 9.0 / 10.8; 25 of 64, 512 after 512 (200) 12.0 / 12.6.
-// Calls for dQ alone come here by the line of dK / dV: below it tp_attn_bwd_fused gives the bits that the two launches give.
+// 128, 128 after 128 (128) 9.0 / 10.8; 25 of 64, 512 after 512 (200) 12.0 / 12.6.  And from dK / dV's line on: 18 of 64, 1408 (396)
+// 24.5 / 20.4, 24 of 64, 1088 (408) 19.2 / 16.4.
+// Calls for dQ alone come here by that line only: below it tp_attn_bwd_fused gives the bits that the two launches give.
 static bool shares_queries(const tp_attn_desc* d) {
     if (d->dtype == TP_F32 || !tiled16(d->head_dim)) return false;
     if (d->reserved2 & (32 | 64)) return d->reserved2 & 32;
-    if (d->dq_only) return shares_bwd(d->batch, d->heads, d->head_dim, d->T);
+    if (shares_bwd(d->batch, d->heads, d->head_dim, d->T)) return true;
+    if (d->dq_only) return false;
     const long w = (long)d->batch * d->heads * ((d->T + 63) / 64), least = d->head_dim > 64 ? 160 : 256;
     return d->T >= 64 && w >= (d->cache_len >= d->T || d->cache_len + d->T <= 1024 ? least : 2 * least);
 }
