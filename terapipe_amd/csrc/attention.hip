@@ -1867,8 +1867,10 @@ static bool shares_bwd(int batch, int heads, int head_dim, int rows) {
 // 128, 128 after 128 (128) 9.0 / 10.8; 25 of 64, 512 after 512 (200) 12.0 / 12.6.  And from dK / dV's line on: 18 of 64, 1408 (396)
 // 24.5 / 20.4, 24 of 64, 1088 (408) 19.2 / 16.4.
 // Calls for dQ alone come here by that line only: below it tp_attn_bwd_fused gives the bits that the two launches give.
+// The kernel's lanes address a head's rows by 32 bits (64-bit tile origins cost it 1 to 2 % at head dimension 64): not beyond 2 GiB of them.
 static bool shares_queries(const tp_attn_desc* d) {
     if (d->dtype == TP_F32 || !tiled16(d->head_dim)) return false;
+    if (((long)d->cache_len + d->T + 512) * d->head_dim * 2 > 1L << 31) return false;
     if (d->reserved2 & (32 | 64)) return d->reserved2 & 32;
     if (shares_bwd(d->batch, d->heads, d->head_dim, d->T)) return true;
     if (d->dq_only) return false;

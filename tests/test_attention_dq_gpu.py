@@ -68,3 +68,27 @@ def test_long_sequences_of_few_heads(BH, T, P, D, dtype):
         p = torch.softmax((q[h].double() @ kd.t()).masked_fill(unseen, float("-inf")), -1)
         want = (p * (dod @ vd.t() - (od * dod).sum(-1, keepdim=True))) @ kd * sc
         assert_close(got[h], want, dtype, "dq of head %d" % h)
+
+
+@pytest.mark.parametrize("D", [80, 128])
+def test_keys_beyond_4_gib(D):
+    """A head whose K and V rows are more than 4 GiB each: two rows near the end take all of a query's weight but what 16 million
+    zeros share."""
+    S = ((1 << 32) // (2 * D) // 32 + 4) * 32
+    k, v = (torch.zeros(1, S, D, device=DEV, dtype=torch.float16) for _ in range(2))
+    g = torch.Generator(device=DEV).manual_seed(D)
+    rnd = lambda *s: torch.randn(*s, generator=g, device=DEV)
+    T, P, sc, far = 1, S - 1, D ** -0.5, [S - 70, S - 1]
+    q = (rnd(1, T, D) * 0.5).half()
+    for at, score in zip(far, (20.0, 21.0)):
+        k[0, at] = (q[0, 0].double() * score / q[0, 0].double().square().sum()).half()
+        v[0, at] = rnd(D).half()
+    do = rnd(T, 1, D).half()
+    kd, vd, dod = k[0, far].double(), v[0, far].double(), do[0, 0].double()
+    s = kd @ q[0, 0].double()
+    lse = torch.logsumexp(torch.cat([s, torch.tensor([S - 2.0], device=DEV, dtype=torch.float64).log()]), 0)
+    p = (s - lse).exp()
+    o = (p @ vd).half()
+    want = (p * (vd @ dod - (o.double() * dod).sum())) @ kd * sc
+    got = _dq(q, k, v, o.view(T, 1, D), lse.float().view(1, T), do, P)
+    assert_close(got[0, 0], want, torch.float16, "dq")
