@@ -388,11 +388,13 @@ class _LayerFunction(torch.autograd.Function):
 
 def _cache_grads(cache, dk_out, dv_out):
     """Gradients for the two cache inputs, not yet written, and those of the cache outputs as the kernel can read them (None
-    where there are none).  The kernel leaves the latter as they are (grad_cache_output.clone(), reference
+    where neither has one, zeros for one alone without).  The kernel leaves the latter as they are (grad_cache_output.clone(), reference
     transformer_models.py:188): it copies the rows that it does not add to."""
     gk, gv = (torch.empty_like(cache, memory_format=torch.contiguous_format) for _ in range(2))
-    if dk_out is None:
+    if dk_out is None and dv_out is None:
         return gk, gv, None, None
+    if dk_out is None:
+        dk_out = torch.zeros_like(dv_out)
     if dv_out is None:
         dv_out = torch.zeros_like(dk_out)
     # (the kernel's rows are contiguous and read 16 bytes at a time)
