@@ -114,7 +114,7 @@ extern "C" size_t tp_layers_fwd_workspace_bytes(const tp_layer_desc* layers, int
     for (int i = 0; layers && i < n; ++i) {
         const tp_layer_desc &l = layers[i], &f = layers[0];
         if (i && l.T == f.T && l.batch == f.batch && l.hidden == f.hidden && l.ffn == f.ffn && l.heads == f.heads &&
-            l.cache_len == f.cache_len && l.dtype == f.dtype && l.activation == f.activation)
+            l.cache_len == f.cache_len && l.dtype == f.dtype && l.activation == f.activation && !l.no_backward == !f.no_backward)
             continue;           // as the first one
         if (tp::validate_layer(&layers[i], "tp_layers_fwd") != TP_OK) return 0;
         const tp::ForwardPlan p = tp::forward_plan(layers[i]);
