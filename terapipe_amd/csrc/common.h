@@ -439,8 +439,8 @@ struct VecSum {
 constexpr int kVecSums = 6;
 int vec_param_sums(const VecSum (&sums)[kVecSums], bool acc_add, bool dst_add, int dtype, void* stream);
 
-// d, whose A are the rows LayerNorm(x) that nobody has taken yet (gemm.hip): whether one launch can take them and run d (d runs on
-// gemm_skinny_kernel and the rows fit its LDS), and that launch, which leaves the rows in A, their statistics in mean and rstd.
+// d, whose A are the rows LayerNorm(x) that nobody has taken yet (gemm.hip): whether one launch can take them and run d (no backward
+// follows, d runs on gemm_skinny_kernel and the rows fit its LDS), and that launch.  It keeps neither the rows nor their statistics.
 struct LayerNormOf { const void* x; const void* gamma; const void* beta; float* mean; float* rstd; };
 bool gemm_takes_layernorm(const tp_gemm_desc& d, const LayerNormOf& ln);
 int gemm_of_layernorm(const tp_gemm_desc& d, const LayerNormOf& ln, float eps, void* stream);

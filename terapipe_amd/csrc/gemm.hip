@@ -702,12 +702,12 @@ static int run_gemm(const tp_gemm_desc* d, const GemmPlan& p, void* workspace, v
 
 bool gemm_takes_layernorm(const tp_gemm_desc& d, const LayerNormOf& l) {
     return (d.reserved & kNoBackward) && runs_skinny(&d) && skinny_takes_ln(d.M, d.K) && d.lda == d.K && l.x && l.gamma && l.beta &&
-           l.mean && l.rstd && !(((uintptr_t)l.x | (uintptr_t)l.gamma | (uintptr_t)l.beta) & 15) && plan_gemm(&d).nsplit <= 1;
+           !(((uintptr_t)l.x | (uintptr_t)l.gamma | (uintptr_t)l.beta) & 15) && plan_gemm(&d).nsplit <= 1;
 }
 int gemm_of_layernorm(const tp_gemm_desc& d, const LayerNormOf& l, float eps, void* stream) {
     const int rc = validate_gemm(&d);
     if (rc != TP_OK) return rc;
-    const SkinnyLn ln = {l.gamma, l.beta, const_cast<void*>(d.A), l.mean, l.rstd, eps};
+    const SkinnyLn ln = {l.gamma, l.beta, eps};
     return run_gemm(&d, plan_gemm(&d), nullptr, stream, &ln, l.x);
 }
 

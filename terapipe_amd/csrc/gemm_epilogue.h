@@ -191,8 +191,8 @@ bool launch_gemm_pipe(int cfg, int op, int dtype, dim3 grid, const GemmArgs& a, 
 // A grouped launch (TN, token-major operands) of `tiles` workgroups on the pipelined 256 x 128 (15) or 128 x 128 (16) tile.
 bool launch_gemm_pipe_group(int cfg, int dtype, int tiles, const GemmGroupArgs& ga, hipStream_t s);
 // Products of up to 32 rows (gemm_skinny.hip; NT, 16-bit): whole k ranges per workgroup, k splits as the arguments say.
-// ln: the activation rows are first the LayerNorm of a.A (skinny_takes_ln; one k range), which it leaves in y, mean and rstd.
-struct SkinnyLn { const void* gamma; const void* beta; void* y; float* mean; float* rstd; float eps; };
+// ln: the activation rows are the LayerNorm of a.A (skinny_takes_ln; one k range).
+struct SkinnyLn { const void* gamma; const void* beta; float eps; };
 bool skinny_takes_ln(int M, int K);
 // half: tiles of 8 weight rows where those of 16 come to at most half of the 256 CUs (their sums are in another order).
 void launch_gemm_skinny(int dtype, const GemmArgs& a, bool half, const SkinnyLn* ln, hipStream_t s);

@@ -20,8 +20,8 @@ namespace tp {
 // of the MFMA are those at two k ranges, and so are its columns; the two diagonal quarters are the tile's sums.  With it a weight of
 // 2048 rows needs no k split.
 // LN (up to 8 rows): the activation rows are the LayerNorm of a.A, taken by each workgroup for itself while its first
-// weight rows come (two-pass fp32 statistics, rounded to T in LDS); the first workgroup leaves the rows and
-// their statistics for whoever reads them later.  A launch less in a chain where a LayerNorm of four rows takes 3.7 us.
+// weight rows come (two-pass fp32 statistics, rounded to T in LDS); neither they nor their statistics are kept.  A launch less in a
+// chain where a LayerNorm of four rows takes 3.7 us.
 template <typename T, int MB, int NT, bool HALF, bool LN>
 __global__ __launch_bounds__(512, MB == 1 && !HALF ? 4 : 2) void gemm_skinny_kernel(GemmArgs a, SkinnyLn ln) {
     constexpr int WAVES = 8, U = HALF ? 8 : NT == 4 ? 2 : 4, UK = HALF ? 64 : 32, STEP = UK * U, TN = HALF ? 8 : 16, PITCH = NT * TN + 4;
@@ -131,8 +131,7 @@ __global__ __launch_bounds__(512, MB == 1 && !HALF ? 4 : 2) void gemm_skinny_ker
                 for (int e = 0; e < 8; ++e) { const float d = v[e] - mu; sq += d * d; }
             }
         const float rs = 1.0f / sqrtf(row_sum(sq, red + WAVES) / (float)a.K + ln.eps);
-        const bool mine = wave / share < a.M, first = mine && blockIdx.x == 0;
-        if (first && part_of == 0 && lane == 0) { ln.mean[row] = mu; ln.rstd[row] = rs; }
+        const bool mine = wave / share < a.M;
 #pragma unroll
         for (int i = 0; i < LNC; ++i)
             if (mine && c0 + i * step < nch) {
@@ -142,7 +141,6 @@ __global__ __launch_bounds__(512, MB == 1 && !HALF ? 4 : 2) void gemm_skinny_ker
 #pragma unroll
                 for (int e = 0; e < 8; ++e) y[e] = (v[e] - mu) * rs * g[e] + b[e];
                 store8<T>(xs, row * (a.K + 8) + c, y);
-                if (first) store8<T>(ln.y, (long)row * a.K + c, y);
             }
         __syncthreads();
     }
