@@ -347,17 +347,27 @@ static void plan_large(const tp_gemm_desc* d, int& cfg, int& ns) {
 
 // Forward products of up to kSkinnyRows rows on a weight of up to 4096 x 4096 run without LDS tiles: the plan's k splits,
 // whatever its tile.  (Beyond, both are bound by the weight stream and the tile kernels read the activation less often:
-// 16 rows on 20480 x 5120 58 us against 49.  A forced tile, and column sums, take the tile kernels.)  Up to 8 rows they take larger
-// weights too, where no k split is called for: us, 4 rows, tile kernels / these: 5120 x 5120 17.8 / 15.0, 8192 x 8192 37 / 31.6,
-// 20480 x 5120 46.6 / 37.8, 12288 x 4096 23.2 / 24.0 and without the LayerNorm before, 4096 x 16384 35.2 / 32.8; but 5120 x 20480, 1.25
-// workgroups of 16 rows to a CU, 40 / 48.  Only where no backward follows: another order of the sums turns ReLU units near zero on or
-// off, and the weight gradients behind them move by 2e-2 in fp16.
+// 16 rows on 20480 x 5120 49 us against 58.  A forced tile, and column sums, take the tile kernels.)
+// Only where no backward follows (another order of the sums turns ReLU units near zero on or off, and the weight gradients behind them
+// move by 2e-2 in fp16), up to 8 rows: without k splits, unless the rows of a weight are longer than 8192 and its tiles of 16 of
+// them do not come to whole rounds of the CUs (5120 x 20480, 1.25 of them: 48 us against 40 on tiles with three splits).
 static inline bool skinny_unsplit(const tp_gemm_desc* d) {
     return (d->reserved & kNoBackward) && d->M <= 8 && (d->K <= 8192 || d->N % 4096 == 0);
 }
+// Those also on larger weights, where tiles of 64 columns, the alternative, would leave half of their last round of CUs or more
+// without one, or split k.  us, 4 and 8 rows, tiles / these: 5120 x 5120 20.4 / 17.9 and 20.1 / 18.5, 7680 x 2560 14.6 / 10.1 and 14.4 / 10.4,
+// 20480 x 5120 48.4 / 41.0 and 47.5 / 43.3, 24576 x 4096 44.6 / 40.1 and 42.2 / 42.5, 4096 x 16384 37.1 / 31.4 and 37.1 / 33.0.  Where
+// they fill it (12288 x 4096 23.8 / 24.9 and 24.0 / 25.3, 15360 x 5120 30.5 / 31.6 and 30.7 / 32.7, 28672 x 4096 48.0 / 51.0) these are taken
+// for the LayerNorm's launch that they save, 3.7 us, and from k = 8192 on (15360 x 8192 57.9 / 53.2 and 57.2 / 52.3).  Weights with few and
+// long rows keep the tiles' k splits: 4608 x 6144 17.8 / 19.4, 5120 x 8192 22.7 / 24.4.
+static inline bool skinny_large(const tp_gemm_desc* d) {
+    const bool filled = ((d->N + 63) / 64 - 1) % kNumCU >= kNumCU / 2;
+    return skinny_unsplit(d) && (long)d->N * d->K <= 256L << 20 && (d->N % 4096 == 0 || 4L * d->K <= 5L * d->N) &&
+           (!filled || d->K >= 8192 || skinny_takes_ln(d->M, d->K));
+}
 static inline bool runs_skinny(const tp_gemm_desc* d) {
     return d->op == TP_GEMM_NT && d->dtype != TP_F32 && d->M <= kSkinnyRows && (d->reserved & 0xff) == 0 && !d->colsum_acc &&
-           (long)d->N * d->K <= (skinny_unsplit(d) ? 256L << 20 : 16L << 20);
+           ((long)d->N * d->K <= 16L << 20 || skinny_large(d));
 }
 
 // fp32 products that run on tiles of 32 x 32 whose waves share k, in one launch (gemm_f32.hip): where the tiles come to at
