@@ -812,9 +812,10 @@ static bool launch_group(const tp_gemm_desc* descs, int n, int cfg, const VecGra
     if (cfg == 15 || cfg == 16) return launch_gemm_pipe_group(cfg, descs[0].dtype, tiles, ga, s);
     return launch_gemm_tall_group(cfg, descs[0].dtype, tiles, ga, vec, s);
 }
-// Vector-parameter gradients behind the group's tiles, where those are of 256 x 256: their blocks run on the CUs that the last round
-// leaves, and what is left when it ends spreads over all of them.  Four layers' four products of 1024 over 4096 rows (64 CUs left): 108 us
-// and 23 for a launch of its own, 108 so; five layers of 2048 over 2048 (three full rounds, none left) a pass of 4013 us, 3953 so.
+// Whether a layer's vector-parameter gradients run as blocks behind the group's tiles, where those are of 256 x 256: on the CUs that the
+// tiles' last round leaves, then, when it ends, on all of them.  A layer's four weight gradients alone / its vector gradients alone /
+// the two launches / this one, us: 1024 wide, 4096 rows (64 CUs left) 100 / 24 / 125 / 102; 2048 wide, 2048 rows (three full rounds,
+// none left) 177 / 25 / 197 / 191; 2560 wide, 2048 rows 294 / 26 / 314 / 295; 6144 wide, 4096 rows 2974 / 116 / 3077 / 3073.
 static bool takes_vec_grads(const tp_gemm_desc* descs, int n, int cfg) {
     return (cfg == 2 && !runs_short(descs, n)) || cfg == 19 || cfg == 20;
 }

@@ -198,7 +198,9 @@ __global__ __launch_bounds__(512, MB == 1 && !HALF ? 4 : 2) void gemm_skinny_ker
 
 // Weight tiles per workgroup: two workgroups fit a CU, so the estimate counts half rounds of 256 workgroups (the first)
 // and rounds of 512, each as long as the tiles a workgroup has; the activation rows' reads, M / (16 NT) of the weight's,
-// cost half as much as those (they hit the caches).
+// cost half as much as those (they hit the caches).  (Of 17 to 32 rows one fits: two turns of loads take 130 to 174 registers.  Its
+// estimate is the same, since the tiles decide a forward's order of sums.  Two workgroups of one turn are slower: 24 rows, us, 6144 x 2048 10.3 /
+// 10.8, 8192 x 2048 11.9 / 12.4, 2048 x 8192 14.3 / 15.0; one turn of twice the loads, as before: 10.9, 12.1, 14.4.)
 static int skinny_tiles(const GemmArgs& a) {
     const int tiles = (a.N + 15) / 16;
     int best = 1;
