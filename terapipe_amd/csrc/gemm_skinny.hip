@@ -11,10 +11,10 @@ namespace tp {
 // registers the MFMA takes (lane l: row l & 15, k 8 * (l >> 4) .. + 7 of each 32), the activation rows the same way
 // (they stay in the caches; NT weight tiles share one read of them), the next turn's loads under way meanwhile.  No LDS and no
 // barrier until the eight partial tiles are added at the end.
-// Measured (4 rows, weights from memory, the same launch back to back, us): 8192 x 2048 9.0 (3.7 TB/s; without the second turn's
-// loads under way 9.8), 6144 x 2048 7.8 (8.3), 4096 x 4096 9.0, 20480 x 5120 37.8 (5.5 TB/s); tiles of 8 rows: 2048 x 2048 4.4 (of
-// 16: 5.2), 2048 x 8192 9.5 (of 16 with four k splits and the launch that adds them 12.5), 768 x 3072 4.8 (6.3).  In a decoding
-// step's chain with the LayerNorm: 8192 x 2048 12.2 (11.9 + 3.7), 6144 x 2048 10.9 (9.9 + 3.7).
+// Measured (4 rows, weights from memory, launches of one graph back to back, us): 8192 x 2048 9.6 (3.5 TB/s; without the second turn's
+// loads under way 10.3), 6144 x 2048 8.7 (9.0), 4096 x 4096 12.3 (13.0; without k splits 10.2), 20480 x 5120 41.0 (5.1 TB/s); tiles of 8
+// rows: 2048 x 2048 4.9 (of 16: 5.7), 2048 x 8192 10.3 (of 16 with four k splits and the launch that adds them 12.6), 768 x 3072 5.2 (6.6).  In a
+// decoding step's chain with the LayerNorm: 8192 x 2048 12.2 (10.5 + 3.6), 6144 x 2048 11.0 (9.4 + 3.6).
 // ---------------------------------------------------------------------------------------------
 // HALF (up to 8 rows, where tiles of 16 weight rows would leave half of the CUs without one): a tile is 8 weight rows, the 16 rows
 // of the MFMA are those at two k ranges, and so are its columns; the two diagonal quarters are the tile's sums.  With it a weight of
